@@ -18,18 +18,17 @@ Differences from the reference that callers can observe:
 import torch
 
 from . import _lib
-from ._lib import c_f32, c_i64, c_int, c_size, check, ptr, stream_ptr
+from ._lib import c_i64, c_size, check, ptr, stream_ptr
 
 
 def _mm(a, b, trans_a=False, trans_b=False):
     """Dense fp32 product on the matrix cores (the reference calls torch::mm)."""
-    from .graph_ext import sgemm
-    return sgemm(a.contiguous(), b.contiguous(), trans_a, trans_b)
+    return _lib.ops().sgemm(a.contiguous(), b.contiguous(), trans_a, trans_b, None)
 
 
 def _check_inputs(*tensors):
     # CHECK_INPUT of the reference: CUDA + contiguous (YiTu_GNN.cpp:65-69)
-    return _lib.require_device(*tensors)
+    _lib.ops().check_inputs(list(tensors))
 
 
 def edge_scale(column_index, degrees):
@@ -38,52 +37,14 @@ def edge_scale(column_index, degrees):
     ``backward`` the aggregation reads them in edge order instead of gathering ``degrees``
     once per edge. The caller owns the tensor: it must be rebuilt when ``column_index`` or
     ``degrees`` change."""
-    _lib.require_device(column_index, degrees)
-    _lib.require_dtype(column_index, torch.int32, "column_index")
-    _lib.require_dtype(degrees, torch.float32, "degrees")
-    out = torch.empty(column_index.numel(), dtype=torch.float32, device=column_index.device)
-    with torch.cuda.device(column_index.device):
-        rc = _lib.lib().yitu_edge_scale(ptr(out), ptr(column_index), ptr(degrees),
-                                        c_i64(column_index.numel()), c_i64(degrees.numel()),
-                                        stream_ptr(column_index.device))
-    check(rc, "yitu_edge_scale")
-    return out
+    return _lib.ops().edge_scale(column_index, degrees)
 
 
 def _aggregate(x, row_pointers, column_index, degrees, alpha, edge_scale=None):
     """out[r] = alpha * s_r * sum_j s_j x[j] over the CSR row r (s = degrees or 1)."""
-    _lib.require_dtype(row_pointers, torch.int32, "row_pointers")
-    _lib.require_dtype(column_index, torch.int32, "column_index")
-    if x.dtype not in (torch.float32, torch.bfloat16):
-        raise RuntimeError("features must be float32 or bfloat16, got %s" % x.dtype)
-    if x.dim() != 2:
-        raise RuntimeError("features must be 2-D [n_nodes, dim]")
-    if degrees is not None:
-        _lib.require_dtype(degrees, torch.float32, "degrees")
-    n_rows = row_pointers.numel() - 1
-    n_src, dim = x.shape
-    nnz = column_index.numel()
-    if degrees is not None and degrees.numel() < max(n_rows, n_src):
-        raise RuntimeError("degrees is shorter than the number of nodes")
-    if edge_scale is not None:
-        _lib.require_device(edge_scale)
-        _lib.require_dtype(edge_scale, torch.float32, "edge_scale")
-        if edge_scale.numel() != nnz:
-            raise RuntimeError("edge_scale must hold one value per edge")
-    out = torch.empty((n_rows, dim), dtype=torch.float32, device=x.device)
-    maxdeg = _lib.max_degree(row_pointers)
-    plan = _lib.row_plan(row_pointers, column_index, n_src, 0x7FFFFFFF)
-    need = _lib.size_fn("yitu_spmm_workspace_bytes")(c_i64(nnz), c_i64(dim), c_int(1)) \
-        if plan is not None and maxdeg >= 64 else 0
-    ws = _lib.workspace(need, x.device)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().yitu_agg_csr(
-            ptr(out), ptr(x), c_int(1 if x.dtype == torch.bfloat16 else 0), ptr(row_pointers),
-            ptr(column_index), ptr(degrees), c_i64(n_rows), c_i64(n_src), c_i64(nnz), c_i64(dim),
-            c_f32(alpha), c_i64(maxdeg), ptr(plan), ptr(edge_scale), ptr(ws), c_size(ws.numel()),
-            stream_ptr(x.device))
-    check(rc, "yitu_agg_csr")
-    return out
+    return _lib.ops().agg(x, row_pointers, column_index, degrees, edge_scale, alpha,
+                          _lib.max_degree(row_pointers),
+                          _lib.row_plan(row_pointers, column_index, x.size(0), 0x7FFFFFFF))
 
 
 def SAG(input, row_pointers, column_index, degrees, part_pointers, part2Node, partSize, dimWorker,

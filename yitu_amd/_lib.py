@@ -49,10 +49,22 @@ def lib():
     return _lib
 
 
-def _declare(name, restype=ctypes.c_int):
-    fn = getattr(lib(), name)
-    fn.restype = restype
-    return fn
+_ops = None
+
+
+def ops():
+    """The native side of the op modules (csrc/bind): checks, allocation, per-graph state and
+    autograd nodes over the same library; raises if it has not been built."""
+    global _ops
+    if _ops is None:
+        lib()  # present, and of the version these bindings were written for
+        try:
+            from . import _ops as native
+        except ImportError as exc:
+            raise RuntimeError("yitu_amd/_ops.so is not built; run `python -m yitu_amd.build` "
+                               "(there is no CPU fallback): %s" % exc) from exc
+        _ops = native
+    return _ops
 
 
 def check(rc, what):
@@ -108,8 +120,8 @@ def workspace(n_bytes, device):
 
 # ---- state derived from a graph ----------------------------------------------------
 # The widest row, the row plan, the by-source view and by-source weight copies are
-# functions of the index tensors and are kept per tensor OBJECT (id, address, version
-# counter) for as long as the tensor lives. The version counter moves when torch writes
+# functions of the index tensors and are kept per tensor OBJECT (implementation, address,
+# version counter) for as long as the tensor lives (csrc/bind/graph_state.cpp). The version counter moves when torch writes
 # the tensor; it does NOT move when a buffer is refilled through its raw pointer, which is
 # how every kernel of this library (yitu_coo_to_csr, the device sampler, ...), DLPack
 # consumers and foreign extensions write. Whoever refills an index or weight tensor in
@@ -135,68 +147,49 @@ class _Built:
         return self.value
 
 
+def watch(tensor):
+    """Drops what is kept for ``tensor`` (csrc/bind/graph_state.cpp) when it dies."""
+    native = ops()
+    weakref.finalize(tensor, native.drop, native.impl_of(tensor)).atexit = False
+
+
 def forget(*tensors):
     """Drops every cached widest row and row plan derived from the given index tensors
     (call after refilling one of them in place through a raw pointer)."""
-    idents = {id(t) for t in tensors if t is not None}
-    for key in [k for k in _max_degree if k[0] in idents]:
-        _max_degree.pop(key, None)
-    for key in [k for k in _plans if k[0] in idents or k[3] in idents]:
-        _plans.pop(key, None)
-
-
-# Widest-row cache: the kernels skip their hub-row machinery when they are told
-# that no row reaches the hub threshold. Computed once per indptr tensor.
-_max_degree = {}
+    for t in tensors:
+        if t is not None:
+            ops().drop(ops().impl_of(t))
 
 
 def max_degree(indptr):
-    """Longest row of a CSR, computed once per ``indptr`` tensor. The entry lives as long
-    as the tensor object: an address alone is no identity, the allocator hands a freed
-    block to the next graph of the same size."""
-    key = (id(indptr), indptr.data_ptr(), indptr.numel(), indptr._version)
-    v = _max_degree.get(key)
-    if v is None:
-        if indptr.numel() <= 1:
-            v = 0
-        else:
-            v = int((indptr[1:] - indptr[:-1]).max().item())
-        _max_degree[key] = v
-        weakref.finalize(indptr, _max_degree.pop, key, None)
+    """Longest row of a CSR, computed once per ``indptr`` tensor (the kernels skip their
+    hub-row machinery when no row reaches the hub threshold). The entry lives as long as the
+    tensor object: an address alone is no identity, the allocator hands a freed block to the
+    next graph of the same size."""
+    native = ops()
+    v = native.find_max_degree(indptr)
+    if v < 0:
+        v = int((indptr[1:] - indptr[:-1]).max().item()) if indptr.numel() > 1 else 0
+        native.put_max_degree(indptr, v)
+        watch(indptr)
     return v
 
 
-# Row plans (band-ordered items of the long rows) are a function of the graph
-# only: built on the device on first use and kept while the index tensor lives.
-_plans = {}
-
-
 def row_plan(indptr, indices, n_src, col_mask):
-    """Device buffer holding the row plan of (indptr, indices), or None when no
-    row reaches the planning threshold and the graph is small. A large graph without
-    long rows still gets one: its header tells the row kernels whether most sources of
-    a row lie near the row's own id, which decides how rows are dealt to the XCDs."""
+    """Device buffer holding the row plan of (indptr, indices): band-ordered items of the long
+    rows, a function of the graph only, built on the device on first use and kept while the
+    index tensor lives. None when no row reaches the planning threshold and the graph is
+    small. A large graph without long rows still gets one: its header tells the row kernels
+    whether most sources of a row lie near the row's own id, which decides how rows are dealt
+    to the XCDs."""
     if max_degree(indptr) < 64 and indices.numel() < (1 << 20):
         return None
-    key = (id(indices), indices.data_ptr(), indices._version, id(indptr), indptr.data_ptr(),
-           indptr._version, int(n_src), int(col_mask))
-    hit = _plans.get(key)
-    if hit is not None:
-        return hit.get(indices.device)
-    L = lib()
-    L.yitu_plan_bytes.restype = c_size
-    L.yitu_plan_workspace_bytes.restype = c_size
-    dev = indices.device
-    nnz = indices.numel()
-    plan = torch.empty(int(L.yitu_plan_bytes(c_i64(nnz))), dtype=torch.uint8, device=dev)
-    ws = workspace(L.yitu_plan_workspace_bytes(c_i64(nnz)), dev)
-    with torch.cuda.device(dev):
-        rc = L.yitu_plan_build(ptr(plan), c_size(plan.numel()), ptr(indptr), ptr(indices),
-                               c_i64(indptr.numel() - 1), c_i64(n_src), c_i64(nnz), c_int(col_mask),
-                               ptr(ws), c_size(ws.numel()), stream_ptr(dev))
-    check(rc, "yitu_plan_build")
-    _plans[key] = _Built(plan, dev)
-    weakref.finalize(indices, _plans.pop, key, None)
+    native = ops()
+    plan = native.find_plan(indptr, indices, int(n_src), col_mask)
+    if plan is None:
+        plan = native.build_plan(indptr, indices, int(n_src), col_mask)
+        native.put_plan(indptr, indices, int(n_src), col_mask, _Built(plan, indices.device))
+        watch(indices)
     return plan
 
 

@@ -1,4 +1,5 @@
-"""Builds libyitu_hip.so (gfx950) in-tree with hipcc.
+"""Builds libyitu_hip.so (gfx950, hipcc), libyitu_host.so and the extension module _ops.so
+(g++) in-tree.
 
 Usage: ``python -m yitu_amd.build [-j N] [--force]``. Objects are cached under
 ``yitu_amd/csrc/build/`` and rebuilt when a source or header is newer.
@@ -67,16 +68,61 @@ def build_host(force=False):
     return HOST_LIB
 
 
+OPS_LIB = os.path.join(HERE, "_ops.so")
+
+
+def _compile_bind(src, force):
+    """One source of _ops.so (csrc/bind: the Python-facing side, compiled against torch)."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+    obj = os.path.join(OBJ, os.path.basename(src) + ".o")
+    deps = glob.glob(os.path.join(CSRC, "bind", "*.hpp")) + \
+        glob.glob(os.path.join(HERE, "..", "include", "*.h")) + [src]
+    if not force and os.path.exists(obj) and \
+            os.path.getmtime(obj) > max(os.path.getmtime(d) for d in deps):
+        return obj
+    include = cpp_extension.include_paths("cuda") + [sysconfig.get_paths()["include"]]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H",
+           "-DTORCH_EXTENSION_NAME=_ops"]
+    for path in include:
+        cmd += ["-isystem", path]
+    r = subprocess.run(cmd + ["-c", src, "-o", obj], capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("g++ failed for %s:\n%s" % (src, r.stdout + r.stderr))
+    if r.stderr.strip():
+        sys.stderr.write(r.stderr)
+    return obj
+
+
+def _link_bind(objs):
+    from torch.utils import cpp_extension
+    dirs = cpp_extension.library_paths("cuda")
+    cmd = [os.environ.get("CXX", "g++"), "-shared", "-o", OPS_LIB] + objs + \
+        ["-L" + HERE, "-l:libyitu_hip.so", "-Wl,-rpath,$ORIGIN"]
+    for path in dirs:
+        cmd += ["-L" + path, "-Wl,-rpath," + path]
+    cmd += ["-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("link of _ops.so failed:\n" + r.stdout + r.stderr)
+
+
 def build(force=False, jobs=8):
     build_host(force)
     os.makedirs(OBJ, exist_ok=True)
     srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
+        binds = [ex.submit(_compile_bind, s, force)
+                 for s in sorted(glob.glob(os.path.join(CSRC, "bind", "*.cpp")))]
         objs = list(ex.map(lambda s: _compile(s, force), srcs))
+        binds = [b.result() for b in binds]
     cmd = [HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError("link failed:\n" + r.stdout + r.stderr)
+    _link_bind(binds)
     return LIB
 
 

@@ -1,31 +1,19 @@
 """GIN layer over ``YiTu_GNN_kernel.forward_gin / backward_gin`` (the role of
 YiTu_GNN/nn/GINConv.py)."""
-import torch
-
-from .. import YiTu_GNN_kernel
-from ._common import DenseWeight, graph_arguments
+from .. import _lib
+from ._common import DenseWeight
 
 
-class GNNAFunction_GIN(torch.autograd.Function):
-    """``apply(X, weight, inputInfo, eplison)`` -> ``(eplison * sum of neighbours) . weight``.
-    The aggregate that ``forward_gin`` returns beside the output is what the
-    backward needs in place of X (GINConv.py:24), so X itself is not kept.
-    Gradients: (dX, dW, None, None)."""
+class GNNAFunction_GIN:
+    """``apply(X, weight, inputInfo, eplison)`` -> ``(eplison * sum of neighbours) . weight``,
+    one autograd node (csrc/bind/autograd.cpp). The aggregate that ``forward_gin`` returns
+    beside the output is what the backward needs in place of X (GINConv.py:24), so X itself
+    is not kept."""
 
     @staticmethod
-    def forward(ctx, X, weight, inputInfo, eplison):
-        tail = graph_arguments(inputInfo, eplison)
-        out, aggregate = YiTu_GNN_kernel.forward_gin(X, weight, *tail)
-        ctx.save_for_backward(aggregate, weight)
-        ctx.tail = tail
-        return out
-
-    @staticmethod
-    def backward(ctx, d_output):
-        aggregate, weight = ctx.saved_tensors
-        d_input, d_weight = YiTu_GNN_kernel.backward_gin(d_output.contiguous(), aggregate, weight,
-                                                         *ctx.tail)
-        return d_input, d_weight, None, None
+    def apply(X, weight, inputInfo, eplison):
+        return _lib.ops().gin_conv(X, weight, inputInfo.row_pointers, inputInfo.column_index,
+                                   eplison, inputInfo.partPtr, inputInfo.part2Node)
 
 
 class GINConv(DenseWeight):

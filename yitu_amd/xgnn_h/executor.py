@@ -124,8 +124,7 @@ class Executor:
             count = len(node.inputs)
             xs = [v[str(i)] for i in range(count)]
             if all(x.is_cuda and x.dtype == torch.float32 for x in xs):
-                y = layers._TypedLinear.apply(count, *xs, *node.attrs["weights"],
-                                              *node.attrs["biases"])
+                y = layers.typed_linear(xs, node.attrs["weights"], node.attrs["biases"])
             else:  # host tensors: the same rows from torch
                 y = torch.cat([F.linear(x, w, b) for x, w, b in
                                zip(xs, node.attrs["weights"], node.attrs["biases"])], dim=0)

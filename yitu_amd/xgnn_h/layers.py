@@ -8,6 +8,7 @@ from typing import Union
 import torch
 from torch import nn
 
+from .. import _lib
 from . import block, bundle, sparse
 
 
@@ -130,64 +131,11 @@ class HeteroGraphConv(nn.Module):
         return outputs
 
 
-class _TypedLinear(torch.autograd.Function):
+def typed_linear(xs, weights, biases):
     """y[off_i : off_i + n_i] = x_i . W_i^T (+ b_i) for every (x_i, W_i, b_i), all
     written into one [sum n_i, out] buffer by the MFMA GEMM: the layout the
-    stacked aggregation reads, produced without a concatenation pass."""
-
-    @staticmethod
-    def forward(ctx, n_parts, *args):
-        from .. import graph_ext
-        xs, ws, bs = args[:n_parts], args[n_parts:2 * n_parts], args[2 * n_parts:]
-        total = sum(x.size(0) for x in xs)
-        y = torch.empty((total, ws[0].size(0)), dtype=torch.float32, device=xs[0].device)
-        parts, off = [], 0
-        for x in xs:
-            parts.append(y[off:off + x.size(0)])
-            off += x.size(0)
-        if all(w.shape == ws[0].shape for w in ws):
-            graph_ext.linear_forward_typed(
-                [x.contiguous() for x in xs], [w.contiguous() for w in ws],
-                [None if b is None else b.contiguous() for b in bs], out_list=parts)
-        else:
-            graph_ext.sgemm_typed([x.contiguous() for x in xs], [w.contiguous() for w in ws],
-                                  trans_b=True, out_list=parts)
-            for part, b in zip(parts, bs):
-                if b is not None:
-                    part += b
-        ctx.n_parts = n_parts
-        ctx.has_bias = [b is not None for b in bs]
-        ctx.save_for_backward(*xs, *ws)
-        return y
-
-    @staticmethod
-    def backward(ctx, grad_y):
-        from .. import graph_ext
-        n = ctx.n_parts
-        xs, ws = ctx.saved_tensors[:n], ctx.saved_tensors[n:]
-        grad_y = grad_y.contiguous()
-        gs, off = [], 0
-        for x in xs:
-            gs.append(grad_y[off:off + x.size(0)])
-            off += x.size(0)
-        gx, gw = [None] * n, [None] * n
-        want = [i for i in range(n) if ctx.needs_input_grad[1 + i]]
-        if want:
-            for i, g in zip(want, graph_ext.sgemm_typed([gs[i] for i in want],
-                                                        [ws[i].contiguous() for i in want])):
-                gx[i] = g
-        want = [i for i in range(n) if ctx.needs_input_grad[1 + n + i]]
-        if want:
-            for i, g in zip(want, graph_ext.sgemm_typed([gs[i] for i in want],
-                                                        [xs[i].contiguous() for i in want],
-                                                        trans_a=True)):
-                gw[i] = g
-        gb = [None] * n
-        want = [i for i in range(n) if ctx.has_bias[i] and ctx.needs_input_grad[1 + 2 * n + i]]
-        if want:
-            for i, g in zip(want, graph_ext.column_sum_typed([gs[i] for i in want])):
-                gb[i] = g
-        return (None, *gx, *gw, *gb)
+    stacked aggregation reads, produced without a concatenation pass. One autograd node."""
+    return _lib.ops().typed_linear(list(xs), list(weights), list(biases))
 
 
 class StackedHeteroGCN(nn.Module):
@@ -249,8 +197,7 @@ class StackedHeteroGCN(nn.Module):
         blk, values = stacked if stacked is not None else self._stacked
         parts = [xs[nty] for _, nty in self.segments]
         fcs = [self.fcs[name] for name, _ in self.segments]
-        h = _TypedLinear.apply(len(parts), *parts, *[fc.weight for fc in fcs],
-                               *[fc.bias for fc in fcs])
+        h = typed_linear(parts, [fc.weight for fc in fcs], [fc.bias for fc in fcs])
         out = sparse.gspmm(blk, values, h.unsqueeze(1)).squeeze(1)
         reached = {dty for _, _, dty in self.relations}
         # one split (its backward is one concatenation) rather than a slice per type (each
