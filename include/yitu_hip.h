@@ -415,6 +415,21 @@ int yitu_sgemm_typed(float *const *c_device_ptrs, const float *const *a_device_p
                      size_t workspace_bytes, void *stream);
 
 /*
+ * Weight and bias gradients of Linear layers that share both widths (the backward of
+ * yitu_linear_forward_typed): dw_i [n_out, n_in] = g_i^T . x_i with g_i [rows_i, n_out],
+ * x_i [rows_i, n_in], and db_i [n_out] = the column sums of g_i, taken while g_i is read
+ * for the product. db (or an entry of it) may be NULL. Host arrays of device pointers, as in
+ * yitu_sgemm_typed. Workspace: ..._workspace_bytes(most rows, n_out, n_in, n_problems).
+ */
+size_t yitu_linear_weight_grad_workspace_bytes(int64_t rows, int64_t n_out, int64_t n_in,
+                                               int64_t n_problems);
+int yitu_linear_weight_grad_typed(float *const *dw_device_ptrs, float *const *db_device_ptrs,
+                                  const float *const *g_device_ptrs,
+                                  const float *const *x_device_ptrs, const int64_t *rows,
+                                  int64_t n_problems, int64_t n_out, int64_t n_in,
+                                  void *workspace_device, size_t workspace_bytes, void *stream);
+
+/*
  * hfused_forward (entry.cpp:136-155; hfused_cuda.cu:5-45,96-137): the SpMM of
  * graph A and the SDDMM + LeakyReLU + edge softmax of graph B (same number of
  * rows, same head count) in ONE launch: the first workgroups of the grid run the

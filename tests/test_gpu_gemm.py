@@ -464,3 +464,52 @@ def test_typed_products_of_forty_small_layers(dev):
     long_parts = [torch.randn(9000, 8, generator=g).to(dev), torch.randn(10, 8, generator=g).to(dev)]
     for x, s in zip(long_parts, graph_ext.column_sum_typed(long_parts)):
         assert_close(s, x.double().sum(0), abs_sum=x.double().abs().sum(0))
+
+
+@pytest.mark.parametrize("ki,no", [(4, 4), (1, 7), (7, 1), (33, 31), (100, 47), (96, 192), (333, 77),
+                                   (512, 40), (130, 512), (128, 128), (256, 256)])
+@pytest.mark.parametrize("rows", [[40001], [30000, 1, 17, 9003]])
+def test_linear_weight_and_bias_gradients(dev, rows, ki, no):
+    """dW_i = g_i^T x_i and db_i = column sums of g_i in one call: ragged widths on both sides
+    (a lane's last columns are read twice), rows that are no multiple of a step, several
+    problems, the bias of one of them not asked for; bitwise reproducible."""
+    g = torch.Generator().manual_seed(ki + no)
+    gs = [torch.randn(r, ki, generator=g) for r in rows]
+    xs = [torch.randn(r, no, generator=g) for r in rows]
+    w = [torch.randn(ki, no, generator=g).to(dev).requires_grad_() for _ in rows]
+    b = [None if i == 1 else torch.zeros(ki, device=dev, requires_grad=True) for i in range(len(rows))]
+    from yitu_amd.xgnn_h import layers as xl
+    params = w + [t for t in b if t is not None]
+
+    def run():
+        y = xl.typed_linear([x.to(dev) for x in xs], w, b)
+        return torch.autograd.grad(y, params, torch.cat(gs).to(dev))
+
+    got = run()
+    for i, r in enumerate(rows):
+        assert_close(got[i], _ref(gs[i], xs[i], True, False), atol=1e-4 * max(1.0, r ** 0.5), what="dW %d" % i)
+    for t, i in zip(got[len(w):], [i for i in range(len(rows)) if b[i] is not None]):
+        assert_close(t, gs[i].double().sum(0).float(), atol=1e-4 * rows[i] ** 0.5, what="db %d" % i)
+    assert all(torch.equal(s, t) for s, t in zip(got, run()))
+
+
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("ms,n,k", [([65537], 47, 100), ([70000], 128, 33), ([66001], 136, 136),
+                                    ([20001], 77, 333), ([17003], 16, 500), ([16400], 7, 3),
+                                    ([40000, 5, 0, 30001], 97, 65), ([70000], 64, 63)])
+def test_sgemm_many_rows_small_weight(dev, ms, n, k, tb):
+    """Products whose weight sits in LDS: inner dimensions below, at and beside a chunk (32, 64),
+    not whole 16-byte pieces, outputs of one to four column blocks and of two panels, last row
+    tiles that are not full; with the biases of a Linear where the weight is [n, k]."""
+    g = torch.Generator().manual_seed(sum(ms) + n)
+    xs = [torch.randn(m, k, generator=g) for m in ms]
+    ws = [torch.randn((n, k) if tb else (k, n), generator=g) for _ in ms]
+    got = graph_ext.sgemm_typed([x.to(dev) for x in xs], [w.to(dev) for w in ws], False, tb)
+    for x, w, c in zip(xs, ws, got):
+        assert_close(c, _ref(x, w, False, tb), atol=1e-4 * max(1.0, k ** 0.5 / 4))
+    if tb:
+        bs = [torch.randn(n, generator=g) for _ in ms]
+        lin = graph_ext.linear_forward_typed([x.to(dev) for x in xs], [w.to(dev) for w in ws],
+                                             [b.to(dev) for b in bs])
+        for c, b, y in zip(got, bs, lin):
+            assert_close(y, c.cpu() + b, atol=1e-5 * max(1.0, k ** 0.5))

@@ -117,8 +117,16 @@ struct MfmaLinearFunction : Function<MfmaLinearFunction> {
         const Tensor g = dense(grads[0]);
         Tensor dx, dw, db;
         if (ctx->needs_input_grad(0)) dx = sgemm(g, saved[1], false, false, std::nullopt);
-        if (ctx->needs_input_grad(1)) dw = sgemm(g, saved[0], true, false, std::nullopt);
-        if (ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2)) db = column_sum(g);
+        const bool want_b = ctx->saved_data["bias"].toBool() && ctx->needs_input_grad(2);
+        if (ctx->needs_input_grad(1)) {
+            TensorVec dws;
+            std::vector<OptTensor> dbs;
+            linear_weight_grad({g}, {saved[0]}, {want_b}, &dws, &dbs);
+            dw = dws[0];
+            db = grad_or_none(dbs[0]);
+        } else if (want_b) {
+            db = column_sum(g);
+        }
         return once({dx, dw, db});
     }
 };
@@ -160,18 +168,22 @@ struct LinearPairFunction : Function<LinearPairFunction> {
     static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &w_a,
                                  const Tensor &w_b, const Tensor &b_a, const Tensor &b_b) {
         ctx->save_for_backward({x, w_a, w_b});
-        auto y = b2gemm(x, w_a, w_b);
-        if (b_a.defined()) y[0].add_(b_a);
-        if (b_b.defined()) y[1].add_(b_b);
-        return y;
+        const auto bias = [](const Tensor &b) { return b.defined() ? OptTensor(b) : std::nullopt; };
+        return linear_forward_typed({x, x}, {w_a, w_b}, {bias(b_a), bias(b_b)}, std::nullopt);
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const auto s = ctx->get_saved_variables();
         const Tensor g_a = dense(grads[0]), g_b = dense(grads[1]);
-        auto d = b2gemm_backward(s[0], s[1], s[2], g_a, g_b);
-        d.push_back(ctx->needs_input_grad(3) ? column_sum(g_a) : Tensor());
-        d.push_back(ctx->needs_input_grad(4) ? column_sum(g_b) : Tensor());
-        return once(std::move(d));
+        TensorVec dws;
+        std::vector<OptTensor> dbs;
+        linear_weight_grad({g_a, g_b}, {s[0], s[0]},
+                           {ctx->needs_input_grad(3), ctx->needs_input_grad(4)}, &dws, &dbs);
+        Tensor dx;
+        if (ctx->needs_input_grad(0)) {
+            dx = sgemm(g_a, s[1], false, false, std::nullopt);
+            sgemm(g_b, s[2], false, false, dx, true);
+        }
+        return once({dx, dws[0], dws[1], grad_or_none(dbs[0]), grad_or_none(dbs[1])});
     }
 };
 
@@ -241,19 +253,35 @@ struct TypedLinearFunction : Function<TypedLinearFunction> {
                 b.push_back(dense(saved[count + i]));
             }
         if (!at.empty()) take(sgemm_typed(a, b, false, false, std::nullopt));
-        for (int64_t i = 0; i < count; i++)
-            if (ctx->needs_input_grad(count + i)) {
+        // weight gradients, each with the bias gradient that belongs to it
+        std::vector<bool> want;
+        std::vector<int64_t> bias_slot(count, -1);
+        for (size_t j = 0; j < bias_at.size(); j++)
+            if (ctx->needs_input_grad(2 * count + j)) bias_slot[bias_at[j]] = 1 + 2 * count + j;
+        const bool one_shape = std::all_of(saved.begin() + count, saved.end(), [&](const Tensor &w) {
+            return w.sizes() == saved[count].sizes();
+        });
+        for (int64_t i = 0; i < count; i++) {
+            if (one_shape && ctx->needs_input_grad(count + i)) {
                 at.push_back(1 + count + i);
                 a.push_back(parts[i]);
                 b.push_back(dense(saved[i]));
+                want.push_back(bias_slot[i] >= 0);
+            } else {
+                if (ctx->needs_input_grad(count + i))
+                    out[1 + count + i] = sgemm(parts[i], dense(saved[i]), true, false, std::nullopt);
+                if (bias_slot[i] >= 0) out[bias_slot[i]] = column_sum(dense(parts[i]));
             }
-        if (!at.empty()) take(sgemm_typed(a, b, true, false, std::nullopt));
-        for (size_t j = 0; j < bias_at.size(); j++)
-            if (ctx->needs_input_grad(2 * count + j)) {
-                at.push_back(1 + 2 * count + j);
-                a.push_back(parts[bias_at[j]]);
+        }
+        if (!at.empty()) {
+            TensorVec dws;
+            std::vector<OptTensor> dbs;
+            linear_weight_grad(a, b, want, &dws, &dbs);
+            for (size_t i = 0; i < at.size(); i++) {
+                out[at[i]] = dws[i];
+                if (want[i]) out[bias_slot[at[i] - 1 - count]] = *dbs[i];
             }
-        if (!at.empty()) take(column_sum_typed(a));
+        }
         return out;
     }
 };

@@ -97,13 +97,18 @@ void bind_graph_state(py::module_ &m);
 // ---- ops (ops.cpp) -------------------------------------------------------------------
 Tensor agg(const Tensor &x, const Tensor &rp, const Tensor &ci, const OptTensor &degrees,
            const OptTensor &edge_scale, double alpha, const RowState &rows);
-Tensor sgemm(const Tensor &a, const Tensor &b, bool trans_a, bool trans_b, const OptTensor &out);
+Tensor sgemm(const Tensor &a, const Tensor &b, bool trans_a, bool trans_b, const OptTensor &out,
+             bool accumulate = false);  // accumulate: add to `out`
 Tensor linear_forward(const Tensor &x, const Tensor &w, const OptTensor &bias);
 TensorVec linear_forward_typed(const TensorVec &xs, const TensorVec &ws,
                                const std::vector<OptTensor> &bs,
                                const std::optional<TensorVec> &outs);
 TensorVec sgemm_typed(const TensorVec &as, const TensorVec &bs, bool trans_a, bool trans_b,
                       const std::optional<TensorVec> &outs);
+// dw_i = g_i^T . x_i, and db_i = column sums of g_i where want_bias[i]
+void linear_weight_grad(const TensorVec &gs, const TensorVec &xs,
+                        const std::vector<bool> &want_bias, TensorVec *dws,
+                        std::vector<OptTensor> *dbs);
 TensorVec b2gemm(const Tensor &x, const Tensor &w_a, const Tensor &w_b);
 TensorVec b2gemm_backward(const Tensor &x, const Tensor &w_a, const Tensor &w_b,
                           const Tensor &grad_a, const Tensor &grad_b);

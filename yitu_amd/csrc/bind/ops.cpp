@@ -84,7 +84,8 @@ Tensor edge_scale(const Tensor &ci, const Tensor &degrees) {
 }
 
 // ---- dense products ------------------------------------------------------------------
-Tensor sgemm(const Tensor &a, const Tensor &b, bool trans_a, bool trans_b, const OptTensor &out) {
+Tensor sgemm(const Tensor &a, const Tensor &b, bool trans_a, bool trans_b, const OptTensor &out,
+             bool accumulate) {
     check_f32(a, "a", 2);
     check_f32(b, "b", 2);
     same_device(a, b);
@@ -102,7 +103,7 @@ Tensor sgemm(const Tensor &a, const Tensor &b, bool trans_a, bool trans_b, const
         c = call.empty({m, n});
     }
     Tensor ws = call.scratch(yitu_sgemm_workspace_bytes(m, n, k, 1));
-    ok(yitu_sgemm(f32(c), f32(a), f32(b), m, n, k, trans_a, trans_b, a.size(1), b.size(1), n, 0,
+    ok(yitu_sgemm(f32(c), f32(a), f32(b), m, n, k, trans_a, trans_b, a.size(1), b.size(1), n, accumulate,
                   ws.data_ptr(), ws.numel(), call.stream),
        "yitu_sgemm");
     return c;
@@ -201,6 +202,38 @@ TensorVec sgemm_typed(const TensorVec &as, const TensorVec &bs, bool trans_a, bo
                         ws.numel(), c.stream),
        "yitu_sgemm_typed");
     return outs;
+}
+
+void linear_weight_grad(const TensorVec &gs, const TensorVec &xs,
+                        const std::vector<bool> &want_bias, TensorVec *dws,
+                        std::vector<OptTensor> *dbs) {
+    const int64_t count = (int64_t)gs.size(), n = gs[0].size(1), k = xs[0].size(1);
+    std::vector<int64_t> rows;
+    int64_t most = 0;
+    for (int64_t i = 0; i < count; i++) {
+        check_f32(gs[i], "grad", 2);
+        check_f32(xs[i], "x", 2);
+        same_device(gs[0], gs[i], xs[i]);
+        TORCH_CHECK(gs[i].size(1) == n && xs[i].size(1) == k && gs[i].size(0) == xs[i].size(0),
+                    "linear_weight_grad: grad_i [m_i, ", n, "], x_i [m_i, ", k, "]");
+        rows.push_back(gs[i].size(0));
+        most = std::max(most, rows.back());
+    }
+    Call c(gs[0]);
+    *dws = outputs(c, std::nullopt, std::vector<int64_t>(count, n), k, at::kFloat);
+    dbs->assign(count, std::nullopt);
+    std::vector<float *> db(count, nullptr);
+    for (int64_t i = 0; i < count; i++)
+        if (want_bias[i]) {
+            (*dbs)[i] = c.empty({n});
+            db[i] = f32((*dbs)[i]);
+        }
+    Tensor ws = c.scratch(yitu_linear_weight_grad_workspace_bytes(most, n, k, count));
+    ok(yitu_linear_weight_grad_typed(pointers<float *>(*dws).data(), db.data(),
+                                     pointers<const float *>(gs).data(),
+                                     pointers<const float *>(xs).data(), rows.data(), count, n, k,
+                                     ws.data_ptr(), ws.numel(), c.stream),
+       "yitu_linear_weight_grad_typed");
 }
 
 Tensor gemm_bf16(const Tensor &a, const Tensor &b, bool trans_b, at::ScalarType dtype,
@@ -780,7 +813,9 @@ void bind_ops(py::module_ &m) {
         }
     });
     m.def("edge_scale", &edge_scale);
-    m.def("sgemm", &sgemm);
+    m.def("sgemm", [](const Tensor &a, const Tensor &b, bool ta, bool tb, const OptTensor &out) {
+        return sgemm(a, b, ta, tb, out);
+    });
     m.def("linear_forward", &linear_forward);
     m.def("linear_forward_typed", &linear_forward_typed);
     m.def("sgemm_typed", &sgemm_typed);

@@ -35,7 +35,7 @@ struct GemmProblem {
     // the K range [s * k_chunk, min(K, (s+1) * k_chunk)) and, when n_split > 1,
     // writes its own [M, N] slab of `partial` (slab index = blockIdx.z)
     int z0, n_split, k_chunk;
-    const float *bias = nullptr;  // [N], added to every row (the many-rows kernel only)
+    const float *bias = nullptr;  // [N], added to every row of C
 };
 
 struct GemmParams {
@@ -203,6 +203,7 @@ __global__ __launch_bounds__(256) void sgemm_mfma_kernel(GemmParams p) {
     float *cbase = pr.C;
     int ldc = p.ldc;
     bool accumulate = p.accumulate != 0;
+    const float *bias = pr.n_split > 1 ? nullptr : pr.bias;  // (a split's sum gets it later)
     if (pr.n_split > 1) {
         cbase = p.partial + (size_t)blockIdx.z * p.max_m * p.N;
         ldc = p.N;
@@ -213,6 +214,7 @@ __global__ __launch_bounds__(256) void sgemm_mfma_kernel(GemmParams p) {
 #pragma unroll
         for (int j = 0; j < TM; j++) {
             const int col = n0 + wn + 32 * j + l32;
+            const float add = bias && (FAST || col < p.N) ? bias[col] : 0.0f;
 #pragma unroll
             for (int jj = 0; jj < 4; jj++)
 #pragma unroll
@@ -220,7 +222,7 @@ __global__ __launch_bounds__(256) void sgemm_mfma_kernel(GemmParams p) {
                     const int row = m0 + wm + 32 * i + 8 * jj + 4 * lk + ii;
                     if (FAST || (row < pr.M && col < p.N)) {
                         float *c = cbase + (int64_t)row * ldc + col;
-                        const float v = acc[i][j][4 * jj + ii];
+                        const float v = acc[i][j][4 * jj + ii] + add;
                         *c = accumulate ? *c + v : v;
                     }
                 }
@@ -268,6 +270,7 @@ __global__ __launch_bounds__(256) void sgemm_splitk_reduce_kernel(GemmParams p) 
             float s = red[0][lane_e];
 #pragma unroll
             for (int g = 1; g < kSplitReduceGroups; g++) s += red[g][lane_e];
+            if (pr.bias) s += pr.bias[col];
             float *c = pr.C + (int64_t)row * p.ldc + col;
             *c = p.accumulate ? *c + s : s;
         }
@@ -638,234 +641,24 @@ static int sgemm_rows_try(const GemmParams &p, bool trans_a, bool trans_b, int l
     return sgemm_rows_launch_k<64, false>(r, stream);
 }
 
-// ---- weight gradients C_q[KI, NO] = A_q^T . B_q over many rows (KI, NO = 64, 128 or 256):
-// the output stays in registers. A workgroup of 8 waves owns a chunk of the rows of one
-// problem and the whole KI x NO product of that chunk (256 x 256: wave (wi, wj) the block
-// of rows 64 wi, columns 128 wj, 2 x 4 MFMA tiles, 128 accumulator registers), so every
-// row of A and B is read once, whole, two 16-row stages ahead through a ring of registers
-// into a double-buffered LDS stage, one barrier per stage. Both MFMA operands are columns
-// of the row-major stage (lane = column, the two halves of the wave take the two rows of
-// the step), with stage rows padded by 128 bytes so that the halves fall into different
-// banks. The chunk products go to the slabs of `partial` and are added by
-// sgemm_splitk_reduce_kernel in a fixed order.
-constexpr int TR_STAGE = 16;  // rows per stage
+}  // namespace yitu
 
-// KI x NO = (32 TX WI) x (32 TY WJ): WI x WJ = 8 waves, each TX x TY MFMA tiles.
-template <int WI, int WJ, int TX, int TY>
-struct TnRowsGeom {
-    static_assert(WI * WJ == 8 && TX * TY <= 8, "8 waves, at most 128 accumulator registers");
-    static constexpr int KI = 32 * TX * WI, NO = 32 * TY * WJ;
-    static constexpr int LDA = KI + 32, LDB = NO + 32;  // padded stage rows, floats
-    static constexpr size_t kLds = (size_t)2 * TR_STAGE * (LDA + LDB) * sizeof(float);
-};
+#include "gemm_panel.hpp"
+#include "gemm_tn.hpp"
 
-template <int WI, int WJ, int TX, int TY>
-__global__ __launch_bounds__(512, 1) void sgemm_tn_rows_kernel(GemmParams p) {
-    using G = TnRowsGeom<WI, WJ, TX, TY>;
-    constexpr int KI = G::KI, NO = G::NO, LDA = G::LDA, LDB = G::LDB;
-    constexpr int PA = (TR_STAGE * KI / 4 + 511) / 512, PB = (TR_STAGE * NO / 4 + 511) / 512;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    float *stage_mem = reinterpret_cast<float *>(smem);  // [2 buffers][A stage, B stage]
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int l32 = lane & 31, lk = lane >> 5;
-    const int i0 = (wave / WJ) * 32 * TX, j0 = (wave % WJ) * 32 * TY;
-    const GemmProblem pr = p.prob[problem_of(p, blockIdx.x)];
-    const int split = blockIdx.x - pr.z0;
-    const int m_beg = split * pr.k_chunk, m_end = min(pr.K, m_beg + pr.k_chunk);
-    const int n_stages = (m_end - m_beg + TR_STAGE - 1) / TR_STAGE;
-
-    float16v acc[TX][TY];
-#pragma unroll
-    for (int a = 0; a < TX; a++)
-#pragma unroll
-        for (int b = 0; b < TY; b++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) acc[a][b][e] = 0.0f;
-
-    // loader: thread t takes the 16-byte pieces t, t + 512, ... of a stage of A and of B
-    f4 ra[2][PA], rb[2][PB];
-    auto gload = [&](int slot, int st) {
-        const int r0 = m_beg + st * TR_STAGE;
-#pragma unroll
-        for (int h = 0; h < PA; h++) {
-            const int piece = t + 512 * h, row = r0 + piece / (KI / 4);
-            f4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (piece < TR_STAGE * KI / 4 && row < m_end)  // rows past the chunk add nothing
-                v = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(
-                    pr.A + (int64_t)row * p.a_sk + (piece % (KI / 4)) * 4));
-            ra[slot][h] = v;
-        }
-#pragma unroll
-        for (int h = 0; h < PB; h++) {
-            const int piece = t + 512 * h, row = r0 + piece / (NO / 4);
-            f4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (piece < TR_STAGE * NO / 4 && row < m_end)
-                v = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(
-                    pr.B + (int64_t)row * p.b_sk + (piece % (NO / 4)) * 4));
-            rb[slot][h] = v;
-        }
-    };
-    gload(0, 0);
-    __builtin_amdgcn_sched_barrier(0);  // oldest first
-    gload(1, 1);
-    for (int s0 = 0; s0 < n_stages; s0 += 2) {
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const int st = s0 + u;
-            if (st >= n_stages) break;  // same for the whole workgroup
-            float *As = stage_mem + (size_t)(st & 1) * TR_STAGE * (LDA + LDB);
-            float *Bs = As + TR_STAGE * LDA;
-            // this buffer was last read two stages ago, before the previous barrier
-#pragma unroll
-            for (int h = 0; h < PA; h++) {
-                const int piece = t + 512 * h;
-                if (piece < TR_STAGE * KI / 4)
-                    *reinterpret_cast<f4 *>(As + (piece / (KI / 4)) * LDA + (piece % (KI / 4)) * 4) =
-                        ra[u][h];
-            }
-#pragma unroll
-            for (int h = 0; h < PB; h++) {
-                const int piece = t + 512 * h;
-                if (piece < TR_STAGE * NO / 4)
-                    *reinterpret_cast<f4 *>(Bs + (piece / (NO / 4)) * LDB + (piece % (NO / 4)) * 4) =
-                        rb[u][h];
-            }
-            __syncthreads();
-            gload(u, st + 2);
-#pragma unroll
-            for (int k2 = 0; k2 < TR_STAGE; k2 += 2) {
-                float a[TX], b[TY];
-#pragma unroll
-                for (int x = 0; x < TX; x++) a[x] = As[(k2 + lk) * LDA + i0 + 32 * x + l32];
-#pragma unroll
-                for (int y = 0; y < TY; y++) b[y] = Bs[(k2 + lk) * LDB + j0 + 32 * y + l32];
-#pragma unroll
-                for (int x = 0; x < TX; x++)
-#pragma unroll
-                    for (int y = 0; y < TY; y++)
-                        acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[x], b[y], acc[x][y], 0, 0, 0);
-            }
-        }
-    }
-    // accumulator element 4 jj + ii of tile (x, y) is row i0 + 32 x + 8 jj + 4 (lane / 32) + ii,
-    // column j0 + 32 y + lane % 32 of this chunk's slab
-    float *dst = p.partial + (size_t)blockIdx.x * p.max_m * p.N;
-#pragma unroll
-    for (int x = 0; x < TX; x++)
-#pragma unroll
-        for (int y = 0; y < TY; y++)
-#pragma unroll
-            for (int jj = 0; jj < 4; jj++)
-#pragma unroll
-                for (int ii = 0; ii < 4; ii++) {
-                    const int row = i0 + 32 * x + 8 * jj + 4 * lk + ii;
-                    __builtin_nontemporal_store(acc[x][y][4 * jj + ii],
-                                                dst + (size_t)row * p.N + j0 + 32 * y + l32);
-                }
-}
-
-template <int WI, int WJ, int TX, int TY>
-static int sgemm_tn_rows_launch(const GemmParams &p, int z, hipStream_t stream) {
-    constexpr size_t lds = TnRowsGeom<WI, WJ, TX, TY>::kLds;
-    static bool prepared_on[64] = {};  // more LDS than the default limit: once per device
-    int device = 0;
-    if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) device = 0;
-    if (lds > 65536 && !prepared_on[device]) {
-        hipError_t e = hipFuncSetAttribute(
-            reinterpret_cast<const void *>(&sgemm_tn_rows_kernel<WI, WJ, TX, TY>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) {
-            set_error("hipFuncSetAttribute(dynamic LDS %zu): %s", lds, hipGetErrorString(e));
-            return -1;
-        }
-        prepared_on[device] = true;
-    }
-    sgemm_tn_rows_kernel<WI, WJ, TX, TY><<<z, 512, lds, stream>>>(p);
-    YITU_LAUNCH_CHECK();
-    return 0;
-}
-
-// widths the kernel is built for: 64, 128 or 256 on either side, at least 8 MFMA tiles
-static bool tn_rows_shape(int64_t ki, int64_t no) {
-    const bool ok_i = ki == 64 || ki == 128 || ki == 256, ok_j = no == 64 || no == 128 || no == 256;
-    return ok_i && ok_j && ki * no >= 64 * 128;
-}
-
-// chunks of all problems together: a workgroup per CU when the products keep the matrix
-// pipes busy (256 x 256), two when the rows are narrow and the kernel waits for memory
-static int tn_rows_chunks(int64_t ki, int64_t no) { return ki * no >= 256 * 256 ? 256 : 512; }
-
-// Takes a group of weight-gradient products [rows, KI]^T . [rows, NO] with many rows in
-// all; *taken says whether it did.
-static int sgemm_tn_rows_try(GemmParams &p, bool trans_a, bool trans_b, int lda, int ldb,
-                             void *workspace, size_t workspace_bytes, hipStream_t stream,
-                             bool *taken) {
-    *taken = false;
-    if (!trans_a || trans_b || p.n_prob < 1 || lda % 4 != 0 || ldb % 4 != 0 || !workspace) return 0;
-    const int ki = p.prob[0].M, no = p.N;
-    if (!tn_rows_shape(ki, no)) return 0;
-    int64_t total = 0;
-    for (int i = 0; i < p.n_prob; i++) {
-        const GemmProblem &pr = p.prob[i];
-        if (pr.M != ki || !aligned16(pr.A) || !aligned16(pr.B)) return 0;
-        total += pr.K;
-    }
-    if (total < 49152) return 0;
-    // every problem gets at least two chunks (its slabs are then always summed by the
-    // reduce kernel)
-    const size_t slab = (size_t)ki * no * sizeof(float);
-    const int64_t chunks = tn_rows_chunks(ki, no);
-    int z = 0;
-    GemmProblem saved[kMaxGroup];
-    for (int i = 0; i < p.n_prob; i++) saved[i] = p.prob[i];
-    for (int i = 0; i < p.n_prob; i++) {
-        GemmProblem &pr = p.prob[i];
-        int64_t want = std::max<int64_t>(2, (chunks * (int64_t)pr.K + total / 2) / total);
-        want = std::min<int64_t>(want, std::max<int64_t>(2, ceil_div(pr.K, TR_STAGE)));
-        pr.k_chunk = (int)(ceil_div(ceil_div(pr.K, want), TR_STAGE) * TR_STAGE);
-        pr.n_split = (int)std::max<int64_t>(2, ceil_div(pr.K, pr.k_chunk));
-        pr.z0 = z;
-        z += pr.n_split;
-    }
-    if ((size_t)z * slab > workspace_bytes || !aligned16(workspace)) {
-        for (int i = 0; i < p.n_prob; i++) p.prob[i] = saved[i];
-        return 0;
-    }
-    *taken = true;
-    p.max_m = ki;
-    p.partial = static_cast<float *>(workspace);
-    p.a_sk = lda;
-    p.a_si = 1;
-    p.b_sk = ldb;
-    p.b_sj = 1;
-    int rc = -1;
-    if (ki == 256 && no == 256) rc = sgemm_tn_rows_launch<4, 2, 2, 4>(p, z, stream);
-    else if (ki == 256 && no == 128) rc = sgemm_tn_rows_launch<4, 2, 2, 2>(p, z, stream);
-    else if (ki == 128 && no == 256) rc = sgemm_tn_rows_launch<2, 4, 2, 2>(p, z, stream);
-    else if (ki == 256 && no == 64) rc = sgemm_tn_rows_launch<8, 1, 1, 2>(p, z, stream);
-    else if (ki == 64 && no == 256) rc = sgemm_tn_rows_launch<1, 8, 2, 1>(p, z, stream);
-    else if (ki == 128 && no == 128) rc = sgemm_tn_rows_launch<2, 4, 2, 1>(p, z, stream);
-    else if (ki == 128 && no == 64) rc = sgemm_tn_rows_launch<4, 2, 1, 1>(p, z, stream);
-    else if (ki == 64 && no == 128) rc = sgemm_tn_rows_launch<2, 4, 1, 1>(p, z, stream);
-    if (rc) return rc;
-    dim3 rg((unsigned)std::min<int64_t>(ceil_div((int64_t)ki * no, kSplitReduceCols), 4096),
-            (unsigned)p.n_prob);
-    sgemm_splitk_reduce_kernel<<<rg, 256, 0, stream>>>(p);
-    YITU_LAUNCH_CHECK();
-    return 0;
-}
+namespace yitu {
 
 // trans_a: A is given as [K, M] row-major (else [M, K]); trans_b: B is given as
 // [N, K] row-major (else [K, N]).
 int sgemm_grouped(GemmParams &p, bool trans_a, bool trans_b, int lda, int ldb, void *workspace,
                   size_t workspace_bytes, hipStream_t stream) {
-    // problems with an empty inner dimension: C = 0 (or unchanged); they leave the group
+    // problems with an empty inner dimension and no bias: C = 0 (or unchanged); they leave the
+    // group
     int kept = 0;
     for (int i = 0; i < p.n_prob; i++) {
         const GemmProblem pr = p.prob[i];
         if (pr.M == 0) continue;
-        if (pr.K > 0) {
+        if (pr.K > 0 || pr.bias) {  // (a bias alone is still written)
             p.prob[kept++] = pr;
             continue;
         }
@@ -886,9 +679,13 @@ int sgemm_grouped(GemmParams &p, bool trans_a, bool trans_b, int lda, int ldb, v
         const int rc = sgemm_rows_try(p, trans_a, trans_b, lda, ldb, workspace, workspace_bytes,
                                       stream, &taken);
         if (taken) return rc;
-        const int rc2 = sgemm_tn_rows_try(p, trans_a, trans_b, lda, ldb, workspace, workspace_bytes,
-                                          stream, &taken);
-        if (taken) return rc2;
+        const int rc1 = sgemm_panel_try(p, trans_a, trans_b, lda, ldb, stream, &taken);
+        if (taken) return rc1;
+        if (trans_a && !trans_b) {
+            const int rc2 = sgemm_tn_rows_try(p, nullptr, lda, ldb, workspace, workspace_bytes,
+                                              stream, &taken);
+            if (taken) return rc2;
+        }
     }
     int max_m = 0;
     for (int i = 0; i < p.n_prob; i++) max_m = std::max(max_m, p.prob[i].M);
@@ -935,9 +732,7 @@ YITU_API size_t yitu_sgemm_workspace_bytes(int64_t m, int64_t n, int64_t k, int6
     // (or room for the [N, K] copies of the weights that the many-rows kernel reads, or for
     // the chunk products of the weight-gradient kernel: a chunk per CU and two per problem)
     size_t rows_ws = std::max<size_t>(sgemm_rows_workspace_bytes(n, k, n_problems), 256);
-    if (tn_rows_shape(m, n))
-        rows_ws = std::max(rows_ws, (size_t)(tn_rows_chunks(m, n) + 2 * kMaxGroup) * m * n *
-                                        sizeof(float));
+    rows_ws = std::max(rows_ws, tn_rows_workspace_bytes(m, n, k, n_problems));
     if (tiles <= 0 || tiles >= 256 || k < 2 * kMinSplitK) return rows_ws;
     const int64_t splits = std::min<int64_t>(ceil_div(k, kMinSplitK), ceil_div(1024, tiles));
     return std::max(rows_ws, align_up((size_t)(splits * m * n * n_problems) * sizeof(float), 256));
@@ -961,27 +756,6 @@ YITU_API int yitu_sgemm(float *c, const float *a, const float *b, int64_t m, int
                          workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
-namespace yitu {
-// y[i, j] += bias[j]: the bias of a Linear whose product did not run on the kernel that adds it
-__global__ __launch_bounds__(256) void bias_add_kernel(float *__restrict__ y,
-                                                       const float *__restrict__ bias, int64_t m,
-                                                       int n, int64_t ldy) {
-    const int64_t total = m * n, stride = (int64_t)gridDim.x * 256;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += stride)
-        y[(i / n) * ldy + i % n] += bias[i % n];
-}
-// The same for every problem of a group in one launch (blockIdx.y = problem): the per-relation
-// Linears of a small heterogeneous graph are dozens of products of a few hundred rows.
-__global__ __launch_bounds__(256) void bias_add_group_kernel(GemmParams p) {
-    const GemmProblem &pr = p.prob[blockIdx.y];
-    if (!pr.bias) return;
-    const int n = p.N;
-    const int64_t total = (int64_t)pr.M * n, stride = (int64_t)gridDim.x * 256;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += stride)
-        pr.C[(i / n) * p.ldc + i % n] += pr.bias[i % n];
-}
-}  // namespace yitu
-
 YITU_API int yitu_linear_forward(float *y, const float *x, const float *w, const float *bias,
                                  int64_t m, int64_t n, int64_t k, void *workspace,
                                  size_t workspace_bytes, void *stream_) {
@@ -996,19 +770,7 @@ YITU_API int yitu_linear_forward(float *y, const float *x, const float *w, const
     p.n_prob = 1;
     p.N = (int)n;
     p.ldc = (int)n;
-    if (k > 0) {
-        bool taken = false;
-        const int rc = sgemm_rows_try(p, false, true, (int)k, (int)k, workspace, workspace_bytes,
-                                      stream, &taken);
-        if (taken) return rc;
-    }
-    p.prob[0].bias = nullptr;
-    const int rc = sgemm_grouped(p, false, true, (int)k, (int)k, workspace, workspace_bytes, stream);
-    if (rc || !bias) return rc;
-    const int grid = (int)std::min<int64_t>(ceil_div(m * n, 256), 16384);
-    bias_add_kernel<<<grid, 256, 0, stream>>>(y, bias, m, (int)n, n);
-    YITU_LAUNCH_CHECK();
-    return 0;
+    return sgemm_grouped(p, false, true, (int)k, (int)k, workspace, workspace_bytes, stream);
 }
 
 YITU_API int yitu_linear_forward_typed(float *const *y, const float *const *x,
@@ -1036,29 +798,9 @@ YITU_API int yitu_linear_forward_typed(float *const *y, const float *const *x,
             pr.bias = bias ? bias[first + i] : nullptr;
             p.prob[p.n_prob++] = pr;
         }
-        if (p.n_prob == 0) continue;
-        if (k > 0) {
-            bool taken = false;
-            const int rc = sgemm_rows_try(p, false, true, (int)k, (int)k, workspace,
-                                          workspace_bytes, stream, &taken);
-            if (rc) return rc;
-            if (taken) continue;
-        }
-        // (the grouped call drops problems from its table: keep what the bias pass needs)
-        const GemmParams all = p;
-        for (int i = 0; i < p.n_prob; i++) p.prob[i].bias = nullptr;
         const int rc = sgemm_grouped(p, false, true, (int)k, (int)k, workspace, workspace_bytes,
                                      stream);
         if (rc) return rc;
-        int64_t most = 0;
-        for (int i = 0; i < all.n_prob; i++)
-            if (all.prob[i].bias) most = std::max<int64_t>(most, (int64_t)all.prob[i].M * n);
-        if (most > 0) {
-            const dim3 grid((unsigned)std::min<int64_t>(ceil_div(most, 256), 16384),
-                            (unsigned)all.n_prob);
-            bias_add_group_kernel<<<grid, 256, 0, stream>>>(all);
-            YITU_LAUNCH_CHECK();
-        }
     }
     return 0;
 }
@@ -1093,6 +835,72 @@ YITU_API int yitu_sgemm_typed(float *const *c, const float *const *a, const floa
         if (rc) return rc;
     }
     return 0;
+}
+
+// Weight and bias gradients of Linear layers that share both widths: dw_i = g_i^T . x_i and
+// db_i = the column sums of g_i (db, or an entry of it, may be null).
+YITU_API int yitu_linear_weight_grad_typed(float *const *dw, float *const *db,
+                                           const float *const *g, const float *const *x,
+                                           const int64_t *rows, int64_t n_problems, int64_t n_out,
+                                           int64_t n_in, void *workspace, size_t workspace_bytes,
+                                           void *stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    YITU_REQUIRE(n_problems >= 0 && n_out >= 0 && n_in >= 0, "negative size");
+    if (n_problems == 0 || n_out == 0) return 0;
+    YITU_REQUIRE(dw && g && x && rows, "null problem table");
+    YITU_REQUIRE(n_out < INT32_MAX && n_in < INT32_MAX, "size out of range");
+    for (int64_t first = 0; first < n_problems; first += kMaxGroup) {
+        GemmParams p{};
+        p.n_prob = (int)std::min<int64_t>(kMaxGroup, n_problems - first);
+        p.N = (int)n_in;
+        p.ldc = (int)n_in;
+        for (int i = 0; i < p.n_prob; i++) {
+            const int64_t ri = rows[first + i];
+            YITU_REQUIRE(ri >= 0 && ri < INT32_MAX && (n_in == 0 || dw[first + i]) &&
+                             (ri == 0 || (g[first + i] && (n_in == 0 || x[first + i]))),
+                         "problem %d: null operand or size out of range", (int)(first + i));
+            p.prob[i] = GemmProblem{g[first + i], x[first + i], dw[first + i], (int)n_out, (int)ri};
+        }
+        bool taken = false;
+        if (n_in > 0) {
+            int rc = sgemm_tn_rows_try(p, db ? db + first : nullptr, (int)n_out, (int)n_in,
+                                       workspace, workspace_bytes, stream, &taken);
+            if (rc) return rc;
+            if (taken) continue;
+        }
+        const int count = p.n_prob;
+        if (n_in > 0) {
+            int rc = sgemm_grouped(p, true, false, (int)n_out, (int)n_in, workspace,
+                                   workspace_bytes, stream);
+            if (rc) return rc;
+        }
+        // (ordered behind the products on the stream: the workspace is free again)
+        int64_t most = 0;
+        for (int i = 0; i < count; i++) most = std::max<int64_t>(most, rows[first + i]);
+        float *out[kMaxGroup];
+        const float *in[kMaxGroup];
+        int64_t ms[kMaxGroup], n_sums = 0;
+        for (int i = 0; db && i < count; i++) {
+            if (!db[first + i]) continue;
+            out[n_sums] = db[first + i];
+            in[n_sums] = g[first + i];
+            ms[n_sums++] = rows[first + i];
+        }
+        int rc = 0;
+        if (most <= 4096)  // short matrices: all of them in one launch
+            rc = yitu_column_sum_typed(out, in, ms, n_sums, n_out, n_out, stream);
+        else
+            for (int64_t i = 0; i < n_sums && !rc; i++)
+                rc = yitu_column_sum(out[i], in[i], ms[i], n_out, workspace, workspace_bytes, stream);
+        if (rc) return rc;
+    }
+    return 0;
+}
+
+YITU_API size_t yitu_linear_weight_grad_workspace_bytes(int64_t rows, int64_t n_out, int64_t n_in,
+                                                        int64_t n_problems) {
+    return std::max(yitu_sgemm_workspace_bytes(n_out, n_in, rows, n_problems),
+                    yitu_column_sum_workspace_bytes(rows, n_out));
 }
 
 YITU_API int yitu_b2gemm(float *y_a, float *y_b, const float *x, const float *w_a,
