@@ -276,7 +276,8 @@ int yitu_gat_forward(float *out_device, float *attn_device, float *row_stats_dev
  * the heads (test/common/model.py:106) and grad_out_device is its gradient
  * g [n_dst,F], standing for grad_out[r,h,:] = g[r,:] / H. The pass then gathers
  * F floats per edge instead of H*F. One-pass shapes only (rows of 256 floats, or
- * 512 / 1024 with out_device, head width a power of two in 32..256).
+ * 512 / 1024 with out_device, head width a power of two in 32..256); with out_device
+ * also 1, 2, 4 or 8 heads of a multiple of 4 up to 256.
  */
 int yitu_gat_backward(float *grad_query_device, float *grad_key_device,
                       float *grad_features_device, float *grad_attn_scratch_device,

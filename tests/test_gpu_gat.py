@@ -193,6 +193,38 @@ def test_gat_head_mean_gradient(dev, h, f):
         assert_close(got, ref, atol=5e-4, what="grad_%s H=%d F=%d" % (name, h, f))
 
 
+@pytest.mark.parametrize("h,f", [(1, 4), (1, 16), (1, 40), (1, 128), (2, 8), (2, 24), (2, 64), (2, 256),
+                                 (4, 8), (4, 32), (4, 100), (8, 8), (8, 12), (8, 16), (8, 32), (8, 256),
+                                 (16, 32), (32, 32)])
+@pytest.mark.parametrize("with_attn", [False, True])
+def test_gat_head_mean_backward_against_oracle(dev, h, f, with_attn):
+    """The head-mean backward over every lane layout (several source rows of one load for
+    narrow heads, partial lane groups for odd widths), with the stored probabilities and
+    from the row statistics, on rows from empty to hundreds of edges."""
+    n_dst, n_src = 203, 167
+    indptr, indices = random_csr(n_dst, n_src, 0.08, h * 7 + f, hub_rows=(9,), hub_degree=160,
+                                 empty_rows=(0, 202))
+    order = np.random.default_rng(f).permutation(len(indices))  # long by-source rows too
+    skew = torch.where(torch.from_numpy(order % 3 == 0), torch.full_like(indices, 5), indices)
+    g = torch.Generator().manual_seed(h * f + 1)
+    q, k = torch.randn(n_dst, h, generator=g), torch.randn(n_src, h, generator=g)
+    x, gy = torch.randn(n_src, h, f, generator=g), torch.randn(n_dst, f, generator=g)
+    per_head = (gy / h).unsqueeze(1).expand(n_dst, h, f).contiguous()
+    attn_o, want_out, want_gq, want_gk, want_gx = _oracle_gat(indptr, skew, q.numpy(), k.numpy(),
+                                                              x.numpy(), per_head.numpy())
+    _, abs_ga, abs_gx = spmm_abs_sums(attn_o, indptr, skew, x, per_head)
+    abs_gq, abs_gk = softmax_backward_abs_sums(indptr, skew, attn_o, abs_ga, n_src)
+    d = lambda t: t.to(dev)
+    made = graph_ext.gat_forward(d(indptr), d(skew), d(q), d(k), d(x), stats_only=not with_attn)
+    gq, gk, gx = graph_ext.gat_backward(d(indptr), d(skew), d(q), d(k), d(x), made[1], d(gy),
+                                        out=made[0], head_mean=True,
+                                        stats=None if with_attn else made[2])
+    what = "H=%d F=%d" % (h, f)
+    assert_close(gq, want_gq, abs_sum=abs_gq[0], what="grad_q " + what)
+    assert_close(gk, want_gk, abs_sum=abs_gk, what="grad_k " + what)
+    assert_close(gx, want_gx, abs_sum=abs_gx, what="grad_x " + what)
+
+
 @pytest.mark.parametrize("n,h,f", [(1000, 4, 64), (37, 1, 4), (513, 8, 32), (300, 2, 256),
                                    (129, 16, 16), (64, 4, 256), (5, 3, 8)])
 @pytest.mark.parametrize("two", [True, False])

@@ -360,7 +360,7 @@ struct FusedGatFunction : Function<FusedGatFunction> {
     static Tensor forward(AutogradContext *ctx, const Tensor &query, const Tensor &key,
                           const Tensor &x, bool head_mean, KeptPtr k) {
         // one-pass shapes: each row's softmax statistics are kept instead of the probabilities
-        k->flag = gat_one_pass_shape(x.size(1), x.size(2)) && k->indices.numel() > 0;
+        k->flag = stats_suffice(x, head_mean) && k->indices.numel() > 0;
         k->flag2 = head_mean;
         const GatOut o = gat_forward(k->indptr, k->indices, query, key, x, k->flag, k->rows());
         ctx->save_for_backward({query, key, x, k->flag ? *o.stats : *o.attn, o.out});
@@ -376,6 +376,12 @@ struct FusedGatFunction : Function<FusedGatFunction> {
                                         dense(grads[0]), s[4], k->flag2, stats, k->rows(),
                                         by_source(k->indptr, k->indices, k->n_src));
         return {g.query, g.key, g.x, Tensor(), Tensor()};
+// Whether the backward needs no more of the forward's softmax than its row statistics.
+bool stats_suffice(const Tensor &x, bool head_mean) {
+    return gat_one_pass_shape(x.size(1), x.size(2)) ||
+           (head_mean && gat_mean_shape(x));
+}
+
     }
 };
 
@@ -391,7 +397,7 @@ struct GatHeadsFunction : Function<GatHeadsFunction> {
             query = both.first;
             key = *both.second;
         }
-        k->flag = gat_one_pass_shape(x_src.size(1), x_src.size(2)) && k->indices.numel() > 0;
+        k->flag = stats_suffice(x_src, head_mean) && k->indices.numel() > 0;
         k->flag2 = head_mean;
         const GatOut o = gat_forward(k->indptr, k->indices, query, key, x_src, k->flag, k->rows());
         variable_list saved = {x_src, a_src, a_dst, query, key, k->flag ? *o.stats : *o.attn, o.out};

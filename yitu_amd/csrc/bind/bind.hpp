@@ -75,6 +75,9 @@ inline const int32_t *i32(const Tensor &t) { return static_cast<const int32_t *>
 inline const void *raw(const OptTensor &t) {
     return t.has_value() && t->defined() ? t->data_ptr() : nullptr;
 }
+inline bool aligned16(const Tensor &t) {
+    return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
 inline bool has(const OptTensor &t) { return t.has_value() && t->defined(); }
 
 // ---- state kept per graph (graph_state.cpp) ------------------------------------------
@@ -127,6 +130,7 @@ std::pair<Tensor, Tensor> sddmm_backward(const Tensor &indptr, const Tensor &ind
                                          const Tensor &grad_out, const RowState &rows,
                                          const std::optional<BySource> &t);
 bool gat_one_pass_shape(int64_t heads, int64_t width);
+bool gat_mean_shape(const Tensor &x);  // of the head-mean backward, x [n_src, H, F]
 struct GatOut {
     Tensor out;
     OptTensor attn, stats;

@@ -532,6 +532,13 @@ bool gat_one_pass_shape(int64_t heads, int64_t width) {
            (row == 256 || row == 512 || row == 1024);
 }
 
+// Features whose backward takes the gradient of the mean over heads as it is.
+bool gat_mean_shape(const Tensor &x) {
+    const int64_t heads = x.size(1), width = x.size(2);
+    return (heads == 1 || heads == 2 || heads == 4 || heads == 8) && width >= 4 && width <= 256 &&
+           width % 4 == 0 && x.size(0) <= (1 << 24) && aligned16(x);
+}
+
 GatOut gat_forward(const Tensor &indptr, const Tensor &indices, const Tensor &query,
                    const Tensor &key, const Tensor &x, bool stats_only, const RowState &rows) {
     check_i32(indptr, "indptr", 1);
@@ -545,7 +552,7 @@ GatOut gat_forward(const Tensor &indptr, const Tensor &indices, const Tensor &qu
     TORCH_CHECK(query.size(0) == n_dst && query.size(1) == h && key.size(0) == n_src &&
                     key.size(1) == h,
                 "query must be [n_dst, H] and key [n_src, H]");
-    TORCH_CHECK(!stats_only || gat_one_pass_shape(h, f),
+    TORCH_CHECK(!stats_only || gat_one_pass_shape(h, f) || gat_mean_shape(x),
                 "stats_only needs a one-pass shape (see gat_one_pass_shape)");
     Call c(x);
     GatOut o;
@@ -581,8 +588,9 @@ GatGrads gat_backward(const Tensor &indptr, const Tensor &indices, const Tensor 
         check_f32(grad_out, "grad_out", 2);
         TORCH_CHECK(grad_out.size(0) == n_dst && grad_out.size(1) == f,
                     "a head-mean grad_out must be [n_dst, n_features]");
-        if (!(gat_one_pass_shape(h, f) && n_dst > 0 && nnz > 0)) {
-            // shapes outside the one-pass kernels: spell the gradient out per head
+        if (!aligned16(grad_out)) grad_out = grad_out.clone();
+        if (!((gat_one_pass_shape(h, f) || (gat_mean_shape(x) && has(out))) && n_dst > 0 && nnz > 0)) {
+            // shapes outside the head-mean kernels: spell the gradient out per head
             grad_out = (grad_out / (double)h).unsqueeze(1).expand({n_dst, h, f}).contiguous();
             head_mean = false;
         }

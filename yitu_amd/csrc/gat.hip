@@ -20,6 +20,8 @@
 // (attn-weighted sum); the softmax + LeakyReLU backward and the grad_key sum
 // then work on [nnz, H] edge arrays only.
 #include "../../include/yitu_hip.h"
+#include <type_traits>
+
 #include "sddmm_kernels.hpp"
 
 namespace yitu {
@@ -1371,207 +1373,11 @@ __global__ __launch_bounds__(kBlock) void gat_src_items_kernel(GatSrcParams p) {
     }
 }
 
-// ---- head-mean gradient, rows of 256 floats: several edges per load -----------------
-// When the gathered row is the F-float gradient of the head mean, a wave-wide load of
-// the layout above fetches the same F floats once per head, and with F * 4 bytes per
-// edge the pass is bound by the number of loads in flight, not by bandwidth. Here a
-// load instruction fetches SLOTS = 64 / LPH = H different edges: lane (s, sub) holds
-// floats [4 sub, +4) of the gradient row of the s-th edge of a group, and the source's
-// own row as H slices x[c, h, 4 sub .. +4). Per group: H dots (one per head, reduced
-// over the slot's LPH lanes), H x 4 FMAs into acc[h], and the epilogue on lanes
-// sub < H (one head each). Slot sums are folded by a fixed butterfly at the end.
-template <int LPH>
-struct SlotRow {
-    static constexpr int H = kWave / LPH;  // heads = slots (rows of 256 floats)
-    float xh[H][4], acc[H][4];
-    float kc, gk;  // lanes sub < H: key[c, sub] and this slot's share of grad_key[c, sub]
-};
+}  // namespace yitu
 
-template <int LPH>
-__device__ __forceinline__ void slot_begin(SlotRow<LPH> &row, const GatSrcParams &p, int c,
-                                           bool load) {
-    constexpr int H = SlotRow<LPH>::H;
-    const int sub = lane_id() % LPH;
-    row.kc = row.gk = 0.0f;
-#pragma unroll
-    for (int h = 0; h < H; h++) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) row.acc[h][i] = row.xh[h][i] = 0.0f;
-        if (load) RowLoad<4, float>::ld(p.x + (size_t)c * 256 + h * (4 * LPH) + sub * 4, row.xh[h]);
-    }
-    if (load && sub < H) row.kc = p.key[(size_t)c * H + sub];
-}
+#include "gat_slots.hpp"
 
-template <int LPH>
-__device__ __forceinline__ void slot_window(SlotRow<LPH> &row, const GatSrcParams &p,
-                                            const EdgeWindow &win, int first, int n) {
-    // U load groups in flight: 2 measured a little better than 4 (fewer registers)
-    constexpr int H = SlotRow<LPH>::H, SLOTS = H, U = 2;
-    const int lane = lane_id();
-    const int s = lane / LPH, sub = lane % LPH;
-    const float *__restrict__ g = static_cast<const float *>(p.sp.feat);
-    const int F = 4 * LPH;
-    for (int k0 = 0; k0 < n; k0 += SLOTS * U) {
-        float v[U][4], a[U][H];
-        float2 sq[U];
-        int vr[U];
-        bool valid[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (k0 + u * SLOTS < n) {  // wave-uniform
-                const int k = k0 + u * SLOTS + s;
-                valid[u] = k < n;
-                const int src = first + min(k, n - 1);
-                const int r = __shfl(win.col, src, kWave);
-                vr[u] = __shfl(win.vrow, src, kWave);
-                RowLoad<4, float>::ld(g + (size_t)r * F + sub * 4, v[u]);
-                sq[u] = make_float2(0.0f, 0.0f);
-                if (p.recompute) {
-                    // no read of attn: lane sub < H makes the probability of (edge, head sub)
-                    // from the destination's line, the slot's lanes then share the H values
-                    float mine_a = 0.0f;
-                    if (sub < H) {
-                        const float4 t4 = p.row_sq[(size_t)r * H + sub];
-                        sq[u] = make_float2(t4.x, t4.y);
-                        mine_a = expf(leaky(t4.y + row.kc) - t4.z) * t4.w;
-                    }
-#pragma unroll
-                    for (int h = 0; h < H; h++) a[u][h] = __shfl(mine_a, (lane - sub) + h, kWave);
-                } else {
-                    if constexpr (H == 8) {  // two 16-byte halves
-                        float lo[4], hi[4];
-                        RowLoad<4, float>::ld(p.sp.values + (size_t)vr[u] * 8, lo);
-                        RowLoad<4, float>::ld(p.sp.values + (size_t)vr[u] * 8 + 4, hi);
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            a[u][i] = lo[i];
-                            a[u][4 + i] = hi[i];
-                        }
-                    } else {
-                        RowLoad<H, float>::ld(p.sp.values + (size_t)vr[u] * H, a[u]);
-                    }
-                    if (sub < H) {
-                        const float4 t4 = p.row_sq[(size_t)r * H + sub];
-                        sq[u] = make_float2(t4.x, t4.y);
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (k0 + u * SLOTS >= n) break;  // wave-uniform
-            float mine = 0.0f;  // d_attn of (this slot's edge, head sub) on lanes sub < H
-#pragma unroll
-            for (int h = 0; h < H; h++) {
-                float d = row.xh[h][0] * v[u][0] + row.xh[h][1] * v[u][1] + row.xh[h][2] * v[u][2] +
-                          row.xh[h][3] * v[u][3];
-                d = group_sum<LPH>(d);
-                if (sub == h) mine = d;
-                const float w = valid[u] ? a[u][h] * p.g_scale : 0.0f;
-#pragma unroll
-                for (int i = 0; i < 4; i++) row.acc[h][i] += w * v[u][i];
-            }
-            if (valid[u] && sub < H) {
-                float ah = 0.0f;
-#pragma unroll
-                for (int h = 0; h < H; h++)
-                    if (sub == h) ah = a[u][h];
-                const float gl = ah * (mine * p.g_scale - sq[u].x) *
-                                 (sq[u].y + row.kc < 0.0f ? kSlope : 1.0f);
-                p.grad_a[(size_t)vr[u] * H + sub] = gl;
-                row.gk += gl;
-            }
-        }
-    }
-}
-
-template <int LPH>
-__device__ __forceinline__ void slot_end(SlotRow<LPH> &row, float *x_dst, float *k_dst) {
-    constexpr int H = SlotRow<LPH>::H;
-    const int lane = lane_id();
-    const int s = lane / LPH, sub = lane % LPH;
-#pragma unroll
-    for (int o = kWave / 2; o >= LPH; o >>= 1) {
-        row.gk += __shfl_xor(row.gk, o, kWave);
-#pragma unroll
-        for (int h = 0; h < H; h++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) row.acc[h][i] += __shfl_xor(row.acc[h][i], o, kWave);
-    }
-    if (s == 0) {
-#pragma unroll
-        for (int h = 0; h < H; h++) store_row_streaming<4>(x_dst + h * (4 * LPH) + sub * 4, row.acc[h]);
-        if (sub < H) k_dst[sub] = row.gk;
-    }
-}
-
-template <int LPH>
-__global__ __launch_bounds__(kBlock) void gat_slot_rows_kernel(GatSrcParams p) {
-    constexpr int H = kWave / LPH;
-    const int lane = lane_id();
-    const int rpw = rows_per_wave(p.sp.n_rows);
-    const int r0 = (blockIdx.x * kWavesPerBlock + wave_id()) * rpw;
-    if (r0 >= p.sp.n_rows) return;
-    const int n_here = min(rpw, p.sp.n_rows - r0);
-    const int my_ptr = p.sp.indptr[r0 + min(lane, n_here)];
-    const int limit = __builtin_amdgcn_readlane(my_ptr, n_here);
-    EdgeWindow win;
-    win.base = -1;
-    win.col = 0;
-    win.w = 0.0f;
-    win.vrow = 0;
-    for (int i = 0; i < n_here; i++) {
-        const int row = r0 + i;
-        const int beg = __builtin_amdgcn_readlane(my_ptr, i), end = __builtin_amdgcn_readlane(my_ptr, i + 1);
-        if (end - beg >= p.sp.plan.threshold) continue;  // a planned row: the item kernel
-        SlotRow<LPH> acc;
-        slot_begin<LPH>(acc, p, row, end > beg);
-        for (int b = beg; b < end; b += kWave) {
-            const int n = min(kWave, end - b);
-            if (win.base < 0 || b < win.base || b + n > win.base + kWave)
-                load_window<W_EDGEHEAD>(win, p.sp, b, limit);
-            slot_window<LPH>(acc, p, win, b - win.base, n);
-        }
-        slot_end<LPH>(acc, p.sp.out + (size_t)row * 256, p.grad_k + (size_t)row * H);
-    }
-}
-
-template <int LPH>
-__global__ __launch_bounds__(kBlock) void gat_slot_items_kernel(GatSrcParams p) {
-    constexpr int H = kWave / LPH;
-    const int lane = lane_id();
-    if (p.sp.plan.counters->overflow) return;
-    const int n_items = min(p.sp.plan.counters->n_items, p.sp.plan.max_items);
-    const int n_waves = gridDim.x * kWavesPerBlock;
-    for (int pos0 = (blockIdx.x * kWavesPerBlock + wave_id()) * kSrcItems;
-         pos0 < n_items; pos0 += n_waves * kSrcItems) {
-        const int n_here = min(kSrcItems, n_items - pos0);
-        const int4 my_rec = p.sp.plan.records[pos0 + min(lane, n_here - 1)];
-        EdgeWindow win[kSrcItems];
-        int n_edges[kSrcItems], tag[kSrcItems], item[kSrcItems];
-#pragma unroll
-        for (int j = 0; j < kSrcItems; j++) {
-            const int beg = __builtin_amdgcn_readlane(my_rec.x, j);
-            const int end = __builtin_amdgcn_readlane(my_rec.y, j);
-            item[j] = __builtin_amdgcn_readlane(my_rec.z, j);
-            tag[j] = __builtin_amdgcn_readlane(my_rec.w, j);
-            n_edges[j] = j < n_here ? end - beg : 0;
-            if (n_edges[j] > 0) load_window<W_EDGEHEAD>(win[j], p.sp, beg, end);
-        }
-#pragma unroll
-        for (int j = 0; j < kSrcItems; j++) {
-            if (n_edges[j] <= 0) continue;
-            const int row = tag[j] & 0x7fffffff;
-            SlotRow<LPH> acc;
-            slot_begin<LPH>(acc, p, row, true);
-            slot_window<LPH>(acc, p, win[j], 0, n_edges[j]);
-            const bool single = tag[j] < 0;
-            slot_end<LPH>(acc,
-                          single ? p.sp.out + (size_t)row * 256 : p.sp.partial + (size_t)item[j] * 256,
-                          single ? p.grad_k + (size_t)row * H : p.partial_k + (size_t)item[j] * H);
-        }
-    }
-}
+namespace yitu {
 
 template <int LPH, int KT, bool FULL>
 static int gat_src_launch_shape(const GatSrcParams &p, bool has_items, const float *grad_out,
@@ -1588,27 +1394,11 @@ static int gat_src_launch_shape(const GatSrcParams &p, bool has_items, const flo
     // enough workgroups to walk the item list once (a second turn would mix source bands)
     const int item_grid = (int)std::min<int64_t>(
         ceil_div(p.sp.plan.max_items, kWavesPerBlock * kSrcItems), 1 << 20);
-    // a head-mean gradient of F < 256 floats per row: the several-edges-per-load kernels
-    constexpr bool kSlots = FULL && KT == 1 && LPH < kWave;
-    bool slots = false;
-    if constexpr (kSlots) slots = p.head_mean != 0;
-    if constexpr (kSlots) {
-        if (slots) {
-            gat_slot_rows_kernel<LPH><<<row_grid, kBlock, 0, stream>>>(p);
-            YITU_LAUNCH_CHECK();
-            if (has_items) {
-                gat_slot_items_kernel<LPH><<<item_grid, kBlock, 0, stream>>>(p);
-                YITU_LAUNCH_CHECK();
-            }
-        }
-    }
-    if (!slots) {
-        gat_src_rows_kernel<LPH, KT, FULL><<<row_grid, kBlock, 0, stream>>>(p);
+    gat_src_rows_kernel<LPH, KT, FULL><<<row_grid, kBlock, 0, stream>>>(p);
+    YITU_LAUNCH_CHECK();
+    if (has_items) {
+        gat_src_items_kernel<LPH, KT, FULL><<<item_grid, kBlock, 0, stream>>>(p);
         YITU_LAUNCH_CHECK();
-        if (has_items) {
-            gat_src_items_kernel<LPH, KT, FULL><<<item_grid, kBlock, 0, stream>>>(p);
-            YITU_LAUNCH_CHECK();
-        }
     }
     if (!has_items) return 0;
     const int red_grid = (int)std::min<int64_t>(p.sp.plan.max_rows, 1 << 16);
@@ -2040,14 +1830,22 @@ YITU_API int yitu_gat_backward(float *grad_query, float *grad_key, float *grad_f
                             (lph & (lph - 1)) == 0 && n_dst > 0 && nnz > 0 && n_dst < INT32_MAX &&
                             n_src <= (1 << 24) && aligned16(features) && aligned16(grad_out) &&
                             aligned16(grad_features);
-    YITU_REQUIRE(!grad_out_is_head_mean || aligned16(attn), "attn must be 16-byte aligned");
-    YITU_REQUIRE(nnz == 0 || attn || (one_gather && out && aligned16(out)),
+    // When the caller's output was the mean over heads, its gradient is one row of F floats
+    // per destination and the pass gathers just that: any head width that is a multiple of 4
+    // where the forward output is given, otherwise (and for 16 or 32 heads) the shapes above.
+    const bool slots = grad_out_is_head_mean && gat_slots_shape(n_heads, n_features) && n_dst > 0 &&
+                       nnz > 0 && n_dst < INT32_MAX && n_src <= (1 << 24) && aligned16(features) &&
+                       aligned16(grad_out) && aligned16(grad_features) && out && aligned16(out);
+    const bool one_pass = slots || one_gather;
+    YITU_REQUIRE(nnz == 0 || attn || (one_pass && out && aligned16(out)),
                  "without attn the backward needs a one-pass shape and the forward output");
-    YITU_REQUIRE(!grad_out_is_head_mean || one_gather,
+    YITU_REQUIRE(!grad_out_is_head_mean || aligned16(attn), "attn must be 16-byte aligned");
+    YITU_REQUIRE(!grad_out_is_head_mean || one_pass,
                  "a head-mean gradient is taken by the one-pass shapes only (rows of 256, 512 or "
-                 "1024 floats, head width 32..256 a power of two); expand it to [n_dst, H, F] / H "
-                 "for other shapes");
-    if (one_gather) {
+                 "1024 floats, head width 32..256 a power of two; with the forward output also 1, 2, "
+                 "4 or 8 heads of a multiple of 4 up to 256); expand it to [n_dst, H, F] / H for "
+                 "other shapes");
+    if (one_pass) {
         GatSrcParams p{};
         p.sp.indptr = t_indptr;
         p.sp.indices = t_rows;
@@ -2104,7 +1902,8 @@ YITU_API int yitu_gat_backward(float *grad_query, float *grad_key, float *grad_f
         p.recompute = row_stats != nullptr;
         p.key = key;
         p.grad_k = grad_key;
-        rc = gat_src_launch<true>(p, has_items, grad_out, out, query, (int)n_dst, stream);
+        rc = slots ? gat_slots_run(p, has_items, grad_out, out, query, (int)n_dst, stream)
+                   : gat_src_launch<true>(p, has_items, grad_out, out, query, (int)n_dst, stream);
         if (rc) return rc;
         SpmmParams q{};
         q.indptr = indptr;
