@@ -337,6 +337,25 @@ int yitu_skinny_linear_backward(float *grad_x_device, int accumulate, float *gra
                                 size_t workspace_bytes, void *stream);
 
 /*
+ * Two skinny Linears that read the same x as one call: y_a [n, out_a] = x . w_a^T (+ bias_a),
+ * y_b [n, out_b] = x . w_b^T (+ bias_b), out_a + out_b as out_features above (out_b may be 0),
+ * every tensor of its own; and the backward, grad_x (+)= grad_y_a . w_a + grad_y_b . w_b.
+ * Bias arguments may be NULL. Workspace: yitu_skinny_linear_workspace_bytes(n, in_features,
+ * out_a + out_b).
+ */
+int yitu_skinny_pair(float *y_a_device, float *y_b_device, const float *x_device,
+                     const float *w_a_device, const float *w_b_device, const float *bias_a_device,
+                     const float *bias_b_device, int64_t n, int64_t in_features, int64_t out_a,
+                     int64_t out_b, void *stream);
+int yitu_skinny_pair_backward(float *grad_x_device, int accumulate, float *grad_w_a_device,
+                              float *grad_w_b_device, float *grad_bias_a_device,
+                              float *grad_bias_b_device, const float *x_device,
+                              const float *w_a_device, const float *w_b_device,
+                              const float *grad_y_a_device, const float *grad_y_b_device, int64_t n,
+                              int64_t in_features, int64_t out_a, int64_t out_b,
+                              void *workspace_device, size_t workspace_bytes, void *stream);
+
+/*
  * out[j] = sum_r x[r,j] for a row-major [n_rows, n_cols] fp32 matrix: the bias
  * gradient of a Linear layer, in two stages with a fixed order of additions and no
  * cleared accumulator, so the call can be recorded into a HIP graph and replayed.

@@ -7,7 +7,7 @@ from torch import nn
 
 import oracle
 from helpers import assert_close
-from yitu_amd import graph_ext
+from yitu_amd import _lib, graph_ext
 from yitu_amd.xgnn_h import bundle
 
 pytestmark = pytest.mark.gpu
@@ -513,3 +513,43 @@ def test_sgemm_many_rows_small_weight(dev, ms, n, k, tb):
                                              [b.to(dev) for b in bs])
         for c, b, y in zip(got, bs, lin):
             assert_close(y, c.cpu() + b, atol=1e-5 * max(1.0, k ** 0.5))
+
+
+@pytest.mark.parametrize("n,k,ja,jb", [(1, 4, 1, 1), (15, 20, 3, 2), (16, 64, 8, 8), (17, 60, 1, 3),
+                                       (1000, 128, 4, 4), (513, 100, 8, 8), (4099, 256, 8, 8),
+                                       (70, 132, 5, 0), (300, 512, 4, 4), (129, 260, 3, 5),
+                                       (200, 1024, 2, 2), (65, 1020, 1, 3)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_skinny_pair(dev, n, k, ja, jb, accumulate):
+    """Two Linears of a few outputs over one x against float64: outputs and every gradient,
+    at part-filled row tiles, column steps and output lanes."""
+    g = torch.Generator().manual_seed(n + k)
+    mk = lambda *s: torch.randn(*s, generator=g)
+    x, base = mk(n, k), mk(n, k)
+    ws, bs, gs = ([mk(j, k) for j in (ja, jb)], [mk(j) for j in (ja, jb)], [mk(n, j) for j in (ja, jb)])
+    d = lambda t: t.to(dev)
+    ys = [torch.empty(n, j, device=dev) for j in (ja, jb)]
+    p = lambda t: _lib.ptr(t if t.numel() else None)
+    stream = _lib.stream_ptr(dev)
+    c = _lib.c_i64
+    dx, dw, db = d(x), [d(w) for w in ws], [d(b) for b in bs]
+    lib = _lib.lib()
+    _lib.check(lib.yitu_skinny_pair(p(ys[0]), p(ys[1]), p(dx), p(dw[0]), p(dw[1]), p(db[0]), p(db[1]),
+                                    c(n), c(k), c(ja), c(jb), stream), "yitu_skinny_pair")
+    for y, w, b in zip(ys, ws, bs):
+        assert_close(y.cpu(), (x.double() @ w.double().t() + b).float(), atol=2e-5 * k ** 0.5)
+    gx = d(base).clone()
+    gw = [torch.empty(j, k, device=dev) for j in (ja, jb)]
+    gb = [torch.empty(j, device=dev) for j in (ja, jb)]
+    dg = [d(t) for t in gs]
+    size = _lib.size_fn("yitu_skinny_linear_workspace_bytes")(c(n), c(k), c(ja + jb))
+    work = torch.empty(size, dtype=torch.uint8, device=dev)
+    _lib.check(lib.yitu_skinny_pair_backward(
+        p(gx), int(accumulate), p(gw[0]), p(gw[1]), p(gb[0]), p(gb[1]), p(dx), p(dw[0]), p(dw[1]),
+        p(dg[0]), p(dg[1]), c(n), c(k), c(ja), c(jb), p(work), _lib.c_size(size), stream),
+        "yitu_skinny_pair_backward")
+    want = sum(t.double() @ w.double() for t, w in zip(gs, ws))
+    assert_close(gx.cpu(), (want + (base.double() if accumulate else 0)).float(), atol=1e-4)
+    for t, a, b in zip(gs, gw, gb):
+        assert_close(a.cpu(), (t.double().t() @ x.double()).float(), atol=2e-5 * n ** 0.5 + 1e-5)
+        assert_close(b.cpu(), t.double().sum(0).float(), atol=2e-5 * n ** 0.5 + 1e-5)

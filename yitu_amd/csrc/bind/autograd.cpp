@@ -61,6 +61,7 @@ variable_list once(variable_list grads) {
 Tensor dense(const Tensor &t) { return t.is_contiguous() ? t : t.contiguous(); }
 OptTensor dense(const OptTensor &t) { return has(t) ? OptTensor(dense(*t)) : std::nullopt; }
 Tensor grad_or_none(const OptTensor &t) { return has(t) ? *t : Tensor(); }
+OptTensor given(const Tensor &t) { return t.defined() ? OptTensor(dense(t)) : std::nullopt; }
 
 // ---- GCN / GIN over the reference's module-1 ops -----------------------------------------
 Tensor aggregate(const Kept &k, const Tensor &x) {
@@ -136,13 +137,33 @@ struct SkinnyLinearFunction : Function<SkinnyLinearFunction> {
                           const OptTensor &bias) {
         ctx->save_for_backward({x, w});
         ctx->saved_data["bias"] = has(bias);
-        return skinny_linear(x, w, dense(bias));
+        return skinny_pair(x, w, std::nullopt, dense(bias), std::nullopt).first;
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const auto saved = ctx->get_saved_variables();
-        auto [dx, dw, db] = skinny_linear_backward(saved[0], saved[1], dense(grads[0]), std::nullopt,
-                                                   ctx->saved_data["bias"].toBool());
-        return once({dx, dw, grad_or_none(db)});
+        const SkinnyGrads g =
+            skinny_pair_backward(saved[0], saved[1], std::nullopt, dense(grads[0]), std::nullopt,
+                                 std::nullopt, ctx->saved_data["bias"].toBool(), false);
+        return once({g.x, g.w_a, grad_or_none(g.bias_a)});
+    }
+};
+
+// Two skinny Linears over one x; an undefined bias is one that is not there.
+struct SkinnyPairFunction : Function<SkinnyPairFunction> {
+    static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &w_a,
+                                 const Tensor &w_b, const Tensor &b_a, const Tensor &b_b) {
+        ctx->save_for_backward({x, w_a, w_b});
+        ctx->saved_data["bias_a"] = b_a.defined();
+        ctx->saved_data["bias_b"] = b_b.defined();
+        auto [y_a, y_b] = skinny_pair(x, w_a, w_b, given(b_a), given(b_b));
+        return {y_a, *y_b};
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const auto s = ctx->get_saved_variables();
+        const SkinnyGrads g = skinny_pair_backward(
+            s[0], s[1], s[2], dense(grads[0]), dense(grads[1]), std::nullopt,
+            ctx->saved_data["bias_a"].toBool(), ctx->saved_data["bias_b"].toBool());
+        return once({g.x, g.w_a, *g.w_b, grad_or_none(g.bias_a), grad_or_none(g.bias_b)});
     }
 };
 
@@ -168,8 +189,7 @@ struct LinearPairFunction : Function<LinearPairFunction> {
     static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &w_a,
                                  const Tensor &w_b, const Tensor &b_a, const Tensor &b_b) {
         ctx->save_for_backward({x, w_a, w_b});
-        const auto bias = [](const Tensor &b) { return b.defined() ? OptTensor(b) : std::nullopt; };
-        return linear_forward_typed({x, x}, {w_a, w_b}, {bias(b_a), bias(b_b)}, std::nullopt);
+        return linear_forward_typed({x, x}, {w_a, w_b}, {given(b_a), given(b_b)}, std::nullopt);
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const auto s = ctx->get_saved_variables();
@@ -356,6 +376,12 @@ struct SddmmFunction : Function<SddmmFunction> {
 };
 
 // ---- fused attention -----------------------------------------------------------------------
+// Whether the backward needs no more of the forward's softmax than its row statistics.
+bool stats_suffice(const Tensor &x, bool head_mean) {
+    return gat_one_pass_shape(x.size(1), x.size(2)) ||
+           (head_mean && gat_mean_shape(x));
+}
+
 struct FusedGatFunction : Function<FusedGatFunction> {
     static Tensor forward(AutogradContext *ctx, const Tensor &query, const Tensor &key,
                           const Tensor &x, bool head_mean, KeptPtr k) {
@@ -376,12 +402,6 @@ struct FusedGatFunction : Function<FusedGatFunction> {
                                         dense(grads[0]), s[4], k->flag2, stats, k->rows(),
                                         by_source(k->indptr, k->indices, k->n_src));
         return {g.query, g.key, g.x, Tensor(), Tensor()};
-// Whether the backward needs no more of the forward's softmax than its row statistics.
-bool stats_suffice(const Tensor &x, bool head_mean) {
-    return gat_one_pass_shape(x.size(1), x.size(2)) ||
-           (head_mean && gat_mean_shape(x));
-}
-
     }
 };
 
@@ -425,6 +445,54 @@ struct GatHeadsFunction : Function<GatHeadsFunction> {
     }
 };
 
+// The attention layer whose logit terms are Linears of the projected features (reference
+// test/common/model.py:61-106) as one node: h = x W_v^T + b_v, q = h W_q^T + b_q,
+// k = h W_k^T + b_k, attention, mean over heads. As separate nodes the two gradients of h met
+// in an addition pass over [n, H F], beside concatenations and copies of the two projections
+// (140 us of elementwise passes at 2^18 nodes x 4 x 64); here the projections' backward adds
+// to the attention's gradient in place.
+struct GatLayerFunction : Function<GatLayerFunction> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, const Tensor &w_v, const Tensor &b_v,
+                          const Tensor &w_q, const Tensor &b_q, const Tensor &w_k, const Tensor &b_k,
+                          KeptPtr k) {
+        const int64_t heads = w_q.size(0);
+        const Tensor h = linear_forward(x, w_v, given(b_v));
+        auto [q, key] = skinny_pair(h, w_q, w_k, given(b_q), given(b_k));
+        const Tensor h3 = h.view({h.size(0), heads, -1});
+        k->flag = stats_suffice(h3, true) && k->indices.numel() > 0;
+        const GatOut o = gat_forward(k->indptr, k->indices, q, *key, h3, k->flag, k->rows());
+        ctx->save_for_backward({x, w_v, w_q, w_k, h, q, *key, k->flag ? *o.stats : *o.attn, o.out});
+        ctx->saved_data["bias_v"] = b_v.defined();
+        ctx->saved_data["bias_q"] = b_q.defined();
+        ctx->saved_data["bias_k"] = b_k.defined();
+        keep(ctx, k);
+        return o.out.mean(1);
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const auto s = ctx->get_saved_variables();
+        const auto k = kept(ctx);
+        const OptTensor attn = k->flag ? std::nullopt : OptTensor(s[7]);
+        const OptTensor stats = k->flag ? OptTensor(s[7]) : std::nullopt;
+        const Tensor &h = s[4];
+        const GatGrads g = gat_backward(k->indptr, k->indices, s[5], s[6],
+                                        h.view({h.size(0), s[2].size(0), -1}), attn, dense(grads[0]),
+                                        s[8], true, stats, k->rows(),
+                                        by_source(k->indptr, k->indices, k->n_src));
+        const SkinnyGrads p = skinny_pair_backward(
+            h, s[2], s[3], g.query, g.key, g.x.view(h.sizes()), ctx->saved_data["bias_q"].toBool(),
+            ctx->saved_data["bias_k"].toBool());
+        const bool bias_v = ctx->saved_data["bias_v"].toBool();
+        TensorVec dws;
+        std::vector<OptTensor> dbs{std::nullopt};
+        if (ctx->needs_input_grad(1)) linear_weight_grad({p.x}, {s[0]}, {bias_v}, &dws, &dbs);
+        else if (bias_v) dbs[0] = column_sum(p.x);
+        Tensor dx;
+        if (ctx->needs_input_grad(0)) dx = sgemm(p.x, s[1], false, false, std::nullopt);
+        return once({dx, dws.empty() ? Tensor() : dws[0], grad_or_none(dbs[0]), p.w_a,
+                     grad_or_none(p.bias_a), *p.w_b, grad_or_none(p.bias_b), Tensor()});
+    }
+};
+
 }  // namespace
 
 void bind_autograd(py::module_ &m) {
@@ -463,6 +531,11 @@ void bind_autograd(py::module_ &m) {
                             const OptTensor &b_b) {
         return LinearPairFunction::apply(x, w_a, w_b, grad_or_none(b_a), grad_or_none(b_b));
     });
+    m.def("skinny_pair", [](const Tensor &x, const Tensor &w_a, const Tensor &w_b, const OptTensor &b_a,
+                            const OptTensor &b_b) {
+        return SkinnyPairFunction::apply(dense(x), dense(w_a), dense(w_b), grad_or_none(b_a),
+                                         grad_or_none(b_b));
+    });
     m.def("typed_linear", &typed_linear);
     m.def("gspmm", [](const Tensor &ip, const Tensor &ix, const Tensor &values, const Tensor &x) {
         return SpmmFunction::apply(values, x, graph_of(ip, ix, x.size(0)));
@@ -479,6 +552,21 @@ void bind_autograd(py::module_ &m) {
                           bool head_mean) {
         return GatHeadsFunction::apply(x_src, x_dst, a_src, a_dst, head_mean,
                                        graph_of(ip, ix, x_src.size(0)));
+    });
+    m.def("gat_layer", [](const Tensor &ip, const Tensor &ix, const Tensor &x, const Tensor &w_v,
+                          const OptTensor &b_v, const Tensor &w_q, const OptTensor &b_q,
+                          const Tensor &w_k, const OptTensor &b_k) -> OptTensor {
+        // shapes it does not take (the caller composes those): a projection too wide for the
+        // skinny product, values so narrow that they are one themselves, no rows
+        const bool takes = x.dim() == 2 && x.is_cuda() && x.size(0) > 0 &&
+                           x.scalar_type() == at::kFloat && w_v.scalar_type() == at::kFloat &&
+                           w_q.scalar_type() == at::kFloat && w_q.sizes() == w_k.sizes() &&
+                           skinny_linear_shape(w_q.size(1), 2 * w_q.size(0)) &&
+                           !skinny_linear_shape(w_v.size(1), w_v.size(0));
+        if (!takes) return std::nullopt;
+        return GatLayerFunction::apply(dense(x), dense(w_v), grad_or_none(b_v), dense(w_q),
+                                       grad_or_none(b_q), dense(w_k), grad_or_none(b_k),
+                                       graph_of(ip, ix, x.size(0)));
     });
 }
 

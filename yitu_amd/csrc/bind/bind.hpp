@@ -150,11 +150,17 @@ std::tuple<Tensor, Tensor, OptTensor> head_dot_backward(const Tensor &x, const T
                                                         const OptTensor &grad_b,
                                                         const OptTensor &grad_x);
 bool skinny_linear_shape(int64_t in_features, int64_t out_features);
-Tensor skinny_linear(const Tensor &x, const Tensor &w, const OptTensor &bias);
-std::tuple<Tensor, Tensor, OptTensor> skinny_linear_backward(const Tensor &x, const Tensor &w,
-                                                             const Tensor &grad_y,
-                                                             const OptTensor &grad_x,
-                                                             bool need_bias);
+// one Linear with a handful of outputs, or two over the same x (w_b given)
+std::pair<Tensor, OptTensor> skinny_pair(const Tensor &x, const Tensor &w_a, const OptTensor &w_b,
+                                         const OptTensor &bias_a, const OptTensor &bias_b);
+struct SkinnyGrads {
+    Tensor x, w_a;
+    OptTensor w_b, bias_a, bias_b;
+};
+SkinnyGrads skinny_pair_backward(const Tensor &x, const Tensor &w_a, const OptTensor &w_b,
+                                 const Tensor &grad_a, const OptTensor &grad_b,
+                                 const OptTensor &grad_x,  // given: added to in place
+                                 bool bias_a, bool bias_b);
 Tensor column_sum(const Tensor &x);
 TensorVec column_sum_typed(const TensorVec &xs);
 void bind_ops(py::module_ &m);

@@ -669,46 +669,63 @@ bool skinny_linear_shape(int64_t in_features, int64_t out_features) {
            out_features <= 16 && out_features * tiles <= 16;
 }
 
-Tensor skinny_linear(const Tensor &x, const Tensor &w, const OptTensor &bias) {
+std::pair<Tensor, OptTensor> skinny_pair(const Tensor &x, const Tensor &w_a, const OptTensor &w_b,
+                                         const OptTensor &bias_a, const OptTensor &bias_b) {
     check_f32(x, "x", 2);
-    check_f32(w, "weight", 2);
-    if (has(bias)) check_f32(*bias, "bias", 1);
-    same_device(x, w);
-    const int64_t n = x.size(0), k = x.size(1), j = w.size(0);
-    TORCH_CHECK(w.size(1) == k && (!has(bias) || bias->numel() == j),
+    check_f32(w_a, "weight", 2);
+    same_device(x, w_a);
+    const int64_t n = x.size(0), k = x.size(1), ja = w_a.size(0), jb = has(w_b) ? w_b->size(0) : 0;
+    if (has(w_b)) {
+        check_f32(*w_b, "weight", 2);
+        same_device(x, *w_b);
+    }
+    if (has(bias_a)) check_f32(*bias_a, "bias", 1);
+    if (has(bias_b)) check_f32(*bias_b, "bias", 1);
+    TORCH_CHECK(w_a.size(1) == k && (!has(w_b) || w_b->size(1) == k) &&
+                    (!has(bias_a) || bias_a->numel() == ja) && (!has(bias_b) || bias_b->numel() == jb),
                 "weight must be [out, in] and bias [out]");
     Call c(x);
-    Tensor y = c.empty({n, j});
-    ok(yitu_skinny_linear(f32(y), f32(x), f32(w), f32(bias), n, k, j, c.stream),
-       "yitu_skinny_linear");
-    return y;
+    Tensor y_a = c.empty({n, ja});
+    OptTensor y_b;
+    if (jb) y_b = c.empty({n, jb});
+    ok(yitu_skinny_pair(f32(y_a), f32(y_b), f32(x), f32(w_a), f32(w_b), f32(bias_a), f32(bias_b), n, k,
+                        ja, jb, c.stream),
+       "yitu_skinny_pair");
+    return {y_a, y_b};
 }
 
-std::tuple<Tensor, Tensor, OptTensor> skinny_linear_backward(const Tensor &x, const Tensor &w,
-                                                             const Tensor &grad_y,
-                                                             const OptTensor &grad_x,
-                                                             bool need_bias) {
+SkinnyGrads skinny_pair_backward(const Tensor &x, const Tensor &w_a, const OptTensor &w_b,
+                                 const Tensor &grad_a, const OptTensor &grad_b,
+                                 const OptTensor &grad_x, bool bias_a, bool bias_b) {
     check_f32(x, "x", 2);
-    check_f32(w, "weight", 2);
-    check_f32(grad_y, "grad_y", 2);
-    same_device(x, w, grad_y);
-    const int64_t n = x.size(0), k = x.size(1), j = w.size(0);
-    Call c(x);
-    Tensor gx;
+    check_f32(w_a, "weight", 2);
+    check_f32(grad_a, "grad_y", 2);
+    same_device(x, w_a, grad_a);
+    const int64_t n = x.size(0), k = x.size(1), ja = w_a.size(0), jb = has(w_b) ? w_b->size(0) : 0;
+    TORCH_CHECK(w_a.size(1) == k && grad_a.size(0) == n && grad_a.size(1) == ja,
+                "weight must be [out, in] and grad_y [n, out]");
+    if (jb) {
+        check_f32(*w_b, "weight", 2);
+        check_f32(*grad_b, "grad_y", 2);
+        same_device(x, *w_b, *grad_b);
+        TORCH_CHECK(w_b->size(1) == k && grad_b->size(0) == n && grad_b->size(1) == jb,
+                    "weight must be [out, in] and grad_y [n, out]");
+    }
     if (has(grad_x)) {
         check_f32(*grad_x, "grad_x", 2);
-        gx = *grad_x;
-    } else {
-        gx = c.empty({n, k});
+        TORCH_CHECK(grad_x->sizes() == x.sizes(), "grad_x must have the shape of x");
     }
-    Tensor gw = c.empty({j, k});
-    OptTensor gb;
-    if (need_bias) gb = c.empty({j});
-    Tensor ws = c.scratch(yitu_skinny_linear_workspace_bytes(n, k, j));
-    ok(yitu_skinny_linear_backward(f32(gx), has(grad_x), f32(gw), f32(gb), f32(x), f32(w),
-                                   f32(grad_y), n, k, j, ws.data_ptr(), ws.numel(), c.stream),
-       "yitu_skinny_linear_backward");
-    return {gx, gw, gb};
+    Call c(x);
+    SkinnyGrads g{has(grad_x) ? *grad_x : c.empty({n, k}), c.empty({ja, k})};
+    if (jb) g.w_b = c.empty({jb, k});
+    if (bias_a) g.bias_a = c.empty({ja});
+    if (jb && bias_b) g.bias_b = c.empty({jb});
+    Tensor ws = c.scratch(yitu_skinny_linear_workspace_bytes(n, k, ja + jb));
+    ok(yitu_skinny_pair_backward(f32(g.x), has(grad_x), f32(g.w_a), f32(g.w_b), f32(g.bias_a),
+                                 f32(g.bias_b), f32(x), f32(w_a), f32(w_b), f32(grad_a), f32(grad_b),
+                                 n, k, ja, jb, ws.data_ptr(), ws.numel(), c.stream),
+       "yitu_skinny_pair_backward");
+    return g;
 }
 
 Tensor column_sum(const Tensor &x) {
@@ -878,8 +895,15 @@ void bind_ops(py::module_ &m) {
     m.def("head_dot", &head_dot);
     m.def("head_dot_backward", &head_dot_backward);
     m.def("skinny_linear_shape", &skinny_linear_shape);
-    m.def("skinny_linear", &skinny_linear);
-    m.def("skinny_linear_backward", &skinny_linear_backward);
+    m.def("skinny_linear", [](const Tensor &x, const Tensor &w, const OptTensor &bias) {
+        return skinny_pair(x, w, std::nullopt, bias, std::nullopt).first;
+    });
+    m.def("skinny_linear_backward", [](const Tensor &x, const Tensor &w, const Tensor &grad_y,
+                                       const OptTensor &grad_x, bool need_bias) {
+        SkinnyGrads g = skinny_pair_backward(x, w, std::nullopt, grad_y, std::nullopt, grad_x,
+                                             need_bias, false);
+        return std::make_tuple(g.x, g.w_a, g.bias_a);
+    });
     m.def("column_sum", &column_sum);
     m.def("column_sum_typed", &column_sum_typed);
     m.def("coo_to_csr", &coo_to_csr);

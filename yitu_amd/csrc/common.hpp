@@ -197,6 +197,41 @@ __device__ __forceinline__ float dpp_permute(float v) {
     return __int_as_float(
         __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
 }
+// The value of the lane whose index differs in bit O alone (O = 1, 2, 4, 8).
+template <int O>
+__device__ __forceinline__ float lane_xor(float v) {
+    if constexpr (O == 1) return dpp_permute<0xb1>(v);       // quad_perm [1,0,3,2]
+    else if constexpr (O == 2) return dpp_permute<0x4e>(v);  // quad_perm [2,3,0,1]
+    else if constexpr (O == 4) return dpp_permute<0x1b>(dpp_permute<0x141>(v));  // xor 7, xor 3
+    else return dpp_permute<0x128>(v);                       // row_ror 8
+}
+// a[l] + a[l ^ O] in the lanes without bit O, b[l] + b[l ^ O] in those with it.
+template <int O>
+__device__ __forceinline__ float pair_sum(float a, float b) {
+    if constexpr (O == 32) return pair_sum32(a, b);
+    else if constexpr (O == 16) return pair_sum16(a, b);
+    else {
+        const bool upper = lane_id() & O;
+        return (upper ? b : a) + lane_xor<O>(upper ? a : b);
+    }
+}
+// Sums of V values over groups of LANES consecutive lanes, added as the butterfly over xor
+// LANES / 2, .., 2, 1 adds them; lane l of a group ends up with value l / (LANES / V) in v[0].
+template <int V, int O>
+__device__ __forceinline__ void group_sums(float (&v)[V]) {
+    if constexpr (O >= 1) {
+        if constexpr (V > 1) {
+            float half[V / 2];
+#pragma unroll
+            for (int i = 0; i < V / 2; i++) half[i] = pair_sum<O>(v[i], v[i + V / 2]);
+            group_sums<V / 2, O / 2>(half);
+            v[0] = half[0];
+        } else {
+            v[0] = pair_sum<O>(v[0], v[0]);
+            group_sums<1, O / 2>(v);
+        }
+    }
+}
 // Sum over aligned groups of WIDTH consecutive lanes, left in every lane of the group.
 // Up to 16 lanes: pairs, quads (quad permutes), halves of a row (mirror inside 8 lanes),
 // rows (mirror inside 16 lanes); beyond that, shuffles across rows. The order of the

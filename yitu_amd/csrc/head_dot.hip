@@ -323,93 +323,123 @@ YITU_API int yitu_head_dot_backward(float *grad_x, int accumulate, float *grad_v
 
 // ---- skinny Linear: y[n, J] = x[n, K] . w[J, K]^T (+ b), J small ---------------------
 // The dense query / key projections of the reference's GATLayer (H*F -> H Linears with
-// bias, test/common/model.py:70-71) have a handful of outputs per row: as GEMMs they
-// are one read of x each with a tile that is almost empty. Here a wave takes rows of
-// K floats (4 per lane and tile), the J weight rows sit in LDS, and each output is a
-// full-wave butterfly; two Linears that read the same x are one call with their
-// weights stacked. Backward: grad_x (+)= grad_y . w in place, grad_w and grad_b as
-// per-workgroup partial sums added in a fixed order.
+// bias, test/common/model.py:70-71) have a handful of outputs per row, one read of x each.
+// Two Linears that read the same x are one call: outputs [0, ja) are the first one's, the
+// others the second's, each with tensors of its own.
 namespace yitu {
 namespace {
 
 constexpr int kSkinnyMaxJ = 16;
 
 struct SkinnyParams {
-    const float *x, *w, *b;  // [n, K], [J, K], [J] or null
-    float *y;                // [n, J]
-    const float *gy;         // backward: [n, J]
-    float *grad_x;           // backward: [n, K]
-    float *partial;          // backward: [workgroups][J * K + J]
+    const float *x;                   // [n, K]
+    const float *w_a, *w_b;           // [ja, K], [J - ja, K]
+    const float *bias_a, *bias_b;     // or null
+    float *y_a, *y_b;                 // [n, ja], [n, J - ja]
+    const float *gy_a, *gy_b;         // backward: the same shapes
+    float *grad_x;                    // backward: [n, K]
+    float *partial;                   // backward: [workgroups][J * K + J]
     int accumulate;
-    int n, K, J;
+    int n, K, J, ja;
+    int w_vec;                        // both weights 16-byte aligned
+    __device__ __forceinline__ const float *weight(int j, int c) const {
+        return j < ja ? w_a + (size_t)j * K + c : w_b + (size_t)(j - ja) * K + c;
+    }
 };
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = kWave / 2; o >= 1; o >>= 1) v += __shfl_xor(v, o, kWave);
-    return v;
-}
-
-template <int KT>
+// LR lanes share a row (K / 4 rounded up to a power of two, KT tiles of 256 columns where
+// LR = 64), the weights stay in registers over all rows of the wave. The J sums of a row and
+// those of U rows are reduced together: each step of the butterfly halves the values a lane
+// holds instead of repeating itself per value (for 8 outputs of 4 rows 32 lane exchanges, not
+// 192 through LDS), in the same order of additions. Bound: one read of x, 46 us for
+// 2^18 x 256 -> 8 (5.8 TB/s), 19 us for 100,000 x 128 -> 8; a butterfly per output and row took
+// 151 and 61. Wide rows (KT > 1): two workgroups a CU, each reads its weights once.
+template <int LR, int KT, int JP>
 __global__ __launch_bounds__(kBlock) void skinny_linear_kernel(SkinnyParams p) {
-    extern __shared__ __align__(16) float w_lds[];  // [J][256 * KT]
-    constexpr int KP = 256 * KT;
-    for (int i = threadIdx.x; i < p.J * KP; i += kBlock) {
-        const int j = i / KP, c = i % KP;
-        w_lds[i] = c < p.K ? p.w[(size_t)j * p.K + c] : 0.0f;
-    }
-    __syncthreads();
-    const int lane = lane_id();
-    const int n_waves = gridDim.x * kWavesPerBlock;
-    const int wave = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-    for (int r0 = wave * kRowsInFlight; r0 < p.n; r0 += n_waves * kRowsInFlight) {
-        float x[kRowsInFlight][KT][4];
+    constexpr int RW = kWave / LR;                                // row slots of a wave
+    constexpr int U = LR / JP >= kRowsInFlight ? kRowsInFlight : LR / JP;  // rows summed together
+    constexpr int G = kRowsInFlight / U, V = JP * U;
+    const int lane = lane_id(), sub = lane % LR, slot = lane / LR;
+    const bool w_vec = p.w_vec;
+    float w[JP][KT][4];
 #pragma unroll
-        for (int u = 0; u < kRowsInFlight; u++) {
-            const int r = min(r0 + u, p.n - 1);
+    for (int j = 0; j < JP; j++)
+#pragma unroll
+        for (int t = 0; t < KT; t++) {
+            const int c = t * 256 + sub * 4;
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[j][t][i] = 0.0f;
+            if (j < p.J && c < p.K) {
+                if (w_vec) RowLoad<4, float>::ld(p.weight(j, c), w[j][t]);
+                else
+#pragma unroll
+                    for (int i = 0; i < 4; i++) w[j][t][i] = p.weight(j, c)[i];
+            }
+        }
+    // the value this lane ends up with: output j of the u-th row of a group
+    const int index = sub / (LR / V), j = index / U, u_mine = index % U;
+    const bool stores = sub % (LR / V) == 0 && j < p.J;
+    float *const y = j < p.ja ? p.y_a + j : p.y_b + (j - p.ja);
+    const int ld = j < p.ja ? p.ja : p.J - p.ja;
+    const float *const bias = j < p.ja ? p.bias_a : p.bias_b;
+    const float b = stores && bias ? bias[j < p.ja ? j : j - p.ja] : 0.0f;
+    constexpr int kTurn = G * U * RW;  // rows of a wave per turn
+    const int n_waves = gridDim.x * kWavesPerBlock;
+    for (int r0 = (blockIdx.x * kWavesPerBlock + wave_id()) * kTurn; r0 < p.n; r0 += n_waves * kTurn) {
+        float x[G * U][KT][4];
+#pragma unroll
+        for (int u = 0; u < G * U; u++) {
+            const int r = min(r0 + u * RW + slot, p.n - 1);
 #pragma unroll
             for (int t = 0; t < KT; t++) {
-                const int c = t * 256 + lane * 4;
+                const int c = t * 256 + sub * 4;
 #pragma unroll
                 for (int i = 0; i < 4; i++) x[u][t][i] = 0.0f;
                 if (c < p.K) RowLoad<4, float>::ld(p.x + (size_t)r * p.K + c, x[u][t]);
             }
         }
-        for (int j = 0; j < p.J; j++) {
-            float d[kRowsInFlight];
 #pragma unroll
-            for (int u = 0; u < kRowsInFlight; u++) d[u] = 0.0f;
+        for (int g = 0; g < G; g++) {
+            float d[V];
 #pragma unroll
-            for (int t = 0; t < KT; t++) {
-                const float4 w4 = *reinterpret_cast<const float4 *>(&w_lds[j * KP + t * 256 + lane * 4]);
+            for (int jj = 0; jj < JP; jj++)
 #pragma unroll
-                for (int u = 0; u < kRowsInFlight; u++)
-                    d[u] += x[u][t][0] * w4.x + x[u][t][1] * w4.y + x[u][t][2] * w4.z + x[u][t][3] * w4.w;
-            }
-            const float bj = p.b ? p.b[j] : 0.0f;
+                for (int u = 0; u < U; u++) {
+                    float s = 0.0f;
 #pragma unroll
-            for (int u = 0; u < kRowsInFlight; u++) {
-                const float s = wave_sum(d[u]);
-                if (lane == 0 && r0 + u < p.n) p.y[(size_t)(r0 + u) * p.J + j] = s + bj;
-            }
+                    for (int t = 0; t < KT; t++) {
+                        const float *xv = x[g * U + u][t], *wv = w[jj][t];
+                        s += xv[0] * wv[0] + xv[1] * wv[1] + xv[2] * wv[2] + xv[3] * wv[3];
+                    }
+                    d[jj * U + u] = s;
+                }
+            group_sums<V, LR / 2>(d);
+            const int r = r0 + (g * U + u_mine) * RW + slot;
+            if (stores && r < p.n) y[(size_t)r * ld] = d[0] + b;
         }
     }
 }
 
-// JT = outputs whose weight-gradient accumulators a lane keeps (J <= JT).
-template <int KT, int JT>
+// grad_x (+)= grad_y . w in place, grad_w and grad_b as per-workgroup partial sums. LR lanes
+// share a row (K / 4 rounded up to a power of two; KT tiles of 256 columns where LR = 64), a
+// wave takes 64 / LR rows at a time. JT = outputs whose weight-gradient accumulators a lane
+// keeps (J <= JT; the loops over them never leave early, or the arrays go to scratch memory:
+// 285 -> 42 us for 50,000 x 256 -> 16). Bound: HBM (x read, grad_x read and written), 157 us for
+// 2^18 x 256 -> 8, 33 us for 100,000 x 128 -> 8.
+template <int LR, int KT, int JT>
 __global__ __launch_bounds__(kBlock) void skinny_linear_bwd_kernel(SkinnyParams p) {
-    extern __shared__ __align__(16) float lds[];  // [J][256 * KT] weights, then the workgroup reduction
-    constexpr int KP = 256 * KT;
-    for (int i = threadIdx.x; i < p.J * KP; i += kBlock) {
-        const int j = i / KP, c = i % KP;
-        lds[i] = c < p.K ? p.w[(size_t)j * p.K + c] : 0.0f;
-    }
+    constexpr int KP = LR * 4 * KT;        // columns, padded
+    constexpr int RW = kWave / LR;         // rows of a wave
+    constexpr int PARTS = kWavesPerBlock * RW;
+    constexpr int kArea = 4096;            // floats: the weights (J * KP at most), then the sums
+    constexpr int JC = kArea / (PARTS * KP);  // outputs whose sums are combined at a time
+    static_assert(JC >= 1 && JT * KP <= kArea, "LDS area");
+    __shared__ __align__(16) float lds[kArea];
+    for (int i = threadIdx.x; i < p.J * KP; i += kBlock)
+        lds[i] = i % KP < p.K ? *p.weight(i / KP, i % KP) : 0.0f;
     __syncthreads();
-    const int lane = lane_id();
-    const int w_id = threadIdx.x / kWave;
-    const int n_waves = gridDim.x * kWavesPerBlock;
-    const int wave = blockIdx.x * kWavesPerBlock + w_id;
+    const int lane = lane_id(), sub = lane % LR, slot = lane / LR;
+    const int stride = gridDim.x * kWavesPerBlock * RW;
     float gw[JT][KT][4], gb[JT];
 #pragma unroll
     for (int j = 0; j < JT; j++) {
@@ -419,27 +449,33 @@ __global__ __launch_bounds__(kBlock) void skinny_linear_bwd_kernel(SkinnyParams 
 #pragma unroll
             for (int i = 0; i < 4; i++) gw[j][t][i] = 0.0f;
     }
-    for (int r = wave; r < p.n; r += n_waves) {
+    const int first = (blockIdx.x * kWavesPerBlock + wave_id()) * RW;
+    for (int r0 = first; r0 < p.n; r0 += stride) {
+        const int r = r0 + slot;
+        const bool there = r < p.n;
         float x[KT][4], out[KT][4];
 #pragma unroll
         for (int t = 0; t < KT; t++) {
-            const int c = t * 256 + lane * 4;
+            const int c = t * 256 + sub * 4;
 #pragma unroll
             for (int i = 0; i < 4; i++) x[t][i] = out[t][i] = 0.0f;
-            if (c < p.K) {
+            if (there && c < p.K) {
                 RowLoad<4, float>::ld(p.x + (size_t)r * p.K + c, x[t]);
                 if (p.accumulate) RowLoad<4, float>::ld(p.grad_x + (size_t)r * p.K + c, out[t]);
             }
         }
-        const float g_lane = lane < p.J ? p.gy[(size_t)r * p.J + lane] : 0.0f;
+        float g_lane = 0.0f;
+        if (there && sub < p.J)
+            g_lane = sub < p.ja ? p.gy_a[(size_t)r * p.ja + sub]
+                                : p.gy_b[(size_t)r * (p.J - p.ja) + sub - p.ja];
 #pragma unroll
         for (int j = 0; j < JT; j++) {
-            if (j >= p.J) break;
-            const float g = __shfl(g_lane, j, kWave);
+            if (j >= p.J) continue;
+            const float g = __shfl(g_lane, (lane - sub) + j, kWave);
             gb[j] += g;
 #pragma unroll
             for (int t = 0; t < KT; t++) {
-                const float4 w4 = *reinterpret_cast<const float4 *>(&lds[j * KP + t * 256 + lane * 4]);
+                const float4 w4 = *reinterpret_cast<const float4 *>(&lds[j * KP + t * 256 + sub * 4]);
                 out[t][0] += g * w4.x;
                 out[t][1] += g * w4.y;
                 out[t][2] += g * w4.z;
@@ -450,47 +486,57 @@ __global__ __launch_bounds__(kBlock) void skinny_linear_bwd_kernel(SkinnyParams 
         }
 #pragma unroll
         for (int t = 0; t < KT; t++) {
-            const int c = t * 256 + lane * 4;
-            if (c < p.K) store_row<4>(p.grad_x + (size_t)r * p.K + c, out[t]);
+            const int c = t * 256 + sub * 4;
+            if (there && c < p.K) store_row<4>(p.grad_x + (size_t)r * p.K + c, out[t]);
         }
     }
-    // workgroup partial: the four waves added in wave order, one output row at a time
+    // workgroup partial: the waves' row slots added in order, JC outputs at a time
     float *dst = p.partial + (size_t)blockIdx.x * (p.J * p.K + p.J);
-    for (int j = 0; j < p.J; j++) {
-        __syncthreads();  // the weights (first pass) or the previous row are no longer needed
+    const int part = wave_id() * RW + slot;
+    __shared__ float bias_part[PARTS][JT];
+    if (sub == 0)
 #pragma unroll
-        for (int jj = 0; jj < JT; jj++) {
-            if (jj != j) continue;
+        for (int j = 0; j < JT; j++) bias_part[part][j] = gb[j];
+#pragma unroll
+    for (int j0 = 0; j0 < JT; j0 += JC) {
+        if (j0 >= p.J) break;
+        __syncthreads();  // the weights (first pass) or the previous sums are no longer needed
+#pragma unroll
+        for (int jj = 0; jj < JC && j0 + jj < JT; jj++)
 #pragma unroll
             for (int t = 0; t < KT; t++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) lds[w_id * KP + t * 256 + lane * 4 + i] = gw[jj][t][i];
-            if (lane == 0) lds[kWavesPerBlock * KP + w_id] = gb[jj];
-        }
+                store_row<4>(&lds[(jj * PARTS + part) * KP + t * 256 + sub * 4], gw[j0 + jj][t]);
         __syncthreads();
-        for (int c = threadIdx.x; c < p.K; c += kBlock) {
+        for (int i = threadIdx.x; i < JC * KP; i += kBlock) {
+            const int jj = i / KP, c = i % KP;
+            if (j0 + jj >= p.J || c >= p.K) continue;
             float s = 0.0f;
 #pragma unroll
-            for (int q = 0; q < kWavesPerBlock; q++) s += lds[q * KP + c];
-            dst[(size_t)j * p.K + c] = s;
+            for (int q = 0; q < PARTS; q++) s += lds[(jj * PARTS + q) * KP + c];
+            dst[(size_t)(j0 + jj) * p.K + c] = s;
         }
-        if (threadIdx.x == 0) {
-            float s = 0.0f;
+    }
+    if ((int)threadIdx.x < p.J) {
+        float s = 0.0f;
 #pragma unroll
-            for (int q = 0; q < kWavesPerBlock; q++) s += lds[kWavesPerBlock * KP + q];
-            dst[(size_t)p.J * p.K + j] = s;
-        }
+        for (int q = 0; q < PARTS; q++) s += bias_part[q][threadIdx.x];
+        dst[(size_t)p.J * p.K + threadIdx.x] = s;
     }
 }
 
+// Up to four outputs side by side in a partial row: output i holds columns [end[i-1], end[i]).
+struct SumOutputs {
+    float *out[4];
+    int end[4];
+};
+
 // out[j] = sum over partial rows of partial[row][j], rows added by kSumGroups thread
 // groups and the group sums in order (the same scheme as head_dot_sum_kernel).
-__global__ __launch_bounds__(kBlock) void partial_sum_kernel(float *__restrict__ out_a, int n_a,
-                                                             float *__restrict__ out_b, int n_b,
+__global__ __launch_bounds__(kBlock) void partial_sum_kernel(SumOutputs o,
                                                              const float *__restrict__ partial,
                                                              int n_rows) {
     __shared__ float red[kSumGroups][kSumCols];
-    const int width = n_a + n_b;
+    const int width = o.end[3];
     const int c = threadIdx.x % kSumCols, g = threadIdx.x / kSumCols;
     const int j = blockIdx.x * kSumCols + c;
     float s = 0.0f;
@@ -503,10 +549,9 @@ __global__ __launch_bounds__(kBlock) void partial_sum_kernel(float *__restrict__
         float t = 0.0f;
 #pragma unroll
         for (int q = 0; q < kSumGroups; q++) t += red[q][c];
-        if (j < n_a)
-            out_a[j] = t;
-        else if (out_b)
-            out_b[j - n_a] = t;
+        int i = 0;
+        while (j >= o.end[i]) i++;
+        if (o.out[i]) o.out[i][j - (i ? o.end[i - 1] : 0)] = t;
     }
 }
 
@@ -521,17 +566,36 @@ int skinny_check(int64_t n, int64_t k, int64_t j) {
     return 0;
 }
 
-int skinny_bwd_grid(int64_t n) {
-    return (int)std::min<int64_t>(ceil_div(std::max<int64_t>(n, 1), kWavesPerBlock * 8), 1024);
+// A wave's rows are a chain of memory round trips: two of them on small inputs, so that the
+// chip is full first; four of the wide rows, whose partial sums (J * K a workgroup) would
+// otherwise be a good part of the traffic.
+int skinny_bwd_grid(int64_t n, int64_t k) {
+    const int64_t rows = kWavesPerBlock * (k <= 64 ? 8 : k <= 256 ? (k <= 128 ? 4 : 2) : 4);
+    return (int)std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, rows), 1024));
 }
 
-template <int KT>
-int skinny_bwd_launch(const SkinnyParams &p, int grid, size_t lds_bytes, hipStream_t stream) {
-    if (p.J <= 4) skinny_linear_bwd_kernel<KT, 4><<<grid, kBlock, lds_bytes, stream>>>(p);
+template <int LR, int KT>
+int skinny_launch(const SkinnyParams &p, hipStream_t stream) {
+    const int grid = (int)std::min<int64_t>(
+        ceil_div(p.n, kWavesPerBlock * kRowsInFlight * (kWave / LR)), KT == 1 ? 2048 : 512);
+    if (p.J <= 2) skinny_linear_kernel<LR, KT, 2><<<grid, kBlock, 0, stream>>>(p);
+    else if (p.J <= 4) skinny_linear_kernel<LR, KT, 4><<<grid, kBlock, 0, stream>>>(p);
     else if (p.J <= 8) {
-        if constexpr (KT <= 2) skinny_linear_bwd_kernel<KT, 8><<<grid, kBlock, lds_bytes, stream>>>(p);
+        if constexpr (KT <= 2) skinny_linear_kernel<LR, KT, 8><<<grid, kBlock, 0, stream>>>(p);
     } else {
-        if constexpr (KT == 1) skinny_linear_bwd_kernel<KT, 16><<<grid, kBlock, lds_bytes, stream>>>(p);
+        if constexpr (KT == 1) skinny_linear_kernel<LR, KT, 16><<<grid, kBlock, 0, stream>>>(p);
+    }
+    YITU_LAUNCH_CHECK();
+    return 0;
+}
+
+template <int LR, int KT>
+int skinny_bwd_launch(const SkinnyParams &p, int grid, hipStream_t stream) {
+    if (p.J <= 4) skinny_linear_bwd_kernel<LR, KT, 4><<<grid, kBlock, 0, stream>>>(p);
+    else if (p.J <= 8) {
+        if constexpr (KT <= 2) skinny_linear_bwd_kernel<LR, KT, 8><<<grid, kBlock, 0, stream>>>(p);
+    } else {
+        if constexpr (KT == 1) skinny_linear_bwd_kernel<LR, KT, 16><<<grid, kBlock, 0, stream>>>(p);
     }
     YITU_LAUNCH_CHECK();
     return 0;
@@ -540,78 +604,106 @@ int skinny_bwd_launch(const SkinnyParams &p, int grid, size_t lds_bytes, hipStre
 }  // namespace
 }  // namespace yitu
 
-YITU_API int yitu_skinny_linear(float *y, const float *x, const float *w, const float *bias,
-                                int64_t n, int64_t in_features, int64_t out_features,
-                                void *stream_) {
+YITU_API int yitu_skinny_pair(float *y_a, float *y_b, const float *x, const float *w_a,
+                              const float *w_b, const float *bias_a, const float *bias_b, int64_t n,
+                              int64_t in_features, int64_t out_a, int64_t out_b, void *stream_) {
     hipStream_t stream = static_cast<hipStream_t>(stream_);
-    if (int rc = skinny_check(n, in_features, out_features)) return rc;
+    if (int rc = skinny_check(n, in_features, out_a + out_b)) return rc;
     if (n == 0) return 0;
-    YITU_REQUIRE(y && x && w && aligned16(x), "null or misaligned pointer");
+    YITU_REQUIRE(out_a > 0 && out_b >= 0 && y_a && x && w_a && (out_b == 0 || (y_b && w_b)) &&
+                     aligned16(x), "null or misaligned pointer");
     SkinnyParams p{};
     p.x = x;
-    p.w = w;
-    p.b = bias;
-    p.y = y;
+    p.w_a = w_a;
+    p.w_b = w_b;
+    p.bias_a = bias_a;
+    p.bias_b = bias_b;
+    p.y_a = y_a;
+    p.y_b = y_b;
     p.n = (int)n;
     p.K = (int)in_features;
-    p.J = (int)out_features;
-    const int kt = (int)((in_features + 255) / 256);
-    const int grid = head_dot_grid(n);
-    switch (kt) {
-        case 1: skinny_linear_kernel<1><<<grid, kBlock, sizeof(float) * p.J * 256, stream>>>(p); break;
-        case 2: skinny_linear_kernel<2><<<grid, kBlock, sizeof(float) * p.J * 512, stream>>>(p); break;
-        default: skinny_linear_kernel<4><<<grid, kBlock, sizeof(float) * p.J * 1024, stream>>>(p);
-    }
-    YITU_LAUNCH_CHECK();
-    return 0;
+    p.J = (int)(out_a + out_b);
+    p.ja = (int)out_a;
+    p.w_vec = aligned16(w_a) && (out_b == 0 || aligned16(w_b));
+    if (in_features <= 64) return skinny_launch<16, 1>(p, stream);
+    if (in_features <= 128) return skinny_launch<32, 1>(p, stream);
+    if (in_features <= 256) return skinny_launch<64, 1>(p, stream);
+    if (in_features <= 512) return skinny_launch<64, 2>(p, stream);
+    return skinny_launch<64, 4>(p, stream);
+}
+
+YITU_API int yitu_skinny_linear(float *y, const float *x, const float *w, const float *bias,
+                                int64_t n, int64_t in_features, int64_t out_features,
+                                void *stream) {
+    return yitu_skinny_pair(y, nullptr, x, w, nullptr, bias, nullptr, n, in_features, out_features,
+                            0, stream);
 }
 
 YITU_API size_t yitu_skinny_linear_workspace_bytes(int64_t n, int64_t in_features,
                                                    int64_t out_features) {
     return sizeof(float) * (size_t)(out_features * in_features + out_features) *
-           (size_t)skinny_bwd_grid(n);
+           (size_t)skinny_bwd_grid(n, in_features);
+}
+
+YITU_API int yitu_skinny_pair_backward(float *grad_x, int accumulate, float *grad_w_a,
+                                       float *grad_w_b, float *grad_bias_a, float *grad_bias_b,
+                                       const float *x, const float *w_a, const float *w_b,
+                                       const float *grad_y_a, const float *grad_y_b, int64_t n,
+                                       int64_t in_features, int64_t out_a, int64_t out_b,
+                                       void *workspace, size_t workspace_bytes, void *stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    const int64_t k = in_features, j = out_a + out_b;
+    if (int rc = skinny_check(n, k, j)) return rc;
+    YITU_REQUIRE(out_a > 0 && out_b >= 0 && grad_w_a && (out_b == 0 || grad_w_b) &&
+                     (n == 0 || (grad_x && x && w_a && grad_y_a && (out_b == 0 || (w_b && grad_y_b)))),
+                 "null pointer");
+    YITU_REQUIRE(aligned16(x) && aligned16(grad_x), "pointers must be 16-byte aligned");
+    if (n == 0) {
+        int rc = fill_zero(grad_w_a, out_a * k, stream);
+        if (!rc && out_b) rc = fill_zero(grad_w_b, out_b * k, stream);
+        if (!rc && grad_bias_a) rc = fill_zero(grad_bias_a, out_a, stream);
+        if (!rc && grad_bias_b) rc = fill_zero(grad_bias_b, out_b, stream);
+        return rc;
+    }
+    YITU_REQUIRE(workspace && workspace_bytes >= yitu_skinny_linear_workspace_bytes(n, k, j),
+                 "workspace too small: need %zu bytes", yitu_skinny_linear_workspace_bytes(n, k, j));
+    SkinnyParams p{};
+    p.x = x;
+    p.w_a = w_a;
+    p.w_b = w_b;
+    p.gy_a = grad_y_a;
+    p.gy_b = grad_y_b;
+    p.grad_x = grad_x;
+    p.partial = static_cast<float *>(workspace);
+    p.accumulate = accumulate;
+    p.n = (int)n;
+    p.K = (int)k;
+    p.J = (int)j;
+    p.ja = (int)out_a;
+    const int grid = skinny_bwd_grid(n, k);
+    int rc;
+    if (k <= 64) rc = skinny_bwd_launch<16, 1>(p, grid, stream);
+    else if (k <= 128) rc = skinny_bwd_launch<32, 1>(p, grid, stream);
+    else if (k <= 256) rc = skinny_bwd_launch<64, 1>(p, grid, stream);
+    else if (k <= 512) rc = skinny_bwd_launch<64, 2>(p, grid, stream);
+    else rc = skinny_bwd_launch<64, 4>(p, grid, stream);
+    if (rc) return rc;
+    const int wa = (int)(out_a * k), wall = (int)(j * k);
+    const SumOutputs o{{grad_w_a, grad_w_b, grad_bias_a, grad_bias_b},
+                       {wa, wall, wall + (int)out_a, wall + (int)j}};
+    partial_sum_kernel<<<(int)ceil_div(wall + j, kSumCols), kBlock, 0, stream>>>(o, p.partial, grid);
+    YITU_LAUNCH_CHECK();
+    return 0;
 }
 
 YITU_API int yitu_skinny_linear_backward(float *grad_x, int accumulate, float *grad_w,
                                          float *grad_bias, const float *x, const float *w,
                                          const float *grad_y, int64_t n, int64_t in_features,
                                          int64_t out_features, void *workspace,
-                                         size_t workspace_bytes, void *stream_) {
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
-    if (int rc = skinny_check(n, in_features, out_features)) return rc;
-    YITU_REQUIRE(grad_x && grad_w && x && w && grad_y && aligned16(x) && aligned16(grad_x),
-                 "null or misaligned pointer");
-    YITU_REQUIRE(workspace && aligned16(workspace) &&
-                     workspace_bytes >= yitu_skinny_linear_workspace_bytes(n, in_features, out_features),
-                 "workspace too small: need %zu bytes",
-                 yitu_skinny_linear_workspace_bytes(n, in_features, out_features));
-    SkinnyParams p{};
-    p.x = x;
-    p.w = w;
-    p.gy = grad_y;
-    p.grad_x = grad_x;
-    p.partial = static_cast<float *>(workspace);
-    p.accumulate = accumulate;
-    p.n = (int)n;
-    p.K = (int)in_features;
-    p.J = (int)out_features;
-    const int kt = (int)((in_features + 255) / 256);
-    const int grid = skinny_bwd_grid(n);
-    // LDS: the weights, later per-wave rows of one output plus the four bias sums
-    const size_t kp = 256 * (kt == 3 ? 4 : kt);
-    const size_t lds_bytes = sizeof(float) * std::max<size_t>(p.J * kp, kWavesPerBlock * kp + kWavesPerBlock);
-    int rc;
-    switch (kt) {
-        case 1: rc = skinny_bwd_launch<1>(p, grid, lds_bytes, stream); break;
-        case 2: rc = skinny_bwd_launch<2>(p, grid, lds_bytes, stream); break;
-        default: rc = skinny_bwd_launch<4>(p, grid, lds_bytes, stream);
-    }
-    if (rc) return rc;
-    const int width = p.J * p.K + p.J;
-    partial_sum_kernel<<<(int)ceil_div(width, kSumCols), kBlock, 0, stream>>>(
-        grad_w, p.J * p.K, grad_bias, p.J, p.partial, grid);
-    YITU_LAUNCH_CHECK();
-    return 0;
+                                         size_t workspace_bytes, void *stream) {
+    return yitu_skinny_pair_backward(grad_x, accumulate, grad_w, nullptr, grad_bias, nullptr, x, w,
+                                     nullptr, grad_y, nullptr, n, in_features, out_features, 0,
+                                     workspace, workspace_bytes, stream);
 }
 
 // ---- column sums: out[j] = sum_r x[r, j] -----------------------------------------------
@@ -778,8 +870,9 @@ YITU_API int yitu_column_sum(float *out, const float *x, int64_t n_rows, int64_t
         column_chunk_sum_kernel<<<chunks, kBlock, 0, stream>>>(partial, x, (int)n_rows,
                                                                (int)n_cols, chunk);
     YITU_LAUNCH_CHECK();
+    const int width = (int)n_cols;
     partial_sum_kernel<<<(int)ceil_div(n_cols, kSumCols), kBlock, 0, stream>>>(
-        out, (int)n_cols, nullptr, 0, partial, chunks);
+        SumOutputs{{out, nullptr, nullptr, nullptr}, {width, width, width, width}}, partial, chunks);
     YITU_LAUNCH_CHECK();
     return 0;
 }

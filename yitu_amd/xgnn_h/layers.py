@@ -54,6 +54,12 @@ class GATLayer(nn.Module):
         self.leaky_relu = nn.LeakyReLU(negative_slope=0.2)
 
     def forward(self, blk: block.Block, x):
+        if self.fused and isinstance(x, torch.Tensor):
+            out = _lib.ops().gat_layer(*blk.adj_sparse, x, self.linear_v.weight, self.linear_v.bias,
+                                       self.linear_q.weight, self.linear_q.bias,
+                                       self.linear_k.weight, self.linear_k.bias)
+            if out is not None:
+                return out
         if isinstance(x, (list, tuple)):
             assert len(x) == 2
             h_src = bundle.linear(x[0], self.linear_v.weight, self.linear_v.bias)
