@@ -794,6 +794,33 @@ int yitu_csr_transpose(int32_t *t_indptr_device, int32_t *t_rows_device, int32_t
                        int64_t n_cols, int64_t nnz, int32_t col_mask, void *workspace_device,
                        size_t workspace_bytes, void *stream);
 
+/*
+ * Sums of row ranges of one matrix: out[range r, row i] = act((sum_k x[source_k + i]) / divisor),
+ * out [n_rows, width], x [.., width], both contiguous. What a heterogeneous layer does behind
+ * its products (sum over the relations of a node type, mean, activation;
+ * test/common/model.py:137-171, 198-236) for all node types in one launch. ranges tile the rows
+ * of out in ascending order; sources holds the first row of x of every source of every range.
+ * The backward writes grad_x at every source row; rows of x that are nobody's source are not
+ * written. The caller vouches for the two device tables (they are read unchecked).
+ */
+enum { YITU_FOLD_NONE = 0, YITU_FOLD_RELU = 1, YITU_FOLD_ELU = 2 };
+typedef struct {
+    int32_t out_begin;    /* first row of the range in out */
+    int32_t rows;
+    int32_t first_source; /* index into sources */
+    int32_t n_sources;    /* 0: the rows are zero */
+    float divisor;
+    int32_t act;          /* YITU_FOLD_* */
+    float alpha;          /* of the ELU */
+    int32_t pad;
+} YituFoldRange;
+int yitu_fold_rows(float *out, const float *x, const YituFoldRange *ranges_device,
+                   const int32_t *sources_device, int64_t n_ranges, int64_t n_rows, int64_t width,
+                   void *stream);
+int yitu_fold_rows_backward(float *grad_x, const float *grad_out, const float *out,
+                            const YituFoldRange *ranges_device, const int32_t *sources_device,
+                            int64_t n_ranges, int64_t n_rows, int64_t width, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,124 @@
+"""The batched form of a heterogeneous dataflow: its row-range ops against plain torch, and
+whole models against the executor that runs one relation at a time."""
+import pytest
+import torch
+
+import pipeline_cases as cases
+from helpers import assert_close
+from yitu_amd import _lib, xgnn_h
+from yitu_amd.xgnn_h import ir, models
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("width", [1, 3, 4, 20, 64])
+def test_fold_of_row_ranges(dev, width):
+    g = torch.Generator().manual_seed(width)
+    x = torch.randn(70, width, generator=g).to(dev).requires_grad_()
+    # rows, sources, divisor, act, alpha: an empty range, one without sources, rows 45..49 unread
+    ranges = [(5, [0, 30], 2.0, 0, 0.0), (0, [7], 1.0, 1, 0.0), (3, [], 1.0, 0, 0.0),
+              (20, [50], 3.0, 1, 0.0), (10, [5, 15, 35], 1.0, 2, 0.7), (4, [25], 1.0, 2, 1.0)]
+    plan = _lib.ops().fold_plan(70, ranges, x)
+    out = _lib.ops().fold_rows(x, plan)
+    want = []
+    for rows, sources, div, act, alpha in ranges:
+        v = sum((x[s:s + rows] for s in sources), torch.zeros(rows, width, device=dev)) / div
+        want.append(v.relu() if act == 1 else torch.nn.functional.elu(v, alpha) if act == 2 else v)
+    want = torch.cat(want)
+    assert_close(out, want)
+    dy = torch.randn(want.shape, generator=g).to(dev)
+    assert_close(torch.autograd.grad(out, x, dy)[0], torch.autograd.grad(want, x, dy)[0])
+
+
+def test_fold_plan_refuses_ranges_outside_or_twice(dev):
+    x = torch.zeros(10, 4, device=dev)
+    with pytest.raises(RuntimeError):
+        _lib.ops().fold_plan(10, [(4, [7], 1.0, 0, 0.0)], x)
+    with pytest.raises(RuntimeError):
+        _lib.ops().fold_plan(10, [(4, [0], 1.0, 0, 0.0), (4, [3], 1.0, 0, 0.0)], x)
+    with pytest.raises(RuntimeError):
+        _lib.ops().fold_rows(x, _lib.ops().fold_plan(9, [(9, [0], 1.0, 0, 0.0)], x))
+
+
+@pytest.mark.parametrize("k,n", [(5, 3), (16, 32), (33, 17)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_linear_over_row_ranges(dev, k, n, bias):
+    """Rows read twice, not at all and in part, from two matrices."""
+    g = torch.Generator().manual_seed(k)
+    t = lambda *s: torch.randn(*s, generator=g).to(dev).requires_grad_()  # noqa: E731
+    a, b = t(40, k), t(9, k)
+    units = [(0, 0, 25), (1, 0, 9), (0, 20, 15), (0, 20, 1), (1, 0, 9)]
+    ws, bs = [t(n, k) for _ in units], [t(n) for _ in units] if bias else []
+    plan = _lib.ops().linear_plan(units, [bias] * len(units), [40, 9], a)
+    y = _lib.ops().linear_rows([a, b], ws, bs, plan)
+    want = torch.cat([(a, b)[m][o:o + r] @ w.t() + (bs[i] if bias else 0.0)
+                      for i, ((m, o, r), w) in enumerate(zip(units, ws))])
+    assert_close(y, want)
+    dy = torch.randn(want.shape, generator=g).to(dev)
+    leaves = [a, b, *ws, *bs]
+    for got, ref in zip(torch.autograd.grad(y, leaves, dy), torch.autograd.grad(want, leaves, dy)):
+        assert_close(got, ref, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("which", ["rgcn", "rgat"])
+@pytest.mark.parametrize("stitch", [False, True])
+@pytest.mark.parametrize("relations", [7, 3])  # several and single relations per type
+def test_batched_model_equals_one_relation_at_a_time(dev, which, stitch, relations):
+    torch.manual_seed(5)
+    hgraph = cases.hetero_graph(device=dev)
+    if relations == 3:
+        kept = [("paper", "written_by", "author"), ("author", "writes", "paper"),
+                ("paper", "appears_in", "venue")]
+        hgraph = cases.mp.HeteroGraph.from_blocks(
+            cases.NTYPES, {r: hgraph.hetero_graph[r].blk for r in kept}, device=dev)
+    kwargs = cases.hetero_kwargs(hgraph, device=dev, with_norms=which == "rgcn")
+    model = (models.RGCNModel(hgraph, 12, 16, 5) if which == "rgcn"
+             else models.RGATModel(hgraph, 12, 16, 8, n_heads=2)).to(dev)
+    flow = xgnn_h.Optimizer().lower(xgnn_h.Module2IR().transform(model, kwargs), kwargs)
+    if stitch:
+        flow = xgnn_h.Stitcher().transform(flow, kwargs)
+    batched = xgnn_h.batch.batch_rows(flow, kwargs)
+    ops = cases.ops_of(batched)
+    core = "spmm" if which == "rgcn" else "gat"
+    if stitch or relations == 3:
+        assert ops[core + "_rows"] == 2 and ops[core] == 0 and ops["linear"] == 0
+    params = list(model.parameters())
+    weights = {}
+    results = []
+    for flag in (False, True):
+        executor = xgnn_h.Executor(group_linears=flag)
+        executor.eval()
+        out = executor.run(flow, kwargs)
+        for i, (k, v) in enumerate(out.items()):
+            weights.setdefault(k, torch.randn_like(v))
+        results.append((out, torch.autograd.grad([out[k] for k in out], params,
+                                                 [weights[k] for k in out], allow_unused=True)))
+        if flag:  # a second pass, and one with other parameters, on the same plans
+            with torch.no_grad():
+                for p in params:
+                    p.mul_(1.1)
+            again = executor.run(flow, kwargs)
+            plain = xgnn_h.Executor(group_linears=False)
+            plain.eval()
+            for k, v in plain.run(flow, kwargs).items():
+                assert_close(again[k], v, rtol=1e-4, atol=1e-5)
+    (out_a, grads_a), (out_b, grads_b) = results
+    for k in out_a:
+        assert_close(out_b[k], out_a[k], rtol=1e-4, atol=1e-5)
+    for a, b in zip(grads_a, grads_b):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert_close(b, a, rtol=1e-4, atol=1e-5)
+
+
+def test_batched_model_in_training_mode_keeps_its_shapes(dev):
+    hgraph = cases.hetero_graph(device=dev)
+    kwargs = cases.hetero_kwargs(hgraph, device=dev)
+    model = models.RGCNModel(hgraph, 8, 8, 4).to(dev)
+    flow = xgnn_h.Module2IR().transform(model, kwargs)
+    executor = xgnn_h.Executor()
+    executor.train()  # dropout is drawn for the whole batch
+    out = executor.run(flow, kwargs)
+    assert {k: list(v.shape) for k, v in out.items()} == \
+        {k: [n, 4] for k, n in hgraph.nty2num.items()}
+    assert isinstance(flow, dict) and all(isinstance(n, ir.Node) for n in flow.values())

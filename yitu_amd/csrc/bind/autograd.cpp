@@ -1,67 +1,10 @@
 // The differentiable layers and ops as autograd nodes. Forward and backward run without the
 // interpreter (on a small graph it cost more than the kernels did); the sparse structure
 // takes no gradient, and a gradient that nobody asked for is not computed.
-#include <torch/csrc/autograd/custom_function.h>
-#include <torch/csrc/autograd/functions/basic_ops.h>
-
-#include "bind.hpp"
+#include "nodes.hpp"
 
 namespace yitu_bind {
 namespace {
-
-using torch::autograd::AutogradContext;
-using torch::autograd::Function;
-using torch::autograd::variable_list;
-
-// What a node keeps besides its saved tensors.
-struct Kept : torch::CustomClassHolder {
-    Tensor indptr, indices, degrees;
-    OptTensor edge_scale;
-    int64_t n_src = 0;
-    int mask = kColMask;
-    double alpha = 1.0;
-    bool flag = false, flag2 = false;
-    RowState rows() const { return row_state(indptr, indices, n_src, mask); }
-};
-using KeptPtr = c10::intrusive_ptr<Kept>;
-
-void keep(AutogradContext *ctx, const KeptPtr &k) {
-    ctx->saved_data["kept"] = c10::IValue::make_capsule(k);
-}
-KeptPtr kept(AutogradContext *ctx) {
-    return c10::static_intrusive_pointer_cast<Kept>(ctx->saved_data["kept"].toCapsule());
-}
-KeptPtr graph_of(const Tensor &indptr, const Tensor &indices, int64_t n_src) {
-    auto k = c10::make_intrusive<Kept>();
-    k->indptr = indptr;
-    k->indices = indices;
-    k->n_src = n_src;
-    return k;
-}
-
-// The gradients of ops whose backward is not differentiable itself: a second differentiation
-// raises instead of silently giving nothing.
-variable_list once(variable_list grads) {
-    if (!at::GradMode::is_enabled()) return grads;
-    std::vector<size_t> at;
-    variable_list live;
-    for (size_t i = 0; i < grads.size(); i++)
-        if (grads[i].defined()) {
-            at.push_back(i);
-            live.push_back(grads[i].detach().requires_grad_());
-        }
-    torch::autograd::DelayedError error(
-        "trying to differentiate twice a function that was marked with @once_differentiable",
-        (int64_t)live.size());
-    live = error(std::move(live));
-    for (size_t i = 0; i < at.size(); i++) grads[at[i]] = live[i];
-    return grads;
-}
-
-Tensor dense(const Tensor &t) { return t.is_contiguous() ? t : t.contiguous(); }
-OptTensor dense(const OptTensor &t) { return has(t) ? OptTensor(dense(*t)) : std::nullopt; }
-Tensor grad_or_none(const OptTensor &t) { return has(t) ? *t : Tensor(); }
-OptTensor given(const Tensor &t) { return t.defined() ? OptTensor(dense(t)) : std::nullopt; }
 
 // ---- GCN / GIN over the reference's module-1 ops -----------------------------------------
 Tensor aggregate(const Kept &k, const Tensor &x) {
@@ -376,17 +319,11 @@ struct SddmmFunction : Function<SddmmFunction> {
 };
 
 // ---- fused attention -----------------------------------------------------------------------
-// Whether the backward needs no more of the forward's softmax than its row statistics.
-bool stats_suffice(const Tensor &x, bool head_mean) {
-    return gat_one_pass_shape(x.size(1), x.size(2)) ||
-           (head_mean && gat_mean_shape(x));
-}
-
 struct FusedGatFunction : Function<FusedGatFunction> {
     static Tensor forward(AutogradContext *ctx, const Tensor &query, const Tensor &key,
                           const Tensor &x, bool head_mean, KeptPtr k) {
         // one-pass shapes: each row's softmax statistics are kept instead of the probabilities
-        k->flag = stats_suffice(x, head_mean) && k->indices.numel() > 0;
+        k->flag = gat_stats_suffice(x, head_mean) && k->indices.numel() > 0;
         k->flag2 = head_mean;
         const GatOut o = gat_forward(k->indptr, k->indices, query, key, x, k->flag, k->rows());
         ctx->save_for_backward({query, key, x, k->flag ? *o.stats : *o.attn, o.out});
@@ -417,7 +354,7 @@ struct GatHeadsFunction : Function<GatHeadsFunction> {
             query = both.first;
             key = *both.second;
         }
-        k->flag = stats_suffice(x_src, head_mean) && k->indices.numel() > 0;
+        k->flag = gat_stats_suffice(x_src, head_mean) && k->indices.numel() > 0;
         k->flag2 = head_mean;
         const GatOut o = gat_forward(k->indptr, k->indices, query, key, x_src, k->flag, k->rows());
         variable_list saved = {x_src, a_src, a_dst, query, key, k->flag ? *o.stats : *o.attn, o.out};
@@ -459,7 +396,7 @@ struct GatLayerFunction : Function<GatLayerFunction> {
         const Tensor h = linear_forward(x, w_v, given(b_v));
         auto [q, key] = skinny_pair(h, w_q, w_k, given(b_q), given(b_k));
         const Tensor h3 = h.view({h.size(0), heads, -1});
-        k->flag = stats_suffice(h3, true) && k->indices.numel() > 0;
+        k->flag = gat_stats_suffice(h3, true) && k->indices.numel() > 0;
         const GatOut o = gat_forward(k->indptr, k->indices, q, *key, h3, k->flag, k->rows());
         ctx->save_for_backward({x, w_v, w_q, w_k, h, q, *key, k->flag ? *o.stats : *o.attn, o.out});
         ctx->saved_data["bias_v"] = b_v.defined();
@@ -576,4 +513,5 @@ PYBIND11_MODULE(_ops, m) {
     yitu_bind::bind_graph_state(m);
     yitu_bind::bind_ops(m);
     yitu_bind::bind_autograd(m);
+    yitu_bind::bind_batched(m);
 }

@@ -1,0 +1,356 @@
+// The nodes of a heterogeneous model whose relations run together (yitu_amd/xgnn_h/batch.py):
+// every batched product writes the rows of all its members into one buffer, and what follows
+// reads row ranges of that buffer in place.
+#include "nodes.hpp"
+
+namespace yitu_bind {
+namespace {
+
+// Row ranges of one matrix summed into ranges of another (yitu_fold_rows). The table is
+// checked here against both row counts; the kernels read it as it is.
+struct FoldPlan : torch::CustomClassHolder {
+    struct Range {
+        int64_t rows;
+        std::vector<int64_t> sources;
+        double divisor;
+        int64_t act;
+        double alpha;
+    };
+    int64_t rows_in = 0, rows_out = 0, n_ranges = 0;
+    bool covers = true;  // every row of x is a source
+    Tensor ranges, sources;
+
+    FoldPlan(int64_t rows_in_, const std::vector<Range> &list, at::Device device)
+        : rows_in(rows_in_), n_ranges((int64_t)list.size()) {
+        std::vector<YituFoldRange> table;
+        std::vector<int32_t> from;
+        std::vector<std::pair<int64_t, int64_t>> used;
+        for (const Range &r : list) {
+            TORCH_CHECK(r.rows >= 0 && r.divisor != 0.0 && r.act >= YITU_FOLD_NONE &&
+                            r.act <= YITU_FOLD_ELU, "fold: bad range");
+            table.push_back({(int32_t)rows_out, (int32_t)r.rows, (int32_t)from.size(),
+                             (int32_t)r.sources.size(), (float)r.divisor, (int32_t)r.act,
+                             (float)r.alpha, 0});
+            rows_out += r.rows;
+            for (int64_t s : r.sources) {
+                TORCH_CHECK(s >= 0 && s + r.rows <= rows_in, "fold: source rows ", s, " to ",
+                            s + r.rows, " of ", rows_in);
+                from.push_back((int32_t)s);
+                used.emplace_back(s, r.rows);
+            }
+        }
+        TORCH_CHECK(!list.empty() && rows_in < INT32_MAX && rows_out < INT32_MAX, "fold: bad size");
+        std::sort(used.begin(), used.end());
+        int64_t at = 0;
+        for (const auto &[begin, rows] : used) {
+            TORCH_CHECK(rows == 0 || begin >= at, "fold: a row is the source of two ranges");
+            covers = covers && (rows == 0 || begin == at);
+            at = std::max(at, begin + rows);
+        }
+        covers = covers && at == rows_in;
+        const auto host = [&](const void *data, size_t words) {
+            Tensor t = torch::empty({std::max<int64_t>((int64_t)words, 1)}, at::kInt);
+            if (words) memcpy(t.data_ptr(), data, 4 * words);
+            return t.to(device);
+        };
+        ranges = host(table.data(), table.size() * sizeof(YituFoldRange) / 4);
+        sources = host(from.data(), from.size());
+    }
+    const YituFoldRange *table() const {
+        return reinterpret_cast<const YituFoldRange *>(ranges.data_ptr());
+    }
+};
+using FoldPlanPtr = c10::intrusive_ptr<FoldPlan>;
+
+Tensor fold(const Tensor &x, const FoldPlan &p) {
+    check_f32(x, "x", 2);
+    TORCH_CHECK(x.size(0) == p.rows_in, "fold: the plan is for ", p.rows_in, " rows, not ", x.size(0));
+    same_device(x, p.ranges);
+    Call c(x);
+    Tensor out = c.empty({p.rows_out, x.size(1)});
+    ok(yitu_fold_rows(f32(out), f32(x), p.table(), i32(p.sources), p.n_ranges, p.rows_out, x.size(1),
+                      c.stream),
+       "yitu_fold_rows");
+    return out;
+}
+
+// Rows of a result as a tensor of their own: the same memory, but for autograd no view of the
+// whole (the caller may write it in place, as any result).
+Tensor own_rows(const Tensor &t, int64_t first, int64_t rows) {
+    at::AutoDispatchBelowADInplaceOrView guard;
+    return t.narrow(0, first, rows);
+}
+
+Tensor fold_backward(const FoldPlan &p, const Tensor &out, const Tensor &g) {
+    Call c(g);
+    Tensor dx = c.empty({p.rows_in, out.size(1)});
+    if (!p.covers) dx.zero_();
+    ok(yitu_fold_rows_backward(f32(dx), f32(g), f32(out), p.table(), i32(p.sources), p.n_ranges,
+                               p.rows_out, out.size(1), c.stream),
+       "yitu_fold_rows_backward");
+    return dx;
+}
+
+struct FoldFunction : Function<FoldFunction> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x, FoldPlanPtr p) {
+        Tensor out = fold(x, *p);
+        ctx->save_for_backward({out});
+        ctx->saved_data["plan"] = c10::IValue::make_capsule(p);
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const auto p =
+            c10::static_intrusive_pointer_cast<FoldPlan>(ctx->saved_data["plan"].toCapsule());
+        return once({fold_backward(*p, ctx->get_saved_variables()[0], dense(grads[0])), Tensor()});
+    }
+};
+
+// The same with the result handed out as `sizes` rows each: the outputs of a model.
+struct FoldSplitFunction : Function<FoldSplitFunction> {
+    static variable_list forward(AutogradContext *ctx, const Tensor &x, FoldPlanPtr p,
+                                 std::vector<int64_t> sizes) {
+        const Tensor out = fold(x, *p);
+        variable_list parts;
+        int64_t at = 0;
+        for (int64_t n : sizes) {
+            parts.push_back(own_rows(out, at, n));
+            at += n;
+        }
+        TORCH_CHECK(at == p->rows_out, "fold: the parts do not add up");
+        variable_list saved = parts;  // a part that was written to is noticed
+        ctx->save_for_backward(std::move(saved));
+        ctx->saved_data["plan"] = c10::IValue::make_capsule(p);
+        ctx->saved_data["out"] = out;
+        return parts;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const auto p =
+            c10::static_intrusive_pointer_cast<FoldPlan>(ctx->saved_data["plan"].toCapsule());
+        const auto parts = ctx->get_saved_variables();
+        for (size_t i = 0; i < grads.size(); i++)
+            if (!grads[i].defined()) grads[i] = at::zeros_like(parts[i]);
+        const Tensor g = at::cat(grads);
+        return once({fold_backward(*p, ctx->saved_data["out"].toTensor(), g), Tensor(), Tensor()});
+    }
+};
+
+// Linears over row ranges of a few matrices: unit u reads rows [offset, offset + rows) of
+// matrix base, and writes the rows behind unit u - 1's in the result.
+struct LinearPlan : torch::CustomClassHolder {
+    struct Unit {
+        int64_t base, offset, rows;
+    };
+    std::vector<Unit> units;
+    std::vector<bool> has_bias;
+    std::vector<int64_t> base_rows;
+    int64_t total = 0;
+    // per-unit gradients [total, k] -> gradients of the bases, one below the other; null where
+    // the units are the bases in order
+    FoldPlanPtr fold;
+
+    LinearPlan(std::vector<Unit> units_, std::vector<bool> has_bias_, std::vector<int64_t> base_rows_,
+               at::Device device)
+        : units(std::move(units_)), has_bias(std::move(has_bias_)), base_rows(std::move(base_rows_)) {
+        TORCH_CHECK(!units.empty() && has_bias.size() == units.size(), "linear_rows: bad plan");
+        std::vector<int64_t> at;
+        for (const Unit &u : units) {
+            TORCH_CHECK(u.base >= 0 && u.base < (int64_t)base_rows.size() && u.offset >= 0 &&
+                            u.rows >= 0 && u.offset + u.rows <= base_rows[u.base],
+                        "linear_rows: unit outside its input");
+            at.push_back(total);
+            total += u.rows;
+        }
+        // each base cut where a unit begins or ends; the units over a piece are its sources
+        std::vector<FoldPlan::Range> ranges;
+        bool same = true;
+        int64_t begin = 0;
+        for (int64_t b = 0; b < (int64_t)base_rows.size(); b++) {
+            std::vector<int64_t> cuts{0, base_rows[b]};
+            for (const Unit &u : units)
+                if (u.base == b) {
+                    cuts.push_back(u.offset);
+                    cuts.push_back(u.offset + u.rows);
+                }
+            std::sort(cuts.begin(), cuts.end());
+            for (size_t i = 0; i + 1 < cuts.size(); i++) {
+                if (cuts[i] == cuts[i + 1]) continue;
+                FoldPlan::Range r{cuts[i + 1] - cuts[i], {}, 1.0, YITU_FOLD_NONE, 0.0};
+                for (size_t u = 0; u < units.size(); u++)
+                    if (units[u].base == b && units[u].offset <= cuts[i] &&
+                        units[u].offset + units[u].rows >= cuts[i + 1])
+                        r.sources.push_back(at[u] + cuts[i] - units[u].offset);
+                same = same && r.sources.size() == 1 && r.sources[0] == begin + cuts[i];
+                ranges.push_back(std::move(r));
+            }
+            begin += base_rows[b];
+        }
+        if (!(same && begin == total) && !ranges.empty())
+            fold = c10::make_intrusive<FoldPlan>(total, ranges, device);
+    }
+};
+using LinearPlanPtr = c10::intrusive_ptr<LinearPlan>;
+
+struct LinearRowsFunction : Function<LinearRowsFunction> {
+    static TensorVec inputs(const LinearPlan &p, const variable_list &bases) {
+        TensorVec xs;
+        for (const auto &u : p.units)
+            xs.push_back(u.rows == bases[u.base].size(0) ? bases[u.base]
+                                                         : bases[u.base].narrow(0, u.offset, u.rows));
+        return xs;
+    }
+    static TensorVec parts(const LinearPlan &p, const Tensor &t) {
+        TensorVec v;
+        int64_t at = 0;
+        for (const auto &u : p.units) {
+            v.push_back(t.narrow(0, at, u.rows));
+            at += u.rows;
+        }
+        return v;
+    }
+    static Tensor forward(AutogradContext *ctx, at::TensorList bases, at::TensorList ws,
+                          at::TensorList bs, LinearPlanPtr p) {
+        variable_list saved;
+        for (const Tensor &t : bases) saved.push_back(dense(t));
+        TensorVec weights;
+        for (const Tensor &t : ws) weights.push_back(dense(t));
+        std::vector<OptTensor> biases;
+        size_t b = 0;
+        for (bool there : p->has_bias)
+            biases.push_back(there ? OptTensor(dense(bs[b++])) : std::nullopt);
+        Tensor y = Call(bases[0]).empty({p->total, ws[0].size(0)});
+        linear_forward_typed(inputs(*p, saved), weights, biases, parts(*p, y));
+        saved.insert(saved.end(), weights.begin(), weights.end());
+        ctx->save_for_backward(std::move(saved));
+        ctx->saved_data["plan"] = c10::IValue::make_capsule(p);
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const auto p =
+            c10::static_intrusive_pointer_cast<LinearPlan>(ctx->saved_data["plan"].toCapsule());
+        const auto saved = ctx->get_saved_variables();
+        const size_t n_bases = p->base_rows.size(), n_units = p->units.size();
+        const variable_list bases(saved.begin(), saved.begin() + n_bases);
+        const TensorVec weights(saved.begin() + n_bases, saved.end());
+        const Tensor g = dense(grads[0]);
+        const TensorVec gs = parts(*p, g);
+        // one entry per argument: bases, weights, the biases that are there, the plan
+        size_t n_biases = 0;
+        for (bool there : p->has_bias) n_biases += there;
+        variable_list out(n_bases + n_units + n_biases + 1);
+        bool any = false;
+        for (size_t b = 0; b < n_bases; b++) any = any || ctx->needs_input_grad(b);
+        if (any) {
+            Tensor dx = Call(g).empty({p->total, weights[0].size(1)});
+            sgemm_typed(gs, weights, false, false, parts(*p, dx));
+            if (p->fold) dx = fold(dx, *p->fold);
+            int64_t at = 0;
+            for (size_t b = 0; b < n_bases; b++) {
+                if (ctx->needs_input_grad(b))
+                    out[b] = n_bases == 1 ? dx : own_rows(dx, at, p->base_rows[b]);
+                at += p->base_rows[b];
+            }
+        }
+        TensorVec want_g, want_x;
+        std::vector<bool> want_b;
+        std::vector<std::pair<size_t, size_t>> slot;  // of the weight and of its bias
+        const TensorVec xs = inputs(*p, bases);
+        size_t bias = n_bases + n_units;
+        for (size_t u = 0; u < n_units; u++) {
+            const size_t at = p->has_bias[u] ? bias++ : 0;
+            const bool b = at && ctx->needs_input_grad(at);
+            if (ctx->needs_input_grad(n_bases + u)) {
+                want_g.push_back(gs[u]);
+                want_x.push_back(xs[u]);
+                want_b.push_back(b);
+                slot.emplace_back(n_bases + u, at);
+            } else if (b) {
+                out[at] = column_sum(gs[u]);
+            }
+        }
+        if (!want_g.empty()) {
+            TensorVec dws;
+            std::vector<OptTensor> dbs;
+            linear_weight_grad(want_g, want_x, want_b, &dws, &dbs);
+            for (size_t i = 0; i < slot.size(); i++) {
+                out[slot[i].first] = dws[i];
+                if (want_b[i]) out[slot[i].second] = *dbs[i];
+            }
+        }
+        return once(std::move(out));
+    }
+};
+
+// Attention whose queries are a row range of the matrix that holds the keys (both projections
+// of all relations are one batched product).
+struct GatRowsFunction : Function<GatRowsFunction> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &qk, const Tensor &x, int64_t first,
+                          bool head_mean, KeptPtr k) {
+        const Tensor query = qk.narrow(0, first, k->indptr.numel() - 1);
+        k->flag = gat_stats_suffice(x, head_mean) && k->indices.numel() > 0;
+        k->flag2 = head_mean;
+        const GatOut o = gat_forward(k->indptr, k->indices, query, qk, x, k->flag, k->rows());
+        ctx->save_for_backward({qk, x, k->flag ? *o.stats : *o.attn, o.out});
+        ctx->saved_data["first"] = first;
+        keep(ctx, k);
+        return head_mean ? o.out.mean(1) : o.out;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const auto s = ctx->get_saved_variables();
+        const auto k = kept(ctx);
+        const int64_t first = ctx->saved_data["first"].toInt(), n_dst = k->indptr.numel() - 1;
+        const OptTensor attn = k->flag ? std::nullopt : OptTensor(s[2]);
+        const OptTensor stats = k->flag ? OptTensor(s[2]) : std::nullopt;
+        GatGrads g = gat_backward(k->indptr, k->indices, s[0].narrow(0, first, n_dst), s[0], s[1],
+                                  attn, dense(grads[0]), s[3], k->flag2, stats, k->rows(),
+                                  by_source(k->indptr, k->indices, k->n_src));
+        g.key.narrow(0, first, n_dst).add_(g.query.view({n_dst, s[0].size(1)}));
+        return once({g.key, g.x, Tensor(), Tensor(), Tensor()});
+    }
+};
+
+}  // namespace
+
+void bind_batched(py::module_ &m) {
+    py::class_<FoldPlan, FoldPlanPtr>(m, "FoldPlan");
+    py::class_<LinearPlan, LinearPlanPtr>(m, "LinearPlan");
+    // ranges: (rows, first rows of the sources, divisor, act, alpha)
+    m.def("fold_plan", [](int64_t rows_in,
+                          const std::vector<std::tuple<int64_t, std::vector<int64_t>, double, int64_t,
+                                                       double>> &ranges,
+                          const Tensor &like) {
+        std::vector<FoldPlan::Range> list;
+        for (const auto &[rows, sources, divisor, act, alpha] : ranges)
+            list.push_back({rows, sources, divisor, act, alpha});
+        return c10::make_intrusive<FoldPlan>(rows_in, list, like.device());
+    });
+    m.def("fold_rows", [](const Tensor &x, FoldPlanPtr p) { return FoldFunction::apply(x, p); });
+    m.def("fold_split", [](const Tensor &x, FoldPlanPtr p, std::vector<int64_t> sizes) {
+        return FoldSplitFunction::apply(x, p, std::move(sizes));
+    });
+    // units: (base, offset, rows)
+    m.def("linear_plan", [](const std::vector<std::tuple<int64_t, int64_t, int64_t>> &units,
+                            const std::vector<bool> &has_bias, const std::vector<int64_t> &base_rows,
+                            const Tensor &like) {
+        std::vector<LinearPlan::Unit> list;
+        for (const auto &[base, offset, rows] : units) list.push_back({base, offset, rows});
+        return c10::make_intrusive<LinearPlan>(list, has_bias, base_rows, like.device());
+    });
+    m.def("linear_rows", [](const TensorVec &bases, const TensorVec &ws, const TensorVec &bs,
+                            LinearPlanPtr p) {
+        TORCH_CHECK(bases.size() == p->base_rows.size() && ws.size() == p->units.size(),
+                    "linear_rows: the plan is for other inputs");
+        for (size_t b = 0; b < bases.size(); b++)
+            TORCH_CHECK(bases[b].dim() == 2 && bases[b].size(0) == p->base_rows[b],
+                        "linear_rows: the plan is for other inputs");
+        TORCH_CHECK(bs.size() == (size_t)std::count(p->has_bias.begin(), p->has_bias.end(), true),
+                    "linear_rows: the plan is for other biases");
+        return LinearRowsFunction::apply(at::TensorList(bases), at::TensorList(ws),
+                                         at::TensorList(bs), p);
+    });
+    m.def("gat_rows", [](const Tensor &ip, const Tensor &ix, const Tensor &qk, const Tensor &x,
+                         int64_t first, bool head_mean) {
+        return GatRowsFunction::apply(qk, x, first, head_mean, graph_of(ip, ix, x.size(0)));
+    });
+}
+
+}  // namespace yitu_bind

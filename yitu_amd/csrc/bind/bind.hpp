@@ -131,6 +131,8 @@ std::pair<Tensor, Tensor> sddmm_backward(const Tensor &indptr, const Tensor &ind
                                          const std::optional<BySource> &t);
 bool gat_one_pass_shape(int64_t heads, int64_t width);
 bool gat_mean_shape(const Tensor &x);  // of the head-mean backward, x [n_src, H, F]
+// whether the backward needs no more of the forward's softmax than its row statistics
+bool gat_stats_suffice(const Tensor &x, bool head_mean);
 struct GatOut {
     Tensor out;
     OptTensor attn, stats;
@@ -166,5 +168,6 @@ TensorVec column_sum_typed(const TensorVec &xs);
 void bind_ops(py::module_ &m);
 
 void bind_autograd(py::module_ &m);
+void bind_batched(py::module_ &m);
 
 }  // namespace yitu_bind

@@ -539,6 +539,10 @@ bool gat_mean_shape(const Tensor &x) {
            width % 4 == 0 && x.size(0) <= (1 << 24) && aligned16(x);
 }
 
+bool gat_stats_suffice(const Tensor &x, bool head_mean) {
+    return gat_one_pass_shape(x.size(1), x.size(2)) || (head_mean && gat_mean_shape(x));
+}
+
 GatOut gat_forward(const Tensor &indptr, const Tensor &indices, const Tensor &query,
                    const Tensor &key, const Tensor &x, bool stats_only, const RowState &rows) {
     check_i32(indptr, "indptr", 1);

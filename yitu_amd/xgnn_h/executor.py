@@ -7,7 +7,11 @@ against."""
 import torch
 from torch.nn import functional as F
 
-from . import bundle, ir, layers, mp, sparse
+from .. import _lib
+from . import batch, bundle, ir, layers, mp, sparse
+
+
+_BATCHED = ("rows", "typed_rows", "fold", "spmm_rows", "gat_rows")
 
 
 def _fill(template, values):
@@ -22,10 +26,14 @@ def _fill(template, values):
 
 class Executor:
     def __init__(self, group_linears: bool = True):
-        """``group_linears``: run the Linears of one depth and one shape as one grouped
-        launch (``Optimizer.group_linears``), decided once per dataflow."""
+        """``group_linears``: run what can run together as one launch, decided once per
+        dataflow: products and aggregations over row ranges of shared buffers on the GPU
+        (``batch.batch_rows``), elsewhere the Linears of one depth and one shape
+        (``Optimizer.group_linears``)."""
         self._group_linears = group_linears
         self._prepared = {}  # id(dataflow) -> (dataflow, the form that is evaluated, its order)
+        self._batched = {}  # (id(dataflow), training) -> (dataflow, batched form, its order) or None
+        self._plans = {}  # node of a batched form -> what its evaluations share
         self._is_training = None
         self._edge_values = {}  # edge_values node -> (state of its inputs, result, inputs)
         self._whole_tables = {}  # embedding node -> (state of its index tensor, is arange, tensor)
@@ -90,6 +98,8 @@ class Executor:
         op = node.op
         if op in ("input", "graph"):
             return self._lookup(node.name, kwargs)
+        if op in _BATCHED:
+            return self._eval_batched(node, v)
         if op == "call":
             if node.attrs["fn"] is F.embedding:
                 whole = self._whole_table(node, v)
@@ -155,17 +165,117 @@ class Executor:
     def run(self, dataflow: ir.Dataflow, kwargs: dict):
         """Evaluates the root (or every root of a dict) of ``dataflow``; ``kwargs``
         are the model's arguments, plus ``stitch`` when the stitcher has run."""
+        batched = self._batched_form(dataflow, kwargs) \
+            if self._group_linears and self._is_training is not None else None
+        if batched is not None:
+            values = {}
+            if self._leaves(batched, kwargs, values):
+                return self._evaluate(batched[1], batched[3], values, kwargs)
         kept = self._prepared.get(id(dataflow))
         if kept is None or kept[0] is not dataflow:
             from .optimizer import Optimizer
             flow = Optimizer.group_linears(dataflow) if self._group_linears else dataflow
             kept = (dataflow, flow, ir.walk(flow))
             self._prepared[id(dataflow)] = kept
-        _, dataflow, order = kept
-        values = {}
+        return self._evaluate(kept[1], kept[2], {}, kwargs)
+
+    def _evaluate(self, dataflow, order, values, kwargs):
         for node in order:
             ins = {k: values[id(c)] for k, c in node.inputs.items()}
             values[id(node)] = self._eval(node, ins, kwargs)
         if isinstance(dataflow, ir.Node):
             return values[id(dataflow)]
         return {k: values[id(n)] for k, n in dataflow.items()}
+
+    # -- batched form ---------------------------------------------------------------
+    def _batched_form(self, dataflow, kwargs):
+        """(dataflow, its batched form, leaves, the other nodes in order), or None."""
+        key = (id(dataflow), bool(self._is_training))
+        kept = self._batched.get(key)
+        if kept is None or kept[0] is not dataflow:
+            ws = [w for n in ir.walk(dataflow) if n.op in ("linear", "bundle", "typed_linear")
+                  for w, _ in batch.weights_of(n)]
+            flow = batch.batch_rows(dataflow, kwargs, key[1]) \
+                if ws and all(w.is_cuda and w.dtype == torch.float32 for w in ws) else None
+            order = [] if flow is None else ir.walk(flow)
+            leaf = lambda n: n.op in ("input", "graph")  # noqa: E731
+            kept = (dataflow, flow, [n for n in order if leaf(n)], [n for n in order if not leaf(n)])
+            self._batched[key] = kept
+        return None if kept[1] is None else (kept[0], kept[1], kept[2], kept[3])
+
+    def _leaves(self, batched, kwargs, values):
+        """Looks up the arguments; False when they are not shaped as they were captured (row
+        ranges are fixed in the batched form) or are no device floats."""
+        for node in batched[2]:
+            t = self._lookup(node.name, kwargs)
+            if node.op == "graph":
+                if list(t.size) != node.size:
+                    return False
+            elif not t.is_cuda or list(t.shape) != node.size or \
+                    (t.is_floating_point() and t.dtype != torch.float32):
+                return False
+            values[id(node)] = t
+        return True
+
+    def _edge_weights(self, node, v, blocks, kept):
+        """Edge weights of a batched aggregation: ones, or each relation's row scales spread over
+        its edges; kept while the same scale tensors come by (unless they train)."""
+        spec = node.attrs["spec"]
+        scales = [[v["s%d.%d" % (i, j)] for j in range(n)] for i, (_, n) in enumerate(spec)]
+        flat = [t for s in scales for t in s]
+        state = [(id(t), t.data_ptr(), t._version) for t in flat]
+        trains = any(t.requires_grad for t in flat)
+        if not trains and kept.get("state") == state:
+            return kept["weights"]
+        parts = []
+        for blk, s in zip(blocks, scales):
+            if not s:
+                parts.append(torch.ones(blk.num_edges(), device=v["x"].device))
+                continue
+            rows, _, bids = mp.edge_endpoints(blk)
+            parts.append(s[0].reshape(-1)[rows] if len(s) == 1 else
+                         torch.stack([t.reshape(-1) for t in s])[bids, rows])
+        weights = torch.cat(parts).unsqueeze(-1)
+        if not trains:
+            kept.update(state=state, weights=weights, scales=flat)
+        return weights
+
+    def _eval_batched(self, node: ir.Node, v: dict):
+        op, a = node.op, node.attrs
+        if op == "rows":
+            return v["x"].narrow(0, a["first"], a["rows"])
+        plan = self._plans.get(id(node))
+        if op == "typed_rows":
+            bases = [v[str(i)] for i in range(len(node.inputs))]
+            if plan is None:
+                plan = (node, _lib.ops().linear_plan(a["units"], [b is not None for b in a["biases"]],
+                                                     a["base_rows"], bases[0]),
+                        [b for b in a["biases"] if b is not None])
+                self._plans[id(node)] = plan
+            return _lib.ops().linear_rows(bases, a["weights"], plan[2], plan[1])
+        if op == "fold":
+            x = v["x"]
+            if plan is None:
+                plan = (node, _lib.ops().fold_plan(x.size(0), a["ranges"], x))
+                self._plans[id(node)] = plan
+            x = x if x.dim() == 2 else x.reshape(x.size(0), -1)
+            if "split" in a:
+                return _lib.ops().fold_split(x, plan[1], a["split"])
+            out = _lib.ops().fold_rows(x, plan[1])
+            return out if len(a["tail"]) == 1 else out.view([-1] + a["tail"])
+        # aggregation or attention over the members' stacked blocks
+        blocks = [v["g%d" % i] for i in range(sum(1 for k in node.inputs if k[0] == "g"))]
+        adj = [t for b in blocks for t in b.adj_sparse]
+        state = [(id(t), t._version) for t in adj]
+        if plan is None or plan[1] != state:
+            build = batch.spmm_block if op == "spmm_rows" else batch.gat_block
+            plan = (node, state, adj, build(blocks, a["spec"], a["n_cols"]), {})
+            self._plans[id(node)] = plan
+        indptr, indices = plan[3].adj_sparse
+        if op == "spmm_rows":
+            return sparse.GSPMMFunction.apply((indptr, indices),
+                                              self._edge_weights(node, v, blocks, plan[4]), v["x"])
+        if "q" in v:
+            return sparse.FusedGATFunction.apply((indptr, indices), v["q"], v["k"], v["x"],
+                                                 a["head_mean"])
+        return _lib.ops().gat_rows(indptr, indices, v["k"], v["x"], a["first"], a["head_mean"])
