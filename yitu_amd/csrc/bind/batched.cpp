@@ -74,11 +74,14 @@ Tensor fold(const Tensor &x, const FoldPlan &p) {
     return out;
 }
 
-// Rows of a result as a tensor of their own: the same memory, but for autograd no view of the
-// whole (the caller may write it in place, as any result).
-Tensor own_rows(const Tensor &t, int64_t first, int64_t rows) {
-    at::AutoDispatchBelowADInplaceOrView guard;
-    return t.narrow(0, first, rows);
+// Part of a result as a tensor of its own: the same memory, but for autograd no view of the
+// whole (the caller may write it in place, as any result). `first` counts floats.
+Tensor own_part(const Tensor &t, int64_t first, at::IntArrayRef sizes) {
+    Tensor part = at::detail::make_tensor<c10::TensorImpl>(
+        c10::TensorImpl::VIEW, c10::Storage(t.storage()), t.key_set(), t.dtype());
+    part.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
+    part.unsafeGetTensorImpl()->set_storage_offset(t.storage_offset() + first);
+    return part;
 }
 
 Tensor fold_backward(const FoldPlan &p, const Tensor &out, const Tensor &g) {
@@ -113,7 +116,7 @@ struct FoldSplitFunction : Function<FoldSplitFunction> {
         variable_list parts;
         int64_t at = 0;
         for (int64_t n : sizes) {
-            parts.push_back(own_rows(out, at, n));
+            parts.push_back(own_part(out, at * out.size(1), {n, out.size(1)}));
             at += n;
         }
         TORCH_CHECK(at == p->rows_out, "fold: the parts do not add up");
@@ -190,36 +193,64 @@ struct LinearPlan : torch::CustomClassHolder {
 };
 using LinearPlanPtr = c10::intrusive_ptr<LinearPlan>;
 
+// (By address, not by tensor: a narrow() for each unit of each operand took longer than the
+// launches did.)
 struct LinearRowsFunction : Function<LinearRowsFunction> {
-    static TensorVec inputs(const LinearPlan &p, const variable_list &bases) {
-        TensorVec xs;
-        for (const auto &u : p.units)
-            xs.push_back(u.rows == bases[u.base].size(0) ? bases[u.base]
-                                                         : bases[u.base].narrow(0, u.offset, u.rows));
+    static std::vector<const float *> inputs(const LinearPlan &p, const variable_list &bases,
+                                             int64_t k) {
+        std::vector<const float *> xs;
+        for (const auto &u : p.units) xs.push_back(f32(bases[u.base]) + u.offset * k);
         return xs;
     }
-    static TensorVec parts(const LinearPlan &p, const Tensor &t) {
-        TensorVec v;
-        int64_t at = 0;
+    // rows of the units in [total, width]
+    template <typename P>
+    static std::vector<P> parts(const LinearPlan &p, const Tensor &t) {
+        std::vector<P> v;
+        float *at = f32(t);
         for (const auto &u : p.units) {
-            v.push_back(t.narrow(0, at, u.rows));
-            at += u.rows;
+            v.push_back(at);
+            at += u.rows * t.size(1);
         }
+        return v;
+    }
+    static std::vector<int64_t> rows(const LinearPlan &p) {
+        std::vector<int64_t> v;
+        for (const auto &u : p.units) v.push_back(u.rows);
         return v;
     }
     static Tensor forward(AutogradContext *ctx, at::TensorList bases, at::TensorList ws,
                           at::TensorList bs, LinearPlanPtr p) {
+        const int64_t n = ws[0].size(0), k = ws[0].size(1);
         variable_list saved;
-        for (const Tensor &t : bases) saved.push_back(dense(t));
-        TensorVec weights;
-        for (const Tensor &t : ws) weights.push_back(dense(t));
-        std::vector<OptTensor> biases;
+        for (const Tensor &t : bases) {
+            saved.push_back(dense(t));
+            check_f32(saved.back(), "x", 2);
+            TORCH_CHECK(t.size(1) == k, "linear_rows: inputs must have ", k, " columns");
+            same_device(ws[0], t);
+        }
+        std::vector<const float *> weights, biases;
+        for (const Tensor &t : ws) {
+            saved.push_back(dense(t));
+            check_f32(saved.back(), "weight", 2);
+            same_device(ws[0], t);
+            TORCH_CHECK(t.sizes() == ws[0].sizes(), "linear_rows: weights must have one shape");
+            weights.push_back(f32(saved.back()));
+        }
+        TensorVec held;
         size_t b = 0;
-        for (bool there : p->has_bias)
-            biases.push_back(there ? OptTensor(dense(bs[b++])) : std::nullopt);
-        Tensor y = Call(bases[0]).empty({p->total, ws[0].size(0)});
-        linear_forward_typed(inputs(*p, saved), weights, biases, parts(*p, y));
-        saved.insert(saved.end(), weights.begin(), weights.end());
+        for (bool there : p->has_bias) {
+            if (there) {
+                held.push_back(dense(bs[b++]));
+                check_f32(held.back(), "bias", 1);
+                same_device(ws[0], held.back());
+                TORCH_CHECK(held.back().numel() == n, "linear_rows: biases must have ", n, " values");
+            }
+            biases.push_back(there ? f32(held.back()) : nullptr);
+        }
+        Call c(ws[0]);
+        Tensor y = c.empty({p->total, n});
+        linear_forward_at(c, parts<float *>(*p, y), {inputs(*p, saved, k), rows(*p)}, weights, biases,
+                          n, k);
         ctx->save_for_backward(std::move(saved));
         ctx->saved_data["plan"] = c10::IValue::make_capsule(p);
         return y;
@@ -229,10 +260,11 @@ struct LinearRowsFunction : Function<LinearRowsFunction> {
             c10::static_intrusive_pointer_cast<LinearPlan>(ctx->saved_data["plan"].toCapsule());
         const auto saved = ctx->get_saved_variables();
         const size_t n_bases = p->base_rows.size(), n_units = p->units.size();
-        const variable_list bases(saved.begin(), saved.begin() + n_bases);
-        const TensorVec weights(saved.begin() + n_bases, saved.end());
         const Tensor g = dense(grads[0]);
-        const TensorVec gs = parts(*p, g);
+        check_f32(g, "grad", 2);
+        const int64_t n = saved[n_bases].size(0), k = saved[n_bases].size(1);
+        const RowsView gs{parts<const float *>(*p, g), rows(*p)};
+        Call c(g);
         // one entry per argument: bases, weights, the biases that are there, the plan
         size_t n_biases = 0;
         for (bool there : p->has_bias) n_biases += there;
@@ -240,41 +272,49 @@ struct LinearRowsFunction : Function<LinearRowsFunction> {
         bool any = false;
         for (size_t b = 0; b < n_bases; b++) any = any || ctx->needs_input_grad(b);
         if (any) {
-            Tensor dx = Call(g).empty({p->total, weights[0].size(1)});
-            sgemm_typed(gs, weights, false, false, parts(*p, dx));
+            std::vector<const float *> weights;
+            for (size_t u = 0; u < n_units; u++) weights.push_back(f32(saved[n_bases + u]));
+            Tensor dx = c.empty({p->total, k});
+            linear_input_grad_at(c, parts<float *>(*p, dx), gs, weights, n, k);
             if (p->fold) dx = fold(dx, *p->fold);
             int64_t at = 0;
             for (size_t b = 0; b < n_bases; b++) {
                 if (ctx->needs_input_grad(b))
-                    out[b] = n_bases == 1 ? dx : own_rows(dx, at, p->base_rows[b]);
+                    out[b] = n_bases == 1 ? dx : own_part(dx, at * k, {p->base_rows[b], k});
                 at += p->base_rows[b];
             }
         }
-        TensorVec want_g, want_x;
-        std::vector<bool> want_b;
-        std::vector<std::pair<size_t, size_t>> slot;  // of the weight and of its bias
-        const TensorVec xs = inputs(*p, bases);
+        // weight and bias gradients in one buffer, each weight at a multiple of 64 floats
+        RowsView want;
+        std::vector<const float *> want_x;
+        std::vector<std::pair<size_t, size_t>> slot;  // of the weight and of its bias (0: none)
+        const auto xs = inputs(*p, saved, k);
         size_t bias = n_bases + n_units;
         for (size_t u = 0; u < n_units; u++) {
             const size_t at = p->has_bias[u] ? bias++ : 0;
             const bool b = at && ctx->needs_input_grad(at);
             if (ctx->needs_input_grad(n_bases + u)) {
-                want_g.push_back(gs[u]);
+                want.x.push_back(gs.x[u]);
+                want.rows.push_back(gs.rows[u]);
                 want_x.push_back(xs[u]);
-                want_b.push_back(b);
-                slot.emplace_back(n_bases + u, at);
+                slot.emplace_back(n_bases + u, b ? at : 0);
             } else if (b) {
-                out[at] = column_sum(gs[u]);
+                out[at] = column_sum(own_part(g, gs.x[u] - f32(g), {gs.rows[u], n}));
             }
         }
-        if (!want_g.empty()) {
-            TensorVec dws;
-            std::vector<OptTensor> dbs;
-            linear_weight_grad(want_g, want_x, want_b, &dws, &dbs);
+        if (!slot.empty()) {
+            const int64_t step = (n * k + 63) / 64 * 64, bias_step = (n + 63) / 64 * 64,
+                          biases_at = step * (int64_t)slot.size();
+            Tensor buffer = c.empty({biases_at + bias_step * (int64_t)slot.size()});
+            std::vector<float *> dw, db;
             for (size_t i = 0; i < slot.size(); i++) {
-                out[slot[i].first] = dws[i];
-                if (want_b[i]) out[slot[i].second] = *dbs[i];
+                dw.push_back(f32(buffer) + step * i);
+                db.push_back(slot[i].second ? f32(buffer) + biases_at + bias_step * i : nullptr);
+                out[slot[i].first] = own_part(buffer, step * i, {n, k});
+                if (slot[i].second)
+                    out[slot[i].second] = own_part(buffer, biases_at + bias_step * i, {n});
             }
+            linear_weight_grad_at(c, dw, db, want, want_x, n, k);
         }
         return once(std::move(out));
     }

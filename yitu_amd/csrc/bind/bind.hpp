@@ -60,9 +60,14 @@ struct Call {
     Tensor empty(at::IntArrayRef size, at::ScalarType dtype = at::kFloat) const {
         return Tensor(at::detail::empty_cuda(size, dtype, device, std::nullopt));
     }
-    // Scratch for one call; the caching allocator hands it out in stream order.
-    Tensor scratch(size_t bytes) const {
-        return empty({std::max<int64_t>((int64_t)bytes, 256)}, at::kByte);
+    // Scratch for one call, in the allocator's stream order; nothing where nothing is needed.
+    struct Scratch {
+        Tensor buffer;
+        void *data_ptr() const { return buffer.defined() ? buffer.data_ptr() : nullptr; }
+        size_t numel() const { return buffer.defined() ? (size_t)buffer.numel() : 0; }
+    };
+    Scratch scratch(size_t bytes) const {
+        return bytes ? Scratch{empty({(int64_t)bytes}, at::kByte)} : Scratch{};
     }
 };
 inline void ok(int rc, const char *what) {
@@ -108,6 +113,20 @@ TensorVec linear_forward_typed(const TensorVec &xs, const TensorVec &ws,
                                const std::optional<TensorVec> &outs);
 TensorVec sgemm_typed(const TensorVec &as, const TensorVec &bs, bool trans_a, bool trans_b,
                       const std::optional<TensorVec> &outs);
+// The same over matrices given by address and row count (the caller has checked them):
+// y_i [m_i, n] = x_i [m_i, k] . w_i^T + b_i, and dx_i [m_i, k] = g_i [m_i, n] . w_i
+struct RowsView {
+    std::vector<const float *> x;
+    std::vector<int64_t> rows;
+};
+void linear_forward_at(const Call &c, const std::vector<float *> &y, const RowsView &x,
+                       const std::vector<const float *> &w, const std::vector<const float *> &b,
+                       int64_t n, int64_t k);
+void linear_input_grad_at(const Call &c, const std::vector<float *> &dx, const RowsView &g,
+                          const std::vector<const float *> &w, int64_t n, int64_t k);
+void linear_weight_grad_at(const Call &c, const std::vector<float *> &dw,
+                           const std::vector<float *> &db, const RowsView &g,
+                           const std::vector<const float *> &x, int64_t n, int64_t k);
 // dw_i = g_i^T . x_i, and db_i = column sums of g_i where want_bias[i]
 void linear_weight_grad(const TensorVec &gs, const TensorVec &xs,
                         const std::vector<bool> &want_bias, TensorVec *dws,

@@ -64,7 +64,7 @@ Tensor agg(const Tensor &x, const Tensor &rp, const Tensor &ci, const OptTensor 
     Tensor out = c.empty({n_rows, dim});
     const size_t need =
         has(rows.plan) && rows.max_degree >= kLongRow ? yitu_spmm_workspace_bytes(nnz, dim, 1) : 0;
-    Tensor ws = c.scratch(need);
+    const auto ws = c.scratch(need);
     ok(yitu_agg_csr(f32(out), x.data_ptr(), bf16, i32(rp), i32(ci), f32(degrees), n_rows, n_src, nnz,
                     dim, (float)alpha, rows.max_degree, raw(rows.plan), f32(edge_scale),
                     ws.data_ptr(), ws.numel(), c.stream),
@@ -102,7 +102,7 @@ Tensor sgemm(const Tensor &a, const Tensor &b, bool trans_a, bool trans_b, const
     } else {
         c = call.empty({m, n});
     }
-    Tensor ws = call.scratch(yitu_sgemm_workspace_bytes(m, n, k, 1));
+    const auto ws = call.scratch(yitu_sgemm_workspace_bytes(m, n, k, 1));
     ok(yitu_sgemm(f32(c), f32(a), f32(b), m, n, k, trans_a, trans_b, a.size(1), b.size(1), n, accumulate,
                   ws.data_ptr(), ws.numel(), call.stream),
        "yitu_sgemm");
@@ -122,7 +122,7 @@ Tensor linear_forward(const Tensor &x, const Tensor &w, const OptTensor &bias) {
                 "linear_forward: x [m, k], weight [n, k], bias [n]");
     Call c(x);
     Tensor y = c.empty({m, n});
-    Tensor ws = c.scratch(yitu_sgemm_workspace_bytes(m, n, k, 1));
+    const auto ws = c.scratch(yitu_sgemm_workspace_bytes(m, n, k, 1));
     ok(yitu_linear_forward(f32(y), f32(x), f32(w), f32(bias), m, n, k, ws.data_ptr(), ws.numel(),
                            c.stream),
        "yitu_linear_forward");
@@ -155,13 +155,8 @@ TensorVec linear_forward_typed(const TensorVec &xs, const TensorVec &ws,
     }
     Call c(xs[0]);
     TensorVec outs = outputs(c, given, ms, n, at::kFloat);
-    Tensor scratch = c.scratch(
-        yitu_sgemm_workspace_bytes(*std::max_element(ms.begin(), ms.end()), n, k, (int64_t)count));
-    ok(yitu_linear_forward_typed(pointers<float *>(outs).data(), pointers<const float *>(xs).data(),
-                                 pointers<const float *>(ws).data(), biases.data(), ms.data(),
-                                 (int64_t)count, n, k, scratch.data_ptr(), scratch.numel(),
-                                 c.stream),
-       "yitu_linear_forward_typed");
+    linear_forward_at(c, pointers<float *>(outs), {pointers<const float *>(xs), ms},
+                      pointers<const float *>(ws), biases, n, k);
     return outs;
 }
 
@@ -193,7 +188,7 @@ TensorVec sgemm_typed(const TensorVec &as, const TensorVec &bs, bool trans_a, bo
     const int64_t n = bs[0].size(trans_b ? 0 : 1);
     Call c(as[0]);
     TensorVec outs = outputs(c, given, ms, n, at::kFloat);
-    Tensor ws = c.scratch(yitu_sgemm_workspace_bytes(*std::max_element(ms.begin(), ms.end()), n,
+    const auto ws = c.scratch(yitu_sgemm_workspace_bytes(*std::max_element(ms.begin(), ms.end()), n,
                                                      *std::max_element(ks.begin(), ks.end()),
                                                      (int64_t)count));
     ok(yitu_sgemm_typed(pointers<float *>(outs).data(), pointers<const float *>(as).data(),
@@ -209,7 +204,6 @@ void linear_weight_grad(const TensorVec &gs, const TensorVec &xs,
                         std::vector<OptTensor> *dbs) {
     const int64_t count = (int64_t)gs.size(), n = gs[0].size(1), k = xs[0].size(1);
     std::vector<int64_t> rows;
-    int64_t most = 0;
     for (int64_t i = 0; i < count; i++) {
         check_f32(gs[i], "grad", 2);
         check_f32(xs[i], "x", 2);
@@ -217,7 +211,6 @@ void linear_weight_grad(const TensorVec &gs, const TensorVec &xs,
         TORCH_CHECK(gs[i].size(1) == n && xs[i].size(1) == k && gs[i].size(0) == xs[i].size(0),
                     "linear_weight_grad: grad_i [m_i, ", n, "], x_i [m_i, ", k, "]");
         rows.push_back(gs[i].size(0));
-        most = std::max(most, rows.back());
     }
     Call c(gs[0]);
     *dws = outputs(c, std::nullopt, std::vector<int64_t>(count, n), k, at::kFloat);
@@ -228,11 +221,37 @@ void linear_weight_grad(const TensorVec &gs, const TensorVec &xs,
             (*dbs)[i] = c.empty({n});
             db[i] = f32((*dbs)[i]);
         }
-    Tensor ws = c.scratch(yitu_linear_weight_grad_workspace_bytes(most, n, k, count));
-    ok(yitu_linear_weight_grad_typed(pointers<float *>(*dws).data(), db.data(),
-                                     pointers<const float *>(gs).data(),
-                                     pointers<const float *>(xs).data(), rows.data(), count, n, k,
-                                     ws.data_ptr(), ws.numel(), c.stream),
+    linear_weight_grad_at(c, pointers<float *>(*dws), db, {pointers<const float *>(gs), rows},
+                          pointers<const float *>(xs), n, k);
+}
+
+void linear_forward_at(const Call &c, const std::vector<float *> &y, const RowsView &x,
+                       const std::vector<const float *> &w, const std::vector<const float *> &b,
+                       int64_t n, int64_t k) {
+    const int64_t count = (int64_t)y.size(), most = *std::max_element(x.rows.begin(), x.rows.end());
+    const auto ws = c.scratch(yitu_sgemm_workspace_bytes(most, n, k, count));
+    ok(yitu_linear_forward_typed(y.data(), x.x.data(), w.data(), b.data(), x.rows.data(), count, n, k,
+                                 ws.data_ptr(), ws.numel(), c.stream),
+       "yitu_linear_forward_typed");
+}
+
+void linear_input_grad_at(const Call &c, const std::vector<float *> &dx, const RowsView &g,
+                          const std::vector<const float *> &w, int64_t n, int64_t k) {
+    const int64_t count = (int64_t)dx.size(), most = *std::max_element(g.rows.begin(), g.rows.end());
+    const std::vector<int64_t> ks(count, n);
+    const auto ws = c.scratch(yitu_sgemm_workspace_bytes(most, k, n, count));
+    ok(yitu_sgemm_typed(dx.data(), g.x.data(), w.data(), g.rows.data(), ks.data(), count, k, 0, 0, n,
+                        k, k, 0, ws.data_ptr(), ws.numel(), c.stream),
+       "yitu_sgemm_typed");
+}
+
+void linear_weight_grad_at(const Call &c, const std::vector<float *> &dw,
+                           const std::vector<float *> &db, const RowsView &g,
+                           const std::vector<const float *> &x, int64_t n, int64_t k) {
+    const int64_t count = (int64_t)dw.size(), most = *std::max_element(g.rows.begin(), g.rows.end());
+    const auto ws = c.scratch(yitu_linear_weight_grad_workspace_bytes(most, n, k, count));
+    ok(yitu_linear_weight_grad_typed(dw.data(), db.data(), g.x.data(), x.data(), g.rows.data(), count,
+                                     n, k, ws.data_ptr(), ws.numel(), c.stream),
        "yitu_linear_weight_grad_typed");
 }
 
@@ -250,7 +269,7 @@ Tensor gemm_bf16(const Tensor &a, const Tensor &b, bool trans_b, at::ScalarType 
     Call call(a);
     Tensor c = outputs(call, has(out) ? std::optional<TensorVec>(TensorVec{*out}) : std::nullopt,
                        {m}, n, dtype)[0];
-    Tensor ws = call.scratch(yitu_gemm_bf16_workspace_bytes(n, k, trans_b));
+    const auto ws = call.scratch(yitu_gemm_bf16_workspace_bytes(n, k, trans_b));
     ok(yitu_gemm_bf16(c.data_ptr(), dtype == at::kBFloat16, a.data_ptr(), b.data_ptr(), m, n, k,
                       trans_b, k, b.size(1), n, ws.data_ptr(), ws.numel(), call.stream),
        "yitu_gemm_bf16");
@@ -281,7 +300,7 @@ TensorVec gemm_bf16_typed(const TensorVec &as, const TensorVec &bs, bool trans_b
                 "out_dtype must be float32 or bfloat16");
     Call c(as[0]);
     TensorVec outs = outputs(c, given, ms, n, dtype);
-    Tensor ws = c.scratch(yitu_gemm_bf16_typed_workspace_bytes((int64_t)count, n, k, trans_b));
+    const auto ws = c.scratch(yitu_gemm_bf16_typed_workspace_bytes((int64_t)count, n, k, trans_b));
     ok(yitu_gemm_bf16_typed(pointers<void *>(outs).data(), dtype == at::kBFloat16,
                             pointers<const void *>(as).data(), pointers<const void *>(bs).data(),
                             ms.data(), (int64_t)count, n, k, trans_b, k, bs[0].size(1), n,
@@ -316,7 +335,7 @@ TensorVec gemm_bf16_tn_typed(const TensorVec &as, const TensorVec &bs,
     TORCH_CHECK(!accumulate || given, "accumulate needs outputs to add to");
     Call c(as[0]);
     TensorVec outs = outputs(c, given, std::vector<int64_t>(count, ki), no, at::kFloat);
-    Tensor ws = c.scratch(yitu_gemm_bf16_tn_typed_workspace_bytes(ms.data(), (int64_t)count, ki, no));
+    const auto ws = c.scratch(yitu_gemm_bf16_tn_typed_workspace_bytes(ms.data(), (int64_t)count, ki, no));
     ok(yitu_gemm_bf16_tn_typed(pointers<float *>(outs).data(), pointers<const void *>(as).data(),
                                pointers<const void *>(bs).data(), ms.data(), (int64_t)count, ki, no,
                                std::max(lda, ki), std::max(ldb, no), no, accumulate, ws.data_ptr(),
@@ -337,7 +356,7 @@ Tensor gemm_bf16_tn(const Tensor &a, const Tensor &b, const OptTensor &out, bool
     Call c(a);
     Tensor o = outputs(c, has(out) ? std::optional<TensorVec>(TensorVec{*out}) : std::nullopt, {ki},
                        no, at::kFloat)[0];
-    Tensor ws = c.scratch(yitu_gemm_bf16_tn_workspace_bytes(m, ki, no));
+    const auto ws = c.scratch(yitu_gemm_bf16_tn_workspace_bytes(m, ki, no));
     ok(yitu_gemm_bf16_tn(f32(o), a.data_ptr(), b.data_ptr(), m, ki, no, a.stride(0), b.stride(0), no,
                          accumulate, ws.data_ptr(), ws.numel(), c.stream),
        "yitu_gemm_bf16_tn");
@@ -373,7 +392,7 @@ TensorVec b2gemm_backward(const Tensor &x, const Tensor &w_a, const Tensor &w_b,
     TORCH_CHECK(grad_a.size(0) == n && grad_a.size(1) == m, "grad_* must be [n, m]");
     Call c(x);
     Tensor dx = c.empty({n, k}), dw_a = c.empty({m, k}), dw_b = c.empty({m, k});
-    Tensor ws = c.scratch(yitu_sgemm_workspace_bytes(m, k, n, 2));
+    const auto ws = c.scratch(yitu_sgemm_workspace_bytes(m, k, n, 2));
     ok(yitu_b2gemm_backward(f32(dx), f32(dw_a), f32(dw_b), f32(x), f32(w_a), f32(w_b), f32(grad_a),
                             f32(grad_b), n, k, m, ws.data_ptr(), ws.numel(), c.stream),
        "yitu_b2gemm_backward");
@@ -397,7 +416,7 @@ Tensor spmm_forward(const Tensor &values, const Tensor &indptr, const Tensor &in
                 "multiple of 8");
     Call c(features);
     Tensor out = c.empty({n_dst, h, f}, bf16_out ? at::kBFloat16 : at::kFloat);
-    Tensor ws = c.scratch(has(rows.plan) ? spmm_scratch(nnz, h * f, rows.max_degree) : 0);
+    const auto ws = c.scratch(has(rows.plan) ? spmm_scratch(nnz, h * f, rows.max_degree) : 0);
     int rc;
     if (bf16_out)
         rc = yitu_spmm_forward_bf16_rows(out.data_ptr(), f32(values), i32(indptr), i32(indices),
@@ -434,7 +453,7 @@ std::pair<OptTensor, OptTensor> spmm_backward(const Tensor &values, const Tensor
     OptTensor grad_a, grad_x;
     if (need_a) grad_a = c.empty(values.sizes());
     if (need_x) grad_x = c.empty(features.sizes());
-    Tensor ws = c.scratch(spmm_scratch(nnz, h * f, std::max(rows.max_degree, t.max_degree)));
+    const auto ws = c.scratch(spmm_scratch(nnz, h * f, std::max(rows.max_degree, t.max_degree)));
     ok(yitu_spmm_backward(f32(grad_a), f32(grad_x), f32(values), i32(indptr), i32(indices),
                           f32(features), f32(grad_out), i32(t.t_indptr), i32(t.t_rows),
                           i32(t.t_perm), n_dst, n_src, nnz, h, f, rows.max_degree, t.max_degree,
@@ -456,7 +475,7 @@ Tensor edge_dot(const Tensor &indptr, const Tensor &indices, const Tensor &dst, 
                 "dst_feat must be [n_dst, H, F] matching src_feat's H and F");
     Call c(src);
     Tensor out = c.empty({nnz, h});
-    Tensor ws = c.scratch(0);
+    const auto ws = c.scratch(0);
     ok(yitu_spmm_backward(f32(out), nullptr, nullptr, i32(indptr), i32(indices), f32(src), f32(dst),
                           nullptr, nullptr, nullptr, n_dst, n_src, nnz, h, f, rows.max_degree, -1,
                           raw(rows.plan), nullptr, ws.data_ptr(), ws.numel(), c.stream),
@@ -487,7 +506,7 @@ Tensor sddmm_forward(const Tensor &indptr, const Tensor &indices, const Tensor &
     const int64_t n_src = key.size(0), h = key.size(1), n_bid = query.size(0);
     Call c(key);
     Tensor attn = c.empty({nnz, h});
-    Tensor ws = c.scratch(rows.max_degree >= kLongRow
+    const auto ws = c.scratch(rows.max_degree >= kLongRow
                               ? yitu_sddmm_workspace_bytes(n_dst, nnz, h, n_bid, 1)
                               : 0);
     ok(yitu_sddmm_forward(f32(attn), i32(indptr), i32(indices), f32(query), f32(key), n_dst, n_src,
@@ -514,7 +533,7 @@ std::pair<Tensor, Tensor> sddmm_backward(const Tensor &indptr, const Tensor &ind
     OptTensor grad_edge;
     if (t) grad_edge = c.empty({nnz, h});
     const bool wide = rows.max_degree >= kLongRow || (t && t->max_degree >= kLongRow);
-    Tensor ws = c.scratch(wide ? yitu_sddmm_workspace_bytes(n_dst, nnz, h, n_bid, 1) : 0);
+    const auto ws = c.scratch(wide ? yitu_sddmm_workspace_bytes(n_dst, nnz, h, n_bid, 1) : 0);
     ok(yitu_sddmm_backward(f32(grad_q), f32(grad_k), f32(grad_edge), i32(indptr), i32(indices),
                            f32(query), f32(key), f32(attn), f32(grad_out),
                            t ? i32(t->t_indptr) : nullptr, t ? i32(t->t_perm) : nullptr, n_dst, n_src,
@@ -563,7 +582,7 @@ GatOut gat_forward(const Tensor &indptr, const Tensor &indices, const Tensor &qu
     o.out = c.empty({n_dst, h, f});
     if (stats_only) o.stats = c.empty({n_dst, h, 2});
     else o.attn = c.empty({nnz, h});
-    Tensor ws = c.scratch(
+    const auto ws = c.scratch(
         rows.max_degree >= kLongRow ? yitu_gat_workspace_bytes(n_dst, nnz, h, f, 1) : 0);
     ok(yitu_gat_forward(f32(o.out), f32(o.attn), f32(o.stats), i32(indptr), i32(indices), f32(query),
                         f32(key), f32(x), n_dst, n_src, nnz, h, f, rows.max_degree, raw(rows.plan),
@@ -610,7 +629,7 @@ GatGrads gat_backward(const Tensor &indptr, const Tensor &indices, const Tensor 
     Tensor s1 = c.empty({nnz, h});
     Tensor s2 = has(attn) ? c.empty({nnz, h}) : s1;  // unused by the one-pass path
     const bool wide = std::max(rows.max_degree, t.max_degree) >= kLongRow || has(out);
-    Tensor ws =
+    const auto ws =
         c.scratch(wide ? yitu_gat_workspace_bytes(std::max(n_dst, n_src), nnz, h, f, 1) : 0);
     ok(yitu_gat_backward(f32(g.query), f32(g.key), f32(g.x), f32(s1), f32(s2), i32(indptr),
                          i32(indices), f32(query), f32(key), f32(x), f32(attn), f32(stats), f32(out),
@@ -660,7 +679,7 @@ std::tuple<Tensor, Tensor, OptTensor> head_dot_backward(const Tensor &x, const T
     Tensor gva = c.empty(a.sizes());
     OptTensor gvb;
     if (has(b)) gvb = c.empty(b->sizes());
-    Tensor ws = c.scratch(yitu_head_dot_workspace_bytes(n, h, f));
+    const auto ws = c.scratch(yitu_head_dot_workspace_bytes(n, h, f));
     ok(yitu_head_dot_backward(f32(gx), has(grad_x), f32(gva), f32(gvb), f32(x), f32(a), f32(b),
                               f32(grad_a), f32(grad_b), n, h, f, ws.data_ptr(), ws.numel(), c.stream),
        "yitu_head_dot_backward");
@@ -724,7 +743,7 @@ SkinnyGrads skinny_pair_backward(const Tensor &x, const Tensor &w_a, const OptTe
     if (jb) g.w_b = c.empty({jb, k});
     if (bias_a) g.bias_a = c.empty({ja});
     if (jb && bias_b) g.bias_b = c.empty({jb});
-    Tensor ws = c.scratch(yitu_skinny_linear_workspace_bytes(n, k, ja + jb));
+    const auto ws = c.scratch(yitu_skinny_linear_workspace_bytes(n, k, ja + jb));
     ok(yitu_skinny_pair_backward(f32(g.x), has(grad_x), f32(g.w_a), f32(g.w_b), f32(g.bias_a),
                                  f32(g.bias_b), f32(x), f32(w_a), f32(w_b), f32(grad_a), f32(grad_b),
                                  n, k, ja, jb, ws.data_ptr(), ws.numel(), c.stream),
@@ -737,7 +756,7 @@ Tensor column_sum(const Tensor &x) {
     const int64_t m = x.size(0), n = x.size(1);
     Call c(x);
     Tensor out = c.empty({n});
-    Tensor ws = c.scratch(yitu_column_sum_workspace_bytes(m, n));
+    const auto ws = c.scratch(yitu_column_sum_workspace_bytes(m, n));
     ok(yitu_column_sum(f32(out), f32(x), m, n, ws.data_ptr(), ws.numel(), c.stream),
        "yitu_column_sum");
     return out;
@@ -785,7 +804,7 @@ std::tuple<Tensor, Tensor, Tensor> coo_to_csr(const Tensor &rows, const Tensor &
     Tensor indptr = c.empty({n_rows + 1}, at::kInt);
     Tensor indices = c.empty({std::max<int64_t>(n_edges, 1)}, at::kInt);
     Tensor nnz = c.empty({1}, at::kLong);
-    Tensor ws = c.scratch(yitu_coo_to_csr_workspace_bytes(n_edges, n_rows));
+    const auto ws = c.scratch(yitu_coo_to_csr_workspace_bytes(n_edges, n_rows));
     ok(yitu_coo_to_csr(static_cast<int32_t *>(indptr.data_ptr()),
                        static_cast<int32_t *>(indices.data_ptr()),
                        static_cast<long long *>(nnz.data_ptr()), i32(rows), i32(cols), n_edges,
@@ -802,7 +821,7 @@ std::tuple<Tensor, Tensor, Tensor> csr_transpose(const Tensor &indptr, const Ten
     Call c(indices);
     Tensor t_indptr = c.empty({n_src + 1}, at::kInt), t_rows = c.empty({nnz}, at::kInt),
            t_perm = c.empty({nnz}, at::kInt);
-    Tensor ws = c.scratch(yitu_csr_transpose_workspace_bytes(nnz, n_src));
+    const auto ws = c.scratch(yitu_csr_transpose_workspace_bytes(nnz, n_src));
     ok(yitu_csr_transpose(static_cast<int32_t *>(t_indptr.data_ptr()),
                           static_cast<int32_t *>(t_rows.data_ptr()),
                           static_cast<int32_t *>(t_perm.data_ptr()), i32(indptr), i32(indices),
@@ -817,7 +836,7 @@ Tensor build_plan(const Tensor &indptr, const Tensor &indices, int64_t n_src, in
     const int64_t nnz = indices.numel();
     Call c(indices);
     Tensor plan = c.empty({(int64_t)yitu_plan_bytes(nnz)}, at::kByte);
-    Tensor ws = c.scratch(yitu_plan_workspace_bytes(nnz));
+    const auto ws = c.scratch(yitu_plan_workspace_bytes(nnz));
     ok(yitu_plan_build(plan.data_ptr(), plan.numel(), i32(indptr), i32(indices), indptr.numel() - 1,
                        n_src, nnz, mask, ws.data_ptr(), ws.numel(), c.stream),
        "yitu_plan_build");

@@ -88,6 +88,17 @@ class Executor:
             self._whole_tables[id(node)] = kept
         return weight.view_as(weight) if kept[1] else None
 
+    def _read_only_table(self, node: ir.Node, v: dict):
+        """The same where only products read the rows: the table itself."""
+        kept = self._whole_tables.get(id(node))
+        if kept is not None and kept[1] and torch.is_grad_enabled():
+            idx = next(iter(v.values()))
+            weight = node.attrs["args"][1]
+            if kept[2] is idx and kept[0] == (idx.data_ptr(), idx._version, idx.numel()) and \
+                    torch.is_tensor(weight) and weight.requires_grad:
+                return weight
+        return self._whole_table(node, v)
+
     def forget_tables(self):
         """Drops what is remembered about embedding index tensors (call after refilling one
         through a raw pointer, which leaves its version counter unchanged)."""
@@ -102,7 +113,8 @@ class Executor:
             return self._eval_batched(node, v)
         if op == "call":
             if node.attrs["fn"] is F.embedding:
-                whole = self._whole_table(node, v)
+                whole = self._read_only_table(node, v) if node.attrs.get("read_only") else \
+                    self._whole_table(node, v)
                 if whole is not None:
                     return whole
             return node.attrs["fn"](*_fill(node.attrs["args"], v), **_fill(node.attrs["kwargs"], v))
@@ -198,21 +210,22 @@ class Executor:
             flow = batch.batch_rows(dataflow, kwargs, key[1]) \
                 if ws and all(w.is_cuda and w.dtype == torch.float32 for w in ws) else None
             order = [] if flow is None else ir.walk(flow)
-            leaf = lambda n: n.op in ("input", "graph")  # noqa: E731
-            kept = (dataflow, flow, [n for n in order if leaf(n)], [n for n in order if not leaf(n)])
+            leaves = [(n, n.size if n.op == "graph" else torch.Size(n.size), n.op == "graph")
+                      for n in order if n.op in ("input", "graph")]
+            kept = (dataflow, flow, leaves, [n for n in order if n.op not in ("input", "graph")])
             self._batched[key] = kept
-        return None if kept[1] is None else (kept[0], kept[1], kept[2], kept[3])
+        return None if kept[1] is None else kept
 
     def _leaves(self, batched, kwargs, values):
         """Looks up the arguments; False when they are not shaped as they were captured (row
         ranges are fixed in the batched form) or are no device floats."""
-        for node in batched[2]:
+        for node, size, graph in batched[2]:
             t = self._lookup(node.name, kwargs)
-            if node.op == "graph":
-                if list(t.size) != node.size:
+            if graph:
+                if t.size != size:
                     return False
-            elif not t.is_cuda or list(t.shape) != node.size or \
-                    (t.is_floating_point() and t.dtype != torch.float32):
+            elif t.shape != size or not t.is_cuda or \
+                    (t.dtype is not torch.float32 and t.is_floating_point()):
                 return False
             values[id(node)] = t
         return True
