@@ -760,6 +760,15 @@ int yitu_coo_to_csr(int32_t *indptr_device, int32_t *indices_device, long long *
                     const int32_t *rows_device, const int32_t *cols_device, int64_t n_edges,
                     int64_t n_rows, int64_t n_cols, void *workspace_device, size_t workspace_bytes,
                     void *stream);
+/* The same from ids of 4 or 8 bytes (id_bytes), with info_device[2] = {distinct edges or -1,
+ * edges of the longest row}. */
+int yitu_coo_to_csr_ids(int32_t *indptr_device, int32_t *indices_device, long long *info_device,
+                        const void *rows_device, const void *cols_device, int id_bytes,
+                        int64_t n_edges, int64_t n_rows, int64_t n_cols, void *workspace_device,
+                        size_t workspace_bytes, void *stream);
+/* *longest_device = edges of the longest row of a CSR (0 without rows). */
+int yitu_longest_row(long long *longest_device, const int32_t *indptr_device, int64_t n_rows,
+                     void *stream);
 
 /*
  * build_part on the device (ccsrc/kernel/YiTu_GNN.cpp:203-245, which walks the rows on

@@ -169,10 +169,21 @@ def max_degree(indptr):
     native = ops()
     v = native.find_max_degree(indptr)
     if v < 0:
-        v = int((indptr[1:] - indptr[:-1]).max().item()) if indptr.numel() > 1 else 0
-        native.put_max_degree(indptr, v)
-        watch(indptr)
+        if indptr.numel() <= 1:
+            v = 0
+        elif indptr.is_cuda and indptr.dtype == torch.int32 and indptr.dim() == 1 and \
+                indptr.is_contiguous():
+            v = int(native.longest_row(indptr).item())
+        else:
+            v = int((indptr[1:] - indptr[:-1]).max().item())
+        put_max_degree(indptr, v)
     return v
+
+
+def put_max_degree(indptr, value):
+    """Keeps the longest row of a CSR whose builder knows it."""
+    ops().put_max_degree(indptr, value)
+    watch(indptr)
 
 
 def row_plan(indptr, indices, n_src, col_mask):
@@ -182,7 +193,7 @@ def row_plan(indptr, indices, n_src, col_mask):
     small. A large graph without long rows still gets one: its header tells the row kernels
     whether most sources of a row lie near the row's own id, which decides how rows are dealt
     to the XCDs."""
-    if max_degree(indptr) < 64 and indices.numel() < (1 << 20):
+    if indices.numel() < (1 << 20) and max_degree(indptr) < 64:
         return None
     native = ops()
     plan = native.find_plan(indptr, indices, int(n_src), col_mask)

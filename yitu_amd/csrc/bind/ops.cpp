@@ -795,22 +795,38 @@ TensorVec column_sum_typed(const TensorVec &xs) {
 
 // ---- graph preparation -----------------------------------------------------------------
 namespace {
+// indptr, indices (as many as edges went in), {distinct edges or -1, longest row}
 std::tuple<Tensor, Tensor, Tensor> coo_to_csr(const Tensor &rows, const Tensor &cols, int64_t n_rows,
                                               int64_t n_cols) {
-    check_i32(rows, "rows", 1);
-    check_i32(cols, "cols", 1);
+    const at::ScalarType ids = rows.scalar_type();
+    TORCH_CHECK(ids == at::kInt || ids == at::kLong, "ids must be int32 or int64");
+    check(rows, ids, "rows", 1);
+    check(cols, ids, "cols", 1);
+    same_device(rows, cols);
     const int64_t n_edges = rows.numel();
+    TORCH_CHECK(cols.numel() == n_edges, "rows and cols must be equally long");
     Call c(rows);
     Tensor indptr = c.empty({n_rows + 1}, at::kInt);
     Tensor indices = c.empty({std::max<int64_t>(n_edges, 1)}, at::kInt);
-    Tensor nnz = c.empty({1}, at::kLong);
+    Tensor info = c.empty({2}, at::kLong);
     const auto ws = c.scratch(yitu_coo_to_csr_workspace_bytes(n_edges, n_rows));
-    ok(yitu_coo_to_csr(static_cast<int32_t *>(indptr.data_ptr()),
-                       static_cast<int32_t *>(indices.data_ptr()),
-                       static_cast<long long *>(nnz.data_ptr()), i32(rows), i32(cols), n_edges,
-                       n_rows, n_cols, ws.data_ptr(), ws.numel(), c.stream),
-       "yitu_coo_to_csr");
-    return {indptr, indices, nnz};
+    ok(yitu_coo_to_csr_ids(static_cast<int32_t *>(indptr.data_ptr()),
+                           static_cast<int32_t *>(indices.data_ptr()),
+                           static_cast<long long *>(info.data_ptr()), rows.data_ptr(),
+                           cols.data_ptr(), ids == at::kInt ? 4 : 8, n_edges, n_rows, n_cols,
+                           ws.data_ptr(), ws.numel(), c.stream),
+       "yitu_coo_to_csr_ids");
+    return {indptr, indices, info};
+}
+
+Tensor longest_row(const Tensor &indptr) {
+    check_i32(indptr, "indptr", 1);
+    Call c(indptr);
+    Tensor out = c.empty({1}, at::kLong);
+    ok(yitu_longest_row(static_cast<long long *>(out.data_ptr()), i32(indptr), indptr.numel() - 1,
+                        c.stream),
+       "yitu_longest_row");
+    return out;
 }
 
 std::tuple<Tensor, Tensor, Tensor> csr_transpose(const Tensor &indptr, const Tensor &indices,
@@ -931,6 +947,7 @@ void bind_ops(py::module_ &m) {
     m.def("column_sum_typed", &column_sum_typed);
     m.def("coo_to_csr", &coo_to_csr);
     m.def("csr_transpose", &csr_transpose);
+    m.def("longest_row", &longest_row);
     m.def("build_plan", &build_plan);
 }
 

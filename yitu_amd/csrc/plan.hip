@@ -1,12 +1,15 @@
-// Builds the row plan on the device: queue the long rows (one atomic per
-// workgroup), cut every long row where its sorted columns cross the boundaries
-// of its source bands and into items of at most 64 edges, key every item by its
-// middle source id, stable radix sort, write the records.
+// Builds the row plan on the device: queue the long rows, cut every long row where its
+// sorted columns cross the boundaries of its source bands and into items of at most 64
+// edges, and deal the items into 2^16 bins by their middle source id. An item draws its rank
+// in its bin when it is made, so a prefix sum of the bins gives its place; the order inside
+// a bin does not matter to the kernels.
+// Bound by atomics on one address, which the memory side takes one at a time (about 8 ns
+// each): so the workgroups are of 1,024 threads and claim rows and items for all of them
+// with one add. 200,000 rows, 3 M edges: 55 us in five launches, where a radix sort of the
+// items (all slots, used or not) and narrower workgroups took 175.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
-
-#include <rocprim/device/device_radix_sort.hpp>
 
 #include "../../include/yitu_hip.h"
 #include "plan.hpp"
@@ -15,7 +18,9 @@ namespace yitu {
 
 namespace {
 
-constexpr int kBandBits = 16;  // sort key = middle source id reduced to this many bits
+constexpr int kBins = 1 << 16;      // of items, by middle source id
+constexpr int kPlanBlock = 1024;    // threads of the building kernels
+constexpr int kPlanWaves = kPlanBlock / kWave;
 
 struct BuildBuffers {
     PlanCounters *counters;
@@ -23,36 +28,27 @@ struct BuildBuffers {
     int4 *records;
     int *band_info;   // {log2 of the band width, number of bands, local edges, sampled edges}, in the plan header
     int4 *items;      // {first edge, end edge, index into rows[], row} in queue order
-    uint32_t *keys_in, *keys_out;
-    int32_t *vals_in, *order;
-    void *sort_temp;
-    size_t sort_temp_bytes;
-    int key_shift;    // sort key = middle source id >> key_shift (16 bits)
+    int2 *place;      // {bin, rank in it} of every item, in queue order
+    int *bin_start;   // items of every bin, then its first place
+    int key_shift;    // bin = middle source id >> key_shift
     int band_shift;   // band of a source = id >> band_shift
     int n_bands;      // 1 = no cuts
     int max_rows, max_items;
 };
 
-__global__ __launch_bounds__(kBlock) void plan_init_kernel(BuildBuffers b) {
-    const int64_t i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const int64_t stride = (int64_t)gridDim.x * kBlock;
-    if (i0 == 0) {
+__global__ __launch_bounds__(kPlanBlock) void plan_init_kernel(BuildBuffers b) {
+    const int i = blockIdx.x * kPlanBlock + threadIdx.x;
+    if (i == 0) {
         b.counters->n_items = 0;
         b.counters->n_rows = 0;
         b.counters->overflow = 0;
         b.counters->pad = 0;
-    }
-    if (i0 == 0) {
         b.band_info[0] = b.band_shift;
         b.band_info[1] = b.n_bands;
         b.band_info[kPlanInfoLocal] = 0;
         b.band_info[kPlanInfoSampled] = 0;
     }
-    // slots that get no item sort behind every real key
-    for (int64_t i = i0; i < b.max_items; i += stride) {
-        b.keys_in[i] = 0xffffu;
-        b.vals_in[i] = (int32_t)i;
-    }
+    if (i < kBins) b.bin_start[i] = 0;
 }
 
 // Every lane owns one row; the long rows of a workgroup are numbered with a
@@ -72,7 +68,7 @@ __device__ __forceinline__ int block_rank(bool flag, int *wave_sums, int *block_
     __syncthreads();
     if (threadIdx.x == 0) {
         int br = 0;
-        for (int w = 0; w < kWavesPerBlock; w++) br += wave_sums[w];
+        for (int w = 0; w < kPlanWaves; w++) br += wave_sums[w];
         *block_base = br > 0 ? atomicAdd(counter, br) : 0;
     }
     __syncthreads();
@@ -87,13 +83,13 @@ __device__ __forceinline__ int block_rank(bool flag, int *wave_sums, int *block_
 // spaced, are sampled, and an edge counts as local when its source lies within
 // 1/64 of the id space (at least 1,024 ids) of the row's own relative position.
 // One add per workgroup and counter.
-__global__ __launch_bounds__(kBlock) void plan_queue_kernel(BuildBuffers b,
+__global__ __launch_bounds__(kPlanBlock) void plan_queue_kernel(BuildBuffers b,
                                                             const int32_t *__restrict__ indptr,
                                                             const int32_t *__restrict__ indices,
                                                             int n_rows, int n_src, int col_mask) {
-    __shared__ int wave_sums[kWavesPerBlock];
+    __shared__ int wave_sums[kPlanWaves];
     __shared__ int block_base;
-    const int row = blockIdx.x * kBlock + threadIdx.x;
+    const int row = blockIdx.x * kPlanBlock + threadIdx.x;
     int deg = 0, beg = 0;
     if (row < n_rows) {
         beg = indptr[row];
@@ -143,18 +139,18 @@ __global__ __launch_bounds__(kBlock) void plan_queue_kernel(BuildBuffers b,
 // crossings into segments (none shorter than kPlanMinSegment), the wave then
 // writes the items of every segment: ceil(len / 64) pieces of equal size. Item
 // ids of a row are consecutive; a workgroup takes its ids with one atomic.
-__global__ __launch_bounds__(kBlock) void plan_items_kernel(BuildBuffers b,
+__global__ __launch_bounds__(kPlanBlock) void plan_items_kernel(BuildBuffers b,
                                                             const int32_t *__restrict__ indptr,
                                                             const int32_t *__restrict__ indices,
                                                             int col_mask) {
-    __shared__ int cut[kWavesPerBlock][kPlanMaxBands + 1];
-    __shared__ int seg_beg[kWavesPerBlock][kPlanMaxBands + 1];    // [n_seg] = end of the row
-    __shared__ int seg_first[kWavesPerBlock][kPlanMaxBands + 1];  // first item of the segment, [n_seg] = total
-    __shared__ int n_seg[kWavesPerBlock];
-    __shared__ int wave_first[kWavesPerBlock];
+    __shared__ int cut[kPlanWaves][kPlanMaxBands + 1];
+    __shared__ int seg_beg[kPlanWaves][kPlanMaxBands + 1];    // [n_seg] = end of the row
+    __shared__ int seg_first[kPlanWaves][kPlanMaxBands + 1];  // first item of the segment, [n_seg] = total
+    __shared__ int n_seg[kPlanWaves];
+    __shared__ int wave_first[kPlanWaves];
     const int lane = lane_id();
     const int wave = threadIdx.x / kWave;
-    const int slot = blockIdx.x * kWavesPerBlock + wave;
+    const int slot = blockIdx.x * kPlanWaves + wave;
     const int n_rows = b.counters->overflow ? 0 : min(b.counters->n_rows, b.max_rows);
     const bool active = slot < n_rows;
     int row = 0, beg = 0, end = 0;
@@ -213,12 +209,12 @@ __global__ __launch_bounds__(kBlock) void plan_items_kernel(BuildBuffers b,
     __syncthreads();
     if (threadIdx.x == 0) {
         int sum = 0;
-        for (int w = 0; w < kWavesPerBlock; w++) {
+        for (int w = 0; w < kPlanWaves; w++) {
             wave_first[w] = sum;
             sum += seg_first[w][n_seg[w]];
         }
         const int base = sum > 0 ? atomicAdd(&b.counters->n_items, sum) : 0;
-        for (int w = 0; w < kWavesPerBlock; w++) wave_first[w] += base;
+        for (int w = 0; w < kPlanWaves; w++) wave_first[w] += base;
     }
     __syncthreads();
     if (!active) return;
@@ -240,32 +236,59 @@ __global__ __launch_bounds__(kBlock) void plan_items_kernel(BuildBuffers b,
         const int ie = min(se, ib + size);
         const int mid_col = indices[(ib + ie) >> 1] & col_mask;
         b.items[first_item + i] = make_int4(ib, ie, slot, row);
-        b.keys_in[first_item + i] =
-            min((uint32_t)mid_col >> b.key_shift, (1u << kBandBits) - 1u);
+        const int bin = min(mid_col >> b.key_shift, kBins - 1);
+        b.place[first_item + i] = make_int2(bin, atomicAdd(&b.bin_start[bin], 1));
+    }
+}
+
+// Exclusive prefix sum of the bins, by one workgroup: 64 bins per thread, four at a time.
+__global__ __launch_bounds__(kPlanBlock) void plan_bin_starts_kernel(BuildBuffers b) {
+    __shared__ int wave_sums[kPlanWaves];
+    constexpr int kEach = kBins / kPlanBlock / 4;
+    int4 *bins = reinterpret_cast<int4 *>(b.bin_start) + threadIdx.x * kEach;
+    int4 v[kEach];
+    int sum = 0;
+#pragma unroll
+    for (int k = 0; k < kEach; k++) v[k] = bins[k];
+#pragma unroll
+    for (int k = 0; k < kEach; k++) sum += v[k].x + v[k].y + v[k].z + v[k].w;
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    int pre = sum;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int x = __shfl_up(pre, o, kWave);
+        if (lane >= o) pre += x;
+    }
+    if (lane == kWave - 1) wave_sums[wave] = pre;
+    __syncthreads();
+    pre -= sum;
+    for (int w = 0; w < wave; w++) pre += wave_sums[w];
+#pragma unroll
+    for (int k = 0; k < kEach; k++) {
+        int4 o;
+        o.x = pre;
+        o.y = o.x + v[k].x;
+        o.z = o.y + v[k].y;
+        o.w = o.z + v[k].z;
+        pre = o.w + v[k].w;
+        bins[k] = o;
     }
 }
 
 __global__ __launch_bounds__(kBlock) void plan_records_kernel(BuildBuffers b) {
-    const int pos = blockIdx.x * kBlock + threadIdx.x;
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= b.max_items) return;
     const int n_items = b.counters->overflow ? 0 : min(b.counters->n_items, b.max_items);
-    if (pos >= b.max_items) return;
-    int4 rec = make_int4(0, 0, 0, 0);
-    if (pos < n_items) {
-        const int item = b.order[pos];  // stable sort: real items precede the padding
-        const int4 it = b.items[item];
-        // a row that is a single item is finished by the item kernel itself
-        const int single = b.rows[it.z].z == 1 ? (int)0x80000000 : 0;
-        rec = make_int4(it.x, it.y, item, it.w | single);
+    if (i >= n_items) {  // slots behind the last item
+        b.records[i] = make_int4(0, 0, 0, 0);
+        return;
     }
-    b.records[pos] = rec;
-}
-
-size_t sort_temp_bytes(int64_t n) {
-    size_t bytes = 0;
-    uint32_t *k = nullptr;
-    int32_t *v = nullptr;
-    (void)rocprim::radix_sort_pairs(nullptr, bytes, k, k, v, v, (size_t)n, 0, 16);
-    return bytes;
+    const int2 at = b.place[i];
+    const int4 it = b.items[i];
+    // a row that is a single item is finished by the item kernel itself
+    const int single = b.rows[it.z].z == 1 ? (int)0x80000000 : 0;
+    const int place = b.bin_start[at.x] + at.y;
+    if (place < n_items) b.records[place] = make_int4(it.x, it.y, i, it.w | single);
 }
 
 constexpr size_t kHeaderBytes = 512;  // counters | at byte 256: {log2 band width, bands}
@@ -279,8 +302,8 @@ size_t plan_bytes(int64_t nnz) {
 
 size_t plan_build_workspace_bytes(int64_t nnz) {
     const size_t items = (size_t)plan_max_items(nnz);
-    return align_up(sizeof(int4) * items, 256) + 4 * align_up(sizeof(int32_t) * items, 256) +
-           align_up(sort_temp_bytes((int64_t)items), 256);
+    return align_up(sizeof(int4) * items, 256) + align_up(sizeof(int2) * items, 256) +
+           sizeof(int) * kBins;
 }
 
 size_t plan_temp_bytes(int64_t nnz) { return plan_bytes(nnz) + plan_build_workspace_bytes(nnz); }
@@ -322,37 +345,28 @@ int plan_build(void *plan, size_t plan_size, const int32_t *indptr, const int32_
     char *w = static_cast<char *>(workspace);
     b.items = reinterpret_cast<int4 *>(w);
     w += align_up(sizeof(int4) * (size_t)b.max_items, 256);
-    const size_t arr = align_up(sizeof(int32_t) * (size_t)b.max_items, 256);
-    b.keys_in = reinterpret_cast<uint32_t *>(w);
-    b.keys_out = reinterpret_cast<uint32_t *>(w + arr);
-    b.vals_in = reinterpret_cast<int32_t *>(w + 2 * arr);
-    b.order = reinterpret_cast<int32_t *>(w + 3 * arr);
-    w += 4 * arr;
-    b.sort_temp = w;
-    b.sort_temp_bytes = sort_temp_bytes(b.max_items);
-    w += align_up(b.sort_temp_bytes, 256);
+    b.place = reinterpret_cast<int2 *>(w);
+    b.bin_start = reinterpret_cast<int *>(w + align_up(sizeof(int2) * (size_t)b.max_items, 256));
     const int64_t span = std::max<int64_t>(n_src, 1) - 1;  // largest source id
     b.key_shift = 0;
-    while ((span >> b.key_shift) >= ((int64_t)1 << kBandBits)) b.key_shift++;
+    while ((span >> b.key_shift) >= kBins) b.key_shift++;
     b.band_shift = kPlanBandShift;
     while ((span >> b.band_shift) + 1 > kPlanMaxBands) b.band_shift++;
     b.n_bands = with_bands ? (int)((span >> b.band_shift) + 1) : 1;
 
-    const int item_grid = (int)ceil_div(b.max_items, kBlock);
-    plan_init_kernel<<<std::min(item_grid, 4096), kBlock, 0, stream>>>(b);
+    plan_init_kernel<<<kBins / kPlanBlock, kPlanBlock, 0, stream>>>(b);
     YITU_LAUNCH_CHECK();
     if (n_rows > 0) {
-        plan_queue_kernel<<<(int)ceil_div(n_rows, kBlock), kBlock, 0, stream>>>(
+        plan_queue_kernel<<<(int)ceil_div(n_rows, kPlanBlock), kPlanBlock, 0, stream>>>(
             b, indptr, indices, (int)n_rows, (int)n_src, col_mask);
         YITU_LAUNCH_CHECK();
     }
-    plan_items_kernel<<<(int)ceil_div(b.max_rows, kWavesPerBlock), kBlock, 0, stream>>>(
+    plan_items_kernel<<<(int)ceil_div(b.max_rows, kPlanWaves), kPlanBlock, 0, stream>>>(
         b, indptr, indices, col_mask);
     YITU_LAUNCH_CHECK();
-    size_t temp_bytes = b.sort_temp_bytes;
-    YITU_HIP(rocprim::radix_sort_pairs(b.sort_temp, temp_bytes, b.keys_in, b.keys_out, b.vals_in,
-                                       b.order, (size_t)b.max_items, 0, 16, stream));
-    plan_records_kernel<<<item_grid, kBlock, 0, stream>>>(b);
+    plan_bin_starts_kernel<<<1, kPlanBlock, 0, stream>>>(b);
+    YITU_LAUNCH_CHECK();
+    plan_records_kernel<<<(int)ceil_div(b.max_items, kBlock), kBlock, 0, stream>>>(b);
     YITU_LAUNCH_CHECK();
     return 0;
 }

@@ -14,10 +14,11 @@ def coo_to_csr(rows, cols, n_rows, n_cols=None):
     _lib.require_device(rows, cols)
     if rows.shape != cols.shape or rows.dim() != 1:
         raise RuntimeError("rows and cols must be 1-D and equally long")
-    rows = rows.to(torch.int32).contiguous()
-    cols = cols.to(torch.int32).contiguous()
-    indptr, indices, nnz = _lib.ops().coo_to_csr(rows, cols, n_rows, n_cols)
-    count = int(nnz.item())
+    if rows.dtype != cols.dtype or rows.dtype not in (torch.int32, torch.int64):
+        rows, cols = rows.to(torch.int64), cols.to(torch.int64)
+    indptr, indices, info = _lib.ops().coo_to_csr(rows, cols, n_rows, n_cols)
+    count, longest = info.tolist()
     if count < 0:
         raise RuntimeError("edge list holds a node id outside [0, n_rows) x [0, n_cols)")
+    _lib.put_max_degree(indptr, longest)
     return indptr, indices[:count].clone()
