@@ -54,6 +54,13 @@ size_t yitu_plan_workspace_bytes(int64_t nnz);
 int yitu_plan_build(void *plan_device, size_t plan_bytes, const int32_t *indptr_device,
                     const int32_t *indices_device, int64_t n_rows, int64_t n_src, int64_t nnz,
                     int32_t col_mask, void *workspace_device, size_t workspace_bytes, void *stream);
+/* The plan of a graph without a row of 64 edges: the header alone (yitu_plan_header_bytes(), 256-byte
+ * aligned), which tells the row kernels how to deal rows to the XCDs. Valid only beside a
+ * max_degree below 64. */
+size_t yitu_plan_header_bytes(void);
+int yitu_plan_build_header(void *plan_device, const int32_t *indptr_device,
+                           const int32_t *indices_device, int64_t n_rows, int64_t n_src, int64_t nnz,
+                           int32_t col_mask, void *stream);
 
 /* ------------------------------------------------------------------------- */
 /* Module 1: YiTu_GNN.YiTu_GNN_kernel  (ccsrc/kernel/YiTu_GNN.cpp:247-258)     */

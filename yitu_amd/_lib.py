@@ -190,15 +190,16 @@ def row_plan(indptr, indices, n_src, col_mask):
     """Device buffer holding the row plan of (indptr, indices): band-ordered items of the long
     rows, a function of the graph only, built on the device on first use and kept while the
     index tensor lives. None when no row reaches the planning threshold and the graph is
-    small. A large graph without long rows still gets one: its header tells the row kernels
+    small. A larger graph without long rows gets the plan's header: it tells the row kernels
     whether most sources of a row lie near the row's own id, which decides how rows are dealt
     to the XCDs."""
-    if indices.numel() < (1 << 20) and max_degree(indptr) < 64:
+    longest = max_degree(indptr)
+    if longest < 64 and indices.numel() < ops().plan_min_edges:
         return None
     native = ops()
     plan = native.find_plan(indptr, indices, int(n_src), col_mask)
     if plan is None:
-        plan = native.build_plan(indptr, indices, int(n_src), col_mask)
+        plan = native.build_plan(indptr, indices, int(n_src), col_mask, longest)
         native.put_plan(indptr, indices, int(n_src), col_mask, _Built(plan, indices.device))
         watch(indices)
     return plan

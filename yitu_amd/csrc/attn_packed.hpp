@@ -170,7 +170,7 @@ __global__ __launch_bounds__(kBlock) void gat_rows_packed_kernel(GatParams p, in
     const int H = p.sp.H;
     const PackedGat<HV, KT> pg(p);
     packed_walk(
-        p.sp, R, blockIdx.x * kWavesPerBlock + threadIdx.x / kWave,
+        p.sp, R, row_block(p.sp, blockIdx.x, gridDim.x) * kWavesPerBlock + threadIdx.x / kWave,
         [&](const PackedChunk &c) {
             const bool act = lane < c.n;
             const int e = c.base + min(lane, c.n - 1);

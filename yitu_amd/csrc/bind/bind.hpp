@@ -22,6 +22,9 @@ using TensorVec = std::vector<Tensor>;
 constexpr int kColMask = 0xFFFFFF;
 constexpr int kAllBits = 0x7FFFFFFF;
 constexpr int64_t kLongRow = 64;  // rows of this many edges use the plan and its workspace
+// Graphs of fewer edges and no long row have no plan: their rows fit every L2, and a call is
+// its launch (at 124,000 edges in communities dealing the rows to the XCDs made 9.3 us 6.1).
+constexpr int64_t kPlanMinEdges = 1 << 15;
 
 // ---- checks ------------------------------------------------------------------------
 inline void check_device(const Tensor &t) {

@@ -159,7 +159,7 @@ RowState row_state(const Tensor &indptr, const Tensor &indices, int64_t n_src, i
     RowState s;
     s.max_degree = max_degree(indptr);
     // as _lib.row_plan: no plan for small graphs without long rows
-    if (s.max_degree < kLongRow && indices.numel() < (1 << 20)) return s;
+    if (s.max_degree < kLongRow && indices.numel() < kPlanMinEdges) return s;
     PyObject *wait = nullptr;
     if (find_built(plans, indptr, indices, n_src, mask, &wait, [&](Built &b) { s.plan = b.plan; })) {
         wait_for(wait, indices);

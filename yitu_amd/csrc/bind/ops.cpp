@@ -846,11 +846,19 @@ std::tuple<Tensor, Tensor, Tensor> csr_transpose(const Tensor &indptr, const Ten
     return {t_indptr, t_rows, t_perm};
 }
 
-Tensor build_plan(const Tensor &indptr, const Tensor &indices, int64_t n_src, int mask) {
+Tensor build_plan(const Tensor &indptr, const Tensor &indices, int64_t n_src, int mask,
+                  int64_t max_degree) {
     check_i32(indptr, "indptr", 1);
     check_i32(indices, "indices", 1);
     const int64_t nnz = indices.numel();
     Call c(indices);
+    if (max_degree >= 0 && max_degree < kLongRow) {
+        Tensor plan = c.empty({(int64_t)yitu_plan_header_bytes()}, at::kByte);
+        ok(yitu_plan_build_header(plan.data_ptr(), i32(indptr), i32(indices), indptr.numel() - 1,
+                                  n_src, nnz, mask, c.stream),
+           "yitu_plan_build_header");
+        return plan;
+    }
     Tensor plan = c.empty({(int64_t)yitu_plan_bytes(nnz)}, at::kByte);
     const auto ws = c.scratch(yitu_plan_workspace_bytes(nnz));
     ok(yitu_plan_build(plan.data_ptr(), plan.numel(), i32(indptr), i32(indices), indptr.numel() - 1,
@@ -948,7 +956,9 @@ void bind_ops(py::module_ &m) {
     m.def("coo_to_csr", &coo_to_csr);
     m.def("csr_transpose", &csr_transpose);
     m.def("longest_row", &longest_row);
-    m.def("build_plan", &build_plan);
+    m.def("build_plan", &build_plan, py::arg("indptr"), py::arg("indices"), py::arg("n_src"),
+          py::arg("mask"), py::arg("max_degree") = -1);
+    m.attr("plan_min_edges") = kPlanMinEdges;
 }
 
 }  // namespace yitu_bind

@@ -135,7 +135,7 @@ __device__ __forceinline__ void dot_rows_body(const DotParams &p, int block) {
 
 template <int VEC, int G, int KT>
 __global__ __launch_bounds__(kBlock) void dot_rows_kernel(DotParams p) {
-    dot_rows_body<VEC, G, KT>(p, blockIdx.x);
+    dot_rows_body<VEC, G, KT>(p, row_block(p.sp, blockIdx.x, gridDim.x));
 }
 
 }  // namespace yitu

@@ -144,7 +144,7 @@ template <int VEC, int G, int KT>
 __global__ __launch_bounds__(kBlock) void gat_rows_kernel(GatParams p) {
     const int lane = lane_id();
     const int rpw = rows_per_wave(p.sp.n_rows);
-    const int r0 = (blockIdx.x * kWavesPerBlock + wave_id()) * rpw;
+    const int r0 = (row_block(p.sp, blockIdx.x, gridDim.x) * kWavesPerBlock + wave_id()) * rpw;
     if (r0 >= p.sp.n_rows) return;
     const int n_here = min(rpw, p.sp.n_rows - r0);
     const int my_ptr = p.sp.indptr[r0 + min(lane, n_here)];
@@ -1307,7 +1307,7 @@ template <int LPH, int KT, bool FULL>
 __global__ __launch_bounds__(kBlock) void gat_src_rows_kernel(GatSrcParams p) {
     const int lane = lane_id();
     const int rpw = rows_per_wave(p.sp.n_rows);
-    const int r0 = (blockIdx.x * kWavesPerBlock + wave_id()) * rpw;
+    const int r0 = (row_block(p.sp, blockIdx.x, gridDim.x) * kWavesPerBlock + wave_id()) * rpw;
     if (r0 >= p.sp.n_rows) return;
     const int n_here = min(rpw, p.sp.n_rows - r0);
     const int my_ptr = p.sp.indptr[r0 + min(lane, n_here)];
@@ -1390,11 +1390,10 @@ static int gat_src_launch_shape(const GatSrcParams &p, bool has_items, const flo
                 p.head_mean, p.g_scale);
         YITU_LAUNCH_CHECK();
     }
-    const int row_grid = (int)ceil_div(p.sp.n_rows, kWavesPerBlock * rows_per_wave(p.sp.n_rows));
     // enough workgroups to walk the item list once (a second turn would mix source bands)
     const int item_grid = (int)std::min<int64_t>(
         ceil_div(p.sp.plan.max_items, kWavesPerBlock * kSrcItems), 1 << 20);
-    gat_src_rows_kernel<LPH, KT, FULL><<<row_grid, kBlock, 0, stream>>>(p);
+    gat_src_rows_kernel<LPH, KT, FULL><<<row_grid(p.sp.n_rows), kBlock, 0, stream>>>(p);
     YITU_LAUNCH_CHECK();
     if (has_items) {
         gat_src_items_kernel<LPH, KT, FULL><<<item_grid, kBlock, 0, stream>>>(p);
@@ -1525,14 +1524,13 @@ static int gat_fwd_launch(GatParams &p, bool has_items, hipStream_t stream) {
         // gather per edge, more waves in flight are worth more than longer chunk runs
         // (24 / 63 rows: 1.94 / 2.05 ms on a 2^21-node graph)
         const int R = std::min(packed_rows_per_wave(p.sp.n_rows), 24);
-        const int grid = (int)ceil_div(p.sp.n_rows, (int64_t)kWavesPerBlock * R);
+        int grid = (int)ceil_div(p.sp.n_rows, (int64_t)kWavesPerBlock * R);
+        if (grid >= 64) grid = (grid + 7) / 8 * 8;  // whole eighths for row_block
         if (hv == 4) gat_rows_packed_kernel<4, KT><<<grid, kBlock, 0, stream>>>(p, R);
         else if (hv == 2) gat_rows_packed_kernel<2, KT><<<grid, kBlock, 0, stream>>>(p, R);
         else gat_rows_packed_kernel<1, KT><<<grid, kBlock, 0, stream>>>(p, R);
     } else {
-        gat_rows_kernel<VEC, G, KT>
-            <<<(int)ceil_div(p.sp.n_rows, kWavesPerBlock * rows_per_wave(p.sp.n_rows)), kBlock, 0,
-               stream>>>(p);
+        gat_rows_kernel<VEC, G, KT><<<row_grid(p.sp.n_rows), kBlock, 0, stream>>>(p);
     }
     YITU_LAUNCH_CHECK();
     if (!has_items) return 0;

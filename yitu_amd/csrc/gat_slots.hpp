@@ -182,7 +182,7 @@ template <int LPF, int H>
 __global__ __launch_bounds__(kBlock) void gat_slot_rows_kernel(GatSrcParams p) {
     const int lane = lane_id();
     const int rpw = rows_per_wave(p.sp.n_rows);
-    const int r0 = (blockIdx.x * kWavesPerBlock + wave_id()) * rpw;
+    const int r0 = (row_block(p.sp, blockIdx.x, gridDim.x) * kWavesPerBlock + wave_id()) * rpw;
     if (r0 >= p.sp.n_rows) return;
     const int n_here = min(rpw, p.sp.n_rows - r0);
     const int my_ptr = p.sp.indptr[r0 + min(lane, n_here)];
@@ -301,9 +301,7 @@ static int gat_slots_launch(const GatSrcParams &p, bool has_items, const float *
         <<<(int)ceil_div(n_dst, kWavesPerBlock * 2 * (kWave / LPF)), kBlock, 0, stream>>>(
             const_cast<float4 *>(p.row_sq), g, out, query, p.stats, n_dst, p.sp.F);
     YITU_LAUNCH_CHECK();
-    gat_slot_rows_kernel<LPF, H>
-        <<<(int)ceil_div(p.sp.n_rows, kWavesPerBlock * rows_per_wave(p.sp.n_rows)), kBlock, 0,
-           stream>>>(p);
+    gat_slot_rows_kernel<LPF, H><<<row_grid(p.sp.n_rows), kBlock, 0, stream>>>(p);
     YITU_LAUNCH_CHECK();
     if (!has_items) return 0;
     // enough workgroups to walk the item list once (a second turn would mix source bands)

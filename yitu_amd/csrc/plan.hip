@@ -26,7 +26,7 @@ struct BuildBuffers {
     PlanCounters *counters;
     int4 *rows;
     int4 *records;
-    int *band_info;   // {log2 of the band width, number of bands, local edges, sampled edges}, in the plan header
+    int *band_info;   // the header words (plan.hpp)
     int4 *items;      // {first edge, end edge, index into rows[], row} in queue order
     int2 *place;      // {bin, rank in it} of every item, in queue order
     int *bin_start;   // items of every bin, then its first place
@@ -47,8 +47,10 @@ __global__ __launch_bounds__(kPlanBlock) void plan_init_kernel(BuildBuffers b) {
         b.band_info[1] = b.n_bands;
         b.band_info[kPlanInfoLocal] = 0;
         b.band_info[kPlanInfoSampled] = 0;
+        b.band_info[kPlanInfoLocalEdges] = 0;
+        b.band_info[kPlanInfoEdges] = 0;
     }
-    if (i < kBins) b.bin_start[i] = 0;
+    if (b.bin_start && i < kBins) b.bin_start[i] = 0;
 }
 
 // Every lane owns one row; the long rows of a workgroup are numbered with a
@@ -105,22 +107,27 @@ __global__ __launch_bounds__(kPlanBlock) void plan_queue_kernel(BuildBuffers b,
             local += c - own <= reach && own - c <= reach;
         }
     }
-    __shared__ int seen[2];  // sampled edges, local ones
-    if (threadIdx.x == 0) seen[0] = seen[1] = 0;
+    int weight = sampled ? deg * local / sampled : 0;  // local edges of the row
+    if (row == n_rows - 1) b.band_info[kPlanInfoEdges] = beg + deg;
+    __shared__ int seen[3];  // sampled edges, local ones, local edges
+    if (threadIdx.x == 0) seen[0] = seen[1] = seen[2] = 0;
     __syncthreads();
 #pragma unroll
     for (int o = kWave / 2; o > 0; o >>= 1) {
         sampled += __shfl_xor(sampled, o, kWave);
         local += __shfl_xor(local, o, kWave);
+        weight += __shfl_xor(weight, o, kWave);
     }
     if (lane_id() == 0 && sampled) {
         atomicAdd(&seen[0], sampled);
         atomicAdd(&seen[1], local);
+        atomicAdd(&seen[2], weight);
     }
     __syncthreads();
     if (threadIdx.x == 0 && seen[0]) {
         atomicAdd(&b.band_info[kPlanInfoSampled], seen[0]);
         if (seen[1]) atomicAdd(&b.band_info[kPlanInfoLocal], seen[1]);
+        if (seen[2]) atomicAdd(&b.band_info[kPlanInfoLocalEdges], seen[2]);
     }
     const bool longrow = deg >= kPlanThreshold;
     const int slot = block_rank(longrow, wave_sums, &block_base, &b.counters->n_rows);
@@ -291,12 +298,10 @@ __global__ __launch_bounds__(kBlock) void plan_records_kernel(BuildBuffers b) {
     if (place < n_items) b.records[place] = make_int4(it.x, it.y, i, it.w | single);
 }
 
-constexpr size_t kHeaderBytes = 512;  // counters | at byte 256: {log2 band width, bands}
-
 }  // namespace
 
 size_t plan_bytes(int64_t nnz) {
-    return kHeaderBytes + align_up(sizeof(int4) * (size_t)plan_max_rows(nnz), 256) +
+    return kPlanHeaderBytes + align_up(sizeof(int4) * (size_t)plan_max_rows(nnz), 256) +
            align_up(sizeof(int4) * (size_t)plan_max_items(nnz), 256);
 }
 
@@ -312,7 +317,7 @@ PlanView plan_view(const void *plan, int64_t nnz) {
     PlanView v{};
     const char *w = static_cast<const char *>(plan);
     v.counters = reinterpret_cast<const PlanCounters *>(w);
-    w += kHeaderBytes;
+    w += kPlanHeaderBytes;
     v.max_rows = (int)plan_max_rows(nnz);
     v.max_items = (int)plan_max_items(nnz);
     v.rows = reinterpret_cast<const int4 *>(w);
@@ -321,6 +326,33 @@ PlanView plan_view(const void *plan, int64_t nnz) {
     v.threshold = kPlanThreshold;
     v.info = reinterpret_cast<const int *>(static_cast<const char *>(plan) + 256);
     return v;
+}
+
+static void set_bands(BuildBuffers &b, int64_t n_src, bool with_bands) {
+    const int64_t span = std::max<int64_t>(n_src, 1) - 1;  // largest source id
+    b.key_shift = 0;
+    while ((span >> b.key_shift) >= kBins) b.key_shift++;
+    b.band_shift = kPlanBandShift;
+    while ((span >> b.band_shift) + 1 > kPlanMaxBands) b.band_shift++;
+    b.n_bands = with_bands ? (int)((span >> b.band_shift) + 1) : 1;
+}
+
+int plan_build_header(void *plan, const int32_t *indptr, const int32_t *indices, int64_t n_rows,
+                      int64_t n_src, int64_t nnz, int32_t col_mask, hipStream_t stream) {
+    YITU_REQUIRE(plan && (reinterpret_cast<uintptr_t>(plan) & 255u) == 0,
+                 "plan must be 256-byte aligned");
+    YITU_REQUIRE(n_rows < INT32_MAX && n_src < INT32_MAX && nnz < INT32_MAX, "size out of range");
+    BuildBuffers b{};  // (no room for rows or items: a long row would be an overflow)
+    b.counters = static_cast<PlanCounters *>(plan);
+    b.band_info = reinterpret_cast<int *>(static_cast<char *>(plan) + 256);
+    set_bands(b, n_src, true);
+    plan_init_kernel<<<1, kPlanBlock, 0, stream>>>(b);
+    YITU_LAUNCH_CHECK();
+    if (n_rows == 0) return 0;
+    plan_queue_kernel<<<(int)ceil_div(n_rows, kPlanBlock), kPlanBlock, 0, stream>>>(
+        b, indptr, indices, (int)n_rows, (int)n_src, col_mask);
+    YITU_LAUNCH_CHECK();
+    return 0;
 }
 
 int plan_build(void *plan, size_t plan_size, const int32_t *indptr, const int32_t *indices,
@@ -347,12 +379,7 @@ int plan_build(void *plan, size_t plan_size, const int32_t *indptr, const int32_
     w += align_up(sizeof(int4) * (size_t)b.max_items, 256);
     b.place = reinterpret_cast<int2 *>(w);
     b.bin_start = reinterpret_cast<int *>(w + align_up(sizeof(int2) * (size_t)b.max_items, 256));
-    const int64_t span = std::max<int64_t>(n_src, 1) - 1;  // largest source id
-    b.key_shift = 0;
-    while ((span >> b.key_shift) >= kBins) b.key_shift++;
-    b.band_shift = kPlanBandShift;
-    while ((span >> b.band_shift) + 1 > kPlanMaxBands) b.band_shift++;
-    b.n_bands = with_bands ? (int)((span >> b.band_shift) + 1) : 1;
+    set_bands(b, n_src, with_bands);
 
     plan_init_kernel<<<kBins / kPlanBlock, kPlanBlock, 0, stream>>>(b);
     YITU_LAUNCH_CHECK();
@@ -417,4 +444,14 @@ YITU_API int yitu_plan_build(void *plan, size_t plan_size, const int32_t *indptr
     YITU_REQUIRE(indptr && (nnz == 0 || indices), "null CSR");
     return plan_build(plan, plan_size, indptr, indices, n_rows, n_src, nnz, col_mask, true,
                       workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+YITU_API size_t yitu_plan_header_bytes(void) { return kPlanHeaderBytes; }
+YITU_API int yitu_plan_build_header(void *plan, const int32_t *indptr, const int32_t *indices,
+                                    int64_t n_rows, int64_t n_src, int64_t nnz, int32_t col_mask,
+                                    void *stream) {
+    YITU_REQUIRE(n_rows >= 0 && n_src >= 0 && nnz >= 0, "negative size");
+    YITU_REQUIRE(indptr && (nnz == 0 || indices), "null CSR");
+    return plan_build_header(plan, indptr, indices, n_rows, n_src, nnz, col_mask,
+                             static_cast<hipStream_t>(stream));
 }

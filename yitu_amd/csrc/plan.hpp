@@ -57,21 +57,25 @@ struct PlanView {
     const int *info;  // header words behind the counters (kPlanInfo*), or null
 };
 
-// Header words: {log2 of the band width, number of bands, local edges, sampled edges}.
+// Header words: {log2 of the band width, number of bands, local edges and sampled edges of the
+// builder's sample, local edges of all short rows as the sample has them, edges}.
 // The builder samples edges of the short rows; an edge is local when its source lies
-// near the row's own relative position in the id space. A graph three quarters of
-// whose sampled edges are local (community structure with ids to match, as planted
-// or as a reorder leaves them) has its short rows walked XCD by XCD. Measured on two
-// graphs of 2^21 vertices and 62 M edges, fp32 rows of 128 floats: planted
-// communities of 512 (97 % local) 4.43 ms round robin, 2.69 ms XCD by XCD (16 rows
-// per wave; 2.07 ms with 4); an R-MAT graph after the Rabbit-Order reorder (51 %
-// local: its rows of one or two edges sit next to their source, its hot sources are
-// everybody's) 2.70 and 2.94 ms.
+// near the row's own relative position in the id space. A graph one fifth of whose
+// edges are local ones of short rows (community structure with ids to match, as planted
+// or as a reorder leaves them) has its short rows walked XCD by XCD. Counted in edges, not
+// in sampled ones: an R-MAT graph after the Rabbit-Order reorder has half of its sampled
+// edges local, but those are rows of one or two edges; of all its edges it is 4 %, its hot
+// sources are everybody's, and it is 0.97 times as fast that way. Measured, round robin and
+// XCD by XCD, 150,000 vertices of 15 edges in communities of 512, fp32 rows of 100 floats:
+// 21 % local 171 and 152 us, 38 % 159 and 119, 51 % 152 and 99, 82 % 122 and 69; R-MAT
+// graphs, shuffled (1 %) or reordered (4 %), of 2^17, 2^18 and 2^21 vertices: 0.96 to 1.01.
 constexpr int kPlanInfoLocal = 2;
 constexpr int kPlanInfoSampled = 3;
+constexpr int kPlanInfoLocalEdges = 4;
+constexpr int kPlanInfoEdges = 5;
 
 __device__ __forceinline__ bool plan_says_local(const PlanView &v) {
-    return v.info && 4ll * v.info[kPlanInfoLocal] > 3ll * v.info[kPlanInfoSampled];
+    return v.info && 5ll * v.info[kPlanInfoLocalEdges] > v.info[kPlanInfoEdges];
 }
 
 inline int64_t plan_max_rows(int64_t nnz) { return nnz / kPlanThreshold + 1; }
@@ -88,6 +92,10 @@ int plan_build(void *plan, size_t plan_size, const int32_t *indptr, const int32_
                int64_t n_rows, int64_t n_src, int64_t nnz, int32_t col_mask, bool with_bands,
                void *workspace, size_t workspace_bytes, hipStream_t stream);
 PlanView plan_view(const void *plan, int64_t nnz);
+// A plan of a graph without rows of kPlanThreshold edges: its header alone (kPlanHeaderBytes).
+constexpr size_t kPlanHeaderBytes = 512;  // counters | at byte 256: the header words
+int plan_build_header(void *plan, const int32_t *indptr, const int32_t *indices, int64_t n_rows,
+                      int64_t n_src, int64_t nnz, int32_t col_mask, hipStream_t stream);
 // A view that plans nothing (every row is handled by the row kernels).
 inline PlanView plan_none() {
     PlanView v{};

@@ -46,8 +46,7 @@ __global__ __launch_bounds__(kBlock) void dot_items_kernel(DotParams p) {
 template <int VEC, int G, int KT>
 static int dot_launch(const DotParams &p, bool has_items, hipStream_t stream) {
     if (!p.long_rows_only) {
-        dot_rows_kernel<VEC, G, KT>
-            <<<(int)ceil_div(p.sp.n_rows, kWavesPerBlock * rows_per_wave(p.sp.n_rows)), kBlock, 0, stream>>>(p);
+        dot_rows_kernel<VEC, G, KT><<<row_grid(p.sp.n_rows), kBlock, 0, stream>>>(p);
         YITU_LAUNCH_CHECK();
     }
     if (has_items) {

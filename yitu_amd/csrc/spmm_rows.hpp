@@ -293,6 +293,11 @@ __device__ __forceinline__ int row_block(const SpmmParams &p, int block, int n_b
     return (block & 7) * (n_blocks >> 3) + (block >> 3);
 }
 
+inline int row_grid(int n_rows) {
+    const int grid = (int)ceil_div(n_rows, kWavesPerBlock * rows_per_wave(n_rows));
+    return grid >= 64 ? (grid + 7) / 8 * 8 : grid;  // whole eighths for row_block
+}
+
 // Row kernel: a wave walks rows_per_wave consecutive rows. Their bounds come from
 // one coalesced indptr load, their edges from a sliding 64-edge window, so a
 // short row costs one round of feature gathers and nothing else that waits on

@@ -57,9 +57,8 @@ def transposed(indptr, indices, n_src):
         t = _Transposed()
         t.n_src = int(n_src)
         t.t_indptr, t.t_rows, t.t_perm = native.csr_transpose(indptr, indices, int(n_src))
-        # (the plan of a large graph needs no word from the GPU: it is under way before the wait)
-        t.plan_t = _lib.row_plan(t.t_indptr, t.t_rows, indptr.numel() - 1, 0x7FFFFFFF)
         t.max_degree_t = _lib.max_degree(t.t_indptr)
+        t.plan_t = _lib.row_plan(t.t_indptr, t.t_rows, indptr.numel() - 1, 0x7FFFFFFF)
         native.put_by_source(indptr, indices, int(n_src), _lib._Built(t, indices.device))
         _lib.watch(indices)
     return t
