@@ -628,7 +628,8 @@ int yitu_gemm_bf16_tn_typed(float *const *c_device_ptrs, const void *const *a_bf
  * Backward: yitu_relu_layernorm_backward (d_pre with a row stride, partial sums
  * of the affine gradients: [yitu_tattn_partial_rows(n_rows), 2 n_cols], gamma's
  * then beta's), dx_r = d_pre . w_r, yitu_tattn_backward (dq2 [n_dst, 2 dim_out]
- * columns 0..dim_out-1, dkv [n_edges, 2 dim_out]; scratch [n_edges, n_heads, 2]),
+ * columns 0..dim_out-1, dkv [n_edges, 2 dim_out]; scratch [n_edges, n_heads, 2]; ld is
+ * the row length of dx_r),
  * dx_kv = dkv . w_kv, dx_q = dq2 . w_q2, the weight gradients as transposed
  * products, yitu_tattn_finalize (grad_h [n_dst + n_edges, dim_node], grad_f, either
  * may be NULL; partial sums of the time encoder's gradients
@@ -649,6 +650,18 @@ int yitu_tattn_prepare(float *x_kv_device, float *x_q_device, float *x_r_device,
                        const float *w_out_device, const float *b_out_device, int64_t n_dst,
                        int64_t n_edges, int64_t dim_node, int64_t dim_edge, int64_t dim_time,
                        int64_t dim_out, int64_t ld, void *stream);
+/* The same with node i's features in row nodes[i] of h (nodes NULL: row i; unchecked). */
+int yitu_tattn_prepare_nodes(float *x_kv_device, float *x_q_device, float *x_r_device,
+                             float *w_kv_device, float *w_q2_device, float *w_r_device,
+                             const float *h_device, const int32_t *nodes_device,
+                             const float *f_device, const float *dt_device,
+                             const float *time_w_device, const float *time_b_device,
+                             const float *w_q_device, const float *b_q_device,
+                             const float *w_k_device, const float *b_k_device,
+                             const float *w_v_device, const float *b_v_device,
+                             const float *w_out_device, const float *b_out_device, int64_t n_dst,
+                             int64_t n_edges, int64_t dim_node, int64_t dim_edge, int64_t dim_time,
+                             int64_t dim_out, int64_t ld, void *stream);
 int yitu_tattn_forward(float *x_r_device, float *attn_device, const float *q2_device,
                        const float *kv_device, const int32_t *indptr_device, int64_t n_dst,
                        int64_t n_edges, int64_t dim_out, int64_t n_heads, int64_t ld, void *stream);
@@ -670,6 +683,17 @@ int yitu_tattn_finalize(float *grad_h_device, float *grad_f_device, float *parti
                         const float *time_w_device, const float *time_b_device, int64_t n_dst,
                         int64_t n_edges, int64_t dim_node, int64_t dim_edge, int64_t dim_time,
                         int64_t dim_out, int64_t ld, void *stream);
+/* The same with the input gradients given as column windows: dx_kv holds ld_kv columns of the
+ * augmented input from first_kv on (from dim_node + dim_edge at most where neither grad_h nor
+ * grad_f is wanted, from dim_node where grad_h is not), dx_q likewise, dx_r (rows of ld_r) its
+ * first dim_out (+ dim_node) columns. */
+int yitu_tattn_finalize_windows(float *grad_h_device, float *grad_f_device, float *partial_device,
+                                const float *dx_kv_device, int64_t ld_kv, int64_t first_kv,
+                                const float *dx_q_device, int64_t ld_q, int64_t first_q,
+                                const float *dx_r_device, int64_t ld_r, const float *dt_device,
+                                const float *time_w_device, const float *time_b_device,
+                                int64_t n_dst, int64_t n_edges, int64_t dim_node, int64_t dim_edge,
+                                int64_t dim_time, int64_t dim_out, int64_t ld, void *stream);
 int yitu_partial_sums(float *out_a_device, const float *partial_a_device, int64_t rows_a,
                       int64_t cols_a, float *out_b_device, const float *partial_b_device,
                       int64_t rows_b, int64_t cols_b, void *stream);
@@ -716,6 +740,17 @@ int yitu_tsample_recent(int32_t *row_device, int32_t *col_device, int32_t *eid_o
                         const int32_t *roots_device, const float *root_ts_device, int64_t n_roots,
                         int fan, int prop_time, void *workspace_device, size_t workspace_bytes,
                         void *stream);
+/* The same, with the by-root structure of the sampled block: block_indptr [n_roots + 1], and the
+ * count also in block_indptr[n_roots]. */
+int yitu_tsample_recent_block(int32_t *block_indptr_device, int32_t *row_device,
+                              int32_t *col_device, int32_t *eid_out_device, float *ts_out_device,
+                              float *dts_out_device, int32_t *nodes_out_device,
+                              long long *n_edges_out_device, int32_t *cursor_device,
+                              const int32_t *indptr_device, const int32_t *indices_device,
+                              const int32_t *eid_device, const float *ts_device, int64_t n_nodes,
+                              const int32_t *roots_device, const float *root_ts_device,
+                              int64_t n_roots, int fan, int prop_time, void *workspace_device,
+                              size_t workspace_bytes, void *stream);
 
 /*
  * The other modes of ParallelSampler (sampler_core.cpp:201-359), as the two pieces its
@@ -811,7 +846,7 @@ int yitu_csr_transpose(int32_t *t_indptr_device, int32_t *t_rows_device, int32_t
                        size_t workspace_bytes, void *stream);
 
 /*
- * Sums of row ranges of one matrix: out[range r, row i] = act((sum_k x[source_k + i]) / divisor),
+ * Sums of row ranges of one matrix: out[range r, row i] = act((sum_k x[source_k + i]) * factor),
  * out [n_rows, width], x [.., width], both contiguous. What a heterogeneous layer does behind
  * its products (sum over the relations of a node type, mean, activation;
  * test/common/model.py:137-171, 198-236) for all node types in one launch. ranges tile the rows
@@ -825,7 +860,7 @@ typedef struct {
     int32_t rows;
     int32_t first_source; /* index into sources */
     int32_t n_sources;    /* 0: the rows are zero */
-    float divisor;
+    float factor;
     int32_t act;          /* YITU_FOLD_* */
     float alpha;          /* of the ELU */
     int32_t pad;

@@ -514,4 +514,5 @@ PYBIND11_MODULE(_ops, m) {
     yitu_bind::bind_ops(m);
     yitu_bind::bind_autograd(m);
     yitu_bind::bind_batched(m);
+    yitu_bind::bind_temporal(m);
 }

@@ -28,8 +28,9 @@ struct FoldPlan : torch::CustomClassHolder {
         for (const Range &r : list) {
             TORCH_CHECK(r.rows >= 0 && r.divisor != 0.0 && r.act >= YITU_FOLD_NONE &&
                             r.act <= YITU_FOLD_ELU, "fold: bad range");
+            // (torch divides by a number as it multiplies by its reciprocal)
             table.push_back({(int32_t)rows_out, (int32_t)r.rows, (int32_t)from.size(),
-                             (int32_t)r.sources.size(), (float)r.divisor, (int32_t)r.act,
+                             (int32_t)r.sources.size(), 1.0f / (float)r.divisor, (int32_t)r.act,
                              (float)r.alpha, 0});
             rows_out += r.rows;
             for (int64_t s : r.sources) {

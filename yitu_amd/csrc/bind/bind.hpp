@@ -191,5 +191,6 @@ void bind_ops(py::module_ &m);
 
 void bind_autograd(py::module_ &m);
 void bind_batched(py::module_ &m);
+void bind_temporal(py::module_ &m);
 
 }  // namespace yitu_bind

@@ -1,4 +1,4 @@
-// Sums of row ranges: out[range r, row i] = act_r((sum_k x[source_rk + i]) / div_r), and its
+// Sums of row ranges: out[range r, row i] = act_r((sum_k x[source_rk + i]) * factor_r), and its
 // backward. The batched form of a heterogeneous model keeps the rows of all its relations in
 // one buffer (yitu_amd/xgnn_h/batch.py); what stands between two batched products (the sum
 // over the relations that reach a node type, the division by their number, the activation;
@@ -48,14 +48,14 @@ __global__ __launch_bounds__(kBlock) void fold_rows_kernel(float *__restrict__ o
     }
 #pragma unroll
     for (int j = 0; j < VEC; j++) {
-        if (r.divisor != 1.0f) v[j] /= r.divisor;
+        if (r.factor != 1.0f) v[j] *= r.factor;
         if (r.act == YITU_FOLD_RELU) v[j] = v[j] > 0.0f || v[j] != v[j] ? v[j] : 0.0f;
         if (r.act == YITU_FOLD_ELU) v[j] = v[j] > 0.0f ? v[j] : r.alpha * expm1f(v[j]);
     }
     store_row<VEC>(out + i * VEC, v);
 }
 
-// grad_x of every source of a range = grad_out act'(out) / div. ReLU and ELU are
+// grad_x of every source of a range = grad_out act'(out) factor. ReLU and ELU are
 // differentiated at their own result (out > 0; alpha e^v = out + alpha).
 template <int VEC>
 __global__ __launch_bounds__(kBlock) void fold_rows_bwd_kernel(
@@ -79,7 +79,7 @@ __global__ __launch_bounds__(kBlock) void fold_rows_bwd_kernel(
     }
 #pragma unroll
     for (int j = 0; j < VEC; j++)
-        if (r.divisor != 1.0f) g[j] /= r.divisor;
+        if (r.factor != 1.0f) g[j] *= r.factor;
     for (int k = 0; k < r.n_sources; k++) {
         const int64_t to = (int64_t)sources[r.first_source + k] + row - r.out_begin;
         store_row<VEC>(grad_x + (to * row_vecs + c) * VEC, g);

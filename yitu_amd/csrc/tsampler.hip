@@ -37,80 +37,154 @@ __global__ __launch_bounds__(kBlock) void ts_reset_kernel(int32_t *__restrict__ 
     if (i < n_nodes) cursor[i] = indptr[i];
 }
 
+// A wave per root in each of these: two thousand roots one per thread were 32 waves, each
+// walking a chain of dependent loads (count, scan and fill of 2,048 roots x 20: 6 + 8 + 17 us, now
+// 4 + 5 + 4).
+//
+// The last edge with ts <= thr by a search of 64 probes a step: lane l looks at the last edge of
+// the l-th of 64 equal parts.
 __global__ __launch_bounds__(kBlock) void ts_advance_kernel(
     int32_t *__restrict__ cursor, const int32_t *__restrict__ indptr, const float *__restrict__ ts,
     const int32_t *__restrict__ roots, const float *__restrict__ root_ts, int64_t n_roots,
-    int32_t n_nodes, int *__restrict__ bad) {
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    int32_t n_nodes) {
+    const int64_t i = (int64_t)blockIdx.x * kWavesPerBlock + wave_id();
     if (i >= n_roots) return;
     const int32_t n = roots[i];
-    if (n < 0 || n >= n_nodes) {
-        atomicExch(bad, 1);
-        return;
-    }
+    if (n < 0 || n >= n_nodes) return;  // (the count below reports it)
     const float thr = query_threshold(root_ts[i]);
-    int32_t lo = indptr[n], hi = indptr[n + 1];  // first edge with ts > thr
-    const int32_t first = lo;
+    const int32_t first = indptr[n];
+    int32_t lo = first, hi = indptr[n + 1];  // the first edge with ts > thr is in [lo, hi]
     while (lo < hi) {
-        const int32_t mid = lo + ((hi - lo) >> 1);
-        if (ts[mid] <= thr) lo = mid + 1; else hi = mid;
+        const int32_t step = (hi - lo + kWave - 1) / kWave;
+        const int64_t at = (int64_t)lo + (int64_t)(lane_id() + 1) * step - 1;
+        const unsigned long long beyond = __ballot(at >= hi || !(ts[at] <= thr));
+        if (!beyond) {  // (64 parts cover [lo, hi): the last lane's probe was not beyond it)
+            lo = hi;
+            break;
+        }
+        const int part = __ffsll(beyond) - 1;
+        const int64_t end = (int64_t)lo + (int64_t)(part + 1) * step - 1;
+        lo += part * step;
+        hi = (int32_t)min((int64_t)hi, end);
     }
-    if (lo - 1 >= first) atomicMax(&cursor[n], lo - 1);
+    if (lane_id() == 0 && lo - 1 >= first) atomicMax(&cursor[n], lo - 1);
 }
 
+// Edges a root keeps, of the `fan` before its cursor; -1 for a root that is no node.
 __global__ __launch_bounds__(kBlock) void ts_count_kernel(
     int32_t *__restrict__ counts, const int32_t *__restrict__ cursor,
     const int32_t *__restrict__ indptr, const float *__restrict__ ts,
     const int32_t *__restrict__ roots, const float *__restrict__ root_ts, int64_t n_roots,
     int32_t n_nodes, int fan) {
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * kWavesPerBlock + wave_id();
     if (i >= n_roots) return;
     const int32_t n = roots[i];
-    int32_t cnt = 0;
+    int32_t cnt = -1;
     if (n >= 0 && n < n_nodes) {
         const float thr = query_threshold(root_ts[i]);
-        const int32_t first = indptr[n], e = cursor[n];
-        for (int32_t k = e; k > max(first, e - fan); k--) cnt += ts[k] < thr ? 1 : 0;
+        const int32_t e = cursor[n], stop = max(indptr[n], e - fan);
+        cnt = 0;
+        for (int32_t k = e; k > stop; k -= kWave) {
+            const int32_t mine = k - lane_id();
+            cnt += __popcll(__ballot(mine > stop && ts[max(mine, stop)] < thr));
+        }
     }
-    counts[i] = cnt;
+    if (lane_id() == 0) counts[i] = cnt;
+}
+
+// block_indptr = exclusive prefix sums of the counts, by one workgroup in chunks of 16,384;
+// *n_edges_out = their total, or -1 with a root that is no node.
+__global__ __launch_bounds__(1024) void ts_starts_kernel(int32_t *__restrict__ block_indptr,
+                                                         long long *__restrict__ n_edges_out,
+                                                         const int32_t *__restrict__ counts,
+                                                         int64_t n_roots) {
+    constexpr int kEach = 16, kChunk = 1024 * kEach;
+    __shared__ int sums[16];
+    __shared__ int bad;
+    const int lane = lane_id(), wave = threadIdx.x / kWave;
+    if (threadIdx.x == 0) bad = 0;
+    __syncthreads();
+    int carry = 0;
+    for (int64_t base = 0; base < n_roots; base += kChunk) {
+        int v[kEach], own = 0;
+#pragma unroll
+        for (int k = 0; k < kEach; k++) {
+            const int64_t i = base + (int64_t)threadIdx.x * kEach + k;
+            v[k] = i < n_roots ? counts[i] : 0;
+            if (v[k] < 0) {
+                bad = 1;
+                v[k] = 0;
+            }
+            own += v[k];
+        }
+        int pre = own;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const int x = __shfl_up(pre, o, kWave);
+            if (lane >= o) pre += x;
+        }
+        if (lane == kWave - 1) sums[wave] = pre;
+        __syncthreads();
+        int at = carry + pre - own, all = 0;
+        for (int w = 0; w < 16; w++) {
+            at += w < wave ? sums[w] : 0;
+            all += sums[w];
+        }
+#pragma unroll
+        for (int k = 0; k < kEach; k++) {
+            const int64_t i = base + (int64_t)threadIdx.x * kEach + k;
+            if (i < n_roots) block_indptr[i] = at;
+            at += v[k];
+        }
+        carry += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        block_indptr[n_roots] = carry;
+        *n_edges_out = bad ? -1 : carry;
+    }
 }
 
 struct FillArgs {
     int32_t *row, *col, *eid_out, *nodes_out;
     float *ts_out, *dts_out;
-    long long *n_edges_out;
-    const int32_t *offsets, *counts, *cursor, *indptr, *indices, *eid, *roots;
+    const int32_t *offsets, *cursor, *indptr, *indices, *eid, *roots;
     const float *ts, *root_ts;
-    const int *bad;
     int64_t n_roots;
     int32_t n_nodes;
     int fan, prop_time;
 };
 
 __global__ __launch_bounds__(kBlock) void ts_fill_kernel(FillArgs a) {
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * kWavesPerBlock + wave_id();
     if (i >= a.n_roots) return;
-    if (i == a.n_roots - 1)
-        *a.n_edges_out = *a.bad ? -1 : (long long)a.offsets[i] + a.counts[i];
+    const int lane = lane_id();
     const int32_t n = a.roots[i];
     const float t = a.root_ts[i];
-    a.nodes_out[i] = n;
-    a.ts_out[i] = t;
-    a.dts_out[i] = 0.0f;
+    if (lane == 0) {
+        a.nodes_out[i] = n;
+        a.ts_out[i] = t;
+        a.dts_out[i] = 0.0f;
+    }
     if (n < 0 || n >= a.n_nodes) return;
     const float thr = query_threshold(t);
-    const int32_t first = a.indptr[n], e = a.cursor[n];
-    int64_t w = a.offsets[i];
-    for (int32_t k = e; k > max(first, e - a.fan); k--) {
-        if (a.ts[k] < thr) {
+    const int32_t e = a.cursor[n], stop = max(a.indptr[n], e - a.fan);
+    int64_t base = a.offsets[i];
+    for (int32_t k = e; k > stop; k -= kWave) {
+        const int32_t mine = k - lane;
+        const float when = a.ts[max(mine, stop)];
+        const bool keep = mine > stop && when < thr;
+        const unsigned long long kept = __ballot(keep);
+        if (keep) {
+            const int64_t w = base + __popcll(kept & ((1ull << lane) - 1));
             a.row[w] = (int32_t)i;
             a.col[w] = (int32_t)(a.n_roots + w);
-            a.eid_out[w] = a.eid[k];
-            a.ts_out[a.n_roots + w] = a.prop_time ? t : a.ts[k];
-            a.dts_out[a.n_roots + w] = t - a.ts[k];
-            a.nodes_out[a.n_roots + w] = a.indices[k];
-            w++;
+            a.eid_out[w] = a.eid[mine];
+            a.ts_out[a.n_roots + w] = a.prop_time ? t : when;
+            a.dts_out[a.n_roots + w] = t - when;
+            a.nodes_out[a.n_roots + w] = a.indices[mine];
         }
+        base += __popcll(kept);
     }
 }
 
@@ -306,7 +380,47 @@ YITU_API int yitu_tsample_reset(int32_t *cursor, const int32_t *indptr, int64_t 
 
 YITU_API size_t yitu_tsample_workspace_bytes(int64_t n_roots) {
     const int64_t n = std::max<int64_t>(n_roots, 1);
-    return 256 + 2 * align_up(sizeof(int32_t) * (size_t)n, 256) + align_up(scan_bytes(n), 256);
+    return 2 * align_up(sizeof(int32_t) * (size_t)(n + 1), 256);
+}
+
+YITU_API int yitu_tsample_recent_block(int32_t *block_indptr, int32_t *row, int32_t *col,
+                                       int32_t *eid_out, float *ts_out, float *dts_out,
+                                       int32_t *nodes_out, long long *n_edges_out, int32_t *cursor,
+                                       const int32_t *indptr, const int32_t *indices,
+                                       const int32_t *eid, const float *ts, int64_t n_nodes,
+                                       const int32_t *roots, const float *root_ts, int64_t n_roots,
+                                       int fan, int prop_time, void *workspace,
+                                       size_t workspace_bytes, void *stream_) {
+    hipStream_t stream = static_cast<hipStream_t>(stream_);
+    YITU_REQUIRE(n_nodes >= 0 && n_roots >= 0 && fan >= 0, "negative size");
+    YITU_REQUIRE(n_nodes < INT32_MAX && n_roots * (int64_t)(fan + 1) < INT32_MAX,
+                 "size out of range");
+    YITU_REQUIRE(n_edges_out && block_indptr, "null output");
+    YITU_REQUIRE(workspace && workspace_bytes >= yitu_tsample_workspace_bytes(n_roots) &&
+                     (reinterpret_cast<uintptr_t>(workspace) & 255u) == 0,
+                 "workspace too small or not 256-byte aligned: need %zu bytes",
+                 yitu_tsample_workspace_bytes(n_roots));
+    int32_t *counts = static_cast<int32_t *>(workspace);
+    if (n_roots > 0) {
+        YITU_REQUIRE(row && col && eid_out && ts_out && dts_out && nodes_out && cursor && indptr &&
+                         roots && root_ts,
+                     "null pointer");
+        const int grid = (int)ceil_div(n_roots, kWavesPerBlock);
+        ts_advance_kernel<<<grid, kBlock, 0, stream>>>(cursor, indptr, ts, roots, root_ts, n_roots,
+                                                       (int32_t)n_nodes);
+        YITU_LAUNCH_CHECK();
+        ts_count_kernel<<<grid, kBlock, 0, stream>>>(counts, cursor, indptr, ts, roots, root_ts,
+                                                     n_roots, (int32_t)n_nodes, fan);
+        YITU_LAUNCH_CHECK();
+    }
+    ts_starts_kernel<<<1, 1024, 0, stream>>>(block_indptr, n_edges_out, counts, n_roots);
+    YITU_LAUNCH_CHECK();
+    if (n_roots == 0) return 0;
+    const FillArgs a{row, col, eid_out, nodes_out, ts_out, dts_out, block_indptr, cursor, indptr,
+                     indices, eid, roots, ts, root_ts, n_roots, (int32_t)n_nodes, fan, prop_time};
+    ts_fill_kernel<<<(int)ceil_div(n_roots, kWavesPerBlock), kBlock, 0, stream>>>(a);
+    YITU_LAUNCH_CHECK();
+    return 0;
 }
 
 YITU_API int yitu_tsample_recent(int32_t *row, int32_t *col, int32_t *eid_out, float *ts_out,
@@ -315,69 +429,17 @@ YITU_API int yitu_tsample_recent(int32_t *row, int32_t *col, int32_t *eid_out, f
                                  const int32_t *eid, const float *ts, int64_t n_nodes,
                                  const int32_t *roots, const float *root_ts, int64_t n_roots,
                                  int fan, int prop_time, void *workspace, size_t workspace_bytes,
-                                 void *stream_) {
-    hipStream_t stream = static_cast<hipStream_t>(stream_);
-    YITU_REQUIRE(n_nodes >= 0 && n_roots >= 0 && fan >= 0, "negative size");
-    YITU_REQUIRE(n_nodes < INT32_MAX && n_roots * (int64_t)(fan + 1) < INT32_MAX,
-                 "size out of range");
-    YITU_REQUIRE(n_edges_out, "null output");
-    YITU_REQUIRE(workspace && workspace_bytes >= yitu_tsample_workspace_bytes(n_roots) &&
-                     (reinterpret_cast<uintptr_t>(workspace) & 255u) == 0,
-                 "workspace too small or not 256-byte aligned: need %zu bytes",
-                 yitu_tsample_workspace_bytes(n_roots));
-    int rc = fill_zero(static_cast<float *>(workspace), 64, stream);  // flag, and the count below
-    if (rc) return rc;
-    if (n_roots == 0) {
-        // *n_edges_out = 0: reuse the zeroed words
-        YITU_HIP(hipMemcpyAsync(n_edges_out, workspace, sizeof(long long), hipMemcpyDeviceToDevice,
-                                stream));
-        return 0;
-    }
-    YITU_REQUIRE(row && col && eid_out && ts_out && dts_out && nodes_out && cursor && indptr &&
-                     roots && root_ts,
-                 "null pointer");
-    char *w = static_cast<char *>(workspace);
-    int *bad = reinterpret_cast<int *>(w);
-    w += 256;
-    const size_t arr = align_up(sizeof(int32_t) * (size_t)n_roots, 256);
-    int32_t *counts = reinterpret_cast<int32_t *>(w);
-    int32_t *offsets = reinterpret_cast<int32_t *>(w + arr);
-    void *temp = w + 2 * arr;
-    const int grid = (int)ceil_div(n_roots, kBlock);
-    ts_advance_kernel<<<grid, kBlock, 0, stream>>>(cursor, indptr, ts, roots, root_ts, n_roots,
-                                                   (int32_t)n_nodes, bad);
-    YITU_LAUNCH_CHECK();
-    ts_count_kernel<<<grid, kBlock, 0, stream>>>(counts, cursor, indptr, ts, roots, root_ts,
-                                                 n_roots, (int32_t)n_nodes, fan);
-    YITU_LAUNCH_CHECK();
-    size_t bytes = scan_bytes(n_roots);
-    YITU_HIP(rocprim::exclusive_scan(temp, bytes, counts, offsets, 0, (size_t)n_roots,
-                                     rocprim::plus<int32_t>(), stream));
-    FillArgs a{};
-    a.row = row;
-    a.col = col;
-    a.eid_out = eid_out;
-    a.nodes_out = nodes_out;
-    a.ts_out = ts_out;
-    a.dts_out = dts_out;
-    a.n_edges_out = n_edges_out;
-    a.offsets = offsets;
-    a.counts = counts;
-    a.cursor = cursor;
-    a.indptr = indptr;
-    a.indices = indices;
-    a.eid = eid;
-    a.roots = roots;
-    a.ts = ts;
-    a.root_ts = root_ts;
-    a.bad = bad;
-    a.n_roots = n_roots;
-    a.n_nodes = (int32_t)n_nodes;
-    a.fan = fan;
-    a.prop_time = prop_time;
-    ts_fill_kernel<<<grid, kBlock, 0, stream>>>(a);
-    YITU_LAUNCH_CHECK();
-    return 0;
+                                 void *stream) {
+    YITU_REQUIRE(n_roots >= 0 && workspace &&
+                     workspace_bytes >= yitu_tsample_workspace_bytes(n_roots),
+                 "workspace too small: need %zu bytes", yitu_tsample_workspace_bytes(n_roots));
+    int32_t *block_indptr = reinterpret_cast<int32_t *>(
+        static_cast<char *>(workspace) +
+        align_up(sizeof(int32_t) * (size_t)(std::max<int64_t>(n_roots, 1) + 1), 256));
+    return yitu_tsample_recent_block(block_indptr, row, col, eid_out, ts_out, dts_out, nodes_out,
+                                     n_edges_out, cursor, indptr, indices, eid, ts, n_nodes, roots,
+                                     root_ts, n_roots, fan, prop_time, workspace, workspace_bytes,
+                                     stream);
 }
 
 YITU_API int yitu_tsample_advance(int32_t *cursor, const int32_t *indptr, const float *ts,

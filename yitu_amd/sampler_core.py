@@ -124,9 +124,10 @@ class DeviceTemporalGraphBlock:
     """A sampled block whose arrays are torch tensors on the GPU; the accessors
     mirror TemporalGraphBlock (``.cpu_block()`` converts to the numpy form)."""
 
-    def __init__(self, row, col, eid, ts, dts, nodes, dim_in, dim_out):
+    def __init__(self, row, col, eid, ts, dts, nodes, dim_in, dim_out, indptr=None, id_bound=None):
         self._a = (row, col, eid, ts, dts, nodes)
         self._dim_in, self._dim_out = int(dim_in), int(dim_out)
+        self._indptr, self._id_bound = indptr, id_bound
 
     def row(self):
         return self._a[0]
@@ -151,6 +152,14 @@ class DeviceTemporalGraphBlock:
 
     def dim_out(self):
         return self._dim_out
+
+    def indptr(self):
+        """First edge of every root slot, [dim_out + 1] int32; None if the sampler made none."""
+        return self._indptr
+
+    def id_bound(self):
+        """Every id in ``nodes`` is below this; None if the sampler knows no bound."""
+        return self._id_bound
 
     def cpu_block(self):
         return TemporalGraphBlock(*[t.cpu().numpy() for t in self._a], self._dim_in, self._dim_out)
@@ -179,6 +188,10 @@ class GpuParallelSampler:
         self._eid = to(eid, np.int32)
         self._ts = to(ts, np.float32)
         self._n_nodes = self._indptr.numel() - 1
+        # roots are nodes (checked on the device), neighbours are what indices holds
+        neighbours = np.asarray(indices)
+        self._id_bound = None if neighbours.size and int(neighbours.min()) < 0 else \
+            max(self._n_nodes, int(neighbours.max()) + 1 if neighbours.size else 0)
         self._fan = [int(x) for x in num_neighbors[:num_layers]]
         self._prop_time = bool(prop_time)
         self._recent = bool(recent)
@@ -217,20 +230,11 @@ class GpuParallelSampler:
                                         nodes[:n + m], n + m, n)
 
     def _layer(self, roots, root_ts, fan):
-        import torch
         from . import _lib
         n = roots.numel()
-        outs = self._outputs(n, fan)
-        ws = _lib.workspace(_lib.size_fn("yitu_tsample_workspace_bytes")(_lib.c_i64(n)), self._dev)
-        with torch.cuda.device(self._dev):
-            rc = _lib.lib().yitu_tsample_recent(
-                *[_lib.ptr(t) for t in outs], _lib.ptr(self._cursor), _lib.ptr(self._indptr),
-                _lib.ptr(self._indices), _lib.ptr(self._eid), _lib.ptr(self._ts),
-                _lib.c_i64(self._n_nodes), _lib.ptr(roots), _lib.ptr(root_ts), _lib.c_i64(n),
-                _lib.c_int(fan), _lib.c_int(int(self._prop_time)), _lib.ptr(ws),
-                _lib.c_size(ws.numel()), _lib.stream_ptr(self._dev))
-        _lib.check(rc, "yitu_tsample_recent")
-        return self._block(outs, n)
+        *block, indptr = _lib.ops().tsample_recent(self._cursor, self._indptr, self._indices, self._eid,
+                                                   self._ts, roots, root_ts, fan, self._prop_time)
+        return DeviceTemporalGraphBlock(*block, block[5].numel(), n, indptr, self._id_bound)
 
     def _advance(self, k, roots, root_ts, offset):
         import torch
