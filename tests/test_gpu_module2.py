@@ -677,3 +677,24 @@ def test_spmm_backward_constant_weights_take_the_by_source_copy(dev):
     for _ in range(3):
         got = graph_ext.spmm_backward(values, ip, ix, xd, gyd, need_grad_a=False)[1]
         assert_close(got, 2 * torch.as_tensor(want), abs_sum=2 * abs_gx)
+
+
+def test_spmm_backward_refuses_other_shapes_with_kept_weights(dev):
+    """With a kept by-source copy of the weights grad_x is a forward product over the by-source
+    structure, which reads grad_out by destination: operands are compared first."""
+    indptr, indices = (t.to(dev) for t in random_csr(20, 30, 0.3, 3))
+    values = torch.rand(indices.numel(), 2, device=dev)
+    x, gy = torch.randn(30, 2, 8, device=dev), torch.randn(20, 2, 8, device=dev)
+    want = graph_ext.spmm_backward(values, indptr, indices, x, gy)[1]
+    for _ in range(3):
+        for bad_x, bad_gy in ((x, gy[:19]), (x, torch.cat([gy, gy])), (x, gy[:, :, :4].contiguous()),
+                              (x, gy[:, :1].contiguous()), (x[:, :, :4].contiguous(), gy),
+                              (x.bfloat16(), gy), (x, gy.double()), (x, gy.transpose(1, 2))):
+            with pytest.raises(RuntimeError):
+                graph_ext.spmm_backward(values, indptr, indices, bad_x, bad_gy, need_grad_a=False)
+        assert_close(graph_ext.spmm_backward(values, indptr, indices, x, gy, need_grad_a=False)[1], want)
+    for _ in range(3):  # fp32 out of bf16 features: their gradient is not offered
+        x16 = x.bfloat16().requires_grad_()
+        out = sparse.GSPMMFunction.apply((indptr, indices), values, x16)
+        with pytest.raises(RuntimeError, match="features"):
+            out.sum().backward()

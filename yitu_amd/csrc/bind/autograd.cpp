@@ -274,6 +274,7 @@ struct SpmmFunction : Function<SpmmFunction> {
         const auto k = kept(ctx);
         const Tensor g = dense(grads[0]);
         const bool need_a = ctx->needs_input_grad(0), need_x = ctx->needs_input_grad(1);
+        spmm_backward_check(saved[0], k->indptr, k->indices, saved[1], g);
         if (!need_a && !need_x) return {Tensor(), Tensor(), Tensor()};
         const int64_t n_dst = k->indptr.numel() - 1;
         if (!need_a && k->indices.numel() > 0 && n_dst <= kColMask) {

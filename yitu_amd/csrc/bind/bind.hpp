@@ -139,6 +139,8 @@ TensorVec b2gemm_backward(const Tensor &x, const Tensor &w_a, const Tensor &w_b,
                           const Tensor &grad_a, const Tensor &grad_b);
 Tensor spmm_forward(const Tensor &values, const Tensor &indptr, const Tensor &indices,
                     const Tensor &features, bool bf16_out, const RowState &rows);
+void spmm_backward_check(const Tensor &values, const Tensor &indptr, const Tensor &indices,
+                         const Tensor &features, const Tensor &grad_out);
 std::pair<OptTensor, OptTensor> spmm_backward(const Tensor &values, const Tensor &indptr,
                                               const Tensor &indices, const Tensor &features,
                                               const Tensor &grad_out, bool need_a, bool need_x,

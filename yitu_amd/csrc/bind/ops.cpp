@@ -435,20 +435,34 @@ Tensor spmm_forward(const Tensor &values, const Tensor &indptr, const Tensor &in
     return out;
 }
 
+// What every form of the backward asks of its operands, before any of them is chosen: each
+// kernel reads grad_out by destination and values by edge. Rows of grad_out in bf16 take bf16
+// features too (they are not read).
+void spmm_backward_check(const Tensor &values, const Tensor &indptr, const Tensor &indices,
+                         const Tensor &features, const Tensor &grad_out) {
+    check_f32(values, "values", 2);
+    check_i32(indptr, "indptr", 1);
+    check_i32(indices, "indices", 1);
+    const bool bf16 = grad_out.scalar_type() == at::kBFloat16;
+    check(features, bf16 && features.scalar_type() == at::kBFloat16 ? at::kBFloat16 : at::kFloat,
+          "features", 3);
+    check(grad_out, bf16 ? at::kBFloat16 : at::kFloat, "grad_out", 3);
+    same_device(values, indptr, indices, features, grad_out);
+    TORCH_CHECK(grad_out.size(0) == indptr.numel() - 1 && grad_out.size(1) == features.size(1) &&
+                    grad_out.size(2) == features.size(2),
+                "grad_out must be [n_dst, n_heads, n_features]");
+    TORCH_CHECK(values.size(0) >= indices.numel() && values.size(1) == features.size(1),
+                "values must be [n_edges, n_heads]");
+}
+
 std::pair<OptTensor, OptTensor> spmm_backward(const Tensor &values, const Tensor &indptr,
                                               const Tensor &indices, const Tensor &features,
                                               const Tensor &grad_out, bool need_a, bool need_x,
                                               const RowState &rows, const BySource &t) {
-    check_f32(values, "values", 2);
-    check_i32(indptr, "indptr", 1);
-    check_i32(indices, "indices", 1);
-    check_f32(features, "features", 3);
     check_f32(grad_out, "grad_out", 3);
-    same_device(values, indptr, indices, features, grad_out);
+    spmm_backward_check(values, indptr, indices, features, grad_out);
     const int64_t n_dst = indptr.numel() - 1, nnz = indices.numel();
     const int64_t n_src = features.size(0), h = features.size(1), f = features.size(2);
-    TORCH_CHECK(grad_out.size(0) == n_dst && grad_out.size(1) == h && grad_out.size(2) == f,
-                "grad_out must be [n_dst, n_heads, n_features]");
     Call c(features);
     OptTensor grad_a, grad_x;
     if (need_a) grad_a = c.empty(values.sizes());
@@ -905,6 +919,7 @@ void bind_ops(py::module_ &m) {
                              bool bf16_out, int64_t md, const OptTensor &plan) {
         return spmm_forward(v, ip, ix, x, bf16_out, rows_of(md, plan));
     });
+    m.def("spmm_backward_check", &spmm_backward_check);
     m.def("spmm_backward", [](const Tensor &v, const Tensor &ip, const Tensor &ix, const Tensor &x,
                               const Tensor &g, bool need_a, bool need_x, int64_t md,
                               const OptTensor &plan, const py::object &t) {

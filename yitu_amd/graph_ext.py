@@ -100,11 +100,7 @@ def spmm_backward(values, indptr, indices, features, grad_out, need_grad_a=True,
         if need_grad_a:
             raise RuntimeError("spmm_backward with bf16 rows computes grad_x only "
                                "(need_grad_a=False): the reference's op is fp32")
-        if features.dtype not in (torch.float32, torch.bfloat16) or features.dim() != 3:
-            raise RuntimeError("features must be a [n_src, H, F] tensor")
-        if grad_out.dim() != 3 or grad_out.shape[0] != n_dst or \
-                grad_out.shape[1:] != features.shape[1:]:
-            raise RuntimeError("grad_out must be [n_dst, n_heads, n_features]")
+        native.spmm_backward_check(values, indptr, indices, features, grad_out)
         if not need_grad_x:
             return [None, None]
         if n_dst > COL_MASK:
@@ -115,6 +111,9 @@ def spmm_backward(values, indptr, indices, features, grad_out, need_grad_a=True,
         values_t = native.by_source_values(values, indptr, indices, n_src, True)
         return [None, spmm_forward(values_t, tr.t_indptr, tr.t_rows, grad_out,
                                    out_dtype=grad_x_dtype)]
+    # before anything reads them: the by-source branch below hands grad_out to a forward
+    # product that cannot know how many rows or columns it should have
+    native.spmm_backward_check(values, indptr, indices, features, grad_out)
     if not (need_grad_a or need_grad_x):
         return [None, None]
     if grad_x_dtype != torch.float32:
