@@ -111,6 +111,27 @@ def test_batched_model_equals_one_relation_at_a_time(dev, which, stitch, relatio
             assert_close(b, a, rtol=1e-4, atol=1e-5)
 
 
+def test_two_dropouts_of_the_same_rows_differ(dev):
+    """F.dropout(h, .5) - F.dropout(h, .5): about half of the entries
+    are not zero, whatever the batch."""
+    hgraph = cases.hetero_graph(device=dev)
+    kwargs = cases.hetero_kwargs(hgraph, device=dev)
+
+    class Model(models.RGCNModel):
+        def forward(self, hgraph, norms, xs):
+            drop = lambda h: torch.nn.functional.dropout(h, 0.5)  # noqa: E731
+            return {t: drop(h) - drop(h) for t, h in self._run(hgraph, xs, norms).items()}
+
+    model = Model(hgraph, 8, 8, 16).to(dev)
+    flow = xgnn_h.Optimizer().lower(xgnn_h.Module2IR().transform(model, kwargs), kwargs)
+    executor = xgnn_h.Executor()
+    executor.train()
+    for form in (flow, xgnn_h.Stitcher().transform(flow, kwargs)):
+        out = executor.run(form, kwargs)
+        share = torch.cat(list(out.values())).ne(0).float().mean()
+        assert 0.4 < float(share) < 0.6  # 117 x 16 fair draws: a standard error of 0.012
+
+
 def test_batched_model_in_training_mode_keeps_its_shapes(dev):
     hgraph = cases.hetero_graph(device=dev)
     kwargs = cases.hetero_kwargs(hgraph, device=dev)

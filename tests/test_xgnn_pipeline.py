@@ -334,3 +334,47 @@ def test_grouped_linears_equal_one_linear_at_a_time(which):
         assert (ga is None) == (gb is None)
         if ga is not None:
             assert_close(gb, ga, rtol=1e-5, atol=1e-6)
+
+
+class _Drops(nn.Module):
+    """One relational layer whose results meet two dropouts and their difference."""
+
+    def __init__(self, hgraph):
+        super().__init__()
+        self.em = models.REmbedding(hgraph, 8)
+        self.conv = models.HeteroGraphConv({e: models.GCNLayer(8, 6) for e in hgraph.etypes})
+
+    def forward(self, hgraph, norms, xs):
+        drop = lambda h: nn.functional.dropout(h, 0.5)  # noqa: E731
+        return {t: drop(h) - drop(h) for t, h in self.conv(hgraph, self.em(hgraph, xs), norms).items()}
+
+
+@pytest.mark.parametrize("stitch", [False, True])
+def test_every_dropout_of_a_batched_model_draws_for_itself(stitch):
+    """Dropouts of different node types share a draw over the batch, two dropouts of the same
+    rows never do."""
+    hgraph = cases.hetero_graph()
+    kwargs = cases.hetero_kwargs(hgraph)
+    flow = xgnn_h.Optimizer().lower(xgnn_h.Module2IR().transform(_Drops(hgraph), kwargs), kwargs)
+    if stitch:
+        flow = xgnn_h.Stitcher().transform(flow, kwargs)
+    batched = xgnn_h.batch.batch_rows(flow, kwargs, training=True)
+    for root in batched.values():
+        a, b = root.inputs.values()
+        assert a is not b
+        drawn = [next(n for n in ir.walk(x) if n.op == "dropout") for x in (a, b)]
+        assert drawn[0] is not drawn[1]
+    assert cases.ops_of(batched)["dropout"] >= 2
+    if stitch:
+        assert cases.ops_of(batched)["dropout"] == 2
+    assert cases.ops_of(xgnn_h.batch.batch_rows(flow, kwargs))["dropout"] == 0
+
+
+def test_dropout_of_rows_read_twice_is_not_one_draw_over_the_batch():
+    x = ir.Node("input", size=[5, 4], name="x")
+    h, k = (ir.Node("linear", {"x": x}, {"weight": torch.randn(4, 4), "bias": None}, [5, 4])
+            for _ in range(2))
+    both = ir.Node("concat", {"0": h, "1": h, "2": k}, size=[15, 4])
+    flow = ir.Node("dropout", {"x": both}, {"p": 0.5}, [15, 4])
+    batched = xgnn_h.batch.batch_rows(flow, {"x": torch.randn(5, 4)}, training=True)
+    assert [n.size for n in ir.walk(batched) if n.op == "dropout"] == [[15, 4]]

@@ -165,10 +165,24 @@ class _Batcher:
                 slot, attrs = "0", {"fn": torch.Tensor.view, "kwargs": {},
                                     "args": (ir.Slot("0"), [-1] + list(tail))}
         key = (id(v.node), node.op, str(attrs))
+        if node.op == "dropout":
+            # each dropout draws for itself: one draw over the batch serves dropouts of
+            # different rows, never two of the same row
+            draws = self.memo.setdefault(key, [])
+            made = next((d for d in draws if not any(self._overlap(s, v.segs) for s in d[1])), None)
+            if made is None:
+                made = (ir.Node("dropout", {slot: v.node}, attrs, [self._rows_of(v.node)] + list(tail)), [])
+                draws.append(made)
+            made[1].append(v.segs)
+            return _Value(made[0], v.segs)
         if key not in self.memo:
             self.memo[key] = ir.Node(node.op, {slot: v.node}, attrs,
                                      [self._rows_of(v.node)] + list(tail))
         return _Value(self.memo[key], v.segs)
+
+    @staticmethod
+    def _overlap(a, b):
+        return any(x < y + m and y < x + n for x, n in a for y, m in b)
 
     # -- nodes that need no batch ----------------------------------------------------------
     def _immediate(self, node):
@@ -195,7 +209,11 @@ class _Batcher:
                     return self._whole_batch(node, v, node.size[1:])
                 if fn == "squeeze" and node.attrs["kwargs"].get("dim") == 1 and child.size[1] == 1:
                     return self._whole_batch(node, v, node.size[1:])
-                if op == "dropout" or (fn in _ROWWISE and self._plain(node)):
+                if op == "dropout":
+                    twice = any(self._overlap([a], v.segs[:i]) for i, a in enumerate(v.segs))
+                    if not twice:  # (rows read twice are drawn for twice)
+                        return self._whole_batch(node, v, node.size[1:])
+                elif fn in _ROWWISE and self._plain(node):
                     return self._whole_batch(node, v, node.size[1:])
         ins = {k: self._tensor(c) for k, c in node.inputs.items()}
         if op == "call" and node.attrs["fn"] is F.embedding:
