@@ -650,18 +650,6 @@ int yitu_tattn_prepare(float *x_kv_device, float *x_q_device, float *x_r_device,
                        const float *w_out_device, const float *b_out_device, int64_t n_dst,
                        int64_t n_edges, int64_t dim_node, int64_t dim_edge, int64_t dim_time,
                        int64_t dim_out, int64_t ld, void *stream);
-/* The same with node i's features in row nodes[i] of h (nodes NULL: row i; unchecked). */
-int yitu_tattn_prepare_nodes(float *x_kv_device, float *x_q_device, float *x_r_device,
-                             float *w_kv_device, float *w_q2_device, float *w_r_device,
-                             const float *h_device, const int32_t *nodes_device,
-                             const float *f_device, const float *dt_device,
-                             const float *time_w_device, const float *time_b_device,
-                             const float *w_q_device, const float *b_q_device,
-                             const float *w_k_device, const float *b_k_device,
-                             const float *w_v_device, const float *b_v_device,
-                             const float *w_out_device, const float *b_out_device, int64_t n_dst,
-                             int64_t n_edges, int64_t dim_node, int64_t dim_edge, int64_t dim_time,
-                             int64_t dim_out, int64_t ld, void *stream);
 int yitu_tattn_forward(float *x_r_device, float *attn_device, const float *q2_device,
                        const float *kv_device, const int32_t *indptr_device, int64_t n_dst,
                        int64_t n_edges, int64_t dim_out, int64_t n_heads, int64_t ld, void *stream);

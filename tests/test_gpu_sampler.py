@@ -117,6 +117,19 @@ def test_device_block_feeds_the_attention_layer(dev):
     a = layer(TemporalBlock.from_sampler(host.get_ret()[0], memory, device=dev))
     b = layer(TemporalBlock.from_device_block(gpu.get_ret()[0], memory))
     assert torch.equal(a, b)
+    # the block holds the rows as they were: a memory written afterwards, as a memory-based model
+    # does, is not read again, and a block made without gradients carries none
+    blk = TemporalBlock.from_device_block(gpu.get_ret()[0], memory)
+    kept = memory.clone()
+    memory.zero_()
+    assert torch.equal(a, layer(blk)) and torch.equal(blk.h, kept[gpu.get_ret()[0].nodes().long()])
+    kept.requires_grad_()
+    with torch.no_grad():
+        blk = TemporalBlock.from_device_block(gpu.get_ret()[0], kept)
+    layer(blk).sum().backward()
+    assert kept.grad is None and layer.w_q.weight.grad is not None
+    layer(TemporalBlock.from_device_block(gpu.get_ret()[0], kept)).sum().backward()
+    assert kept.grad is not None
 
 
 MODES = np.load(os.path.join(ROOT, "tests", "golden", "sampler_modes.npz"))

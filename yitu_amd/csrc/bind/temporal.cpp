@@ -6,8 +6,6 @@
 namespace yitu_bind {
 namespace {
 
-const int32_t *i32(const OptTensor &t) { return has(t) ? yitu_bind::i32(*t) : nullptr; }
-
 // Consecutive fp32 matrices in one buffer, each at a multiple of 64 floats.
 struct Carver {
     int64_t room = 0;
@@ -48,10 +46,10 @@ void gemm(const Call &c, float *out, const float *a, const float *b, int64_t m, 
 }
 
 std::pair<Tensor, Tensor> tattn_forward(const Tensor &indptr, int64_t n_dst, int64_t heads, double eps,
-                                        const OptTensor &h, const OptTensor &nodes,
-                                        const OptTensor &f, const Tensor &dt, const OptTensor &time_w,
-                                        const OptTensor &time_b, const TensorVec &params,
-                                        const Tensor &ln_w, const Tensor &ln_b) {
+                                        const OptTensor &h, const OptTensor &f, const Tensor &dt,
+                                        const OptTensor &time_w, const OptTensor &time_b,
+                                        const TensorVec &params, const Tensor &ln_w,
+                                        const Tensor &ln_b) {
     check_i32(indptr, "indptr", 1);
     check_f32(dt, "dt");
     for (const OptTensor *t : {&h, &f, &time_w, &time_b})
@@ -67,12 +65,7 @@ std::pair<Tensor, Tensor> tattn_forward(const Tensor &indptr, int64_t n_dst, int
     check_f32(ln_b, "ln_b");
     const Dims d = dims_of(h, f, dt, time_w, params[2], n_dst, heads);
     TORCH_CHECK(indptr.numel() == n_dst + 1, "indptr must be [n_dst + 1]");
-    if (has(nodes)) {
-        check_i32(*nodes, "nodes", 1);
-        same_device(dt, *nodes);
-    }
-    TORCH_CHECK(!has(h) || (has(nodes) ? nodes->numel() : h->size(0)) == d.B + d.E,
-                "node features: one row per root and per edge");
+    TORCH_CHECK(!has(h) || h->size(0) == d.B + d.E, "node features: one row per root and per edge");
     TORCH_CHECK(!has(f) || f->size(0) == d.E, "edge features: one row per edge");
     TORCH_CHECK(!has(time_w) || (time_w->numel() == d.Dt && has(time_b) && time_b->numel() == d.Dt),
                 "the time encoder is a Linear(1, dim_time)");
@@ -85,11 +78,11 @@ std::pair<Tensor, Tensor> tattn_forward(const Tensor &indptr, int64_t n_dst, int
     const Kept k(d);
     Tensor buf = c.empty({std::max<int64_t>(k.c.room, 64)}), out = c.empty({d.B, d.O});
     const auto p = [&](int i) { return f32(buf) + k.c.at[i]; };
-    ok(yitu_tattn_prepare_nodes(p(k.x_kv), p(k.x_q), p(k.x_r), p(k.w_kv), p(k.w_q2), p(k.w_r), f32(h),
-                                i32(nodes), f32(f), f32(dt), f32(time_w), f32(time_b), f32(params[0]),
-                                f32(params[1]), f32(params[2]), f32(params[3]), f32(params[4]),
-                                f32(params[5]), f32(params[6]), f32(params[7]), d.B, d.E, d.Dn, d.De,
-                                d.Dt, d.O, d.LD, c.stream),
+    ok(yitu_tattn_prepare(p(k.x_kv), p(k.x_q), p(k.x_r), p(k.w_kv), p(k.w_q2), p(k.w_r), f32(h), f32(f),
+                          f32(dt), f32(time_w), f32(time_b), f32(params[0]), f32(params[1]),
+                          f32(params[2]), f32(params[3]), f32(params[4]), f32(params[5]),
+                          f32(params[6]), f32(params[7]), d.B, d.E, d.Dn, d.De, d.Dt, d.O, d.LD,
+                          c.stream),
        "yitu_tattn_prepare");
     if (d.E > 0) {
         float *cs[] = {p(k.kv), p(k.q2)};
@@ -101,7 +94,7 @@ std::pair<Tensor, Tensor> tattn_forward(const Tensor &indptr, int64_t n_dst, int
     } else {
         gemm(c, p(k.q2), p(k.x_q), p(k.w_q2), d.B, 2 * d.O, d.LD, false, true, d.LD, d.LD, 2 * d.O);
     }
-    ok(yitu_tattn_forward(p(k.x_r), p(k.attn), p(k.q2), p(k.kv), yitu_bind::i32(indptr), d.B, d.E, d.O,
+    ok(yitu_tattn_forward(p(k.x_r), p(k.attn), p(k.q2), p(k.kv), i32(indptr), d.B, d.E, d.O,
                           d.H, d.LD, c.stream),
        "yitu_tattn_forward");
     gemm(c, p(k.pre), p(k.x_r), p(k.w_r), d.B, d.O, d.LD, false, true, d.LD, d.LD, d.O);
@@ -166,7 +159,7 @@ std::vector<OptTensor> tattn_backward(const Tensor &grad_out, const Tensor &buf,
        "yitu_relu_layernorm_backward");
     gemm(c, w(dx_r), w(d_pre2), p(k.w_r), d.B, n_r, d.O, false, false, 2 * d.O, d.LD, n_r);
     ok(yitu_tattn_backward(w(dq2), w(dkv), w(scratch), w(dx_r), p(k.q2), p(k.kv), p(k.attn),
-                           yitu_bind::i32(indptr), d.B, d.E, d.O, d.H, n_r, c.stream),
+                           i32(indptr), d.B, d.E, d.O, d.H, n_r, c.stream),
        "yitu_tattn_backward");
     if (reads_kv && reads_q && n_kv == n_q) {
         float *cs[] = {w(dx_kv), w(dx_q)};
@@ -236,8 +229,8 @@ TensorVec tsample_recent(const Tensor &cursor, const Tensor &indptr, const Tenso
     const auto out = [](const Tensor &x) { return static_cast<int32_t *>(x.data_ptr()); };
     ok(yitu_tsample_recent_block(out(block), out(row), out(col), out(e), f32(t), f32(dts), out(nodes),
                                  static_cast<long long *>(count.data_ptr()), out(cursor),
-                                 yitu_bind::i32(indptr), yitu_bind::i32(indices), yitu_bind::i32(eid),
-                                 f32(ts), n_nodes, yitu_bind::i32(roots), f32(root_ts), n, (int)fan,
+                                 i32(indptr), i32(indices), i32(eid),
+                                 f32(ts), n_nodes, i32(roots), f32(root_ts), n, (int)fan,
                                  prop_time, ws.data_ptr(), ws.numel(), c.stream),
        "yitu_tsample_recent");
     const int64_t m = count.item<int64_t>();

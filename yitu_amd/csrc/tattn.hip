@@ -72,7 +72,6 @@ __device__ __forceinline__ float time_arg(float dt, float w, float b) {
 struct PrepareArgs {
     float *x_kv, *x_q, *x_r, *w_kv, *w_q2, *w_r;
     const float *h, *f, *dt, *time_w, *time_b;
-    const int32_t *nodes;  // row of h that holds node i's features; null: row i
     const float *wq, *bq, *wk, *bk, *wv, *bv, *wo, *bo;
 };
 
@@ -84,10 +83,9 @@ __global__ __launch_bounds__(kBlock) void tattn_prepare_kernel(TattnDims d, Prep
     const int E = d.n_edges, B = d.n_dst, O = d.O, LD = d.LD;
     const int Dkv = d.Dn + d.De + d.Dt, Dq = d.Dn + d.Dt, Dr = O + d.Dn;
     int64_t r = row;
-    const auto node_row = [&](int64_t i) { return a.h + (a.nodes ? (int64_t)a.nodes[i] : i) * d.Dn; };
     if (r < E) {
         const float t = a.dt[r];
-        const float *h = node_row(B + r);
+        const float *h = a.h + (B + r) * d.Dn;
         float *out = a.x_kv + r * LD;
         for (int c = lane; c < LD; c += kWave) {
             float v = c == LD - 1 ? 1.0f : 0.0f;
@@ -100,7 +98,7 @@ __global__ __launch_bounds__(kBlock) void tattn_prepare_kernel(TattnDims d, Prep
     }
     r -= E;
     if (r < B) {
-        const float *h = node_row(r);
+        const float *h = a.h + r * d.Dn;
         float *out = a.x_q + r * LD;
         for (int c = lane; c < LD; c += kWave) {
             float v = c == LD - 1 ? 1.0f : 0.0f;
@@ -112,7 +110,7 @@ __global__ __launch_bounds__(kBlock) void tattn_prepare_kernel(TattnDims d, Prep
     }
     r -= B;
     if (r < B) {
-        const float *h = node_row(r);
+        const float *h = a.h + r * d.Dn;
         float *out = a.x_r + r * LD;
         for (int c = O + lane; c < LD; c += kWave) {
             float v = c == LD - 1 ? 1.0f : 0.0f;
@@ -976,9 +974,9 @@ YITU_API int64_t yitu_tattn_partial_rows(int64_t n_rows) {
     return std::max<int64_t>(1, ceil_div(n_rows, kWavesPerBlock * rows_per_wave_reduce(n_rows)));
 }
 
-YITU_API int yitu_tattn_prepare_nodes(float *x_kv, float *x_q, float *x_r, float *w_kv, float *w_q2,
-                                float *w_r, const float *h, const int32_t *nodes, const float *f,
-                                const float *dt, const float *time_w, const float *time_b, const float *wq,
+YITU_API int yitu_tattn_prepare(float *x_kv, float *x_q, float *x_r, float *w_kv, float *w_q2,
+                                float *w_r, const float *h, const float *f, const float *dt,
+                                const float *time_w, const float *time_b, const float *wq,
                                 const float *bq, const float *wk, const float *bk, const float *wv,
                                 const float *bv, const float *wo, const float *bo, int64_t n_dst,
                                 int64_t n_edges, int64_t dim_node, int64_t dim_edge,
@@ -991,25 +989,13 @@ YITU_API int yitu_tattn_prepare_nodes(float *x_kv, float *x_q, float *x_r, float
                  "null feature input");
     YITU_REQUIRE(dim_node + dim_time > 0, "the query needs node or time features");
     YITU_REQUIRE(wq && bq && wk && bk && wv && bv && wo && bo, "null parameter");
-    PrepareArgs a{x_kv, x_q, x_r, w_kv, w_q2, w_r, h, f, dt, time_w, time_b, nodes,
+    PrepareArgs a{x_kv, x_q, x_r, w_kv, w_q2, w_r, h, f, dt, time_w, time_b,
                   wq, bq, wk, bk, wv, bv, wo, bo};
     const int64_t rows = n_edges + 2 * n_dst + 5 * dim_out;
     tattn_prepare_kernel<<<(int)ceil_div(rows, kWavesPerBlock), kBlock, 0,
                            static_cast<hipStream_t>(stream)>>>(d, a);
     YITU_LAUNCH_CHECK();
     return 0;
-}
-
-YITU_API int yitu_tattn_prepare(float *x_kv, float *x_q, float *x_r, float *w_kv, float *w_q2,
-                                float *w_r, const float *h, const float *f, const float *dt,
-                                const float *time_w, const float *time_b, const float *wq,
-                                const float *bq, const float *wk, const float *bk, const float *wv,
-                                const float *bv, const float *wo, const float *bo, int64_t n_dst,
-                                int64_t n_edges, int64_t dim_node, int64_t dim_edge,
-                                int64_t dim_time, int64_t dim_out, int64_t ld, void *stream) {
-    return yitu_tattn_prepare_nodes(x_kv, x_q, x_r, w_kv, w_q2, w_r, h, nullptr, f, dt, time_w, time_b,
-                                    wq, bq, wk, bk, wv, bv, wo, bo, n_dst, n_edges, dim_node,
-                                    dim_edge, dim_time, dim_out, ld, stream);
 }
 
 YITU_API int yitu_tattn_forward(float *x_r, float *attn, const float *q2, const float *kv,

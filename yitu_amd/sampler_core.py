@@ -124,10 +124,10 @@ class DeviceTemporalGraphBlock:
     """A sampled block whose arrays are torch tensors on the GPU; the accessors
     mirror TemporalGraphBlock (``.cpu_block()`` converts to the numpy form)."""
 
-    def __init__(self, row, col, eid, ts, dts, nodes, dim_in, dim_out, indptr=None, id_bound=None):
+    def __init__(self, row, col, eid, ts, dts, nodes, dim_in, dim_out, indptr=None):
         self._a = (row, col, eid, ts, dts, nodes)
         self._dim_in, self._dim_out = int(dim_in), int(dim_out)
-        self._indptr, self._id_bound = indptr, id_bound
+        self._indptr = indptr
 
     def row(self):
         return self._a[0]
@@ -157,10 +157,6 @@ class DeviceTemporalGraphBlock:
         """First edge of every root slot, [dim_out + 1] int32; None if the sampler made none."""
         return self._indptr
 
-    def id_bound(self):
-        """Every id in ``nodes`` is below this; None if the sampler knows no bound."""
-        return self._id_bound
-
     def cpu_block(self):
         return TemporalGraphBlock(*[t.cpu().numpy() for t in self._a], self._dim_in, self._dim_out)
 
@@ -188,10 +184,6 @@ class GpuParallelSampler:
         self._eid = to(eid, np.int32)
         self._ts = to(ts, np.float32)
         self._n_nodes = self._indptr.numel() - 1
-        # roots are nodes (checked on the device), neighbours are what indices holds
-        neighbours = np.asarray(indices)
-        self._id_bound = None if neighbours.size and int(neighbours.min()) < 0 else \
-            max(self._n_nodes, int(neighbours.max()) + 1 if neighbours.size else 0)
         self._fan = [int(x) for x in num_neighbors[:num_layers]]
         self._prop_time = bool(prop_time)
         self._recent = bool(recent)
@@ -234,7 +226,7 @@ class GpuParallelSampler:
         n = roots.numel()
         *block, indptr = _lib.ops().tsample_recent(self._cursor, self._indptr, self._indices, self._eid,
                                                    self._ts, roots, root_ts, fan, self._prop_time)
-        return DeviceTemporalGraphBlock(*block, block[5].numel(), n, indptr, self._id_bound)
+        return DeviceTemporalGraphBlock(*block, block[5].numel(), n, indptr)
 
     def _advance(self, k, roots, root_ts, offset):
         import torch

@@ -22,24 +22,21 @@ def _dense(t):
 
 
 class TemporalAttentionFunction(torch.autograd.Function):
-    """apply(indptr, n_dst, num_head, eps, nodes, h, f, dt, time_w, time_b, w_q, b_q, w_k, b_k,
-    w_v, b_v, w_out, b_out, ln_w, ln_b) -> [n_dst, dim_out]. ``h`` [n_dst + E, dim_node] or
-    None; or, with ``nodes`` int32 [n_dst + E], a feature table whose row ``nodes[i]`` is taken
-    (it gets no gradient). ``f`` [E, dim_edge] or None, ``time_w`` [dim_time, 1] / ``time_b``
-    or None."""
+    """apply(indptr, n_dst, num_head, eps, h, f, dt, time_w, time_b, w_q, b_q, w_k, b_k, w_v,
+    b_v, w_out, b_out, ln_w, ln_b) -> [n_dst, dim_out]. ``h`` [n_dst + E, dim_node] or None,
+    ``f`` [E, dim_edge] or None, ``time_w`` [dim_time, 1] / ``time_b`` or None."""
 
     @staticmethod
-    def forward(ctx, indptr, n_dst, num_head, eps, nodes, h, f, dt, time_w, time_b, w_q, b_q, w_k,
-                b_k, w_v, b_v, w_out, b_out, ln_w, ln_b):
+    def forward(ctx, indptr, n_dst, num_head, eps, h, f, dt, time_w, time_b, w_q, b_q, w_k, b_k,
+                w_v, b_v, w_out, b_out, ln_w, ln_b):
         h, f, dt, time_w, time_b = _dense(h), _dense(f), _dense(dt), _dense(time_w), _dense(time_b)
         ln_w = _dense(ln_w)
         params = [_dense(t) for t in (w_q, b_q, w_k, b_k, w_v, b_v, w_out, b_out)]
-        out, buf = _lib.ops().tattn_forward(indptr, n_dst, num_head, eps, h, nodes, f, dt, time_w, time_b,
+        out, buf = _lib.ops().tattn_forward(indptr, n_dst, num_head, eps, h, f, dt, time_w, time_b,
                                             params, ln_w, _dense(ln_b))
         ctx.dims = (n_dst, dt.numel(), 0 if h is None else h.size(1), 0 if f is None else f.size(1),
                     0 if time_w is None else time_w.size(0), w_k.size(0), num_head)
         ctx.eps = eps
-        ctx.gathered = nodes is not None
         ctx.buf = buf
         ctx.save_for_backward(indptr, dt, time_w, time_b, ln_w)
         return out
@@ -48,7 +45,7 @@ class TemporalAttentionFunction(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, grad_out):
         indptr, dt, time_w, time_b, ln_w = ctx.saved_tensors
-        need_h = ctx.needs_input_grad[5] and not ctx.gathered
         grads = _lib.ops().tattn_backward(grad_out.contiguous(), ctx.buf, indptr, dt, time_w, time_b,
-                                          ln_w, ctx.dims, ctx.eps, need_h, ctx.needs_input_grad[6])
-        return (None, None, None, None, None, grads[0], grads[1], None, *grads[2:])
+                                          ln_w, ctx.dims, ctx.eps, ctx.needs_input_grad[4],
+                                          ctx.needs_input_grad[5])
+        return (None, None, None, None, grads[0], grads[1], None, *grads[2:])

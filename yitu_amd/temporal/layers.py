@@ -89,10 +89,9 @@ class TemporalBlock:
         self._fill(n_dst, row.numel(), row.to(dev), indptr.to(torch.int32).to(dev),
                    torch.as_tensor(np.asarray(dt), dtype=torch.float32).to(dev), h, f)
 
-    def _fill(self, n_dst, n_edges, row, indptr, dt, h, f, table=None):
+    def _fill(self, n_dst, n_edges, row, indptr, dt, h, f):
         self.n_dst, self.n_edges = int(n_dst), int(n_edges)
-        self._row, self.indptr, self.dt, self._h, self.f = row, indptr, dt, h, f
-        self._table = table  # (features of all nodes, ids of this block's): h when it is asked for
+        self._row, self.indptr, self.dt, self.h, self.f = row, indptr, dt, h, f
         self._blk = None
 
     # what only some readers want is made when it is read
@@ -109,25 +108,6 @@ class TemporalBlock:
                                      [self.indptr, torch.arange(self.n_edges, dtype=torch.int32,
                                                                 device=self.indptr.device)])
         return self._blk
-
-    @property
-    def h(self):
-        if self._h is None and self._table is not None:
-            memory, ids = self._table
-            self._h = memory[ids.to(torch.int64)]
-            self._table = None
-        return self._h
-
-    @h.setter
-    def h(self, value):
-        self._h, self._table = value, None
-
-    def gathered(self):
-        """(node features, ids of their rows or None): the table itself as long as nobody asked
-        for the rows and it takes no gradient."""
-        if self._table is not None and not (self._table[0].requires_grad and torch.is_grad_enabled()):
-            return self._table
-        return self.h, None
 
     @staticmethod
     def from_sampler(tgb, memory=None, device="cuda"):
@@ -151,12 +131,8 @@ class TemporalBlock:
             indptr = torch.zeros(n_dst + 1, dtype=torch.int64, device=memory.device)
             indptr[1:] = torch.cumsum(torch.bincount(row.to(torch.int64), minlength=n_dst), 0)
             indptr = indptr.to(torch.int32)
-        h, table = None, (memory, nodes)
-        if memory.device != nodes.device or memory.dtype != torch.float32 or memory.dim() != 2 or \
-                not memory.is_contiguous() or dtgb.id_bound() is None or \
-                memory.size(0) < dtgb.id_bound():
-            h, table = memory[nodes.to(torch.int64)], None
-        b._fill(n_dst, row.numel(), row, indptr, dtgb.dts()[n_dst:], h, None, table)
+        # the rows as they are now: the memory may be written before the layer runs
+        b._fill(n_dst, row.numel(), row, indptr, dtgb.dts()[n_dst:], memory[nodes.to(torch.int64)], None)
         return b
 
     def num_edges(self):
@@ -238,10 +214,9 @@ class TransfomerAttentionLayer(torch.nn.Module):
                                 self.num_head):
             # the whole layer as one autograd node of a dozen launches
             te = self.time_enc.w if self.dim_time > 0 else None
-            h, nodes = b.gathered() if self.dim_node_feat > 0 else (None, None)
             return fused.TemporalAttentionFunction.apply(
-                b.indptr, n_dst, self.num_head, self.layer_norm.eps, nodes, h,
-                b.f if self.dim_edge_feat > 0 else None,
+                b.indptr, n_dst, self.num_head, self.layer_norm.eps,
+                b.h if self.dim_node_feat > 0 else None, b.f if self.dim_edge_feat > 0 else None,
                 b.dt, te.weight if te is not None else None, te.bias if te is not None else None,
                 wq[0], wq[1], wk[0], wk[1], wv[0], wv[1], self.w_out.weight, self.w_out.bias,
                 self.layer_norm.weight, self.layer_norm.bias)
