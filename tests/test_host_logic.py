@@ -114,3 +114,16 @@ def test_auto_knobs_hand_computed():
     assert tuple(k) == (50, 1, 5, 32, 32)
     assert tuple(auto_knobs(11.3, 64, 16, 40.0)) == (11, 8, 8, 32, 16)
     assert worth_reordering(3000.0, 10000) and not worth_reordering(0.5, 10000)
+
+
+def test_temporal_block_parts_can_be_replaced():
+    from yitu_amd.temporal import TemporalBlock
+    from yitu_amd.xgnn_h import Block
+    b = TemporalBlock([0, 0, 2], 3, [1.0, 2.0, 3.0], device="cpu")
+    assert b.row.tolist() == [0, 0, 2] and b.indptr.tolist() == [0, 2, 2, 3]
+    assert b.blk.adj_sparse[1].tolist() == [0, 1, 2]
+    b.row = torch.tensor([1, 1, 2])
+    b.blk = Block([3, 3], [torch.tensor([0, 0, 2, 3], dtype=torch.int32),
+                           torch.arange(3, dtype=torch.int32)])
+    assert b.row.tolist() == [1, 1, 2]
+    assert b.blk.adj_sparse[0].tolist() == b.indptr.tolist() == [0, 0, 2, 3]

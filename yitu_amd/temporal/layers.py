@@ -91,15 +91,19 @@ class TemporalBlock:
 
     def _fill(self, n_dst, n_edges, row, indptr, dt, h, f):
         self.n_dst, self.n_edges = int(n_dst), int(n_edges)
-        self._row, self.indptr, self.dt, self.h, self.f = row, indptr, dt, h, f
-        self._blk = None
+        self.indptr, self.dt, self.h, self.f = indptr, dt, h, f
+        self._sampled_row, self._row, self._blk = row, None, None
 
     # what only some readers want is made when it is read
     @property
     def row(self):
-        if self._row.dtype != torch.int64:
-            self._row = self._row.to(torch.int64)
+        if self._row is None:
+            self._row = self._sampled_row.to(torch.int64)
         return self._row
+
+    @row.setter
+    def row(self, value):
+        self._row = value
 
     @property
     def blk(self):
@@ -108,6 +112,10 @@ class TemporalBlock:
                                      [self.indptr, torch.arange(self.n_edges, dtype=torch.int32,
                                                                 device=self.indptr.device)])
         return self._blk
+
+    @blk.setter
+    def blk(self, value):
+        self._blk, self.indptr = value, value.adj_sparse[0]
 
     @staticmethod
     def from_sampler(tgb, memory=None, device="cuda"):
