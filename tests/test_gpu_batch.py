@@ -30,6 +30,26 @@ def test_fold_of_row_ranges(dev, width):
     assert_close(torch.autograd.grad(out, x, dy)[0], torch.autograd.grad(want, x, dy)[0])
 
 
+@pytest.mark.parametrize("split", [False, True])
+def test_fold_result_may_be_written_where_no_activation_made_it(dev, split):
+    def run(ranges, write):
+        x = torch.randn(12, 4, device=dev).requires_grad_()
+        plan = _lib.ops().fold_plan(12, ranges, x)
+        parts = _lib.ops().fold_split(x, plan, [5, 7]) if split else [_lib.ops().fold_rows(x, plan)]
+        parts[write].mul_(3.0)
+        return torch.autograd.grad([p.sum() for p in parts], x)[0]
+
+    third = [(5, [0], 3.0, 0, 0.0), (7, [5], 3.0, 0, 0.0)]
+    want = torch.full((12, 4), 1 / 3, device=dev)
+    want[:5 if split else 12] = 1.0
+    assert_close(run(third, 0), want)
+    relu = [(5, [0], 1.0, 1, 0.0), (7, [5], 1.0, 0, 0.0)]
+    with pytest.raises(RuntimeError, match="inplace"):
+        run(relu, 0)
+    if split:  # the part beside it is no result of the ReLU
+        assert_close(run(relu, 1)[5:], torch.full((7, 4), 3.0, device=dev))
+
+
 def test_fold_plan_refuses_ranges_outside_or_twice(dev):
     x = torch.zeros(10, 4, device=dev)
     with pytest.raises(RuntimeError):
@@ -109,6 +129,30 @@ def test_batched_model_equals_one_relation_at_a_time(dev, which, stitch, relatio
         assert (a is None) == (b is None)
         if a is not None:
             assert_close(b, a, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("which", ["rgcn", "rgat"])
+def test_outputs_of_a_batched_model_can_be_written_in_place(dev, which):
+    torch.manual_seed(1)
+    hgraph = cases.hetero_graph(device=dev)
+    kwargs = cases.hetero_kwargs(hgraph, device=dev, with_norms=which == "rgcn")
+    model = (models.RGCNModel(hgraph, 12, 16, 5) if which == "rgcn"
+             else models.RGATModel(hgraph, 12, 16, 8, n_heads=2)).to(dev)
+    flow = xgnn_h.Optimizer().lower(xgnn_h.Module2IR().transform(model, kwargs), kwargs)
+    for form in (flow, xgnn_h.Stitcher().transform(flow, kwargs)):
+        grads = []
+        for flag in (False, True):
+            executor = xgnn_h.Executor(group_linears=flag)
+            executor.eval()
+            out = executor.run(form, kwargs)
+            out["paper"].mul_(2.0)
+            out["venue"].add_(1.0)
+            grads.append(torch.autograd.grad([v.square().sum() for v in out.values()],
+                                             list(model.parameters()), allow_unused=True))
+        for a, b in zip(*grads):
+            assert (a is None) == (b is None)
+            if a is not None:
+                assert_close(b, a, rtol=1e-4, atol=1e-4)
 
 
 def test_two_dropouts_of_the_same_rows_differ(dev):

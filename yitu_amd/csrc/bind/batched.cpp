@@ -18,6 +18,7 @@ struct FoldPlan : torch::CustomClassHolder {
     };
     int64_t rows_in = 0, rows_out = 0, n_ranges = 0;
     bool covers = true;  // every row of x is a source
+    std::vector<std::pair<int64_t, int64_t>> active;  // output rows [begin, end) of an activation
     Tensor ranges, sources;
 
     FoldPlan(int64_t rows_in_, const std::vector<Range> &list, at::Device device)
@@ -32,6 +33,7 @@ struct FoldPlan : torch::CustomClassHolder {
             table.push_back({(int32_t)rows_out, (int32_t)r.rows, (int32_t)from.size(),
                              (int32_t)r.sources.size(), 1.0f / (float)r.divisor, (int32_t)r.act,
                              (float)r.alpha, 0});
+            if (r.act != YITU_FOLD_NONE && r.rows > 0) active.emplace_back(rows_out, rows_out + r.rows);
             rows_out += r.rows;
             for (int64_t s : r.sources) {
                 TORCH_CHECK(s >= 0 && s + r.rows <= rows_in, "fold: source rows ", s, " to ",
@@ -56,6 +58,11 @@ struct FoldPlan : torch::CustomClassHolder {
         };
         ranges = host(table.data(), table.size() * sizeof(YituFoldRange) / 4);
         sources = host(from.data(), from.size());
+    }
+    // Whether the backward reads output rows [begin, end): only an activation's.
+    bool reads(int64_t begin, int64_t end) const {
+        return std::any_of(active.begin(), active.end(),
+                           [&](const auto &a) { return a.first < end && begin < a.second; });
     }
     const YituFoldRange *table() const {
         return reinterpret_cast<const YituFoldRange *>(ranges.data_ptr());
@@ -85,12 +92,13 @@ Tensor own_part(const Tensor &t, int64_t first, at::IntArrayRef sizes) {
     return part;
 }
 
+// (`out` is read in the rows of an activation only; undefined where there are none)
 Tensor fold_backward(const FoldPlan &p, const Tensor &out, const Tensor &g) {
     Call c(g);
-    Tensor dx = c.empty({p.rows_in, out.size(1)});
+    Tensor dx = c.empty({p.rows_in, g.size(1)});
     if (!p.covers) dx.zero_();
-    ok(yitu_fold_rows_backward(f32(dx), f32(g), f32(out), p.table(), i32(p.sources), p.n_ranges,
-                               p.rows_out, out.size(1), c.stream),
+    ok(yitu_fold_rows_backward(f32(dx), f32(g), f32(out.defined() ? out : g), p.table(),
+                               i32(p.sources), p.n_ranges, p.rows_out, g.size(1), c.stream),
        "yitu_fold_rows_backward");
     return dx;
 }
@@ -98,7 +106,8 @@ Tensor fold_backward(const FoldPlan &p, const Tensor &out, const Tensor &g) {
 struct FoldFunction : Function<FoldFunction> {
     static Tensor forward(AutogradContext *ctx, const Tensor &x, FoldPlanPtr p) {
         Tensor out = fold(x, *p);
-        ctx->save_for_backward({out});
+        // kept where the backward reads it: a result without an activation may be written in place
+        ctx->save_for_backward({p->active.empty() ? Tensor() : out});
         ctx->saved_data["plan"] = c10::IValue::make_capsule(p);
         return out;
     }
@@ -114,27 +123,34 @@ struct FoldSplitFunction : Function<FoldSplitFunction> {
     static variable_list forward(AutogradContext *ctx, const Tensor &x, FoldPlanPtr p,
                                  std::vector<int64_t> sizes) {
         const Tensor out = fold(x, *p);
-        variable_list parts;
+        variable_list parts, saved;
         int64_t at = 0;
         for (int64_t n : sizes) {
             parts.push_back(own_part(out, at * out.size(1), {n, out.size(1)}));
+            // a part whose values the backward reads: a write to it is noticed
+            saved.push_back(p->reads(at, at + n) ? parts.back() : Tensor());
             at += n;
         }
         TORCH_CHECK(at == p->rows_out, "fold: the parts do not add up");
-        variable_list saved = parts;  // a part that was written to is noticed
         ctx->save_for_backward(std::move(saved));
         ctx->saved_data["plan"] = c10::IValue::make_capsule(p);
-        ctx->saved_data["out"] = out;
+        ctx->saved_data["sizes"] = std::move(sizes);
+        ctx->saved_data["width"] = out.size(1);
+        if (!p->active.empty()) ctx->saved_data["out"] = out;
         return parts;
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads) {
         const auto p =
             c10::static_intrusive_pointer_cast<FoldPlan>(ctx->saved_data["plan"].toCapsule());
-        const auto parts = ctx->get_saved_variables();
+        ctx->get_saved_variables();  // (raises where a part that is read was written to)
+        const auto sizes = ctx->saved_data["sizes"].toIntVector();
+        const int64_t width = ctx->saved_data["width"].toInt();
         for (size_t i = 0; i < grads.size(); i++)
-            if (!grads[i].defined()) grads[i] = at::zeros_like(parts[i]);
-        const Tensor g = at::cat(grads);
-        return once({fold_backward(*p, ctx->saved_data["out"].toTensor(), g), Tensor(), Tensor()});
+            if (!grads[i].defined())
+                grads[i] = at::zeros({sizes[i], width}, p->ranges.options().dtype(at::kFloat));
+        const Tensor g = at::cat(grads),
+                     out = p->active.empty() ? Tensor() : ctx->saved_data["out"].toTensor();
+        return once({fold_backward(*p, out, g), Tensor(), Tensor()});
     }
 };
 
