@@ -245,6 +245,16 @@ __global__ __launch_bounds__(kBlock) void gat_slot_items_kernel(GatSrcParams p) 
     }
 }
 
+// The row of a lane's slot when every wave takes U * SLOTS consecutive rows. Counted in rows:
+// threads (a row is LPF of them) pass 32 bits from 2^26 rows of 256 floats on.
+template <int LPF>
+constexpr int slot_row(unsigned wave, int u_per_wave, int lane) {
+    return (int)(wave * (unsigned)(u_per_wave * (kWave / LPF)) + (unsigned)(lane / LPF));
+}
+static_assert(slot_row<64>(1u << 25, 2, 63) == 1 << 26 && slot_row<16>(1u << 26, 2, 17) == (1 << 29) + 1 &&
+                  slot_row<2>(3, 2, 5) == 3 * 64 + 2,
+              "rows beyond a 32-bit thread count");
+
 // (S, query, max, 1 / sum) of every destination and head, S[r,h] = <g[r,:], out[r,h,:]> / H:
 // a row per slot, read front to back once.
 template <int LPF, int H>
@@ -258,7 +268,7 @@ __global__ __launch_bounds__(kBlock) void gat_slot_dot_kernel(float4 *__restrict
     typedef float f4 __attribute__((ext_vector_type(4)));
     constexpr int U = 2;
     const int lane = lane_id(), sub = lane % LPF;
-    const int r0 = ((blockIdx.x * kWavesPerBlock + wave_id()) * U * kWave + lane) / LPF;
+    const int r0 = slot_row<LPF>(blockIdx.x * kWavesPerBlock + wave_id(), U, lane);
     f4 gv[U], ov[U][H];
 #pragma unroll
     for (int u = 0; u < U; u++) {
