@@ -225,6 +225,38 @@ def test_gat_head_mean_backward_against_oracle(dev, h, f, with_attn):
     assert_close(gx, want_gx, abs_sum=abs_gx, what="grad_x " + what)
 
 
+@pytest.mark.parametrize("h,f", [(1, 20), (2, 24), (4, 32), (4, 8), (8, 12), (1, 256), (8, 64)])
+def test_gat_head_mean_backward_of_an_infinite_gradient_row(dev, h, f):
+    """The last destination's gradient holds +inf in its last column. Its sources get +inf there
+    in grad_x and nowhere a NaN (the slots without an edge load that row once more, and so do
+    lanes past a ragged width); rows that are no neighbours of it stay bitwise the same."""
+    n = 300
+    indptr, indices = random_csr(n, n, 0.01, h * 100 + f, hub_rows=(3, n - 1), hub_degree=150,
+                                 empty_rows=(9,))
+    blk = xblock.Block([n, n], [indptr, indices]).to(dev)
+    g = torch.Generator().manual_seed(f)
+    sources = indices[indptr[n - 1]:indptr[n]].long()
+    x = torch.rand(n, h, f, generator=g) + 0.5
+    odd = int(sources[5])
+    x[odd, :, f - 1] = -0.01
+    leaves = [t.to(dev).requires_grad_() for t in (torch.randn(n, h, generator=g) * 0.3,
+                                                   torch.randn(n, h, generator=g) * 0.3, x)]
+    gy = torch.randn(n, f, generator=g)
+    gy_inf = gy.clone()
+    gy_inf[n - 1, f - 1] = float("inf")
+    base, got = ([t.cpu() for t in torch.autograd.grad(
+        sparse.fused_gat(blk, *leaves, head_mean=True), leaves, grad.to(dev))] for grad in (gy, gy_inf))
+    hit = torch.zeros(n, dtype=torch.bool)
+    hit[sources] = True
+    assert torch.all(torch.isposinf(got[2][hit][:, :, f - 1]))
+    assert torch.equal(got[2][hit][:, :, :f - 1], base[2][hit][:, :, :f - 1])
+    # d logits = a (d - S): +inf less +inf for the others, -inf less +inf for the odd source
+    assert torch.all(torch.isneginf(got[1][odd]))
+    for a, b, same in ((got[2], base[2], ~hit), (got[1], base[1], ~hit),
+                       (got[0], base[0], torch.arange(n) != n - 1)):
+        assert torch.equal(a[same], b[same])
+
+
 @pytest.mark.parametrize("n,h,f", [(1000, 4, 64), (37, 1, 4), (513, 8, 32), (300, 2, 256),
                                    (129, 16, 16), (64, 4, 256), (5, 3, 8)])
 @pytest.mark.parametrize("two", [True, False])

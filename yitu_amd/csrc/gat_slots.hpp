@@ -92,6 +92,11 @@ __device__ __forceinline__ void slot_window(SlotRow<LPF, H> &row, const GatSrcPa
 #pragma unroll
         for (int u = 0; u < U; u++) {
             if (k0 + u * SLOTS >= n) break;  // wave-uniform
+            // a slot without an edge has loaded the last edge's row again, and lanes past a head's
+            // width its last floats: dropped here, where they are added up (0 x inf is not 0)
+            const bool live = valid[u] && 4 * sub < F;
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[u][i] = live ? v[u][i] : 0.0f;
             float mine[HPL];  // d_attn of (this slot's edge, own head)
 #pragma unroll
             for (int i = 0; i < HPL; i++) mine[i] = 0.0f;
