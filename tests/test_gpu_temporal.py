@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from yitu_amd import sampler_core
+from yitu_amd import _lib, sampler_core
 from yitu_amd.temporal import TemporalBlock, TimeEncode, TransfomerAttentionLayer
 from helpers import assert_close, dense_temporal_attention
 
@@ -277,3 +277,45 @@ def test_combined_branch(dev, dims):
         assert got is not None, name
         scale = 1e4 if name == "time_enc.w.weight" else 1.0
         assert_close(got, ref_grad.float(), rtol=1e-4, atol=1e-4 * scale, what=name)
+
+
+@pytest.mark.parametrize("O,H", [(32, 1), (100, 2), (200, 4)])
+def test_attention_of_an_infinite_value_row(dev, O, H):
+    """The last neighbour's value row holds +inf in one column: the root's aggregate is +inf
+    there, every other number of the forward keeps its bits, and the logit gradients of the
+    other neighbours are infinite, not NaN (rows past the last neighbour are copies of it, for
+    groups of four and of eight)."""
+    L, p, c = _lib.lib(), _lib.ptr, _lib.c_i64
+    counts = torch.tensor([1, 2, 3, 5, 8, 9, 31, 32, 33, 64, 66])
+    B, E, LD, col = counts.numel(), int(counts.sum()), O + 4, O // 2 + 1
+    indptr = torch.cat([torch.zeros(1, dtype=torch.int64), counts.cumsum(0)])
+    g = torch.Generator().manual_seed(O)
+    mk = lambda *s: torch.randn(*s, generator=g).to(dev)  # noqa: E731
+    q2, kv, dx_r = mk(B, 2 * O), 0.1 * mk(E, 2 * O), mk(B, LD)
+    ip = indptr.to(torch.int32).to(dev)
+    last = (indptr[1:] - 1).to(dev)
+
+    def run(kv):
+        x_r, attn = torch.zeros(B, LD, device=dev), torch.zeros(E, H, device=dev)
+        dq2, dkv = torch.zeros(B, 2 * O, device=dev), torch.zeros(E, 2 * O, device=dev)
+        scratch = torch.zeros(E, H, 2, device=dev)
+        s = _lib.stream_ptr(dev)
+        assert L.yitu_tattn_forward(p(x_r), p(attn), p(q2), p(kv), p(ip), c(B), c(E), c(O), c(H),
+                                    c(LD), s) == 0
+        assert L.yitu_tattn_backward(p(dq2), p(dkv), p(scratch), p(dx_r), p(q2), p(kv), p(attn), p(ip),
+                                     c(B), c(E), c(O), c(H), c(LD), s) == 0
+        return x_r, attn, dkv
+
+    base = run(kv)
+    kv_inf = kv.clone()
+    kv_inf[last, O + col] = float("inf")
+    x_r, attn, dkv = run(kv_inf)
+    assert torch.all(torch.isposinf(x_r[:, col]))
+    rest = torch.arange(LD, device=dev) != col
+    assert torch.equal(x_r[:, rest], base[0][:, rest]) and torch.equal(attn, base[1])
+    assert torch.equal(dkv[:, O:], base[2][:, O:])
+    head = torch.arange(O, device=dev) // (O // H) == col // (O // H)
+    assert torch.equal(dkv[:, :O][:, ~head], base[2][:, :O][:, ~head])
+    others = torch.ones(E, dtype=torch.bool, device=dev)
+    others[last] = False
+    assert torch.all(torch.isinf(dkv[:, :O][others][:, head]))

@@ -236,8 +236,8 @@ __device__ __noinline__ void forward_many(const TattnDims &d, float *__restrict_
             for (int u = 0; u < kEdgesInFlight; u++) {
 #pragma unroll
                 for (int h = 0; h < kTattnMaxHeads; h++) {
-                    if (h < H) {
-                        const float pj = j + u < n ? __shfl(p[h], (j + u) & (kWave - 1), kWave) : 0.0f;
+                    if (h < H && j + u < n) {  // (no row past the last: 0 x inf is not 0)
+                        const float pj = __shfl(p[h], (j + u) & (kWave - 1), kWave);
 #pragma unroll
                         for (int t = 0; t < kT; t++)
                             if (head[t] == h) acc[t] += pj * v[u][t];
@@ -515,7 +515,7 @@ __device__ __forceinline__ void forward_few(const TattnDims &d, float *__restric
     for (int e0 = 0; e0 < kFew; e0 += kFewGroup) {
         if (e0 < n) {
 #pragma unroll
-            for (int e = e0; e < e0 + kFewGroup; e++) {  // (zero weights past the last neighbour)
+            for (int e = e0; e < e0 + kFewGroup; e++) {
                 float pe[HM];
 #pragma unroll
                 for (int h = 0; h < HM; h++) pe[h] = lane_value(p[h], 2 * e);
@@ -524,7 +524,8 @@ __device__ __forceinline__ void forward_few(const TattnDims &d, float *__restric
                     float w = pe[0];
 #pragma unroll
                     for (int h = 1; h < HM; h++) w = head[t] == h ? pe[h] : w;
-                    acc[t] = fmaf(w, row[e][t], acc[t]);
+                    // (no copy of the last row: 0 x inf is not 0)
+                    acc[t] = e < n ? fmaf(w, row[e][t], acc[t]) : acc[t];
                 }
             }
         }
@@ -571,7 +572,7 @@ __device__ __forceinline__ void backward_few(const TattnDims &d, float *__restri
             const float ah = lane / 2 < n ? attn[(int64_t)(beg + lane / 2) * H + h] : 0.0f;
             const float slope = few_dots<NV>(q, key, head, h, n) > 0.0f ? 1.0f : 0.2f;
             const float d_att = few_dots<NV>(g, val, head, h, n);
-            const float row_s = few_sum(rounded_product(ah, d_att));
+            const float row_s = few_sum(lane / 2 < n ? rounded_product(ah, d_att) : 0.0f);
             set_head(a, h, ah);
             set_head(dl, h, ah * (d_att - row_s) * slope);
         }
@@ -597,7 +598,7 @@ __device__ __forceinline__ void backward_few(const TattnDims &d, float *__restri
                         aj = head[t] == h ? ae[h] : aj;
                         dlj = head[t] == h ? dle[h] : dlj;
                     }
-                    dq[t] = fmaf(dlj, key[e][t], dq[t]);
+                    dq[t] = e < n ? fmaf(dlj, key[e][t], dq[t]) : dq[t];
                     if (i < O && e < n) {
                         drow[i] = dlj * q[t];
                         drow[O + i] = aj * g[t];
