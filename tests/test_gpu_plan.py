@@ -14,7 +14,7 @@ import pytest
 import torch
 
 from helpers import powerlaw_graph, random_csr
-from yitu_amd import _lib
+from yitu_amd import _lib, graph_ext
 
 pytestmark = pytest.mark.gpu
 
@@ -176,3 +176,26 @@ def test_locality_of_a_planted_graph_and_of_its_shuffle(dev):
                                               torch.from_numpy(shuffle[src]), n, n)
     p = check_plan(indptr, indices, n, 0x7fffffff, dev)
     assert p["local"] * 8 < p["sampled"]
+
+
+def test_state_in_use_on_another_stream_is_not_handed_out_again(dev):
+    """The plan and the by-source view belong to the stream they were built on. Forgotten while a
+    second stream still reads them, their memory waits for that stream."""
+    indptr, indices = (t.to(dev) for t in powerlaw_graph(12, 60000, 5))
+    n = indptr.numel() - 1
+    plan = _lib.row_plan(indptr, indices, n, graph_ext.COL_MASK)
+    view = graph_ext.transposed(indptr, indices, n)
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(100_000_000)
+        assert _lib.row_plan(indptr, indices, n, graph_ext.COL_MASK) is plan
+        assert graph_ext.transposed(indptr, indices, n) is view
+        busy = side.record_event()
+    held = [(t.data_ptr(), t.numel(), t.dtype) for t in (plan, view.t_rows, view.t_perm)]
+    del plan, view
+    graph_ext.forget(indptr, indices)
+    fresh = [torch.empty(numel, dtype=dtype, device=dev) for _, numel, dtype in held for _ in range(4)]
+    assert not busy.query(), "the second stream ended too early to tell"
+    assert not {t.data_ptr() for t in fresh} & {address for address, _, _ in held}
+    torch.cuda.synchronize()

@@ -129,7 +129,8 @@ def workspace(n_bytes, device):
 # the builders in data/csr.py and the samplers return fresh tensors and need not.
 #
 # Derived buffers are built on the stream that was current at the time; a later use on
-# another stream waits for the build through an event recorded right behind it.
+# another stream waits for the build through an event recorded right behind it, and the
+# buffers are not handed to anybody else before that use is over.
 
 
 class _Built:
@@ -143,7 +144,13 @@ class _Built:
 
     def get(self, device):
         if stream_ptr(device).value != self.raw_stream:  # two integers in the common case
-            torch.cuda.current_stream(device).wait_event(self.event)
+            stream = torch.cuda.current_stream(device)
+            stream.wait_event(self.event)
+            held = [self.value] if torch.is_tensor(self.value) else \
+                [getattr(self.value, name) for name in self.value.__slots__]
+            for t in held:
+                if torch.is_tensor(t) and t.is_cuda:
+                    t.record_stream(stream)
         return self.value
 
 
