@@ -199,3 +199,43 @@ def test_state_in_use_on_another_stream_is_not_handed_out_again(dev):
     assert not busy.query(), "the second stream ended too early to tell"
     assert not {t.data_ptr() for t in fresh} & {address for address, _, _ in held}
     torch.cuda.synchronize()
+
+
+def test_state_forgotten_while_a_backward_waits_for_it(dev):
+    """A backward on another stream than the plan's finds the plan without the interpreter lock
+    and then waits for the lock to wait for the plan's event; another thread forgets the
+    graph in between. The entry has to outlive that."""
+    import sys
+    import threading
+    import time
+    from yitu_amd.xgnn_h import sparse
+    indptr, indices = (t.to(dev) for t in powerlaw_graph(12, 60000, 5))
+    n = indptr.numel() - 1
+    values = torch.rand(indices.numel(), 1, device=dev)
+    x = torch.randn(n, 1, 16, device=dev, requires_grad=True)
+    out = sparse.GSPMMFunction.apply((indptr, indices), values, x)
+    want = torch.autograd.grad(out.sum(), x, retain_graph=True)[0]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        out = sparse.GSPMMFunction.apply((indptr, indices), values, x)
+    torch.cuda.synchronize()
+    got = []
+    for _ in range(3):
+        worker = threading.Thread(target=lambda: got.append(
+            torch.autograd.grad(out.sum(), x, retain_graph=True)[0]))
+        interval = sys.getswitchinterval()
+        worker.start()
+        try:
+            sys.setswitchinterval(0.2)  # this thread keeps the lock while the backward asks for it
+            until = time.monotonic() + 0.05
+            while time.monotonic() < until:
+                pass
+            graph_ext.forget(indptr, indices)
+        finally:
+            sys.setswitchinterval(interval)
+        worker.join()
+        torch.cuda.synchronize()
+    assert len(got) == 3
+    for g in got:
+        assert torch.allclose(g, want, rtol=1e-5, atol=1e-5)

@@ -4,6 +4,7 @@
 // entries on a miss (yitu_amd/_lib.py, yitu_amd/graph_ext.py), stores them here and drops
 // them when the tensor dies or is named to forget(). A use on another stream than the one
 // an entry was built on waits for the build's event (_lib._Built).
+#include <memory>
 #include <mutex>
 
 #include "bind.hpp"
@@ -43,9 +44,19 @@ struct Degree {
     Owner indptr;
     int64_t value;
 };
+// A Python object that threads without the interpreter lock may take and give back.
+struct Held {
+    py::object object;
+    explicit Held(py::object o) : object(std::move(o)) {}
+    ~Held() {
+        py::gil_scoped_acquire gil;
+        object = py::object();
+    }
+};
+using HeldPtr = std::shared_ptr<Held>;
 struct Built {
     Owner indptr, indices;
-    py::object built;  // _lib._Built
+    HeldPtr built;     // _lib._Built
     py::object value;  // the plan tensor, or graph_ext's by-source object
     void *stream;
     BySource view;  // by-source entries only
@@ -77,23 +88,24 @@ int64_t find_degree(const Tensor &indptr) {
     return it != degrees.end() && it->second.indptr.is(indptr) ? it->second.value : -1;
 }
 
-// Calls found(entry) under the lock; false when there is no entry. *built is set when the
-// caller has to wait for the entry's event (with the interpreter lock, after this returns).
+// Calls found(entry) under the lock; false when there is no entry. *wait is set when the
+// caller has to wait for the entry's event (with the interpreter lock, after this returns):
+// a reference of its own, another thread may drop the entry meanwhile.
 template <typename F>
 bool find_built(BuiltMap &map, const Tensor &indptr,
-                const Tensor &indices, int64_t n_src, int mask, PyObject **wait, F found) {
+                const Tensor &indices, int64_t n_src, int mask, HeldPtr *wait, F found) {
     std::lock_guard<std::mutex> g(lock);
     auto it = map.find(Key{id(indices), id(indptr), n_src, mask});
     if (it == map.end() || !it->second.indices.is(indices) || !it->second.indptr.is(indptr))
         return false;
-    *wait = it->second.stream != stream_of(indices) ? it->second.built.ptr() : nullptr;
+    *wait = it->second.stream != stream_of(indices) ? it->second.built : nullptr;
     found(it->second);
     return true;
 }
-void wait_for(PyObject *built, const Tensor &t) {
+void wait_for(const HeldPtr &built, const Tensor &t) {
     if (!built) return;
     py::gil_scoped_acquire gil;
-    py::reinterpret_borrow<py::object>(built).attr("get")(py::cast(t.device()));
+    built->object.attr("get")(py::cast(t.device()));
 }
 
 int64_t max_degree(const Tensor &indptr) {
@@ -106,7 +118,7 @@ int64_t max_degree(const Tensor &indptr) {
 void put_built(BuiltMap &map, const Tensor &indptr,
                const Tensor &indices, int64_t n_src, int mask, const py::object &built,
                bool view) {
-    Built b{Owner(indptr), Owner(indices), built, built.attr("value"), stream_of(indices), {}, {}};
+    Built b{Owner(indptr), Owner(indices), std::make_shared<Held>(built), built.attr("value"), stream_of(indices), {}, {}};
     if (view) b.view = by_source_of(b.value);
     else b.plan = b.value.cast<Tensor>();
     std::optional<Built> old;  // destroyed after the lock is given back
@@ -160,7 +172,7 @@ RowState row_state(const Tensor &indptr, const Tensor &indices, int64_t n_src, i
     s.max_degree = max_degree(indptr);
     // as _lib.row_plan: no plan for small graphs without long rows
     if (s.max_degree < kLongRow && indices.numel() < kPlanMinEdges) return s;
-    PyObject *wait = nullptr;
+    HeldPtr wait;
     if (find_built(plans, indptr, indices, n_src, mask, &wait, [&](Built &b) { s.plan = b.plan; })) {
         wait_for(wait, indices);
         return s;
@@ -174,7 +186,7 @@ RowState row_state(const Tensor &indptr, const Tensor &indices, int64_t n_src, i
 
 BySource by_source(const Tensor &indptr, const Tensor &indices, int64_t n_src) {
     BySource s;
-    PyObject *wait = nullptr;
+    HeldPtr wait;
     if (find_built(views, indptr, indices, n_src, 0, &wait, [&](Built &b) { s = b.view; })) {
         wait_for(wait, indices);
         return s;
@@ -229,7 +241,7 @@ void bind_graph_state(py::module_ &m) {
     const auto find = [](auto &map, const Tensor &indptr, const Tensor &indices, int64_t n_src,
                          int mask) -> py::object {
         py::object value = py::none();
-        PyObject *wait = nullptr;
+        HeldPtr wait;
         if (find_built(map, indptr, indices, n_src, mask, &wait, [&](Built &b) { value = b.value; }))
             wait_for(wait, indices);
         return value;
