@@ -2,6 +2,8 @@
 edge softmax, hfused, the transposed-structure builder) against the CPU oracle,
 through the C ABI, plus the reference's own dense-torch checks run end to end
 through the autograd wrappers."""
+import time
+
 import numpy as np
 import pytest
 import torch
@@ -9,7 +11,7 @@ from torch import nn
 
 import oracle
 from helpers import softmax_backward_abs_sums, spmm_abs_sums, assert_close, powerlaw_graph, random_csr
-from yitu_amd import graph_ext
+from yitu_amd import _lib, graph_ext
 from yitu_amd.xgnn_h import block as xblock
 from yitu_amd.xgnn_h import sparse
 
@@ -698,3 +700,31 @@ def test_spmm_backward_refuses_other_shapes_with_kept_weights(dev):
         out = sparse.GSPMMFunction.apply((indptr, indices), values, x16)
         with pytest.raises(RuntimeError, match="features"):
             out.sum().backward()
+
+
+def test_by_source_weights_made_on_another_stream_are_waited_for(dev):
+    """The copy of the weights in by-source order is made on the stream of the call that makes it;
+    a call on another stream that finds it waits for it."""
+    indptr, indices = (t.to(dev) for t in powerlaw_graph(12, 50000, 17))
+    n = indptr.numel() - 1
+    values = torch.rand(indices.numel(), 1, device=dev)
+    x, gy = torch.randn(n, 1, 24, device=dev), torch.randn(n, 1, 24, device=dev)
+    args = (values, indptr, indices, x, gy)
+    want = graph_ext.spmm_backward(*args, need_grad_a=False)[1]  # seen once
+    view = graph_ext.transposed(indptr, indices, n)
+    _lib.row_plan(view.t_indptr, view.t_rows, n, graph_ext.COL_MASK)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(200_000_000)
+    first = graph_ext.spmm_backward(*args, need_grad_a=False)[1]  # makes the copy, behind the sleep
+    made = torch.cuda.current_stream().record_event()
+    with torch.cuda.stream(side):
+        second = graph_ext.spmm_backward(*args, need_grad_a=False)[1]
+        used = side.record_event()
+    time.sleep(0.01)
+    early = used.query()
+    assert not made.query(), "the first stream ended too early to tell"
+    assert not early
+    torch.cuda.synchronize()
+    assert_close(first, want, atol=1e-3)
+    assert torch.equal(first, second)

@@ -67,6 +67,8 @@ struct Weights {  // edge weights that came by, and their copy in by-source orde
     Owner values, indptr, indices;
     int64_t n_src;
     OptTensor copy;
+    HeldPtr built;  // _lib._Built of the copy
+    void *stream;
 };
 
 std::mutex lock;
@@ -134,14 +136,14 @@ void put_built(BuiltMap &map, const Tensor &indptr,
 
 void drop(const void *impl) {
     std::vector<Built> old;  // destroyed after the lock is given back
-    OptTensor old_copy;
+    std::vector<Weights> old_weights;
     {
         std::lock_guard<std::mutex> g(lock);
         degrees.erase(impl);
         for (auto it = weights.begin(); it != weights.end();)
             if (it->first == impl || it->second.indptr.ref._unsafe_get_target() == impl ||
                 it->second.indices.ref._unsafe_get_target() == impl) {
-                old_copy = std::move(it->second.copy);
+                old_weights.push_back(std::move(it->second));
                 it = weights.erase(it);
             } else
                 ++it;
@@ -204,6 +206,8 @@ BySource by_source(const Tensor &indptr, const Tensor &indices, int64_t n_src) {
 OptTensor by_source_values(const Tensor &values, const Tensor &indptr, const Tensor &indices,
                            int64_t n_src, bool force) {
     bool known = false, seen = false;
+    OptTensor copy;
+    HeldPtr wait;
     {
         std::lock_guard<std::mutex> g(lock);
         auto it = weights.find(id(values));
@@ -212,22 +216,35 @@ OptTensor by_source_values(const Tensor &values, const Tensor &indptr, const Ten
                it->second.indptr.ref._unsafe_get_target() == id(indptr) &&
                it->second.indices.ref._unsafe_get_target() == id(indices) &&
                it->second.indptr.is(indptr) && it->second.indices.is(indices);
-        if (seen && it->second.copy) return it->second.copy;
+        if (seen && it->second.copy) {
+            copy = it->second.copy;
+            if (it->second.stream != stream_of(values)) wait = it->second.built;
+        }
+    }
+    if (copy) {
+        wait_for(wait, values);
+        return copy;
     }
     if (!known) {
         py::gil_scoped_acquire gil;
         py::module_::import("yitu_amd._lib").attr("watch")(values);
     }
-    OptTensor copy;
-    if (seen || force) copy = values.index_select(0, by_source(indptr, indices, n_src).t_perm);
-    OptTensor old_copy;
+    HeldPtr built;
+    if (seen || force) {
+        copy = values.index_select(0, by_source(indptr, indices, n_src).t_perm);
+        py::gil_scoped_acquire gil;
+        built = std::make_shared<Held>(
+            py::module_::import("yitu_amd._lib").attr("_Built")(*copy, py::cast(values.device())));
+    }
+    std::optional<Weights> old;  // destroyed after the lock is given back
     std::lock_guard<std::mutex> g(lock);
     auto it = weights.find(id(values));
     if (it != weights.end()) {
-        old_copy = std::move(it->second.copy);
+        old = std::move(it->second);
         weights.erase(it);
     }
-    weights.emplace(id(values), Weights{Owner(values), Owner(indptr), Owner(indices), n_src, copy});
+    weights.emplace(id(values), Weights{Owner(values), Owner(indptr), Owner(indices), n_src, copy,
+                                        built, stream_of(values)});
     return copy;
 }
 
