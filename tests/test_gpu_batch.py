@@ -5,7 +5,7 @@ import torch
 
 import pipeline_cases as cases
 from helpers import assert_close
-from yitu_amd import _lib, xgnn_h
+from yitu_amd import _lib, graph_ext, xgnn_h
 from yitu_amd.xgnn_h import ir, models
 
 pytestmark = pytest.mark.gpu
@@ -129,6 +129,35 @@ def test_batched_model_equals_one_relation_at_a_time(dev, which, stitch, relatio
         assert (a is None) == (b is None)
         if a is not None:
             assert_close(b, a, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("which", ["rgcn", "rgat"])
+def test_forget_reaches_what_a_batched_model_keeps(dev, which):
+    """Index and norm tensors refilled past torch's version counter and named to forget(): the
+    executor's block-diagonal copies and edge weights are made again."""
+    torch.manual_seed(2)
+    hgraph = cases.hetero_graph(device=dev)
+    kwargs = cases.hetero_kwargs(hgraph, device=dev, with_norms=which == "rgcn")
+    model = (models.RGCNModel(hgraph, 12, 16, 5) if which == "rgcn"
+             else models.RGATModel(hgraph, 12, 16, 8, n_heads=2)).to(dev)
+    flow = xgnn_h.Optimizer().lower(xgnn_h.Module2IR().transform(model, kwargs), kwargs)
+    executor, plain = xgnn_h.Executor(), xgnn_h.Executor(group_linears=False)
+    for e in (executor, plain):
+        e.eval()
+    before = executor.run(flow, kwargs)
+    for g in hgraph.hetero_graph.values():
+        indices = g.blk.adj_sparse[1]
+        version = indices._version
+        indices.data.copy_((indices + 1) % g.blk.size[1])
+        assert indices._version == version
+        graph_ext.forget(*g.blk.adj_sparse)
+    for norm in kwargs.get("norms", {}).values():
+        norm.data.mul_(3.0)
+        graph_ext.forget(norm)
+    after, want = executor.run(flow, kwargs), plain.run(flow, kwargs)
+    for t in want:
+        assert_close(after[t], want[t], rtol=1e-4, atol=1e-5)
+        assert not torch.allclose(after[t], before[t], rtol=1e-2, atol=1e-2)
 
 
 @pytest.mark.parametrize("which", ["rgcn", "rgat"])

@@ -160,12 +160,24 @@ def watch(tensor):
     weakref.finalize(tensor, native.drop, native.impl_of(tensor)).atexit = False
 
 
+_forgotten = {}  # id of a live tensor -> how often it was named to forget()
+
+
 def forget(*tensors):
     """Drops every cached widest row and row plan derived from the given index tensors
     (call after refilling one of them in place through a raw pointer)."""
     for t in tensors:
         if t is not None:
             ops().drop(ops().impl_of(t))
+            if id(t) not in _forgotten:
+                weakref.finalize(t, _forgotten.pop, id(t), None).atexit = False
+            _forgotten[id(t)] = _forgotten.get(id(t), 0) + 1
+
+
+def state_of(tensors):
+    """What changes when one of the tensors (which the caller keeps alive) is replaced, written
+    by torch, or named to ``forget``: for copies kept beside what they were made from."""
+    return [(id(t), t.data_ptr(), t._version, _forgotten.get(id(t), 0)) for t in tensors]
 
 
 def max_degree(indptr):

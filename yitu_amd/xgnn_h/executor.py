@@ -156,14 +156,15 @@ class Executor:
             # per-edge weights of a stitched block from the relations' row scales: constants
             # of the graph, so they are kept for as long as the same scale tensors come by
             parts = [v[str(i)] for i in range(len(node.inputs) - 1)]
-            state = tuple((id(t), t.data_ptr(), t._version) for t in parts) + (id(v["g"]),)
+            adj = list(v["g"].adj_sparse)
+            state = _lib.state_of(parts + adj)
             kept = self._edge_values.get(id(node))
             if any(t.requires_grad for t in parts):
                 kept = None  # scales that train: compute (and differentiate) every time
             if kept is None or kept[0] != state:
                 scales = torch.stack([t.reshape(-1) for t in parts])
                 rows, _, bids = mp.edge_endpoints(v["g"])
-                kept = (state, scales[bids, rows].unsqueeze(-1).contiguous(), parts)
+                kept = (state, scales[bids, rows].unsqueeze(-1).contiguous(), parts + adj)
                 if not any(t.requires_grad for t in parts):
                     self._edge_values[id(node)] = kept
             return kept[1]
@@ -236,7 +237,7 @@ class Executor:
         spec = node.attrs["spec"]
         scales = [[v["s%d.%d" % (i, j)] for j in range(n)] for i, (_, n) in enumerate(spec)]
         flat = [t for s in scales for t in s]
-        state = [(id(t), t.data_ptr(), t._version) for t in flat]
+        state = _lib.state_of(flat)
         trains = any(t.requires_grad for t in flat)
         if not trains and kept.get("state") == state:
             return kept["weights"]
@@ -279,7 +280,7 @@ class Executor:
         # aggregation or attention over the members' stacked blocks
         blocks = [v["g%d" % i] for i in range(sum(1 for k in node.inputs if k[0] == "g"))]
         adj = [t for b in blocks for t in b.adj_sparse]
-        state = [(id(t), t._version) for t in adj]
+        state = _lib.state_of(adj)
         if plan is None or plan[1] != state:
             build = batch.spmm_block if op == "spmm_rows" else batch.gat_block
             plan = (node, state, adj, build(blocks, a["spec"], a["n_cols"]), {})
