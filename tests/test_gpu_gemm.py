@@ -515,6 +515,24 @@ def test_sgemm_many_rows_small_weight(dev, ms, n, k, tb):
             assert_close(y, c.cpu() + b, atol=1e-5 * max(1.0, k ** 0.5))
 
 
+@pytest.mark.parametrize("tb", [False, True])
+@pytest.mark.parametrize("m,n,k", [(100_000, 128, 100), (150_000, 47, 100), (100_001, 96, 192),
+                                   (70_001, 128, 128), (66_000, 136, 136), (20_001, 77, 333),
+                                   (17_003, 16, 500), (16_400, 7, 3), (70_000, 64, 63)])
+def test_sgemm_bits_do_not_depend_on_the_row_count(dev, m, n, k, tb):
+    """Many rows take the kernel that holds the weight in LDS, fewer the tiled one: a row's sums
+    are added in the same order, so that what follows a product (a LeakyReLU of millions of
+    logits has some within a last bit of zero) does not change with the number of rows."""
+    g = torch.Generator().manual_seed(m + n)
+    x = torch.randn(m, k, generator=g).to(dev)
+    w = torch.randn((n, k) if tb else (k, n), generator=g).to(dev)
+    whole = graph_ext.sgemm_typed([x], [w], False, tb)[0]
+    few = 16_383  # (enough tiles that no inner dimension is split)
+    for first in (0, (m - few) // 2, m - few):
+        part = graph_ext.sgemm_typed([x[first:first + few].clone()], [w], False, tb)[0]
+        assert torch.equal(whole[first:first + few], part)
+
+
 @pytest.mark.parametrize("n,k,ja,jb", [(1, 4, 1, 1), (15, 20, 3, 2), (16, 64, 8, 8), (17, 60, 1, 3),
                                        (1000, 128, 4, 4), (513, 100, 8, 8), (4099, 256, 8, 8),
                                        (70, 132, 5, 0), (300, 512, 4, 4), (129, 260, 3, 5),

@@ -6,8 +6,10 @@
 // every wave walks 32-row tiles of A on its own, KC columns at a time through an LDS area of
 // its own: no barrier in the loop, and nothing that one wave waits for holds up another. The
 // next chunk (or the next tile's first) is requested before the products of this one. MFMA
-// step s of lane (i, half) takes k = half * KC / 2 + s of the chunk, so the operands of four
-// steps are one 16-byte LDS read of either side; rows of both areas are padded by 16 bytes
+// step s takes columns 2 s and 2 s + 1 of the chunk, one per half of the wave: the order of the
+// tiled kernel, so a product keeps its bits when its row count moves it from one to the
+// other. Both areas hold every eight columns as four even ones, then four odd ones, so the operands
+// of four steps are one 16-byte LDS read of either side; rows of both areas are padded by 16 bytes
 // (an odd number of 16-byte pieces: conflict-free). The weight is the first MFMA operand: a
 // lane holds four consecutive columns of a row, and rows leave through the wave's LDS area as
 // 128-byte segments. A workgroup takes a run of consecutive tiles of the list of all
@@ -43,6 +45,11 @@ __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Place of a column in its row: 0 2 4 6 1 3 5 7 of every eight.
+constexpr __device__ __forceinline__ int panel_column(int k) {
+    return (k & ~7) | ((k & 1) << 2) | ((k >> 1) & 3);
+}
+
 template <int KC>
 constexpr int panel_chunk_floats() {
     return 32 * (KC + 4);
@@ -51,6 +58,7 @@ constexpr int panel_chunk_floats() {
 template <int NCW, int KC, bool VEC>
 __global__ __launch_bounds__(64 * kPanelWaves, 1) void sgemm_panel_kernel(PanelParams p) {
     typedef float f4 __attribute__((ext_vector_type(4)));
+    typedef float f2 __attribute__((ext_vector_type(2)));
     constexpr int A_LD = KC + 4;
     constexpr int LPR = VEC ? KC / 4 : KC;  // lanes that cover a row of a chunk (at most 64)
     constexpr int RPI = 64 / LPR;           // rows per load instruction
@@ -114,7 +122,7 @@ __global__ __launch_bounds__(64 * kPanelWaves, 1) void sgemm_panel_kernel(PanelP
                 const int64_t from = p.b_kcont ? (int64_t)(n0 + n) * p.ldb + k
                                                : (int64_t)k * p.ldb + n0 + n;
                 w[i] = in ? b_q[from] : 0.0f;
-                to[i] = n * p.ldw + k;
+                to[i] = n * p.ldw + panel_column(k);
                 major += major_step;
                 at += minor_step;
                 if (at >= minor) at -= minor, major++;
@@ -138,11 +146,12 @@ __global__ __launch_bounds__(64 * kPanelWaves, 1) void sgemm_panel_kernel(PanelP
                 const bool tail = (c + 1) * KC > p.K;  // the chunk holds columns past K
 #pragma unroll
                 for (int i = 0; i < LI; i++) {
-                    float *dst = At + (lrow + RPI * i) * A_LD + lcol;
+                    float *dst = At + (lrow + RPI * i) * A_LD + panel_column(lcol);
                     if constexpr (VEC) {
                         f4 v = r4[i];
                         if (tail && c * KC + lcol >= p.K) v = f4{0.0f, 0.0f, 0.0f, 0.0f};
-                        *reinterpret_cast<f4 *>(dst) = v;
+                        *reinterpret_cast<f2 *>(dst) = f2{v[0], v[2]};
+                        *reinterpret_cast<f2 *>(dst + 4) = f2{v[1], v[3]};
                     } else {
                         *dst = tail && c * KC + lcol >= p.K ? 0.0f : r1[i];
                     }
@@ -150,16 +159,16 @@ __global__ __launch_bounds__(64 * kPanelWaves, 1) void sgemm_panel_kernel(PanelP
                 if (c + 1 < n_chunks) gload(tile, c + 1);
                 else if (tile + n_waves < hi) gload(tile + n_waves, 0);
                 wave_lds_fence();
-                // the two halves of the wave take the two halves of the chunk
+                // the halves of the wave take the even and the odd columns
                 const int half = min(KC, p.k_pad - c * KC) / 2;
-                const float *arow = At + l32 * A_LD + lk * half;
-                const float *wrow = Wl + (size_t)l32 * p.ldw + c * KC + lk * half;
+                const float *arow = At + l32 * A_LD + 4 * lk;
+                const float *wrow = Wl + (size_t)l32 * p.ldw + c * KC + 4 * lk;
                 const auto step4 = [&](int s) {
-                    const f4 a = *reinterpret_cast<const f4 *>(arow + s);
+                    const f4 a = *reinterpret_cast<const f4 *>(arow + 2 * s);
                     f4 w[NCW];
 #pragma unroll
                     for (int j = 0; j < NCW; j++)
-                        w[j] = *reinterpret_cast<const f4 *>(wrow + (size_t)32 * j * p.ldw + s);
+                        w[j] = *reinterpret_cast<const f4 *>(wrow + (size_t)32 * j * p.ldw + 2 * s);
 #pragma unroll
                     for (int e = 0; e < 4; e++)
 #pragma unroll
