@@ -370,11 +370,46 @@ def test_every_dropout_of_a_batched_model_draws_for_itself(stitch):
     assert cases.ops_of(xgnn_h.batch.batch_rows(flow, kwargs))["dropout"] == 0
 
 
+def _call(fn, *nodes, size, extra=()):
+    slots = tuple(ir.Slot(str(i)) for i in range(len(nodes)))
+    return ir.Node("call", {str(i): n for i, n in enumerate(nodes)},
+                   {"fn": fn, "args": slots + tuple(extra), "kwargs": {}}, size)
+
+
 def test_dropout_of_rows_read_twice_is_not_one_draw_over_the_batch():
     x = ir.Node("input", size=[5, 4], name="x")
     h, k = (ir.Node("linear", {"x": x}, {"weight": torch.randn(4, 4), "bias": None}, [5, 4])
             for _ in range(2))
+    for fn in (torch.tanh, torch.sigmoid, torch.tanh, torch.sigmoid):
+        h, k = _call(fn, h, size=[5, 4]), _call(fn, k, size=[5, 4])
     both = ir.Node("concat", {"0": h, "1": h, "2": k}, size=[15, 4])
     flow = ir.Node("dropout", {"x": both}, {"p": 0.5}, [15, 4])
     batched = xgnn_h.batch.batch_rows(flow, {"x": torch.randn(5, 4)}, training=True)
     assert [n.size for n in ir.walk(batched) if n.op == "dropout"] == [[15, 4]]
+
+
+def test_sum_over_relations_is_part_of_the_batch():
+    """The relations of a node type, one at a time in the dataflow: their sum, its division and
+    the activation are one pass, without a slice of the batch; a sum whose order would change
+    stays as it is."""
+    hgraph = cases.hetero_graph()
+    kwargs = cases.hetero_kwargs(hgraph)
+    flow = xgnn_h.Optimizer().lower(
+        xgnn_h.Module2IR().transform(models.RGCNModel(hgraph, 8, 8, 4), kwargs), kwargs)
+    ops = cases.ops_of(xgnn_h.batch.batch_rows(flow, kwargs))
+    assert ops["fold"] == 2 and ops["rows"] == 0 and ops["spmm_rows"] == 2
+    x = ir.Node("input", size=[9, 4], name="x")
+    g = [ir.Node("graph", size=[9, 9], name="g.%d" % i) for i in range(4)]
+    agg = [ir.Node("spmm", {"g": n, "x": _call(torch.Tensor.view, ir.Node(
+        "linear", {"x": x}, {"weight": torch.randn(4, 4), "bias": None}, [9, 4]), size=[9, 1, 4],
+        extra=([-1, 1, 4],))}, size=[9, 1, 4]) for n in g]
+    left = _call(torch.add, _call(torch.add, _call(torch.add, agg[0], agg[1], size=[9, 1, 4]), agg[2],
+                                  size=[9, 1, 4]), agg[3], size=[9, 1, 4])
+    (fold,) = [n for n in ir.walk(xgnn_h.batch.batch_rows(left, {"g": None})) if n.op == "fold"]
+    assert [r[1] for r in fold.attrs["ranges"]] == [[0, 9, 18, 27]]
+    pairs = _call(torch.add, _call(torch.add, agg[0], agg[1], size=[9, 1, 4]),
+                  _call(torch.add, agg[2], agg[3], size=[9, 1, 4]), size=[9, 1, 4])
+    batched = xgnn_h.batch.batch_rows(pairs, {"g": None})
+    (fold,) = [n for n in ir.walk(batched) if n.op == "fold"]
+    assert sorted(r[1] for r in fold.attrs["ranges"]) == [[0, 9], [18, 27]]
+    assert batched.op == "call" and batched.fn_name() == "add"

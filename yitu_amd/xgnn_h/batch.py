@@ -20,7 +20,7 @@ import torch
 from torch.nn import functional as F
 
 from . import block, ir, mp
-from .stitcher import _match_term
+from .stitcher import _is_add, _match_term
 
 MAX_COLUMNS = 1 << 24  # what a packed CSR holds (block.py:53)
 
@@ -78,7 +78,7 @@ class _Batcher:
                 self.readers.setdefault(id(c), []).append(n)
         self.is_root = {id(r) for r in self.roots}
         self.value, self.parts, self.memo = {}, {}, {}
-        self.joined = 0  # members of groups of two or more
+        self.together = False  # a group of two or more has been joined
         self.depth = {}
         for n in self.order:
             self.depth[id(n)] = 1 + max([self.depth[id(c)] for c in n.inputs.values()], default=0)
@@ -263,6 +263,9 @@ class _Batcher:
                 return ("gat", id(q.node), id(k.node), id(x.node), bool(node.attrs.get("head_mean")))
         return None
 
+    def _count(self, members):
+        self.together = self.together or len(members) > 1
+
     def _linears(self, members):
         units = []  # (query side, node, which, weight, bias, original input)
         for m in members:
@@ -287,11 +290,14 @@ class _Batcher:
             if at == len(bases):
                 bases.append(base)
             refs.append((at, first, rows))
-        if len(units) == 1 and refs[0][1:] == (0, self._rows_of(bases[0])):
-            m = units[0][1]
+        m = members[0]
+        if len(members) == 1 and (len(units) == 1 or m.op == "bundle") and \
+                refs[0][1:] == (0, self._rows_of(bases[0])):
+            # nobody to join: a product is a launch, and so are the two of a bundle (with a few
+            # outputs a kernel of their own that reads x once)
             self._done(m, _Value(m.with_inputs({k: bases[0] for k in m.inputs})))
             return
-        self.joined += len(units)
+        self._count(members)
         made = ir.Node("typed_rows", {str(i): b for i, b in enumerate(bases)},
                        {"units": refs, "weights": [u[3] for u in units], "biases": [u[4] for u in units],
                         "base_rows": [self._rows_of(b) for b in bases]},
@@ -333,15 +339,50 @@ class _Batcher:
                 return node, divisor, 0, 0.0, tail
             node = nxt
 
+    def _sums(self, members, places):
+        """The members, those whose results are only ever added up joined: [(nodes that the sum
+        makes unnecessary, its last node, its row ranges in the order of the additions)]."""
+        parts = {}  # id of a member's last view -> what stands in the result
+        for m, p in zip(members, places):
+            through = []
+            while len(self.readers.get(id(m), [])) == 1 and id(m) not in self.is_root:
+                nxt = self.readers[id(m)][0]
+                if not (nxt.op == "call" and nxt.fn_name() == "squeeze" and len(nxt.inputs) == 1 and
+                        nxt.attrs["kwargs"].get("dim") == 1 and len(m.size) == 3 and m.size[1] == 1):
+                    break
+                through.append(m)
+                m = nxt
+            parts[id(m)] = (through, m, p)
+        waiting = list(parts)
+        while waiting:
+            first = parts.get(waiting.pop())
+            if first is None:
+                continue
+            readers = self.readers.get(id(first[1]), [])
+            add = readers[0] if len(readers) == 1 else None
+            if add is None or not _is_add(add) or id(first[1]) in self.is_root:
+                continue
+            a, b = (add.inputs[s.key] for s in add.attrs["args"])
+            # a left-hand chain, so that the sum adds in its order; ((a + b) + c)
+            if a is b or id(a) not in parts or id(b) not in parts or a.size != b.size or \
+                    len(parts[id(b)][2]) != 1 or \
+                    any(len(self.readers[id(c)]) != 1 or id(c) in self.is_root for c in (a, b)):
+                continue
+            (ta, _, pa), (tb, _, pb) = parts.pop(id(a)), parts.pop(id(b))
+            parts[id(add)] = (ta + [a] + tb + [b], add, pa + pb)
+            waiting.append(id(add))
+        return list(parts.values())
+
     def _fold(self, members, made, places):
         """Values of the members (``places``: the row ranges of each, to be added up)."""
-        ends = [self._chain(m) for m in members]
-        if all(e[1:4] == (1.0, 0, 0.0) and len(p) == 1 for e, p in zip(ends, places)):
+        sums = self._sums(members, places)
+        ends = [self._chain(m) for _, m, _ in sums]
+        if all(e[1:4] == (1.0, 0, 0.0) and len(p) == 1 for e, (_, _, p) in zip(ends, sums)):
             for m, p in zip(members, places):
                 self._done(m, _Value(made, p))
             return
         ranges = [(p[0][1], [o for o, _ in p], d, act, alpha)
-                  for (_, d, act, alpha, _), p in zip(ends, places)]
+                  for (_, d, act, alpha, _), (_, _, p) in zip(ends, sums)]
         off = 0
         groups = {}  # rows of one shape make one value; (they do, but for members of other shapes)
         for e in ends:
@@ -349,8 +390,10 @@ class _Batcher:
         (tail,) = groups if len(groups) == 1 else (tuple(made.size[1:]),)
         node = ir.Node("fold", {"x": made}, {"ranges": ranges, "tail": list(tail)},
                        [sum(r[0] for r in ranges)] + list(tail))
-        for m, (last, _, _, _, own), r in zip(members, ends, ranges):
-            while m is not last:  # the nodes in between exist no longer
+        for (through, m, _), (last, _, _, _, own), r in zip(sums, ends, ranges):
+            for n in through:  # the nodes in between exist no longer
+                self._finish(n)
+            while m is not last:
                 self._finish(m)
                 m = self.readers[id(m)][0]
             v = _Value(node, [(off, r[0])])
@@ -378,7 +421,7 @@ class _Batcher:
             for m in members:
                 self._alone(m)
             return
-        self.joined += len(members)
+        self._count(members)
         inputs, spec, places, off = {"x": xv[0].node}, [], [], 0
         for i, (m, x) in enumerate(zip(members, xv)):
             inputs["g%d" % i] = self._tensor(m.inputs["g"])
@@ -438,7 +481,7 @@ class _Batcher:
             for m in members:
                 self._alone(m)
             return
-        self.joined += len(members)
+        self._count(members)
         q = self.value[id(members[0].inputs["q"])]
         k = self.value[id(members[0].inputs["k"])]
         x = self.value[id(members[0].inputs["x"])]
@@ -508,7 +551,7 @@ class _Batcher:
             taken = {id(n) for n in members}
             waiting = [n for n in waiting if id(n) not in taken]
             {"linear": self._linears, "spmm": self._spmms, "gat": self._gats}[key[0]](members)
-        if self.joined < 2:
+        if not self.together:
             return None
         return self._outputs()
 
