@@ -30,6 +30,26 @@ def test_fold_of_row_ranges(dev, width):
     assert_close(torch.autograd.grad(out, x, dy)[0], torch.autograd.grad(want, x, dy)[0])
 
 
+@pytest.mark.parametrize("width,scale", [(64, 70_000), (3, 400_000), (256, 16_400), (7, 150_001)])
+def test_fold_of_many_rows(dev, width, scale):
+    """Sizes at which a thread takes several vectors: workgroups inside a range, across two and
+    over a row of tiny ones, the last one not full, with every activation."""
+    g = torch.Generator().manual_seed(width)
+    rows = [scale, 3, 1, 5, scale // 3, 2, scale // 5 + 1]
+    starts = torch.tensor([0] + [2 * r for r in rows]).cumsum(0).tolist()
+    total = starts[-1] + 4
+    ranges = [(r, [s, s + r][:1 + i % 2] + ([s + r] if i == 4 else []), (1.0, 3.0)[i % 2], i % 3, 0.8)
+              for i, (r, s) in enumerate(zip(rows, starts))]
+    x = torch.randn(total, width, generator=g).to(dev).requires_grad_()
+    out = _lib.ops().fold_rows(x, _lib.ops().fold_plan(total, ranges, x))
+    want = torch.cat([(lambda v: v.relu() if act == 1 else torch.nn.functional.elu(v, alpha)
+                       if act == 2 else v)(sum(x[s:s + r] for s in sources) / div)
+                      for r, sources, div, act, alpha in ranges])
+    assert_close(out, want)
+    dy = torch.randn(want.shape, generator=g).to(dev)
+    assert_close(torch.autograd.grad(out, x, dy)[0], torch.autograd.grad(want, x, dy)[0])
+
+
 @pytest.mark.parametrize("split", [False, True])
 def test_fold_result_may_be_written_where_no_activation_made_it(dev, split):
     def run(ranges, write):
