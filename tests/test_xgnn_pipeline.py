@@ -388,6 +388,43 @@ def test_dropout_of_rows_read_twice_is_not_one_draw_over_the_batch():
     assert [n.size for n in ir.walk(batched) if n.op == "dropout"] == [[15, 4]]
 
 
+@pytest.mark.parametrize("rows", [1000, 1_000_000])
+def test_batch_cut_into_slices_is_kept_only_where_it_pays(rows):
+    """Eight products whose results each meet something else: a launch instead of eight, but every
+    result is cut out of the batch again (a zero-filled gradient of its full height each)."""
+    w = [torch.randn(64, 64) for _ in range(8)]
+    xs = [ir.Node("input", size=[rows, 64], name="x.%d" % i) for i in range(8)]
+    hs = [ir.Node("linear", {"x": x}, {"weight": v, "bias": None}, [rows, 64]) for x, v in zip(xs, w)]
+    flow = {str(i): _call(torch.add, h, x, size=[rows, 64]) for i, (h, x) in enumerate(zip(hs, xs))}
+    # (eight products become one, eight slices appear: no node less)
+    assert xgnn_h.batch.batch_rows(flow, {}) is None
+    chains = {k: v for k, v in flow.items()}
+    for k, h in zip(chains, hs):  # row-wise functions of each run once for all
+        t = h
+        for fn in (torch.tanh, torch.sigmoid, torch.tanh, torch.sigmoid):
+            t = _call(fn, t, size=[rows, 64])
+        chains[k] = _call(torch.add, t, xs[int(k)], size=[rows, 64])
+    batched = xgnn_h.batch.batch_rows(chains, {})
+    assert (batched is None) == (rows > 1000)
+
+
+@pytest.mark.parametrize("rows", [1000, 200_000])
+def test_attention_over_many_rows_runs_one_relation_at_a_time(rows):
+    def layer(x, g):
+        h = ir.Node("linear", {"x": x}, {"weight": torch.randn(64, 64), "bias": None}, [rows, 64])
+        q, k = (ir.Node("linear", {"x": h}, {"weight": torch.randn(4, 64), "bias": None}, [rows, 4])
+                for _ in range(2))
+        heads = _call(torch.Tensor.view, h, size=[rows, 4, 16], extra=([-1, 4, 16],))
+        return ir.Node("gat", {"g": g, "q": q, "k": k, "x": heads}, {"head_mean": True}, [rows, 16])
+
+    x = ir.Node("input", size=[rows, 64], name="x")
+    flow = {str(i): layer(x, ir.Node("graph", size=[rows, rows], name="g.%d" % i)) for i in range(3)}
+    batched = xgnn_h.batch.batch_rows(flow, {"g": None})
+    assert (batched is None) == (rows > 1000)
+    if batched is not None:
+        assert cases.ops_of(batched)["gat_rows"] == 1
+
+
 def test_sum_over_relations_is_part_of_the_batch():
     """The relations of a node type, one at a time in the dataflow: their sum, its division and
     the activation are one pass, without a slice of the batch; a sum whose order would change

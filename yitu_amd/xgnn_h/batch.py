@@ -16,6 +16,8 @@ squeezes, concatenations and selections cost nothing; only a reader outside the 
 gets its rows as a tensor of their own. Groups form as dynamic batching does it: whatever can
 be answered without a launch is, then the class with the shallowest ready nodes runs all of
 them."""
+import math
+
 import torch
 from torch.nn import functional as F
 
@@ -23,9 +25,22 @@ from . import block, ir, mp
 from .stitcher import _is_add, _match_term
 
 MAX_COLUMNS = 1 << 24  # what a packed CSR holds (block.py:53)
+# Attention models whose products have this many rows on average run one relation at a time: the
+# launches that a batch saves no longer count, while its few-column query and key products go
+# through the grouped GEMM instead of the kernel that reads x once, and the by-source pass writes the
+# rows of all destinations too. Forward and backward, ms, batched against one at a time: 256 -> 4 x 64
+# with 200,000 rows a product 9.1 : 8.2, 123,000 21.2 : 21.0 (stitched 21.2 : 22.2), 60,000
+# 13.1 : 14.8; 128 -> 4 x 32 with 333,000 14.3 : 13.1. (Without attention the batch is the faster one
+# at every size: 256 wide, 491,520 nodes 13.8 : 16.3, stitched 13.4 : 13.3; 400,000 6.3 : 6.6.)
+MANY_ROWS = 1 << 17
 
 _FOLD_ACT = {"relu": 1, "elu": 2}
 _ROWWISE = ("relu", "elu", "leaky_relu", "tanh", "sigmoid", "gelu", "div", "mul", "multiply")
+# A slice of a batch (``rows``) read by an op that is no part of it gets its gradient through a
+# zero-filled buffer of the batch's full height: a node's launches and 0.64 us per MB of the batch
+# (16 slices of 1 GB made a step of 14.3 ms 24.6), against a node's launches and host work, about
+# 20 us in both directions, for each that the batch does without.
+CUT_US_PER_BYTE, US_PER_NODE = 6.4e-7, 20.0
 
 
 class _Value:
@@ -79,6 +94,7 @@ class _Batcher:
         self.is_root = {id(r) for r in self.roots}
         self.value, self.parts, self.memo = {}, {}, {}
         self.together = False  # a group of two or more has been joined
+        self.attention, self.unit_rows = False, []  # of the joined groups
         self.depth = {}
         for n in self.order:
             self.depth[id(n)] = 1 + max([self.depth[id(c)] for c in n.inputs.values()], default=0)
@@ -298,6 +314,7 @@ class _Batcher:
             self._done(m, _Value(m.with_inputs({k: bases[0] for k in m.inputs})))
             return
         self._count(members)
+        self.unit_rows += [rows for _, _, rows in refs]
         made = ir.Node("typed_rows", {str(i): b for i, b in enumerate(bases)},
                        {"units": refs, "weights": [u[3] for u in units], "biases": [u[4] for u in units],
                         "base_rows": [self._rows_of(b) for b in bases]},
@@ -482,6 +499,7 @@ class _Batcher:
                 self._alone(m)
             return
         self._count(members)
+        self.attention = True
         q = self.value[id(members[0].inputs["q"])]
         k = self.value[id(members[0].inputs["k"])]
         x = self.value[id(members[0].inputs["x"])]
@@ -551,9 +569,17 @@ class _Batcher:
             taken = {id(n) for n in members}
             waiting = [n for n in waiting if id(n) not in taken]
             {"linear": self._linears, "spmm": self._spmms, "gat": self._gats}[key[0]](members)
-        if not self.together:
+        if not self.together or (self.attention and
+                                 sum(self.unit_rows) >= MANY_ROWS * len(self.unit_rows)):
             return None
-        return self._outputs()
+        flow = self._outputs()
+        nodes = ir.walk(flow)
+        slices = [n for n in nodes if n.op == "rows"]
+        ops = sum(bool(n.inputs) for n in self.order) - sum(bool(n.inputs) for n in nodes) + len(slices)
+        cut = sum(4 * math.prod(n.inputs["x"].size) for n in slices)
+        if cut * CUT_US_PER_BYTE + len(slices) * US_PER_NODE > ops * US_PER_NODE:
+            return None
+        return flow
 
     def _outputs(self):
         """The roots. Those that tile one fold become its separate outputs (whose backward takes
@@ -587,7 +613,7 @@ class _Batcher:
 
 def batch_rows(dataflow: ir.Dataflow, kwargs: dict, training: bool = False):
     """The batched form of ``dataflow`` for arguments shaped like ``kwargs`` (outputs and
-    gradients as before), or None where nothing runs together."""
+    gradients as before), or None where nothing runs together, or nothing is gained by it."""
     return _Batcher(dataflow, kwargs, training).build()
 
 
