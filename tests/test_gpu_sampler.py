@@ -88,6 +88,32 @@ def test_equals_host_sampler_over_a_stream_of_batches(dev, layers, fans, prop):
     _same(gpu.get_ret()[0], host.get_ret()[0], "after reset")
 
 
+@pytest.mark.parametrize("fan,n_roots", [(100, 300), (64, 64), (65, 500), (20, 16_384), (3, 16_385),
+                                         (2, 50_000)])
+def test_many_neighbours_and_many_roots(dev, fan, n_roots):
+    """Roots whose neighbours are more than a wave's lanes, and more roots than one workgroup
+    takes in the prefix sums of their counts: the same block as the host sampler's, and its
+    structure; a root that is no node is refused wherever it stands."""
+    rng = np.random.default_rng(fan)
+    indptr, indices, eid, tt, src, dst, ts = _tcsr(rng, 40, 8000)
+    assert np.diff(indptr).max() > 128
+    host = sampler_core.ParallelSampler(indptr, indices, eid, tt, 4, 1, 1, [fan], True, False, 1, 0.0)
+    gpu = sampler_core.GpuParallelSampler(indptr, indices, eid, tt, 4, 1, 1, [fan], True, False, 1,
+                                          0.0, device=dev)
+    ev = np.sort(rng.integers(0, 8000, n_roots))
+    host.sample(src[ev], ts[ev])
+    gpu.sample(src[ev], ts[ev])
+    want, got = host.get_ret()[0], gpu.get_ret()[0]
+    _same(got, want, (fan, n_roots))
+    assert np.array_equal(np.diff(got.indptr().cpu().numpy()),
+                          np.bincount(want.row(), minlength=n_roots))
+    for bad in (0, n_roots // 2, n_roots - 1):
+        roots = src[ev].copy()
+        roots[bad] = 40
+        with pytest.raises(RuntimeError, match="out of range"):
+            gpu.sample(roots, ts[ev])
+
+
 def test_empty_batch_and_bad_root(dev):
     rng = np.random.default_rng(1)
     indptr, indices, eid, tt, *_ = _tcsr(rng, 50, 400)

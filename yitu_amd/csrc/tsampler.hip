@@ -92,56 +92,90 @@ __global__ __launch_bounds__(kBlock) void ts_count_kernel(
     if (lane_id() == 0) counts[i] = cnt;
 }
 
-// block_indptr = exclusive prefix sums of the counts, by one workgroup in chunks of 16,384;
-// *n_edges_out = their total, or -1 with a root that is no node.
+// block_indptr = exclusive prefix sums of the counts, a workgroup per chunk of 16,384; *n_edges_out
+// = their total, or -1 with a root that is no node. Up to one chunk is one launch (2,048 roots:
+// 5 us); beyond, the chunks' sums are made first and every workgroup adds up those before it.
+constexpr int kStartsEach = 16, kStartsChunk = 1024 * kStartsEach;
+struct ChunkSum {
+    int32_t sum, bad;
+};
+
+// Sum over the workgroup's 1,024 threads (every thread gets it); red is theirs alone.
+__device__ __forceinline__ int block_sum(int v, int (&red)[16]) {
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, kWave);
+    __syncthreads();  // red may still be read
+    if (lane_id() == 0) red[wave_id()] = v;
+    __syncthreads();
+    int all = 0;
+    for (int w = 0; w < 16; w++) all += red[w];
+    return all;
+}
+
+__global__ __launch_bounds__(1024) void ts_chunk_sums_kernel(ChunkSum *__restrict__ chunks,
+                                                             const int32_t *__restrict__ counts,
+                                                             int64_t n_roots) {
+    __shared__ int red[16];
+    const int64_t base = (int64_t)blockIdx.x * kStartsChunk;
+    int sum = 0, bad = 0;
+    for (int k = 0; k < kStartsEach; k++) {
+        const int64_t i = base + k * 1024 + threadIdx.x;
+        const int v = i < n_roots ? counts[i] : 0;
+        sum += max(v, 0);
+        bad |= v < 0;
+    }
+    sum = block_sum(sum, red);
+    bad = block_sum(bad, red);
+    if (threadIdx.x == 0) chunks[blockIdx.x] = {sum, bad};
+}
+
 __global__ __launch_bounds__(1024) void ts_starts_kernel(int32_t *__restrict__ block_indptr,
                                                          long long *__restrict__ n_edges_out,
                                                          const int32_t *__restrict__ counts,
+                                                         const ChunkSum *__restrict__ chunks,
                                                          int64_t n_roots) {
-    constexpr int kEach = 16, kChunk = 1024 * kEach;
-    __shared__ int sums[16];
-    __shared__ int bad;
-    const int lane = lane_id(), wave = threadIdx.x / kWave;
-    if (threadIdx.x == 0) bad = 0;
-    __syncthreads();
-    int carry = 0;
-    for (int64_t base = 0; base < n_roots; base += kChunk) {
-        int v[kEach], own = 0;
-#pragma unroll
-        for (int k = 0; k < kEach; k++) {
-            const int64_t i = base + (int64_t)threadIdx.x * kEach + k;
-            v[k] = i < n_roots ? counts[i] : 0;
-            if (v[k] < 0) {
-                bad = 1;
-                v[k] = 0;
-            }
-            own += v[k];
+    __shared__ int red[16], sums[16];
+    const int lane = lane_id(), wave = wave_id(), n_chunks = gridDim.x;
+    int carry = 0, bad = 0;
+    if (n_chunks > 1) {
+        for (int w = threadIdx.x; w < n_chunks; w += 1024) {
+            carry += w < (int)blockIdx.x ? chunks[w].sum : 0;
+            bad |= chunks[w].bad;
         }
-        int pre = own;
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
-            const int x = __shfl_up(pre, o, kWave);
-            if (lane >= o) pre += x;
-        }
-        if (lane == kWave - 1) sums[wave] = pre;
-        __syncthreads();
-        int at = carry + pre - own, all = 0;
-        for (int w = 0; w < 16; w++) {
-            at += w < wave ? sums[w] : 0;
-            all += sums[w];
-        }
-#pragma unroll
-        for (int k = 0; k < kEach; k++) {
-            const int64_t i = base + (int64_t)threadIdx.x * kEach + k;
-            if (i < n_roots) block_indptr[i] = at;
-            at += v[k];
-        }
-        carry += all;
-        __syncthreads();
+        carry = block_sum(carry, red);
     }
-    if (threadIdx.x == 0) {
-        block_indptr[n_roots] = carry;
-        *n_edges_out = bad ? -1 : carry;
+    const int64_t base = (int64_t)blockIdx.x * kStartsChunk;
+    int v[kStartsEach], own = 0;
+#pragma unroll
+    for (int k = 0; k < kStartsEach; k++) {
+        const int64_t i = base + (int64_t)threadIdx.x * kStartsEach + k;
+        v[k] = i < n_roots ? counts[i] : 0;
+        bad |= v[k] < 0;
+        v[k] = max(v[k], 0);
+        own += v[k];
+    }
+    int pre = own;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const int x = __shfl_up(pre, o, kWave);
+        if (lane >= o) pre += x;
+    }
+    if (lane == kWave - 1) sums[wave] = pre;
+    bad = block_sum(bad, red);  // (its barriers order the waves' sums too)
+    int at = carry + pre - own, all = 0;
+    for (int w = 0; w < 16; w++) {
+        at += w < wave ? sums[w] : 0;
+        all += sums[w];
+    }
+#pragma unroll
+    for (int k = 0; k < kStartsEach; k++) {
+        const int64_t i = base + (int64_t)threadIdx.x * kStartsEach + k;
+        if (i < n_roots) block_indptr[i] = at;
+        at += v[k];
+    }
+    if ((int)blockIdx.x == n_chunks - 1 && threadIdx.x == 0) {
+        block_indptr[n_roots] = carry + all;
+        *n_edges_out = bad ? -1 : carry + all;
     }
 }
 
@@ -378,9 +412,16 @@ YITU_API int yitu_tsample_reset(int32_t *cursor, const int32_t *indptr, int64_t 
     return 0;
 }
 
+namespace {
+size_t root_array_bytes(int64_t n_roots) {
+    return align_up(sizeof(int32_t) * (size_t)(std::max<int64_t>(n_roots, 1) + 1), 256);
+}
+}  // namespace
+
+// counts, the block's indptr (yitu_tsample_recent), the chunks' sums
 YITU_API size_t yitu_tsample_workspace_bytes(int64_t n_roots) {
-    const int64_t n = std::max<int64_t>(n_roots, 1);
-    return 2 * align_up(sizeof(int32_t) * (size_t)(n + 1), 256);
+    return 2 * root_array_bytes(n_roots) +
+           align_up(sizeof(ChunkSum) * (size_t)ceil_div(n_roots, kStartsChunk), 256);
 }
 
 YITU_API int yitu_tsample_recent_block(int32_t *block_indptr, int32_t *row, int32_t *col,
@@ -413,7 +454,14 @@ YITU_API int yitu_tsample_recent_block(int32_t *block_indptr, int32_t *row, int3
                                                      n_roots, (int32_t)n_nodes, fan);
         YITU_LAUNCH_CHECK();
     }
-    ts_starts_kernel<<<1, 1024, 0, stream>>>(block_indptr, n_edges_out, counts, n_roots);
+    const int n_chunks = (int)std::max<int64_t>(1, ceil_div(n_roots, kStartsChunk));
+    ChunkSum *chunks = reinterpret_cast<ChunkSum *>(static_cast<char *>(workspace) +
+                                                    2 * root_array_bytes(n_roots));
+    if (n_chunks > 1) {
+        ts_chunk_sums_kernel<<<n_chunks, 1024, 0, stream>>>(chunks, counts, n_roots);
+        YITU_LAUNCH_CHECK();
+    }
+    ts_starts_kernel<<<n_chunks, 1024, 0, stream>>>(block_indptr, n_edges_out, counts, chunks, n_roots);
     YITU_LAUNCH_CHECK();
     if (n_roots == 0) return 0;
     const FillArgs a{row, col, eid_out, nodes_out, ts_out, dts_out, block_indptr, cursor, indptr,
@@ -433,9 +481,8 @@ YITU_API int yitu_tsample_recent(int32_t *row, int32_t *col, int32_t *eid_out, f
     YITU_REQUIRE(n_roots >= 0 && workspace &&
                      workspace_bytes >= yitu_tsample_workspace_bytes(n_roots),
                  "workspace too small: need %zu bytes", yitu_tsample_workspace_bytes(n_roots));
-    int32_t *block_indptr = reinterpret_cast<int32_t *>(
-        static_cast<char *>(workspace) +
-        align_up(sizeof(int32_t) * (size_t)(std::max<int64_t>(n_roots, 1) + 1), 256));
+    int32_t *block_indptr = reinterpret_cast<int32_t *>(static_cast<char *>(workspace) +
+                                                        root_array_bytes(n_roots));
     return yitu_tsample_recent_block(block_indptr, row, col, eid_out, ts_out, dts_out, nodes_out,
                                      n_edges_out, cursor, indptr, indices, eid, ts, n_nodes, roots,
                                      root_ts, n_roots, fan, prop_time, workspace, workspace_bytes,
