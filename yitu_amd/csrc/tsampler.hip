@@ -37,17 +37,36 @@ __global__ __launch_bounds__(kBlock) void ts_reset_kernel(int32_t *__restrict__ 
     if (i < n_nodes) cursor[i] = indptr[i];
 }
 
-// A wave per root in each of these: two thousand roots one per thread were 32 waves, each
-// walking a chain of dependent loads (count, scan and fill of 2,048 roots x 20: 6 + 8 + 17 us, now
-// 4 + 5 + 4).
-//
-// The last edge with ts <= thr by a search of 64 probes a step: lane l looks at the last edge of
-// the l-th of 64 equal parts.
+// G lanes per root in each of these: two thousand roots one per thread were 32 waves, each
+// walking a chain of dependent loads (count, scan and fill of 2,048 roots x 20: 6 + 8 + 17 us,
+// now 2.6 + 3.6 + 3.1). As many lanes as a root has neighbours to look at (rounded up to a power
+// of two): a whole wave for each of 131,072 roots x 5 took 21 us to count and 29 to fill, with
+// eight lanes 4.7 and 8.6.
+template <int G>
+struct RootLanes {
+    int64_t root;
+    int lane;
+    __device__ __forceinline__ RootLanes()
+        : root(((int64_t)blockIdx.x * kBlock + threadIdx.x) / G), lane(lane_id() % G) {}
+    // of this root's lanes (which are active together)
+    __device__ __forceinline__ unsigned long long ballot(bool p) const {
+        const unsigned long long all = __ballot(p);
+        return G == 64 ? all : (all >> (lane_id() / G * G)) & ((1ull << (G & 63)) - 1);
+    }
+};
+
+// The last edge with ts <= thr by a search of G probes a step: lane l looks at the last edge of
+// the l-th of G equal parts. A cursor that is there already is not written: the roots of a batch
+// that share a busy node would wait for each other's atomics (131,072 roots of a Zipf stream:
+// 734 us; 157 the first time and 20 once the cursors are there; a value read early is at most
+// too small, and the maximum decides).
+template <int G>
 __global__ __launch_bounds__(kBlock) void ts_advance_kernel(
     int32_t *__restrict__ cursor, const int32_t *__restrict__ indptr, const float *__restrict__ ts,
     const int32_t *__restrict__ roots, const float *__restrict__ root_ts, int64_t n_roots,
     int32_t n_nodes) {
-    const int64_t i = (int64_t)blockIdx.x * kWavesPerBlock + wave_id();
+    const RootLanes<G> me;
+    const int64_t i = me.root;
     if (i >= n_roots) return;
     const int32_t n = roots[i];
     if (n < 0 || n >= n_nodes) return;  // (the count below reports it)
@@ -55,10 +74,10 @@ __global__ __launch_bounds__(kBlock) void ts_advance_kernel(
     const int32_t first = indptr[n];
     int32_t lo = first, hi = indptr[n + 1];  // the first edge with ts > thr is in [lo, hi]
     while (lo < hi) {
-        const int32_t step = (hi - lo + kWave - 1) / kWave;
-        const int64_t at = (int64_t)lo + (int64_t)(lane_id() + 1) * step - 1;
-        const unsigned long long beyond = __ballot(at >= hi || !(ts[at] <= thr));
-        if (!beyond) {  // (64 parts cover [lo, hi): the last lane's probe was not beyond it)
+        const int32_t step = (hi - lo + G - 1) / G;
+        const int64_t at = (int64_t)lo + (int64_t)(me.lane + 1) * step - 1;
+        const unsigned long long beyond = me.ballot(at >= hi || !(ts[at] <= thr));
+        if (!beyond) {  // (G parts cover [lo, hi): the last lane's probe was not beyond it)
             lo = hi;
             break;
         }
@@ -67,16 +86,20 @@ __global__ __launch_bounds__(kBlock) void ts_advance_kernel(
         lo += part * step;
         hi = (int32_t)min((int64_t)hi, end);
     }
-    if (lane_id() == 0 && lo - 1 >= first) atomicMax(&cursor[n], lo - 1);
+    if (me.lane == 0 && lo - 1 >= first &&
+        __hip_atomic_load(&cursor[n], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < lo - 1)
+        atomicMax(&cursor[n], lo - 1);
 }
 
 // Edges a root keeps, of the `fan` before its cursor; -1 for a root that is no node.
+template <int G>
 __global__ __launch_bounds__(kBlock) void ts_count_kernel(
     int32_t *__restrict__ counts, const int32_t *__restrict__ cursor,
     const int32_t *__restrict__ indptr, const float *__restrict__ ts,
     const int32_t *__restrict__ roots, const float *__restrict__ root_ts, int64_t n_roots,
     int32_t n_nodes, int fan) {
-    const int64_t i = (int64_t)blockIdx.x * kWavesPerBlock + wave_id();
+    const RootLanes<G> me;
+    const int64_t i = me.root;
     if (i >= n_roots) return;
     const int32_t n = roots[i];
     int32_t cnt = -1;
@@ -84,17 +107,18 @@ __global__ __launch_bounds__(kBlock) void ts_count_kernel(
         const float thr = query_threshold(root_ts[i]);
         const int32_t e = cursor[n], stop = max(indptr[n], e - fan);
         cnt = 0;
-        for (int32_t k = e; k > stop; k -= kWave) {
-            const int32_t mine = k - lane_id();
-            cnt += __popcll(__ballot(mine > stop && ts[max(mine, stop)] < thr));
+        for (int32_t k = e; k > stop; k -= G) {
+            const int32_t mine = k - me.lane;
+            cnt += __popcll(me.ballot(mine > stop && ts[max(mine, stop)] < thr));
         }
     }
-    if (lane_id() == 0) counts[i] = cnt;
+    if (me.lane == 0) counts[i] = cnt;
 }
 
 // block_indptr = exclusive prefix sums of the counts, a workgroup per chunk of 16,384; *n_edges_out
-// = their total, or -1 with a root that is no node. Up to one chunk is one launch (2,048 roots:
-// 5 us); beyond, the chunks' sums are made first and every workgroup adds up those before it.
+// = their total, or -1 with a root that is no node. Up to one chunk is one launch (2,048 roots
+// 3.6 us, 16,384 5.2); beyond, the chunks' sums are made first and every workgroup adds up those
+// before it (131,072 roots 4.2 + 6.9 us).
 constexpr int kStartsEach = 16, kStartsChunk = 1024 * kStartsEach;
 struct ChunkSum {
     int32_t sum, bad;
@@ -145,11 +169,19 @@ __global__ __launch_bounds__(1024) void ts_starts_kernel(int32_t *__restrict__ b
         carry = block_sum(carry, red);
     }
     const int64_t base = (int64_t)blockIdx.x * kStartsChunk;
+    const int64_t mine = base + (int64_t)threadIdx.x * kStartsEach;
+    const bool whole = mine + kStartsEach <= n_roots;
     int v[kStartsEach], own = 0;
+    if (whole) {  // (counts is the workspace's first array, 256-byte aligned)
+#pragma unroll
+        for (int k = 0; k < kStartsEach; k += 4)
+            *reinterpret_cast<int4 *>(v + k) = *reinterpret_cast<const int4 *>(counts + mine + k);
+    } else {
+#pragma unroll
+        for (int k = 0; k < kStartsEach; k++) v[k] = mine + k < n_roots ? counts[mine + k] : 0;
+    }
 #pragma unroll
     for (int k = 0; k < kStartsEach; k++) {
-        const int64_t i = base + (int64_t)threadIdx.x * kStartsEach + k;
-        v[k] = i < n_roots ? counts[i] : 0;
         bad |= v[k] < 0;
         v[k] = max(v[k], 0);
         own += v[k];
@@ -169,9 +201,18 @@ __global__ __launch_bounds__(1024) void ts_starts_kernel(int32_t *__restrict__ b
     }
 #pragma unroll
     for (int k = 0; k < kStartsEach; k++) {
-        const int64_t i = base + (int64_t)threadIdx.x * kStartsEach + k;
-        if (i < n_roots) block_indptr[i] = at;
-        at += v[k];
+        const int next = at + v[k];
+        v[k] = at;
+        at = next;
+    }
+    if (whole && reinterpret_cast<uintptr_t>(block_indptr) % 16 == 0) {
+#pragma unroll
+        for (int k = 0; k < kStartsEach; k += 4)
+            *reinterpret_cast<int4 *>(block_indptr + mine + k) = *reinterpret_cast<const int4 *>(v + k);
+    } else {
+#pragma unroll
+        for (int k = 0; k < kStartsEach; k++)
+            if (mine + k < n_roots) block_indptr[mine + k] = v[k];
     }
     if ((int)blockIdx.x == n_chunks - 1 && threadIdx.x == 0) {
         block_indptr[n_roots] = carry + all;
@@ -189,10 +230,12 @@ struct FillArgs {
     int fan, prop_time;
 };
 
+template <int G>
 __global__ __launch_bounds__(kBlock) void ts_fill_kernel(FillArgs a) {
-    const int64_t i = (int64_t)blockIdx.x * kWavesPerBlock + wave_id();
+    const RootLanes<G> me;
+    const int64_t i = me.root;
     if (i >= a.n_roots) return;
-    const int lane = lane_id();
+    const int lane = me.lane;
     const int32_t n = a.roots[i];
     const float t = a.root_ts[i];
     if (lane == 0) {
@@ -204,11 +247,11 @@ __global__ __launch_bounds__(kBlock) void ts_fill_kernel(FillArgs a) {
     const float thr = query_threshold(t);
     const int32_t e = a.cursor[n], stop = max(a.indptr[n], e - a.fan);
     int64_t base = a.offsets[i];
-    for (int32_t k = e; k > stop; k -= kWave) {
+    for (int32_t k = e; k > stop; k -= G) {
         const int32_t mine = k - lane;
         const float when = a.ts[max(mine, stop)];
         const bool keep = mine > stop && when < thr;
-        const unsigned long long kept = __ballot(keep);
+        const unsigned long long kept = me.ballot(keep);
         if (keep) {
             const int64_t w = base + __popcll(kept & ((1ull << lane) - 1));
             a.row[w] = (int32_t)i;
@@ -413,6 +456,18 @@ YITU_API int yitu_tsample_reset(int32_t *cursor, const int32_t *indptr, int64_t 
 }
 
 namespace {
+// Roots up to which the search takes a wave each (the chip holds 8,192 at once).
+constexpr int64_t kWaveRoots = 16384;
+
+// f(lanes per root): the power of two from 8 to 64 that covers `neighbours`.
+template <typename F>
+void with_lanes(int neighbours, F f) {
+    if (neighbours <= 8) f(std::integral_constant<int, 8>());
+    else if (neighbours <= 16) f(std::integral_constant<int, 16>());
+    else if (neighbours <= 32) f(std::integral_constant<int, 32>());
+    else f(std::integral_constant<int, 64>());
+}
+
 size_t root_array_bytes(int64_t n_roots) {
     return align_up(sizeof(int32_t) * (size_t)(std::max<int64_t>(n_roots, 1) + 1), 256);
 }
@@ -446,12 +501,18 @@ YITU_API int yitu_tsample_recent_block(int32_t *block_indptr, int32_t *row, int3
         YITU_REQUIRE(row && col && eid_out && ts_out && dts_out && nodes_out && cursor && indptr &&
                          roots && root_ts,
                      "null pointer");
-        const int grid = (int)ceil_div(n_roots, kWavesPerBlock);
-        ts_advance_kernel<<<grid, kBlock, 0, stream>>>(cursor, indptr, ts, roots, root_ts, n_roots,
-                                                       (int32_t)n_nodes);
+        // a whole wave searches while the chip has room for one per root
+        with_lanes(n_roots <= kWaveRoots ? kWave : 8, [&](auto lanes) {
+            constexpr int G = decltype(lanes)::value;
+            ts_advance_kernel<G><<<(int)ceil_div(n_roots, kBlock / G), kBlock, 0, stream>>>(
+                cursor, indptr, ts, roots, root_ts, n_roots, (int32_t)n_nodes);
+        });
         YITU_LAUNCH_CHECK();
-        ts_count_kernel<<<grid, kBlock, 0, stream>>>(counts, cursor, indptr, ts, roots, root_ts,
-                                                     n_roots, (int32_t)n_nodes, fan);
+        with_lanes(fan, [&](auto lanes) {
+            constexpr int G = decltype(lanes)::value;
+            ts_count_kernel<G><<<(int)ceil_div(n_roots, kBlock / G), kBlock, 0, stream>>>(
+                counts, cursor, indptr, ts, roots, root_ts, n_roots, (int32_t)n_nodes, fan);
+        });
         YITU_LAUNCH_CHECK();
     }
     const int n_chunks = (int)std::max<int64_t>(1, ceil_div(n_roots, kStartsChunk));
@@ -466,7 +527,10 @@ YITU_API int yitu_tsample_recent_block(int32_t *block_indptr, int32_t *row, int3
     if (n_roots == 0) return 0;
     const FillArgs a{row, col, eid_out, nodes_out, ts_out, dts_out, block_indptr, cursor, indptr,
                      indices, eid, roots, ts, root_ts, n_roots, (int32_t)n_nodes, fan, prop_time};
-    ts_fill_kernel<<<(int)ceil_div(n_roots, kWavesPerBlock), kBlock, 0, stream>>>(a);
+    with_lanes(fan, [&](auto lanes) {
+        constexpr int G = decltype(lanes)::value;
+        ts_fill_kernel<G><<<(int)ceil_div(n_roots, kBlock / G), kBlock, 0, stream>>>(a);
+    });
     YITU_LAUNCH_CHECK();
     return 0;
 }
