@@ -204,6 +204,47 @@ def test_outputs_of_a_batched_model_can_be_written_in_place(dev, which):
                 assert_close(b, a, rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("which", ["rgcn", "rgat"])
+@pytest.mark.parametrize("stitch", [False, True])
+def test_batched_model_in_training_mode(dev, which, stitch, monkeypatch):
+    """Dropout between the layers: with a mask that depends on the values alone the batched form
+    gives the outputs and gradients of one relation at a time, stitched or not."""
+    torch.manual_seed(3)
+    hgraph = cases.hetero_graph(device=dev)
+    kwargs = cases.hetero_kwargs(hgraph, device=dev, with_norms=which == "rgcn")
+    model = (models.RGCNModel(hgraph, 12, 16, 5) if which == "rgcn"
+             else models.RGATModel(hgraph, 12, 16, 8, n_heads=2)).to(dev)
+    flow = xgnn_h.Optimizer().lower(xgnn_h.Module2IR().transform(model, kwargs), kwargs)
+    if stitch:
+        flow = xgnn_h.Stitcher().transform(flow, kwargs)
+    batched = xgnn_h.batch.batch_rows(flow, kwargs, training=True)
+    assert cases.ops_of(batched)["dropout"] == 1  # one draw for all node types
+    drawn = []
+
+    def dropout(x, p, training):
+        assert p == 0.5 and training
+        drawn.append(x.size(0))
+        return x * (x > -0.05) / (1 - p)
+
+    monkeypatch.setattr(torch.nn.functional, "dropout", dropout)
+    results, weights = [], {}
+    for flag in (False, True):
+        executor = xgnn_h.Executor(group_linears=flag)
+        executor.train()
+        del drawn[:]
+        out = executor.run(flow, kwargs)
+        assert sum(drawn) == sum(cases.NTYPES.values()) and len(drawn) == (1 if flag else 3)
+        for k, v in out.items():
+            weights.setdefault(k, torch.randn_like(v))
+        results.append([out[k] for k in weights] + list(torch.autograd.grad(
+            [out[k] for k in weights], list(model.parameters()), list(weights.values()),
+            allow_unused=True)))
+    for a, b in zip(*results):
+        assert (a is None) == (b is None)
+        if a is not None:
+            assert_close(b, a, rtol=1e-4, atol=1e-4)
+
+
 def test_two_dropouts_of_the_same_rows_differ(dev):
     """F.dropout(h, .5) - F.dropout(h, .5): about half of the entries
     are not zero, whatever the batch."""

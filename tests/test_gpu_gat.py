@@ -7,7 +7,8 @@ import torch
 import oracle
 from helpers import (assert_close, powerlaw_graph, random_csr, scrambled_csr,
                      softmax_backward_abs_sums, spmm_abs_sums)
-from yitu_amd import graph_ext
+from yitu_amd import _lib, graph_ext
+from yitu_amd.data import graphgen
 from yitu_amd.xgnn_h import block as xblock
 from yitu_amd.xgnn_h import sparse
 
@@ -223,6 +224,36 @@ def test_gat_head_mean_backward_against_oracle(dev, h, f, with_attn):
     assert_close(gq, want_gq, abs_sum=abs_gq[0], what="grad_q " + what)
     assert_close(gk, want_gk, abs_sum=abs_gk, what="grad_k " + what)
     assert_close(gx, want_gx, abs_sum=abs_gx, what="grad_x " + what)
+
+
+@pytest.mark.parametrize("h,f", [(4, 64), (4, 32), (3, 20), (1, 16)])
+@pytest.mark.parametrize("long_rows", [False, True])
+def test_gat_rows_dealt_to_the_xcds(dev, h, f, long_rows):
+    """A graph in communities, whose rows the kernels walk eighth by eighth: short rows alone and
+    long rows among them, a row count that is no whole eighths."""
+    n = 20_011
+    src, dst = graphgen.planted_partition(-(-n // 256), 256, 8, 2, 3)
+    keep = (src < n) & (dst < n)
+    src, dst = src[keep], dst[keep]
+    if long_rows:
+        hubs = torch.arange(0, n, 50).repeat_interleave(150)
+        far = torch.randint(0, n, hubs.shape, generator=torch.Generator().manual_seed(1))
+        src, dst = torch.cat([src, far, hubs]), torch.cat([dst, hubs, far])
+    indptr, indices = graphgen.csr_from_edges(dst, src, n, n)
+    plan = _lib.row_plan(indptr.to(dev), indices.to(dev), n, graph_ext.COL_MASK)
+    raw = plan[256:280].view(torch.int32).tolist()
+    assert 5 * raw[4] > raw[5], "not a graph whose rows are dealt"
+    assert ((indptr[1:] - indptr[:-1]).max() >= 64) == long_rows
+    _run(dev, indptr, indices, n, n, h, f, seed=f)
+    if h != 3:
+        blk = xblock.Block([n, n], [indptr, indices]).to(dev)
+        g = torch.Generator().manual_seed(h)
+        leaves = [torch.randn(n, *s, generator=g).to(dev).requires_grad_() for s in ((h,), (h,), (h, f))]
+        w = torch.randn(n, f, generator=g).to(dev)
+        want = torch.autograd.grad(sparse.fused_gat(blk, *leaves).mean(dim=1), leaves, w)
+        got = torch.autograd.grad(sparse.fused_gat(blk, *leaves, head_mean=True), leaves, w)
+        for a, b in zip(got, want):
+            assert_close(a, b, atol=5e-4)
 
 
 @pytest.mark.parametrize("h,f", [(1, 20), (2, 24), (4, 32), (4, 8), (8, 12), (1, 256), (8, 64)])

@@ -33,6 +33,27 @@ def test_matches_scipy(dev, n_rows, n_cols, n_edges, seed):
     assert np.array_equal(indices.cpu().numpy(), want_idx)
 
 
+@pytest.mark.parametrize("n_rows,n_cols", [
+    (65_535, 65_536), (65_536, 65_536), (65_535, 65_537), (32_767, 131_072), (32_768, 131_072),
+    ((1 << 20) - 1, 4096), (1 << 20, 4096), (1, (1 << 31) - 2), (3, 1 << 30), (4_000_000, 5_000_000)])
+def test_ids_at_the_limit_of_32_bit_keys(dev, n_rows, n_cols):
+    """Row and column ids that fill a 32-bit key, and one bit more: corners, duplicates, and ids
+    outside the matrix (whose key is the last one)."""
+    rng = np.random.default_rng(n_rows)
+    rows = np.concatenate([rng.integers(0, n_rows, 3000), [0, n_rows - 1, 0, n_rows - 1, n_rows - 1]])
+    cols = np.concatenate([rng.integers(0, n_cols, 3000), [0, n_cols - 1, n_cols - 1, 0, n_cols - 1]])
+    order = rng.permutation(rows.size)
+    rows, cols = rows[order], cols[order]
+    put = lambda a: torch.from_numpy(a).to(dev)  # noqa: E731
+    indptr, indices = csr.coo_to_csr(put(rows), put(cols), n_rows, n_cols)
+    pairs = np.unique(np.stack([rows, cols]), axis=1)  # by row, then column
+    assert np.array_equal(indices.cpu().numpy(), pairs[1])
+    assert np.array_equal(np.diff(indptr.cpu().numpy()), np.bincount(pairs[0], minlength=n_rows))
+    for bad_row, bad_col in ((n_rows, 0), (0, n_cols), (-1, 0), (0, -1)):
+        with pytest.raises(RuntimeError, match="outside"):
+            csr.coo_to_csr(put(np.append(rows, bad_row)), put(np.append(cols, bad_col)), n_rows, n_cols)
+
+
 def test_power_law_graph_matches_the_host_build(dev):
     """2^18 nodes, 4 M draws with many duplicates: same bits as the torch build."""
     src, dst = graphgen.rmat(18, 4_000_000, 9, self_loops=True, device=dev)

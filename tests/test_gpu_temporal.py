@@ -169,6 +169,41 @@ def test_fused_layer_all_input_combinations(dev, dims):
         assert torch.equal(got, dict(layer.named_parameters())[name].grad), name
 
 
+@pytest.mark.parametrize("dims", [(33, 7, 100, 8, 256), (16, 12, 8, 2, 32), (30, 50, 0, 1, 24),
+                                  (0, 5, 10, 1, 24), (9, 3, 2, 1, 6)])
+def test_fused_layer_gradients_of_some_inputs_only(dev, dims):
+    """The backward makes the columns of the input gradients that are asked for: node features,
+    edge features, both or neither give the same numbers as all of them."""
+    dim_node, dim_edge, dim_time, num_head, dim_out = dims
+    torch.manual_seed(sum(dims))
+    counts = [0, 1, 33, 70, 3, 0, 8] + [5] * 20
+    n_dst, E = len(counts), sum(counts)
+    dt = np.random.default_rng(0).uniform(0, 1e4, E).astype(np.float32)
+    layer = TransfomerAttentionLayer(dim_node, dim_edge, dim_time, num_head, 0.0, 0.0, dim_out).to(dev)
+    h = torch.randn(n_dst + E, dim_node, device=dev) if dim_node else None
+    f = torch.randn(E, dim_edge, device=dev)
+    w = torch.randn(n_dst, dim_out, device=dev)
+
+    def grads(need_h, need_f):
+        leaves = {"h": h.clone().requires_grad_(need_h) if h is not None else None,
+                  "f": f.clone().requires_grad_(need_f)}
+        blk = TemporalBlock(np.repeat(np.arange(n_dst), counts), n_dst, dt, device=dev, **leaves)
+        named = list(layer.named_parameters()) + [
+            (k, t) for k, t in leaves.items() if t is not None and t.requires_grad]
+        made = torch.autograd.grad(layer(blk), [t for _, t in named], w, allow_unused=True)
+        return {k: t for (k, _), t in zip(named, made)}
+
+    want = grads(h is not None, True)
+    for need_h, need_f in ((False, True), (True, False), (False, False)):
+        got = grads(need_h and h is not None, need_f)
+        assert ("h" in got) == (need_h and h is not None) and ("f" in got) == need_f
+        for name, t in got.items():
+            assert (t is None) == (want[name] is None), name
+            if t is not None:
+                scale = 1e4 if name == "time_enc.w.weight" else 1.0  # sums of products with dt <= 10^4
+                assert_close(t, want[name], rtol=1e-4, atol=1e-4 * scale, what=name)
+
+
 def test_fused_layer_equals_the_composed_ops(dev, monkeypatch):
     """The same block through the fused node and through the composition of graph_ext ops
     that the layer used before (and still uses under dropout)."""
