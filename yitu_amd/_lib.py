@@ -177,9 +177,8 @@ def forget(*tensors):
 def state_of(tensors):
     """What changes when one of the tensors (which the caller keeps alive) is replaced, written
     by torch, or named to ``forget``: for copies kept beside what they were made from."""
-    if not _forgotten:
-        return [(id(t), t.data_ptr(), t._version) for t in tensors]
-    return [(id(t), t.data_ptr(), t._version, _forgotten.get(id(t), 0)) for t in tensors]
+    state = ops().tensor_state(tensors)
+    return (state, [_forgotten.get(id(t), 0) for t in tensors]) if _forgotten else state
 
 
 def max_degree(indptr):

@@ -277,6 +277,17 @@ void bind_graph_state(py::module_ &m) {
                               const py::object &built) {
         put_built(views, indptr, indices, n_src, 0, built, true);
     });
+    // identity, address and version of every tensor, as one comparable value
+    m.def("tensor_state", [](const TensorVec &ts) {
+        std::vector<uintptr_t> v;
+        v.reserve(3 * ts.size());
+        for (const Tensor &t : ts) {
+            v.push_back(reinterpret_cast<uintptr_t>(id(t)));
+            v.push_back(reinterpret_cast<uintptr_t>(t.const_data_ptr()));
+            v.push_back(t._version());
+        }
+        return py::bytes(reinterpret_cast<const char *>(v.data()), v.size() * sizeof(v[0]));
+    });
     m.def("impl_of", [](const Tensor &t) { return reinterpret_cast<uintptr_t>(id(t)); });
     m.def("drop", [](uintptr_t impl) { drop(reinterpret_cast<const void *>(impl)); });
 }
