@@ -10,7 +10,7 @@
 // 3.4 TB/s. Where a workgroup's rows lie in one range, the lookup is the workgroup's own, and from
 // kManyVecs 16-byte vectors on (1,024 workgroups of four each) a thread has kPerThread of them
 // under way: 491,520 rows of 256 floats divided 298 -> 156 us (6.4 TB/s), two such ranges added up
-// 430 -> 290 us; 7,262 rows of 32 floats in five ranges 2.5 us, where the division and the ReLU
+// 430 -> 290 us; 7,262 rows of 32 floats in five ranges 3.2 us, where the division and the ReLU
 // of each range were ten launches of 2.3.
 #include <hip/hip_runtime.h>
 

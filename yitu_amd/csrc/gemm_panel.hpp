@@ -10,8 +10,10 @@
 // tiled kernel, so a product keeps its bits when its row count moves it from one to the
 // other. Both areas hold every eight columns as four even ones, then four odd ones, so the operands
 // of four steps are one 16-byte LDS read of either side; rows of both areas are padded by 16 bytes
-// (an odd number of 16-byte pieces: conflict-free). The weight is the first MFMA operand: a
-// lane holds four consecutive columns of a row, and rows leave through the wave's LDS area as
+// (an odd number of 16-byte pieces: reads without bank conflicts; the writes of a chunk, two
+// of 8 bytes a lane, have some, 2 % of the kernel's cycles, and neighbouring lanes that swap
+// values to write 16 bytes each measured no better). The weight is the first MFMA operand: a lane
+// holds four consecutive columns of a row, and rows leave through the wave's LDS area as
 // 128-byte segments. A workgroup takes a run of consecutive tiles of the list of all
 // problems, one workgroup per CU.
 //
