@@ -728,3 +728,30 @@ def test_by_source_weights_made_on_another_stream_are_waited_for(dev):
     torch.cuda.synchronize()
     assert_close(first, want, atol=1e-3)
     assert torch.equal(first, second)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_by_source_weights_are_not_kept_from_a_recording(dev, dtype):
+    """A step recorded into a graph after one eager run: what it reads is its own, the eager steps
+    behind it see weights that are there, and every replay gives the eager result."""
+    indptr, indices = (t.to(dev) for t in powerlaw_graph(12, 50000, 19))
+    n = indptr.numel() - 1
+    values = torch.rand(indices.numel(), 1, device=dev)
+    x, gy = (torch.randn(n, 1, 24, device=dev).to(dtype) for _ in range(2))
+    view = graph_ext.transposed(indptr, indices, n)
+    _lib.row_plan(view.t_indptr, view.t_rows, n, graph_ext.COL_MASK)
+    if dtype == torch.float32:
+        graph_ext.spmm_backward(values, indptr, indices, x, gy, need_grad_a=False)  # seen once
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        got = graph_ext.spmm_backward(values, indptr, indices, x, gy, need_grad_a=False)[1]
+    for _ in range(3):  # before the first replay, and between the replays
+        want = graph_ext.spmm_backward(values, indptr, indices, x, gy, need_grad_a=False)[1]
+        copied = values.index_select(0, view.t_perm.long())
+        check = graph_ext.spmm_forward(copied, view.t_indptr, view.t_rows, gy)
+        assert_close(want, check, atol=1e-3)
+        got.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_close(got, want, atol=1e-3)

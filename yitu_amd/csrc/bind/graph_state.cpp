@@ -198,11 +198,19 @@ BySource by_source(const Tensor &indptr, const Tensor &indices, int64_t n_src) {
         py::module_::import("yitu_amd.graph_ext").attr("transposed")(indptr, indices, n_src));
 }
 
+// Whether the stream of a call on `t` records a graph.
+static bool recording(const Tensor &t) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    C10_HIP_CHECK(hipStreamIsCapturing(static_cast<hipStream_t>(stream_of(t)), &status));
+    return status != hipStreamCaptureStatusNone;
+}
+
 // Edge weights that take no gradient are usually constants of the graph (norms), passed
 // again every step. The backward reads them through the edge permutation, a scattered
 // 4-byte read per edge and head; the second time the same tensor (same version) comes by a
 // copy in by-source order is made and kept for as long as the tensor lives (`force`: at
-// once). Nothing is returned the first time.
+// once). Nothing is returned the first time. While the stream records a graph none is kept: its
+// memory would hold the weights only from the first replay on.
 OptTensor by_source_values(const Tensor &values, const Tensor &indptr, const Tensor &indices,
                            int64_t n_src, bool force) {
     bool known = false, seen = false;
@@ -223,6 +231,10 @@ OptTensor by_source_values(const Tensor &values, const Tensor &indptr, const Ten
     }
     if (copy) {
         wait_for(wait, values);
+        return copy;
+    }
+    if (recording(values)) {
+        if (force) copy = values.index_select(0, by_source(indptr, indices, n_src).t_perm);
         return copy;
     }
     if (!known) {
